@@ -124,8 +124,10 @@ int launch_linear_dual_row(hipStream_t st, int dev, const void *x1, int K1, cons
                            const void *W2, int64_t ldw2, const void *bias2, const void *residual, void *out, int N);
 int launch_gemv_group(hipStream_t st, GemvGroupArgs g);
 
-// f32 tile kernel for the same NT contraction, FMA in f32.
+// The same NT contraction in f32 (gemm_f32.hip), and the scratch (LinearArgs::splitk_ws) with which it cuts K over blocks
+// where M x N alone leaves CUs idle; with less it cuts K less.
 int launch_linear_f32(hipStream_t st, const LinearArgs &a);
+size_t linear_f32_workspace_bytes(int M, int N, int K);
 bool linear_mfma_fuses_norm(int M, int K, int ln_kind);
 
 // Gated pairs only (glu != 0): with a = min(gate, limit) and b = up cut off at +-limit,  a sigmoid(alpha a) (b + 1).

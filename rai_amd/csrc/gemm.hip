@@ -2,7 +2,7 @@
 //   (the bf16 MFMA tile kernel lives in gemm_mfma.hip)
 //   k_linear_bf16_skinny weight-streaming kernel for M <= 8 rows (decode): each wave
 //                        streams whole weight rows with 16-byte loads; HBM-bound.
-//   k_linear_f32         f32 NT tile kernel (FMA) with the same epilogue.
+//   (f32 Linears live in gemm_f32.hip)
 //   k_matmul_generic     any strides / batch broadcast, f32 or f64 accumulate.
 //
 // Reference semantics: rai-core/src/backend/candle.rs:327-443 (MatMul, stride rule),
@@ -411,103 +411,6 @@ __global__ void __launch_bounds__(256) k_gemv_bf16_reg_group(GemvGroupArgs g, in
   gemv_reg_rows<KC, R>(a, (gw - base) * rows_per_wave, rows_per_wave);
 }
 
-// ============================================================ f32 NT tile kernel
-// 64x64 tile, BK=16, 256 threads each computing a 4x4 micro-tile with FMA.
-__device__ __forceinline__ void linear_f32_tile(const LinearArgs &a, int tile_m, int tile_n) {
-  constexpr int BM = 64, BN = 64, BK = 16;
-  __shared__ float As[BK][BM + 4];
-  __shared__ float Bs[BK][BN + 4];
-  const int tid = threadIdx.x;
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const float *A = (const float *)a.A;
-  const float *W = (const float *)a.W;
-  const int tx = tid & 15, ty = tid >> 4;  // 16 x 16 threads
-  float acc[4][4] = {};
-  const int lrow = tid >> 2, lk = (tid & 3) * 4;  // each thread loads 4 consecutive k of one row
-  const bool vec_ok = (a.lda % 4 == 0) && (a.ldw % 4 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0);
-  for (int k0 = 0; k0 < a.K; k0 += BK) {
-    float va[4] = {0.f, 0.f, 0.f, 0.f}, vb[4] = {0.f, 0.f, 0.f, 0.f};
-    {
-      int m = m0 + lrow, k = k0 + lk;
-      if (m < a.M) {
-        const float *p = A + (int64_t)m * a.lda + k;
-        if (vec_ok && k + 3 < a.K) { float4 t = *reinterpret_cast<const float4 *>(p); va[0] = t.x; va[1] = t.y; va[2] = t.z; va[3] = t.w; }
-        else { for (int j = 0; j < 4; ++j) if (k + j < a.K) va[j] = p[j]; }
-      }
-      int n = n0 + lrow;
-      if (n < a.N) {
-        const float *p = W + (int64_t)n * a.ldw + k;
-        if (vec_ok && k + 3 < a.K) { float4 t = *reinterpret_cast<const float4 *>(p); vb[0] = t.x; vb[1] = t.y; vb[2] = t.z; vb[3] = t.w; }
-        else { for (int j = 0; j < 4; ++j) if (k + j < a.K) vb[j] = p[j]; }
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { As[lk + j][lrow] = va[j]; Bs[lk + j][lrow] = vb[j]; }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < BK; ++k) {
-      float4 av = *reinterpret_cast<const float4 *>(&As[k][ty * 4]);
-      float4 bv = *reinterpret_cast<const float4 *>(&Bs[k][tx * 4]);
-      float af[4] = {av.x, av.y, av.z, av.w}, bf[4] = {bv.x, bv.y, bv.z, bv.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(af[i], bf[j], acc[i][j]);
-    }
-  }
-  const float *bias = (const float *)a.bias;
-  const float *bias2 = (const float *)a.bias2;
-  const float *res = (const float *)a.residual;
-  if (a.glu) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int m = m0 + ty * 4 + i;
-      if (m >= a.M) continue;
-#pragma unroll
-      for (int j = 0; j < 4; j += 2) {
-        int n = n0 + tx * 4 + j;
-        if (n + 1 >= a.N) continue;
-        float g = acc[i][j] + (bias ? bias[n] : 0.f), u = acc[i][j + 1] + (bias ? bias[n + 1] : 0.f);
-        ((float *)a.out1)[(int64_t)m * a.ld1 + (n >> 1)] = a.act == kActClampedGlu ? glu_clamped(g, u, a.act_limit, a.act_alpha) : act_eval(a.act, g) * u;
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int m = m0 + ty * 4 + i;
-    if (m >= a.M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      int n = n0 + tx * 4 + j;
-      if (n >= a.N) continue;
-      float v = acc[i][j] + (bias ? bias[n] : 0.f) + (bias2 ? bias2[n] : 0.f);
-      if (a.act >= 0 && n >= a.act_from) v = act_eval(a.act, v);
-      if (a.f32_out) v *= a.out_scale;
-      if (res) v += res[(int64_t)m * a.ldr + n];
-      if (n < a.n_split) ((float *)a.out1)[(int64_t)m * a.ld1 + n] = v;
-      else ((float *)a.out2)[(int64_t)m * a.ld2 + (n - a.n_split)] = v;
-    }
-  }
-}
-
-__global__ void __launch_bounds__(256) k_linear_f32(LinearArgs a) {
-  const int tiles_m = (a.M + 63) / 64;
-  linear_f32_tile(a, blockIdx.x % tiles_m, blockIdx.x / tiles_m);
-}
-
-// The same tile over the rows of one expert (see MoePlan): blockIdx.x = column tile, blockIdx.y = row tile.
-__global__ void __launch_bounds__(256) k_linear_f32_grouped(LinearArgs a, int64_t w_stride, const int4 *tiles, const int *n_tiles) {
-  if ((int)blockIdx.y >= *n_tiles) return;
-  const int4 t = tiles[blockIdx.y];
-  a.A = (const float *)a.A + (int64_t)t.y * a.lda;
-  a.W = (const float *)a.W + (int64_t)t.x * w_stride;
-  a.out1 = (float *)a.out1 + (int64_t)t.y * a.ld1;
-  a.M = t.z;
-  linear_f32_tile(a, 0, blockIdx.x);
-}
-
 // ============================================================ generic strided batched matmul
 struct MatmulArgs {
   int64_t M, N, K;
@@ -801,22 +704,9 @@ template <typename T> static void launch_transpose_2d(hipStream_t st, T *dst, co
     hipLaunchKernelGGL(k_transpose_2d<T>, grid, dim3(256), 0, st, dst, src, K, N);
 }
 
-int launch_linear_f32(hipStream_t st, const LinearArgs &a) {
-  RAI_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0, RAI_ERR_BAD_SHAPE, "linear: empty problem");
-  RAI_REQUIRE(a.ln_kind < 0, RAI_ERR_UNSUPPORTED, "linear f32: no fused norm");
-  const int tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
-  hipLaunchKernelGGL(k_linear_f32, dim3(tiles), dim3(256), 0, st, a);
-  return launch_check("linear_f32");
-}
-
-int launch_linear_f32_grouped(hipStream_t st, const LinearArgs &a, int64_t w_stride, const MoePlan &plan) {
-  hipLaunchKernelGGL(k_linear_f32_grouped, dim3((a.N + 63) / 64, plan.cap_tiles), dim3(256), 0, st, a, w_stride, plan.tiles, plan.n_tiles);
-  return launch_check("linear_f32_grouped");
-}
-
-// Lends the device's scratch block to a tile GEMM that may split K.
-static int splitk_workspace(int dev, LinearArgs *la) {
-  const size_t want = (size_t)8 * la->M * la->N * sizeof(float);
+// Lends up to `want` bytes (at most 256 MB) of the device's scratch block to a tile GEMM that may split K.
+static int splitk_workspace(int dev, LinearArgs *la, size_t want) {
+  if (want == 0) return RAI_OK;
   const size_t cap = (size_t)256 << 20;
   const size_t bytes = want < cap ? want : cap;
   void *ws = nullptr;
@@ -824,6 +714,9 @@ static int splitk_workspace(int dev, LinearArgs *la) {
   la->splitk_ws = ws;
   la->splitk_ws_bytes = bytes;
   return RAI_OK;
+}
+static size_t splitk_bytes(int dtype, const LinearArgs &la) {
+  return dtype == RAI_F32 ? linear_f32_workspace_bytes(la.M, la.N, la.K) : (size_t)8 * la.M * la.N * sizeof(float);
 }
 
 }  // namespace rai
@@ -891,7 +784,7 @@ int rai_hip_matmul(int dev, const rai_hip_tensor *a, const rai_hip_tensor *b, co
       la.K = (int)K;
       la.n_split = (int)N;
       if (a->dtype == RAI_BF16 && la.M > 8 && la.K % 32 != 0) goto generic;
-      if (a->dtype == RAI_BF16 && la.M > 8) RAI_TRY(splitk_workspace(dev, &la));
+      if (a->dtype == RAI_F32 || la.M > 8) RAI_TRY(splitk_workspace(dev, &la, splitk_bytes(a->dtype, la)));
       return a->dtype == RAI_BF16 ? launch_linear_bf16(st, la) : launch_linear_f32(st, la);
     }
   }
@@ -1002,10 +895,9 @@ int rai_hip_linear(int dev, const rai_hip_tensor *x, const rai_hip_tensor *w, co
   la.act_from = 0;
   hipStream_t st = stream_of(dev);
   if (!st) return RAI_ERR_HIP;
-  if (x->dtype == RAI_BF16 && la.M > 8) {
+  if (x->dtype == RAI_BF16 && la.M > 8)
     RAI_REQUIRE(K % 32 == 0, RAI_ERR_UNSUPPORTED, "linear: bf16 with M > 8 needs K %% 32 == 0 (K=%lld)", (long long)K);
-    RAI_TRY(splitk_workspace(dev, &la));
-  }
+  if (x->dtype == RAI_F32 || la.M > 8) RAI_TRY(splitk_workspace(dev, &la, splitk_bytes(x->dtype, la)));
   return x->dtype == RAI_BF16 ? launch_linear_bf16(st, la) : launch_linear_f32(st, la);
 }
 
@@ -1084,7 +976,7 @@ int rai_hip_linear_packed(int dev, const rai_hip_tensor *x, const rai_hip_tensor
   if (!st) return RAI_ERR_HIP;
   if (la.M > 8) {
     RAI_REQUIRE(K % 32 == 0, RAI_ERR_UNSUPPORTED, "linear_packed: M > 8 needs K %% 32 == 0 (K=%lld)", (long long)K);
-    RAI_TRY(splitk_workspace(dev, &la));
+    RAI_TRY(splitk_workspace(dev, &la, splitk_bytes(RAI_BF16, la)));
   }
   return launch_linear_bf16(st, la);
 }

@@ -1,0 +1,60 @@
+"""f32 Linears at the edges of their kernels' tiles: rows around 4, 32 and 64, K around the 32-wide tiles and the cut over
+waves and blocks, odd N, rows that are not 16-byte aligned."""
+import numpy as np
+import pytest
+
+from tests.util import down, rand, up
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def R(hip):
+    from rai_amd import ops
+
+    return ops
+
+
+def bound(x, w, extra):
+    """Every sum of K products in f32, whatever its order, is within K roundings of the absolute sum; the epilogue's
+    few roundings and its activation are within eight of the result's own size and of what was added."""
+    return (x.shape[1] + 8) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T) + 2.0 ** -20 * extra
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 31, 33, 64, 65, 130])
+@pytest.mark.parametrize("k,n", [(4, 1), (36, 70), (33, 129), (252, 64), (260, 63), (1028, 258), (2560, 40)])
+def test_f32_linear_at_tile_edges(R, m, k, n):
+    g = np.random.Generator(np.random.PCG64(31 + m))
+    x, w = rand(g, (m, k), "f32"), rand(g, (n, k), "f32", 0.05)
+    b, r = rand(g, (n,), "f32"), rand(g, (m, n), "f32")
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    got = down(R.linear(up(x, "f32"), up(w, "f32"))).astype(np.float64)
+    assert np.all(np.abs(got - want) <= bound(x, w, 0.0))
+    z = want + b
+    full = 0.5 * z * (1 + np.tanh(np.sqrt(2 / np.pi) * (z + 0.044715 * z ** 3))) + r
+    got = down(R.linear(up(x, "f32"), up(w, "f32"), up(b, "f32"), "new_gelu", up(r, "f32"))).astype(np.float64)
+    assert np.all(np.abs(got - full) <= 2 * bound(x, w, np.abs(z) + np.abs(r) + 1))   # the activation's slope is below 1.13
+
+
+@pytest.mark.parametrize("m", [1, 3, 40])
+def test_f32_linear_of_unaligned_rows(R, m):
+    """A weight matrix and activations that start one element into their buffers, rows an odd number of elements apart."""
+    g = np.random.Generator(np.random.PCG64(77))
+    x, w = rand(g, (m, 133), "f32"), rand(g, (50, 131), "f32", 0.05)
+    got = down(R.linear(up(x, "f32").narrow(1, 1, 128), up(w, "f32").narrow(1, 3, 128))).astype(np.float64)
+    xs, ws = x[:, 1:129], w[:, 3:131]
+    assert np.all(np.abs(got - xs.astype(np.float64) @ ws.astype(np.float64).T) <= bound(xs, ws, 0.0))
+
+
+@pytest.mark.parametrize("m", [1, 20, 100])
+def test_f32_linear_keeps_small_and_infinite_values(R, m):
+    """Denormal products are kept, and infinities and NaNs reach only the outputs that depend on them (K is no multiple
+    of a tile, so zeros stand past its end)."""
+    x = np.full((m, 300), np.float32(2.0 ** -70))
+    w = np.full((70, 300), np.float32(2.0 ** -65))
+    assert np.all(down(R.linear(up(x, "f32"), up(w, "f32"))) == np.float32(300 * 2.0 ** -135))
+    x = np.ones((m, 300), np.float32)
+    w = np.ones((70, 300), np.float32)
+    w[7, 299], w[9, 0] = np.inf, np.nan
+    got = down(R.linear(up(x, "f32"), up(w, "f32")))
+    assert np.all(np.isinf(got[:, 7])) and np.all(np.isnan(got[:, 9])) and np.all(np.delete(got, [7, 9], 1) == 300)
