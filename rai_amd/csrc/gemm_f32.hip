@@ -1,5 +1,6 @@
 // f32 Linears on the f32 matrix instructions (every product and sum in f32).
 //   k_linear_f32_tile    tiles of 64 x 64 or 32 x 128 outputs, operands through LDS, K optionally cut over blocks
+//   k_linear_f32_rows    up to four rows (decoding)
 //   k_linear_f32_sum     adds the partial products of such a cut and applies the epilogue
 //   k_linear_f32_grouped the tile form over the rows of one expert after another
 //
@@ -234,6 +235,82 @@ __global__ void __launch_bounds__(256) k_linear_f32_grouped(LinearArgs a, int64_
   linear_f32_tile<64, 64, VEC>(a, 0, blockIdx.x * 64, 0, a.K, lds, [&](int m, int n, f32x4 v) { f32_finish4(a, m, n, v); });
 }
 
+// ------------------------------------------------------------------ few rows
+// M <= 4 (decoding): bound by the weight matrix's way from HBM.  A block owns two rows of W, a quarter of K to each of its
+// four waves; a wave reads 1 KB of a row with one instruction and multiplies it with the same piece of the M rows of A,
+// which come from L2 and stay in registers.  Few bytes per wave and many small waves in flight do best: 27 registers at
+// M = 1, eight waves a SIMD.  Measured with weights that no cache holds (us; 1 x 2560 x 32768, 1 x 12800 x 2560, 1 x 2560 x
+// 2560): 48.7, 23.2, 7.0 (6.9, 5.6 and 3.7 TB/s), against 57, 23, 8.2 with four pieces of a row requested at a time, 50, 34,
+// 9.1 without the cut of K, and 220, 769, 160 with tiles of 64 x 64 over unsplit K.  Eight rows take 36 us at 2560 x 10240,
+// where the tile form takes 29; four take 26.
+template <int M>
+__global__ void __launch_bounds__(256) k_linear_f32_rows(LinearArgs a) {
+  constexpr int R = 2, U = 2, KW = 4;
+  __shared__ float red[KW][R * M];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * R;
+  const int chunks = (a.K + 255) / 256, each = (chunks + KW - 1) / KW;
+  const int k_end = min((wave + 1) * each * 256, a.K);
+  const float *A = (const float *)a.A, *w[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) w[i] = (const float *)a.W + (int64_t)min(n0 + i, a.N - 1) * a.ldw;
+  float acc[R][M];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[i][m] = 0.f;
+  for (int k0 = wave * each * 256 + 4 * lane; k0 < k_end; k0 += 256 * U) {
+    f32x4 wv[U][R], xv[U][M];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + 256 * u < k_end ? k0 + 256 * u : k0;   // past the end: read again, not added
+#pragma unroll
+      for (int m = 0; m < M; ++m) xv[u][m] = *reinterpret_cast<const f32x4 *>(A + (int64_t)min(m, a.M - 1) * a.lda + k);
+#pragma unroll
+      for (int i = 0; i < R; ++i) wv[u][i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(w[i] + k));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k0 + 256 * u < k_end) {
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+          for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][m] = fmaf(wv[u][i][e], xv[u][m][e], acc[i][m]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[i][m] = wave_sum(acc[i][m]);
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int m = 0; m < M; ++m) red[wave][i * M + m] = acc[i][m];
+  }
+  __syncthreads();
+  if (threadIdx.x >= a.M) return;   // thread m finishes row m
+  const int m = threadIdx.x;
+  float v[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    v[i] = red[0][i * M + m];
+#pragma unroll
+    for (int j = 1; j < KW; ++j) v[i] += red[j][i * M + m];
+    if (n0 + i < a.N) v[i] += f32_bias(a, n0 + i);
+  }
+  if (a.glu) {
+    if (n0 + 1 < a.N) ((float *)a.out1)[(int64_t)m * a.ld1 + (n0 >> 1)] = f32_gated(a, v[0], v[1]);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    if (n0 + i < a.N) f32_finish(a, m, n0 + i, v[i]);
+}
+
 // ------------------------------------------------------------------ launchers
 static bool rows_aligned(const LinearArgs &a) {
   return a.K % 4 == 0 && a.lda % 4 == 0 && a.ldw % 4 == 0 && (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.W % 16 == 0;
@@ -253,6 +330,12 @@ static int launch_tile(hipStream_t st, const LinearArgs &a, int splits, int k_st
   return launch_check("linear_f32_tile");
 }
 
+constexpr int kFewRows = 4;
+template <int M> static int launch_rows(hipStream_t st, const LinearArgs &a) {
+  hipLaunchKernelGGL((k_linear_f32_rows<M>), dim3((a.N + 1) / 2), dim3(256), 0, st, a);
+  return launch_check("linear_f32_rows");
+}
+
 // How many pieces of K to compute side by side, by the time the tiles and the summing pass would take: a tile of full K
 // is 0.017 us of a busy CU's time per k, a CU needs three or four blocks to be busy, the sum is a launch and a trip of
 // the partial products to memory and back.
@@ -270,7 +353,7 @@ static int f32_splits(int M, int N, int K) {
 }
 
 size_t linear_f32_workspace_bytes(int M, int N, int K) {
-  const int s = f32_splits(M, N, K);
+  const int s = M <= kFewRows && K % 4 == 0 ? 1 : f32_splits(M, N, K);
   return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
 
@@ -278,6 +361,7 @@ int launch_linear_f32(hipStream_t st, const LinearArgs &a) {
   RAI_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0, RAI_ERR_BAD_SHAPE, "linear: empty problem");
   RAI_REQUIRE(a.ln_kind < 0, RAI_ERR_UNSUPPORTED, "linear f32: no fused norm");
   const bool vec = rows_aligned(a);
+  if (vec && a.M <= kFewRows) return a.M == 1 ? launch_rows<1>(st, a) : a.M == 2 ? launch_rows<2>(st, a) : launch_rows<4>(st, a);
   int splits = f32_splits(a.M, a.N, a.K);
   const size_t plane = (size_t)a.M * a.N * sizeof(float);
   if ((size_t)splits * plane > a.splitk_ws_bytes) splits = (int)(a.splitk_ws_bytes / plane);   // what the lent scratch holds
