@@ -130,6 +130,19 @@ int launch_linear_f32(hipStream_t st, const LinearArgs &a);
 size_t linear_f32_workspace_bytes(int M, int N, int K);
 bool linear_mfma_fuses_norm(int M, int K, int ln_kind);
 
+// out[z] = A[z] B[z] (rai_hip_matmul), out contiguous.
+struct MatmulArgs {
+  int64_t M, N, K;
+  int64_t a_rs, a_cs, b_rs, b_cs;  // element strides of the last two dims
+  int batch_rank;
+  int64_t batch_shape[RAI_HIP_MAX_RANK];
+  int64_t a_bs[RAI_HIP_MAX_RANK], b_bs[RAI_HIP_MAX_RANK];
+};
+// The MFMA form (matmul_mfma.hip) and what it takes: f32, bf16 or f16, each operand with a unit stride on one of its last
+// two axes.
+bool matmul_mfma_serves(int dtype, const MatmulArgs &g, int64_t batch);
+int launch_matmul_mfma(hipStream_t st, int dtype, void *out, const void *A, const void *B, const MatmulArgs &g, int64_t batch);
+
 // Gated pairs only (glu != 0): with a = min(gate, limit) and b = up cut off at +-limit,  a sigmoid(alpha a) (b + 1).
 constexpr int kActClampedGlu = RAI_UN_COUNT_;
 __device__ __forceinline__ float glu_clamped(float g, float u, float limit, float alpha) {

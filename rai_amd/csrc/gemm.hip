@@ -412,14 +412,6 @@ __global__ void __launch_bounds__(256) k_gemv_bf16_reg_group(GemvGroupArgs g, in
 }
 
 // ============================================================ generic strided batched matmul
-struct MatmulArgs {
-  int64_t M, N, K;
-  int64_t a_rs, a_cs, b_rs, b_cs;  // element strides of the last two dims
-  int batch_rank;
-  int64_t batch_shape[RAI_HIP_MAX_RANK];
-  int64_t a_bs[RAI_HIP_MAX_RANK], b_bs[RAI_HIP_MAX_RANK];
-};
-
 template <typename T>
 __global__ void __launch_bounds__(256) k_matmul_generic(T *out, const T *A, const T *B, MatmulArgs g) {
   typedef typename Scalar<T>::compute C;
@@ -830,6 +822,7 @@ generic:
     g.b_bs[i] = in ? b->stride[i] : 0;
   }
   RAI_REQUIRE(batch <= 65535, RAI_ERR_UNSUPPORTED, "matmul: batch %lld exceeds grid limit", (long long)batch);
+  if (matmul_mfma_serves(a->dtype, g, batch)) return launch_matmul_mfma(st, a->dtype, base_ptr(out), base_ptr(a), base_ptr(b), g, batch);
   dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), (unsigned)batch);
   RAI_DISPATCH_FLOAT(a->dtype, T,
                      hipLaunchKernelGGL((k_matmul_generic<T>), grid, dim3(256), 0, st, (T *)base_ptr(out),

@@ -1,0 +1,264 @@
+// Batched products of strided operands on the matrix instructions: f32, bf16 and f16, each operand contiguous along K or
+// along its other axis, any batch strides.  (Products whose right operand is one shared, K-contiguous matrix are Linears;
+// f64 and operands without a unit stride stay with k_matmul_generic.)
+//
+// Reference semantics: rai-core/src/backend/candle.rs:327-443 (MatMul, stride rule).
+#include "gemm.h"
+
+namespace rai {
+
+typedef __attribute__((ext_vector_type(16))) float mm_f32x16;
+typedef __attribute__((ext_vector_type(4))) float mm_f32x4;
+typedef __attribute__((ext_vector_type(8))) __bf16 mm_bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 mm_f16x8;
+typedef __attribute__((ext_vector_type(4))) uint32_t mm_chunk;   // 16 bytes of an operand
+
+// acc += a b over the chunk's four (f32) or eight consecutive k of each lane half: 32 x 32 outputs.
+template <typename T> __device__ __forceinline__ mm_f32x16 mm_mfma(mm_chunk a, mm_chunk b, mm_f32x16 acc);
+template <> __device__ __forceinline__ mm_f32x16 mm_mfma<float>(mm_chunk a, mm_chunk b, mm_f32x16 acc) {
+  const mm_f32x4 x = __builtin_bit_cast(mm_f32x4, a), y = __builtin_bit_cast(mm_f32x4, b);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y[s], acc, 0, 0, 0);
+  return acc;
+}
+template <> __device__ __forceinline__ mm_f32x16 mm_mfma<bf16_raw>(mm_chunk a, mm_chunk b, mm_f32x16 acc) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mm_bf16x8, a), __builtin_bit_cast(mm_bf16x8, b), acc, 0, 0, 0);
+}
+template <> __device__ __forceinline__ mm_f32x16 mm_mfma<f16_raw>(mm_chunk a, mm_chunk b, mm_f32x16 acc) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mm_f16x8, a), __builtin_bit_cast(mm_f16x8, b), acc, 0, 0, 0);
+}
+
+// One operand's tile of ROWS outputs x KB bytes of K.  KC (contiguous along K): in LDS as rows of KB + 16 bytes.  Otherwise
+// as it lies, BK rows of ROWS elements + 16 bytes, and the fragments are put together on the way out: 16-bit elements
+// with the transposing LDS read (lane i of 16 receives element i % 4 of the 8 bytes that lanes 4j + i / 4, j = 0..3, point
+// at: with lane a pointing at row a / 4, columns 4 (a % 4), it receives column i of four rows), f32 one by one.
+// Memory is read in pieces of 16 bytes whatever their alignment.
+template <typename T, int ROWS, bool KC, int KB>
+struct MmOperand {
+  static constexpr int V = 16 / sizeof(T), BK = KB / sizeof(T), CPR = KC ? KB / 16 : ROWS / V, P = ROWS * KB / 16 / 256;
+  static constexpr int PITCH = (KC ? KB : ROWS * (int)sizeof(T)) + 16;
+  static constexpr int BYTES = (KC ? ROWS : BK) * PITCH;
+  const T *base;      // the tile's first output row (column), k = 0
+  int64_t stride;     // KC: between outputs; otherwise: between consecutive k
+  int valid, K;       // outputs that exist from the tile's first on; the length of K
+  mm_chunk reg[P];
+
+  // place of this thread's piece p: KC: (output, chunk of K); otherwise (k, chunk of outputs)
+  static __device__ __forceinline__ int row(int p) { return (threadIdx.x + 256 * p) / CPR; }
+  static __device__ __forceinline__ int col(int p) { return ((threadIdx.x + 256 * p) % CPR) * V; }
+
+  // The whole tile lies inside the operand (outputs past the end aside, which are read from the last one).
+  __device__ __forceinline__ bool whole(int k0) const { return k0 + BK <= K && (KC || valid >= ROWS); }
+  __device__ __forceinline__ void fetch(int k0) {
+    if (whole(k0)) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const T *at = KC ? base + (int64_t)min(row(p), valid - 1) * stride + k0 + col(p) : base + (int64_t)(k0 + row(p)) * stride + col(p);
+        __builtin_memcpy(&reg[p], at, 16);
+      }
+      return;
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {   // at the ends: zeros past K, the last output repeated
+      const int k = KC ? k0 + col(p) : k0 + row(p), o = KC ? min(row(p), valid - 1) : col(p);
+      const T *at = KC ? base + (int64_t)o * stride + k : base + (int64_t)k * stride + o;
+      if (k >= K) {
+        reg[p] = mm_chunk{0u, 0u, 0u, 0u};
+      } else if (KC ? k + V <= K : o + V <= valid) {
+        __builtin_memcpy(&reg[p], at, 16);
+      } else {
+        T v[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) v[j] = KC ? base[(int64_t)o * stride + min(k + j, K - 1)] : base[(int64_t)k * stride + min(o + j, valid - 1)];
+        if (KC) {
+#pragma unroll
+          for (int j = 0; j < V; ++j)
+            if (k + j >= K) v[j] = T{};
+        }
+        __builtin_memcpy(&reg[p], v, 16);
+      }
+    }
+  }
+  __device__ __forceinline__ void park(char *st) const {
+#pragma unroll
+    for (int p = 0; p < P; ++p) *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = reg[p];
+  }
+  // Outputs first .. first + 31, chunk pair kk of K: lane (r, h) gets chunk 2 kk + h of output first + r.
+  static __device__ __forceinline__ mm_chunk fragment(const char *st, int first, int kk) {
+    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+    if constexpr (KC) {
+      return *reinterpret_cast<const mm_chunk *>(st + (first + r) * PITCH + kk * 32 + h * 16);
+    } else if constexpr (sizeof(T) == 2) {
+      typedef __attribute__((ext_vector_type(4))) short s16x4;
+      typedef __attribute__((address_space(3))) s16x4 *tr_ptr;
+      const int i = lane & 15, o = first + 16 * ((lane >> 4) & 1) + 4 * (i & 3);
+      const char *at = st + (kk * 16 + h * 8 + (i >> 2)) * PITCH + o * 2;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)at);
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 4 * PITCH));
+      const __attribute__((ext_vector_type(8))) short f = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      return __builtin_bit_cast(mm_chunk, f);
+    } else {
+      mm_f32x4 f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[j] = *reinterpret_cast<const float *>(st + (kk * 8 + h * 4 + j) * PITCH + (first + r) * 4);
+      return __builtin_bit_cast(mm_chunk, f);
+    }
+  }
+};
+
+template <typename T> __device__ __forceinline__ void mm_store(T *dst, const float *src, int n) {   // up to V outputs of a row
+  constexpr int V = 16 / sizeof(T);
+  T v[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) Scalar<T>::store(&v[j], src[j]);
+  if (n >= V) {
+    __builtin_memcpy(dst, v, 16);
+  } else {
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+      if (j < n) dst[j] = v[j];
+  }
+}
+
+// Four waves as 2 x 2, each F x F accumulators of 32 x 32 (tiles of 64 F).  Two LDS stages of KB bytes of K, loaded into
+// registers a tile ahead, one barrier per tile, or (ONE: K fits) a single one; the finished tile goes through LDS so that
+// rows are written 16 bytes at a time.  Attention-sized products are bound by a block's chain of trips (operands, LDS,
+// MFMAs, LDS, rows out), so what counts is how many blocks share a CU; long ones by the L2.
+//   Measured (us; 64 x 64 tiles of multiply-adds on the vector units before): bf16 32 x 512 x 80 x 512 (scores) 11.2 (40.5),
+// 32 x 512 x 512 x 80 (values, [K, N]) 13.4 (94.8), 64 x 1024 x 1024 x 1024 200 to 300 (2900 to 3035), one row against 32 x
+// 777 x 128 10.4 (77.5), odd 18 x 410 x 141 x 349 10.8 (31.8); f32 32 x 512 x 80 x 512 24.4 (47.9).
+template <typename T, bool AKC, bool BKC, int F, int KB, bool ONE>
+__global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T *B, MatmulArgs g, int tiles_m, int tiles_n) {
+  constexpr int BT = 64 * F;
+  typedef MmOperand<T, BT, AKC, KB> OpA;
+  typedef MmOperand<T, BT, BKC, KB> OpB;
+  constexpr int STAGE = OpA::BYTES + OpB::BYTES, OP = BT + 4, PAIRS = KB / 32;
+  constexpr int LDS = (ONE ? 1 : 2) * STAGE > BT * OP * 4 ? (ONE ? 1 : 2) * STAGE : BT * OP * 4;
+  __shared__ __attribute__((aligned(16))) char lds[LDS];
+  // every XCD (blocks are dealt out to the eight of them in turn) walks a run of tiles of its own: the tiles of one batch
+  // entry then share its L2
+  const int total = gridDim.x, xcd = blockIdx.x & 7, q = total >> 3, rem = total & 7;
+  const int t = xcd * q + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  const int z = t / (tiles_m * tiles_n), in = t - z * tiles_m * tiles_n;
+  const int m0 = (in % tiles_m) * BT, n0 = (in / tiles_m) * BT;
+  int64_t aoff = 0, boff = 0;
+  for (int d = g.batch_rank - 1, rest = z; d >= 0; --d) {
+    const int n = (int)g.batch_shape[d], i = rest % n;
+    rest /= n;
+    aoff += i * g.a_bs[d];
+    boff += i * g.b_bs[d];
+  }
+  OpA a;
+  a.stride = AKC ? g.a_rs : g.a_cs;
+  a.base = A + aoff + (AKC ? (int64_t)m0 * g.a_rs : (int64_t)m0);
+  a.valid = (int)min<int64_t>(BT, g.M - m0);
+  a.K = (int)g.K;
+  OpB b;
+  b.stride = BKC ? g.b_cs : g.b_rs;
+  b.base = B + boff + (BKC ? (int64_t)n0 * g.b_cs : (int64_t)n0);
+  b.valid = (int)min<int64_t>(BT, g.N - n0);
+  b.K = (int)g.K;
+
+  const int wave = threadIdx.x >> 6, wm = (wave >> 1) * 32 * F, wn = (wave & 1) * 32 * F;
+  mm_f32x16 acc[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  const int steps = ONE ? 1 : ((int)g.K + OpA::BK - 1) / OpA::BK;
+  a.fetch(0);
+  b.fetch(0);
+  a.park(lds);
+  b.park(lds + OpA::BYTES);
+  if (steps > 1) { a.fetch(OpA::BK); b.fetch(OpA::BK); }
+  __syncthreads();
+  for (int s = 0; s < steps; ++s) {
+    const char *sa = lds + (s & 1) * STAGE, *sb = sa + OpA::BYTES;
+    mm_chunk fa[2][F], fb[2][F];
+    auto read = [&](int kk) {
+#pragma unroll
+      for (int i = 0; i < F; ++i) fa[kk & 1][i] = OpA::fragment(sa, wm + 32 * i, kk);
+#pragma unroll
+      for (int j = 0; j < F; ++j) fb[kk & 1][j] = OpB::fragment(sb, wn + 32 * j, kk);
+    };
+    read(0);
+#pragma unroll
+    for (int kk = 0; kk < PAIRS; ++kk) {
+      if (ONE && kk * (32 / (int)sizeof(T)) >= (int)g.K) break;
+      if (kk + 1 < PAIRS) read(kk + 1);
+      if (kk == 2 && s + 1 < steps) {   // to the stage that every wave left before the last barrier
+        char *next = lds + ((s + 1) & 1) * STAGE;
+        a.park(next);
+        b.park(next + OpA::BYTES);
+        if (s + 2 < steps) { a.fetch((s + 2) * OpA::BK); b.fetch((s + 2) * OpA::BK); }
+      }
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = mm_mfma<T>(fa[kk & 1][i], fb[kk & 1][j], acc[i][j]);
+    }
+    __syncthreads();
+  }
+  // accumulator register e of lane (r, h) is row 8 (e / 4) + 4 h + e % 4, column r
+  float *f = reinterpret_cast<float *>(lds);
+  const int r = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) f[(wm + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3)) * OP + wn + 32 * j + r] = acc[i][j][e];
+  __syncthreads();
+  T *o = out + (int64_t)z * g.M * g.N;
+  constexpr int V = OpA::V;
+#pragma unroll 2
+  for (int e = threadIdx.x; e < BT * BT / V; e += 256) {
+    const int row = e / (BT / V), col = (e % (BT / V)) * V;
+    if (row < a.valid && col < b.valid) mm_store<T>(o + (int64_t)(m0 + row) * g.N + n0 + col, f + row * OP + col, b.valid - col);
+  }
+}
+
+template <typename T, bool AKC, bool BKC>
+static int launch_mm(hipStream_t st, void *out, const void *A, const void *B, const MatmulArgs &g, int64_t batch) {
+  // 64 x 64 tiles; 16-bit operands take 128 x 128 (half the operand traffic per product) once those give every CU two and K
+  // is long enough to pay for the larger prologue (64 x 1024 x 1024 x 1024: 200 to 227 against 290 us; 32 x 512 x 80 x 512:
+  // 12.1 against 11.2).  Up to 256 bytes of K a tile needs no second stage: one load phase, and less LDS, so more blocks to
+  // a CU (32 x 512 x 80 x 512: 13.2 us with two stages of 128 bytes, 12.3 with one of 256, 11.2 with one of 192).
+  const int64_t t64 = batch * ((g.M + 63) / 64) * ((g.N + 63) / 64), tm128 = (g.M + 127) / 128, tn128 = (g.N + 127) / 128;
+  const int kb = (int)(g.K * (int64_t)sizeof(T) < 512 ? g.K * sizeof(T) : 512);
+  const int tm = (int)((g.M + 63) / 64), tn = (int)((g.N + 63) / 64);
+  auto go = [&](auto kernel, int64_t blocks, int tiles_m, int tiles_n) -> int {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, (T *)out, (const T *)A, (const T *)B, g, tiles_m, tiles_n);
+    return launch_check("matmul_mfma");
+  };
+  if constexpr (sizeof(T) == 2) {
+    if (batch * tm128 * tn128 >= 2 * kNumCU && g.K >= 256) return go(k_matmul_mfma<T, AKC, BKC, 2, 128, false>, batch * tm128 * tn128, (int)tm128, (int)tn128);
+  }
+  if (kb <= 128) return go(k_matmul_mfma<T, AKC, BKC, 1, 128, true>, t64, tm, tn);
+  if (kb <= 192) return go(k_matmul_mfma<T, AKC, BKC, 1, 192, true>, t64, tm, tn);
+  if (kb <= 256) return go(k_matmul_mfma<T, AKC, BKC, 1, 256, true>, t64, tm, tn);
+  return go(k_matmul_mfma<T, AKC, BKC, 1, 128, false>, t64, tm, tn);
+}
+
+bool matmul_mfma_serves(int dtype, const MatmulArgs &g, int64_t batch) {
+  const bool a = g.a_cs == 1 || g.a_rs == 1 || g.K == 1 || g.M == 1, b = g.b_rs == 1 || g.b_cs == 1 || g.K == 1 || g.N == 1;
+  return (dtype == RAI_F32 || dtype == RAI_BF16 || dtype == RAI_F16) && a && b && g.K < (1 << 30) && g.M < (1LL << 30) && g.N < (1LL << 30) &&
+         batch * ((g.M + 63) / 64) * ((g.N + 63) / 64) < (1LL << 31);
+}
+
+int launch_matmul_mfma(hipStream_t st, int dtype, void *out, const void *A, const void *B, const MatmulArgs &g0, int64_t batch) {
+  MatmulArgs g = g0;
+  // an axis of one element has no stride of its own
+  const bool akc = g.a_cs == 1 || g.K == 1, bkc = g.b_rs == 1 || g.K == 1;
+  auto go = [&](auto t) -> int {
+    typedef decltype(t) T;
+    if (akc) return bkc ? launch_mm<T, true, true>(st, out, A, B, g, batch) : launch_mm<T, true, false>(st, out, A, B, g, batch);
+    return bkc ? launch_mm<T, false, true>(st, out, A, B, g, batch) : launch_mm<T, false, false>(st, out, A, B, g, batch);
+  };
+  if (dtype == RAI_F32) return go(float());
+  return dtype == RAI_BF16 ? go(bf16_raw()) : go(f16_raw());
+}
+
+}  // namespace rai
