@@ -35,11 +35,12 @@ COMMON = [
 ]
 
 
-# Per-file additions.  attention.hip: its MFMA accumulators are rescaled by ordinary vector instructions every
+# Per-file additions.  attention*.hip: their MFMA accumulators are rescaled by ordinary vector instructions every
 # key tile, so they must live in the registers those instructions can address; without this the compiler parks
 # them in the accumulation registers and copies them out and back around every rescale.
 EXTRA = {
     "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attention_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

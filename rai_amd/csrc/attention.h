@@ -36,6 +36,9 @@ struct AttnArgs {
 };
 
 int launch_attention(hipStream_t st, const AttnArgs &a);
+// The f32 form on matrix instructions (attention_f32.hip): 16 rows and more, head sizes and alignments it takes.
+bool attention_f32_serves(const AttnArgs &a);
+int launch_attention_f32(hipStream_t st, const AttnArgs &a);
 
 // One new token per sequence (decode): rotary embedding of q and of the new k,
 // append of k/v to the cache, and attention over the cache plus the new token,

@@ -1300,6 +1300,7 @@ int launch_attention(hipStream_t st, const AttnArgs &a) {
       default: return launch_flash<256>(st, a);
     }
   }
+  if (attention_f32_serves(a)) return launch_attention_f32(st, a);
   switch (a.dtype) {
     case RAI_F32: return launch_row<float>(st, a);
     case RAI_BF16: return launch_row<bf16_raw>(st, a);

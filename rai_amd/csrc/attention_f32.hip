@@ -1,0 +1,325 @@
+// Prefill attention in f32 on the f32 matrix instructions (scores, probabilities and sums all in f32).
+//
+// Reference semantics: rai-models/src/llm/phi2.rs:244-262, qwen2.rs:205-221, gemma.rs:238-254 (see attention.hip).
+#include "attention.h"
+
+namespace rai {
+
+typedef __attribute__((ext_vector_type(4))) float af_f32x4;
+typedef __attribute__((ext_vector_type(16))) float af_f32x16;
+
+__device__ __forceinline__ float af_gate(float z) { return 1.0f / (1.0f + expf(-z)); }
+
+// A wave owns 32 query rows of one head and walks key tiles of 32, both products on v_mfma_f32_32x32x2_f32 in the
+// transposed orientation S^T = K Q^T, O^T = V^T P^T.  Lane (r, h) then owns query r: register e of its scores is key
+// 8 (e / 4) + 4 h + e % 4, and that register is, as it stands, the operand of the e-th MFMA of the second product, whose other
+// operand is feature r of that key.  Tiles go straight from memory into LDS (K with its 16-byte chunks swizzled by row, so
+// that the 16-byte reads of 32 rows spread over the banks; V as it lies); the registers hold the queries, the output and
+// one tile's sums.  (A form without LDS, both operands loaded into registers a tile ahead, was as fast and ran out of those, or kept longer
+// chains of sums: 1.8e-7 instead of 1.4e-7 off at 80 features.)
+//   One wave is one SIMD's 150 GFLOP/s, so where there are few query groups KSP waves share one, each with every KSP-th
+// key tile, and are merged through LDS.  DB: two LDS stages, the next round's tiles requested before this one's are
+// multiplied; otherwise two blocks on a CU cover each other's waits.
+//   Sums of products are kept in short chains, two side by side (32 features of a score, 16 keys of an output): less
+// rounding, and no MFMA waits for the one before it.
+//   A masked probability is zero and must not meet an infinity or a NaN of V in the product (0 x inf): in tiles with masks
+// those are left out, and afterwards added for the queries that see them.
+//   Measured (us; one block per query row on the vector units before): 32 heads x 333 x 80 23 (92), 32 x 512 x 80 32 (174),
+// 16 x 12 x 1024 x 128 on 2 key heads 970 (3755), 4 x 32 x 500 x 64 on 900 keys 165 (1001), 2 x 8 x 512 x 256 130 (173).
+template <int D> struct F32Attn {
+  static constexpr int CPR = D / 4, DT = (D + 31) / 32, TILE = 32 * D, LOADS = D / 8;   // 1 KB pieces of a tile
+  static __device__ __forceinline__ int swizzle(int row) { return D == 80 ? (row >> 2) & 3 : D == 32 ? (row >> 1) & 7 : row & 15; }
+};
+
+template <int D, int KSP, bool DB>
+__global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_flash_prefill_f32(AttnArgs a) {
+  typedef F32Attn<D> F;
+  constexpr int NG = 4 / KSP, KC = D / 8, DT = F::DT, STAGE = KSP * 2 * F::TILE, LW = (F::LOADS + 3) / 4;
+  extern __shared__ __attribute__((aligned(16))) float af_lds[];
+  typedef __attribute__((address_space(3))) void *lds_ptr;
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kh = wave % KSP;
+  const int head = blockIdx.x, b = blockIdx.z, hk = head / (a.Hq / a.Hkv);
+  // The last query groups see the most keys under a causal mask: those of all heads go first.  Heads next to each other
+  // land on different XCDs, whose L2s then hold the keys of few heads each.
+  const int block_q0 = (int)(gridDim.y - 1 - blockIdx.y) * NG * 32, q0 = block_q0 + wave / KSP * 32;
+  const int off = a.T - a.S;
+  const float *Kg = (const float *)a.k + b * a.ks[0] + hk * a.ks[1];
+  const float *Vg = (const float *)a.v + b * a.vs[0] + hk * a.vs[1];
+  const int qrow = q0 + r, q_abs = off + qrow;
+  const float *qp = (const float *)a.q + b * a.qs[0] + head * a.qs[1] + (int64_t)min(qrow, a.S - 1) * a.qs[2] + 4 * h;
+  af_f32x4 qf[KC];
+#pragma unroll
+  for (int c = 0; c < KC; ++c) qf[c] = *reinterpret_cast<const af_f32x4 *>(qp + 8 * c);
+  af_f32x16 o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  bool left_out = false;   // some infinity or NaN of V in a tile with masks
+  const int last_key = a.causal ? min(q_abs, a.T - 1) : a.T - 1;              // newest and oldest key this lane's query sees
+  const int first_key = a.window > 0 ? q_abs - a.window + 1 : 0;
+  auto end_of = [&](int q, int n) { return q >= a.S ? 0 : a.causal ? min(off + min(q + n, a.S), a.T) : a.T; };
+  const int kv_end = end_of(q0, 32), block_end = end_of(block_q0, 32 * NG);  // of any query of the group, of the block
+  const int oldest = a.window > 0 ? max(off + q0 - a.window + 1, 0) : 0;
+  const int begin = a.window > 0 ? max(off + block_q0 - a.window + 1, 0) & ~31 : 0;
+
+  // this thread's 16 bytes of the wave's LW loads of a tile
+  uint32_t k_off[LW], v_off[LW];
+#pragma unroll
+  for (int j = 0; j < LW; ++j) {
+    const int i = (wave + 4 * j) * 64 + lane, row = i / F::CPR, c = i % F::CPR;
+    k_off[j] = (uint32_t)(row * (int)a.ks[2] + 4 * (c ^ F::swizzle(row)));
+    v_off[j] = (uint32_t)(row * (int)a.vs[2] + 4 * c);
+  }
+  // a tile past the end of the keys starts early: what lies before its own first key is masked
+  auto fetch = [&](int base, int stage) {
+#pragma unroll
+    for (int i = 0; i < KSP; ++i) {
+      const int kt = min(base + 32 * i, a.T - 32);
+      const float *kp = Kg + (int64_t)kt * a.ks[2], *vp = Vg + (int64_t)kt * a.vs[2];
+      float *kd = af_lds + stage * STAGE + i * 2 * F::TILE, *vd = kd + F::TILE;
+#pragma unroll
+      for (int j = 0; j < LW; ++j)
+        if (F::LOADS % 4 == 0 || wave + 4 * j < F::LOADS) {
+          __builtin_amdgcn_global_load_lds((const void *)(kp + k_off[j]), (lds_ptr)(kd + (wave + 4 * j) * 256), 16, 0, 0);
+          __builtin_amdgcn_global_load_lds((const void *)(vp + v_off[j]), (lds_ptr)(vd + (wave + 4 * j) * 256), 16, 0, 0);
+        }
+    }
+  };
+  auto landed = [&]() {   // every wave's loads, for every wave
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  if (DB && begin < block_end) fetch(begin, 0);
+  int stage = 0;
+  for (int base = begin; base < block_end; base += 32 * KSP) {
+    if (DB) {
+      landed();   // and everybody is done with the other stage
+      if (base + 32 * KSP < block_end) fetch(base + 32 * KSP, stage ^ 1);
+    } else {
+      if (base > begin) __syncthreads();   // everybody is done with the last round's tiles
+      fetch(base, 0);
+      landed();
+    }
+    const float *Kt = af_lds + stage * STAGE + kh * 2 * F::TILE, *Vt = Kt + F::TILE;
+    if (DB) stage ^= 1;
+    const int k0 = base + 32 * kh, kt = min(k0, a.T - 32);
+    if (k0 >= kv_end || k0 + 31 < oldest) continue;   // nothing this wave's queries see
+    // (the fences keep the compiler from starting several steps' sums at once, which takes more registers than there are)
+    af_f32x16 s;
+#pragma unroll
+    for (int c0 = 0; c0 < KC; c0 += 4) {
+      af_f32x16 sg[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sg[i][e] = 0.f;
+#pragma unroll
+      for (int c = c0; c < KC && c < c0 + 4; ++c) {
+        const af_f32x4 kf = *reinterpret_cast<const af_f32x4 *>(Kt + r * D + 4 * ((2 * c + h) ^ F::swizzle(r)));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sg[j & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j], qf[c][j], sg[j & 1], 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = (c0 ? s[e] : 0.f) + (sg[0][e] + sg[1][e]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // ---- scale, cap, mask
+    const bool masked = k0 != kt || (a.causal && k0 + 31 > off + q0) || (a.window > 0 && k0 <= off + q0 + 31 - a.window);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] *= a.scale;
+    if (a.softcap > 0.f) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = a.softcap * tanhf(s[e] / a.softcap);
+    }
+    if (masked) {
+      const int from = max(first_key, k0);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int key = kt + 8 * (e >> 2) + 4 * h + (e & 3);
+        s[e] = key > last_key || key < from ? -INFINITY : s[e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m_run, mx), m_safe = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = expf(m_run - m_safe);
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      s[e] = expf(s[e] - m_safe);
+      sum[e & 3] += s[e];
+    }
+    m_run = m_new;
+    l_run = l_run * alpha + ((sum[0] + sum[1]) + (sum[2] + sum[3]));
+    // ---- O^T <- alpha O^T + V^T P^T, the products of sixteen keys in a chain
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      const float *vp = Vt + 4 * h * D + (D % 32 && t == DT - 1 ? min(32 * t + r, D - 1) : 32 * t + r);
+      float v[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v[e] = vp[(8 * (e >> 2) + (e & 3)) * D];
+      if (masked) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (!(fabsf(v[e]) < INFINITY)) { v[e] = 0.f; left_out = true; }
+      }
+      af_f32x16 p0, p1;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) p0[e] = p1[e] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        p0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e], s[e], p0, 0, 0, 0);
+        p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e + 8], s[e + 8], p1, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[t][e] = fmaf(o[t][e], alpha, p0[e] + p1[e]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (__builtin_amdgcn_ballot_w64(left_out)) {
+    // What was left out goes to the queries that see it: the tiles with masks once more, key by key.
+#pragma unroll 1
+    for (int k1 = begin + 32 * kh; k1 < kv_end; k1 += 32 * KSP) {
+      if (k1 + 31 < oldest) continue;
+      const int kt = min(k1, a.T - 32), from = max(first_key, k1);
+      if (!(k1 != kt || (a.causal && k1 + 31 > off + q0) || (a.window > 0 && k1 <= off + q0 + 31 - a.window))) continue;
+#pragma unroll 1
+      for (int key = kt; key < kt + 32; ++key) {
+        const float *kp = Kg + (int64_t)key * a.ks[2] + 4 * h, *vp = Vg + (int64_t)key * a.vs[2] + 4 * h;
+        float dot = 0.f;
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            dot = fmaf(kp[8 * c + j], qf[c][j], dot);
+            if (c % 4 == 3 && j == 3) __builtin_amdgcn_sched_barrier(0);
+          }
+        dot = (dot + __shfl_xor(dot, 32, 64)) * a.scale;
+        if (a.softcap > 0.f) dot = a.softcap * tanhf(dot / a.softcap);
+        if (key > last_key || key < from) continue;
+        const float p = expf(dot - m_run);
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            if (32 * t + 8 * (e >> 2) < D) {
+              const float x = vp[32 * t + 8 * (e >> 2) + (e & 3)];
+              o[t][e] = fabsf(x) < INFINITY ? o[t][e] : fmaf(p, x, o[t][e]);
+            }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  }
+  float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  if constexpr (KSP > 1) {
+    constexpr int MS = (2 + DT * 16) * 64;   // floats a wave hands over: value by value, lane by lane
+    __syncthreads();                         // the tiles are no longer read
+    if (kh > 0) {
+      float *mine = af_lds + (wave / KSP * (KSP - 1) + kh - 1) * MS + lane;
+      mine[0] = m_run;
+      mine[64] = l_tot;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mine[(2 + t * 16 + e) * 64] = o[t][e];
+    }
+    __syncthreads();
+    if (kh > 0) return;
+    const float *theirs = af_lds + wave / KSP * (KSP - 1) * MS + lane;
+    float m = m_run;
+#pragma unroll
+    for (int j = 0; j < KSP - 1; ++j) m = fmaxf(m, theirs[j * MS]);
+    const float ms = m == -INFINITY ? 0.f : m, w0 = expf(m_run - ms);
+    l_tot *= w0;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[t][e] *= w0;
+#pragma unroll 1
+    for (int j = 0; j < KSP - 1; ++j) {
+      const float *p = theirs + j * MS, w = expf(p[0] - ms);
+      l_tot = fmaf(p[64], w, l_tot);
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[t][e] = fmaf(p[(2 + t * 16 + e) * 64], w, o[t][e]);
+    }
+    m_run = m;
+  }
+  if (qrow >= a.S) return;
+  float scale = 1.0f;
+  if (a.sink) {   // relative to the larger of the two exponents
+    const float sink = ((const float *)a.sink)[head], m = fmaxf(m_run, sink);
+    scale = expf(m_run - m);
+    l_tot = l_tot * scale + expf(sink - m);
+  }
+  const float inv = scale / l_tot;
+  const int64_t row = (int64_t)b * a.S + qrow;
+  float *op = (float *)a.out + row * a.out_row_stride + (int64_t)head * D;
+  const float *gp = a.gate ? (const float *)a.gate + row * a.gate_row_stride + (int64_t)head * D : nullptr;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; e += 4) {
+      const int d = 32 * t + 2 * e + 4 * h;   // 8 (e / 4)
+      if (d >= D) continue;
+      af_f32x4 w = {o[t][e] * inv, o[t][e + 1] * inv, o[t][e + 2] * inv, o[t][e + 3] * inv};
+      if (gp) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] *= af_gate(gp[d + j]);
+      }
+      *reinterpret_cast<af_f32x4 *>(op + d) = w;
+    }
+}
+
+template <int D, int KSP> static int launch_f32(hipStream_t st, const AttnArgs &a) {
+  constexpr int NG = 4 / KSP;
+  constexpr bool DB = KSP == 1 && D <= 128;
+  constexpr size_t tiles = (size_t)(DB ? 2 : 1) * KSP * 2 * F32Attn<D>::TILE * sizeof(float);
+  constexpr size_t merge = (size_t)NG * (KSP - 1) * (2 + F32Attn<D>::DT * 16) * 64 * sizeof(float), lds = tiles > merge ? tiles : merge;
+  static_assert(lds <= 160 * 1024, "LDS of a block");
+  static bool attr_set = false;
+  if (lds > 64 * 1024 && !attr_set) {
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_flash_prefill_f32<D, KSP, DB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((k_flash_prefill_f32<D, KSP, DB>), dim3(a.Hq, (a.S + 32 * NG - 1) / (32 * NG), a.B), dim3(256), lds, st, a);
+  return launch_check("flash_prefill_f32");
+}
+
+// Waves to a query group: as many as keep all blocks on the chip at once (two to a CU while LDS and registers hold them), no
+// more than there are key tiles.
+template <int D> static int launch_f32_split(hipStream_t st, const AttnArgs &a) {
+  const int64_t groups = (int64_t)((a.S + 31) / 32) * a.Hq * a.B;
+  const int seen = a.window > 0 && a.window + 31 < a.T ? a.window + 31 : a.T, tiles = (seen + 31) / 32;
+  if constexpr (D <= 128) {
+    if (groups <= (D <= 80 ? 2 : 1) * kNumCU && tiles >= 4) return launch_f32<D, 4>(st, a);
+  }
+  if (groups * 2 <= (D <= 128 ? 8 : 4) * kNumCU && tiles >= 2) return launch_f32<D, 2>(st, a);
+  return launch_f32<D, 1>(st, a);
+}
+
+bool attention_f32_serves(const AttnArgs &a) {
+  if (a.dtype != RAI_F32 || a.S < 16 || a.T < 32 || a.t_dev) return false;
+  if (a.D != 32 && a.D != 64 && a.D != 80 && a.D != 128 && a.D != 192 && a.D != 256) return false;
+  auto al = [](const void *p, const int64_t *s) { return (uintptr_t)p % 16 == 0 && s[0] % 4 == 0 && s[1] % 4 == 0 && s[2] % 4 == 0 && s[2] < (1 << 24); };
+  return al(a.q, a.qs) && al(a.k, a.ks) && al(a.v, a.vs) && (uintptr_t)a.out % 16 == 0 && a.out_row_stride % 4 == 0 && (a.S + 31) / 32 <= 65535 && a.B <= 65535;
+}
+
+int launch_attention_f32(hipStream_t st, const AttnArgs &a) {
+  switch (a.D) {
+    case 32: return launch_f32_split<32>(st, a);
+    case 64: return launch_f32_split<64>(st, a);
+    case 80: return launch_f32_split<80>(st, a);
+    case 128: return launch_f32_split<128>(st, a);
+    case 192: return launch_f32_split<192>(st, a);
+    default: return launch_f32_split<256>(st, a);
+  }
+}
+
+}  // namespace rai

@@ -1,0 +1,60 @@
+"""f32 prefill attention on the matrix instructions: query groups of 32, key tiles of 32, one, two or four waves to a group,
+every head size it takes."""
+import numpy as np
+import pytest
+
+from tests.util import down, rand, up
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def R(hip):
+    from rai_amd import ops
+
+    return ops
+
+
+def reference(q, k, v, scale, causal):
+    q, k, v = (t.astype(np.float64) for t in (q, k, v))
+    n = q.shape[1] // k.shape[1]
+    k, v = np.repeat(k, n, 1), np.repeat(v, n, 1)
+    s, size = np.matmul(q, np.swapaxes(k, 2, 3)) * scale, np.matmul(np.abs(q), np.swapaxes(np.abs(k), 2, 3)) * scale
+    S, T = s.shape[2:]
+    if causal:
+        s = np.where(np.arange(T)[None] <= np.arange(T - S, T)[:, None], s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    # A score's sum is within D + 2 roundings of its absolute sum; twice that error of the largest score (numerator and
+    # denominator), and T + 8 roundings of the weighted sum, reach the output relative to sum p |v|.
+    rel = 2 * (q.shape[-1] + 2) * 2.0 ** -24 * size.max() + (T + 8) * 2.0 ** -23
+    flat = lambda t: np.swapaxes(t, 1, 2).reshape(t.shape[0], S, -1)  # noqa: E731
+    with np.errstate(invalid="ignore"):
+        return flat(p @ v), rel * flat(p @ np.abs(v))
+
+
+@pytest.mark.parametrize("causal", [1, 0])
+@pytest.mark.parametrize("b,hq,hkv,s,t,d", [(1, 2, 2, 16, 32, 64), (2, 3, 1, 33, 65, 80), (1, 4, 2, 128, 128, 128), (1, 2, 1, 31, 300, 32), (1, 1, 1, 97, 129, 192),
+                                            (1, 2, 1, 64, 200, 256), (3, 24, 24, 40, 160, 64), (16, 36, 6, 64, 64, 128)])
+def test_against_64_bits(R, b, hq, hkv, s, t, d, causal):
+    g = np.random.Generator(np.random.PCG64(b + s))
+    q, k, v = rand(g, (b, hq, s, d), "f32"), rand(g, (b, hkv, t, d), "f32"), rand(g, (b, hkv, t, d), "f32")
+    want, tol = reference(q, k, v, d ** -0.5, causal)
+    got = down(R.attention(up(q, "f32"), up(k, "f32"), up(v, "f32"), d ** -0.5, causal, 1)).astype(np.float64)
+    assert np.all(np.abs(got - want) <= tol)
+
+
+@pytest.mark.parametrize("s,t", [(40, 70), (200, 200)])
+def test_infinite_values_reach_only_queries_that_see_them(R, s, t):
+    g = np.random.Generator(np.random.PCG64(9))
+    q, k, v = rand(g, (1, 2, s, 64), "f32"), rand(g, (1, 2, t, 64), "f32"), rand(g, (1, 2, t, 64), "f32")
+    clean, tol = reference(q, k, v, 0.125, 1)
+    at = t - s // 2
+    v[0, 0, at, 5], v[0, 0, t - 1, 7], v[0, 1, at, 63] = np.inf, np.nan, -np.inf
+    got = down(R.attention(up(q, "f32"), up(k, "f32"), up(v, "f32"), 0.125, 1, 1)).astype(np.float64)
+    want = clean.copy()
+    first = at - (t - s)   # the query at the key's own position
+    want[0, first:, 5], want[0, s - 1, 7], want[0, first:, 64 + 63] = np.inf, np.nan, -np.inf
+    same = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~same & ~np.isnan(want)], want[~same & ~np.isnan(want)])
+    assert np.all(np.abs(got - clean)[same] <= tol[same])
