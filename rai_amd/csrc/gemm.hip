@@ -411,6 +411,111 @@ __global__ void __launch_bounds__(256) k_gemv_bf16_reg_group(GemvGroupArgs g, in
   gemv_reg_rows<KC, R>(a, (gw - base) * rows_per_wave, rows_per_wave);
 }
 
+// ============================================================ bf16, few rows
+// Up to M rows of A against a row-major W: a block owns R rows of W, a quarter of K to each of its four waves; a wave reads
+// 1 KB of a row with one instruction and multiplies it with the same piece of the rows of A, which come from L2 and stay
+// in registers.  Bound by the weights' way from HBM: few bytes per wave and many small waves in flight do best.
+//   Measured with weights that no cache holds (us; K x N; the kernels that stage A in LDS or keep all of it in registers in
+// brackets): one row 8192 x 8960 24.0 (39.0; 6.1 TB/s), 2048 x 8960 8.6 (12.8), 512 x 512 4.2 (4.6, a launch); two rows
+// 8192 x 8960 26.4 (42.1); four 29.9 (75.1), 2048 x 8960 10.8 (16.7); eight 37.5 (80.8), 2048 x 8960 14.5 (20.6), 8192 x
+// 2048 14.5 (32.8).
+template <int M, int R, int KW>
+__global__ void __launch_bounds__(256) k_linear_bf16_rows(LinearArgs a) {
+  constexpr int U = 2, G = 4 / KW;   // G groups of R rows to a block
+  __shared__ float red[4][R * M];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kw = wave % KW;
+  const int n0 = (blockIdx.x * G + wave / KW) * R;
+  const int chunks = (a.K + 511) / 512, each = (chunks + KW - 1) / KW;
+  const int k_end = min((kw + 1) * each * 512, a.K);
+  const uint16_t *A = (const uint16_t *)a.A, *w[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) w[i] = (const uint16_t *)a.W + (int64_t)min(n0 + i, a.N - 1) * a.ldw;
+  float acc[R][M];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[i][m] = 0.f;
+  for (int k0 = kw * each * 512 + 8 * lane; k0 < k_end; k0 += 512 * U) {
+    u32x4 wv[U][R], xv[U][M];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + 512 * u < k_end ? k0 + 512 * u : k0;   // past the end: read again, not added
+#pragma unroll
+      for (int m = 0; m < M; ++m) xv[u][m] = *reinterpret_cast<const u32x4 *>(A + (int64_t)min(m, a.M - 1) * a.lda + k);
+#pragma unroll
+      for (int i = 0; i < R; ++i) wv[u][i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w[i] + k));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k0 + 512 * u < k_end) {
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+          for (int m = 0; m < M; ++m) acc[i][m] = dot8_bf16(wv[u][i], xv[u][m], acc[i][m]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[i][m] = wave_sum(acc[i][m]);
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int m = 0; m < M; ++m) red[wave][i * M + m] = acc[i][m];
+  }
+  __syncthreads();
+  if (threadIdx.x >= G * R * M) return;   // a thread finishes one output, or one gated pair
+  const int m = threadIdx.x % M, g = threadIdx.x / (R * M), i = threadIdx.x / M % R, n = (blockIdx.x * G + g) * R + i;
+  if (m >= a.M || n >= a.N) return;
+  const uint16_t *bias = (const uint16_t *)a.bias, *bias2 = (const uint16_t *)a.bias2;
+  auto sum = [&](int j) {
+    float v = red[g * KW][j * M + m];
+#pragma unroll
+    for (int q = 1; q < KW; ++q) v += red[g * KW + q][j * M + m];
+    return v;
+  };
+  if (a.glu) {
+    if ((i & 1) || n + 1 >= a.N) return;
+    const float bg = bias ? bf16_bits_to_f32(bias[n]) : 0.f, bu = bias ? bf16_bits_to_f32(bias[n + 1]) : 0.f;
+    ((uint16_t *)a.out1)[(int64_t)m * a.ld1 + (n >> 1)] = f32_to_bf16_bits(glu_bf16(a, sum(i) + bg, sum(i + 1) + bu));
+    return;
+  }
+  float v = sum(i) + ((bias ? bf16_bits_to_f32(bias[n]) : 0.f) + (bias2 ? bf16_bits_to_f32(bias2[n]) : 0.f));
+  if (a.act >= 0 && n >= a.act_from) v = act_eval(a.act, v);
+  if (a.f32_out) {
+    ((float *)a.out1)[(int64_t)m * a.ld1 + n] = fmaf(a.out_scale, v, a.residual ? ((const float *)a.residual)[(int64_t)m * a.ldr + n] : 0.f);
+    return;
+  }
+  if (a.residual) v += bf16_bits_to_f32(((const uint16_t *)a.residual)[(int64_t)m * a.ldr + n]);
+  if (n < a.n_split) ((uint16_t *)a.out1)[(int64_t)m * a.ld1 + n] = f32_to_bf16_bits(v);
+  else ((uint16_t *)a.out2)[(int64_t)m * a.ld2 + (n - a.n_split)] = f32_to_bf16_bits(v);
+}
+
+template <int M, int R, int KW> static int launch_rows_cfg(hipStream_t st, const LinearArgs &a) {
+  constexpr int per_block = 4 / KW * R;
+  hipLaunchKernelGGL((k_linear_bf16_rows<M, R, KW>), dim3((a.N + per_block - 1) / per_block), dim3(256), 0, st, a);
+  return launch_check("linear_bf16_rows");
+}
+template <int M, int R> static int launch_rows_r(hipStream_t st, const LinearArgs &a, bool whole_k) {
+  return whole_k ? launch_rows_cfg<M, R, 1>(st, a) : launch_rows_cfg<M, R, 4>(st, a);
+}
+
+// Who shares what.  A wave's end (R x M sums across its lanes) is paid per wave, so short rows of W are not cut over the
+// waves of a block, and with more rows of A not long ones either while N alone makes enough waves (two rows of A, 448 x 8960:
+// 4.5 us whole, 7.2 in quarters; eight, 2560 x 17920: 24.9 against 42.5; one, 12800 x 2560: 18.0 against 12.6).  Every block
+// reads the rows of A again: four rows of W to a block halve that where it weighs (four rows of A, 12800 x 17920: 80 us
+// against 99) and make half the waves, which costs elsewhere (2560 x 2560: 7.0 against 6.0).
+static int launch_linear_bf16_rows(hipStream_t st, const LinearArgs &a) {
+  const bool whole_k = a.K <= 1024 || (a.M > 2 && a.K <= 2048 && a.N >= 2048) || (a.M > 4 && a.K <= 4096 && a.N >= 8192);
+  const bool r4 = a.M > 2 && ((a.N >= 8192 && a.K >= (a.M > 4 ? 2049 : 4096)) || (a.M > 4 && a.K >= 8192));
+  if (a.M == 1) return launch_rows_r<1, 2>(st, a, whole_k);
+  if (a.M == 2) return launch_rows_r<2, 2>(st, a, whole_k);
+  if (a.M <= 4) return r4 ? launch_rows_r<4, 4>(st, a, whole_k) : launch_rows_r<4, 2>(st, a, whole_k);
+  return r4 ? launch_rows_r<8, 4>(st, a, whole_k) : launch_rows_r<8, 2>(st, a, whole_k);
+}
+
 // ============================================================ generic strided batched matmul
 template <typename T>
 __global__ void __launch_bounds__(256) k_matmul_generic(T *out, const T *A, const T *B, MatmulArgs g) {
@@ -632,6 +737,12 @@ int launch_linear_dual_row(hipStream_t st, int dev, const void *x1, int K1, cons
 }
 
 int launch_linear_bf16(hipStream_t st, const LinearArgs &a) {
+  if (a.M <= 8 && a.ln_kind < 0 && !a.K2) {
+    RAI_TRY(check_linear_args(a, 2));
+    if (a.glu) RAI_REQUIRE(a.N % 2 == 0 && !a.residual && a.n_split == a.N && a.act >= 0, RAI_ERR_BAD_ARG, "linear: bad gated-MLP arguments");
+    RAI_REQUIRE(!a.f32_out || (a.n_split == a.N && !a.glu), RAI_ERR_BAD_ARG, "linear: an f32 output is a single, ungated one");
+    return launch_linear_bf16_rows(st, a);
+  }
   if (a.M <= 8 && (size_t)a.M * a.K * 2 <= 150 * 1024) return launch_linear_bf16_skinny(st, a);
   return launch_linear_bf16_mfma(st, a);
 }
