@@ -15,26 +15,27 @@ __device__ __forceinline__ float af_gate(float z) { return 1.0f / (1.0f + expf(-
 // 8 (e / 4) + 4 h + e % 4, and that register is, as it stands, the operand of the e-th MFMA of the second product, whose other
 // operand is feature r of that key.  Tiles go straight from memory into LDS (K with its 16-byte chunks swizzled by row, so
 // that the 16-byte reads of 32 rows spread over the banks; V as it lies); the registers hold the queries, the output and
-// one tile's sums.  (A form without LDS, both operands loaded into registers a tile ahead, was as fast and ran out of those, or kept longer
-// chains of sums: 1.8e-7 instead of 1.4e-7 off at 80 features.)
+// one tile's sums.  (A form without LDS, both operands loaded into registers a tile ahead, was as fast and ran out of those.)
 //   One wave is one SIMD's 150 GFLOP/s, so where there are few query groups KSP waves share one, each with every KSP-th
 // key tile, and are merged through LDS.  DB: two LDS stages, the next round's tiles requested before this one's are
-// multiplied; otherwise two blocks on a CU cover each other's waits.
-//   Sums of products are kept in short chains, two side by side (32 features of a score, 16 keys of an output): less
-// rounding, and no MFMA waits for the one before it.
+// multiplied; otherwise several waves share the work of a group and cover each other's waits.
+//   Sums of products are kept in short chains, two side by side (16 features of a score, 8 keys of an output; twice that
+// beyond 128 features): less rounding, and no MFMA waits for the one before it.  Up to 64 features that fits 256 registers and
+// two blocks share a CU; beyond, 512 and one (80 features in 256: spilled, 85 us instead of 59 at 32 x 700).
 //   A masked probability is zero and must not meet an infinity or a NaN of V in the product (0 x inf): in tiles with masks
 // those are left out, and afterwards added for the queries that see them.
-//   Measured (us; one block per query row on the vector units before): 32 heads x 333 x 80 23 (92), 32 x 512 x 80 32 (174),
-// 16 x 12 x 1024 x 128 on 2 key heads 970 (3755), 4 x 32 x 500 x 64 on 900 keys 165 (1001), 2 x 8 x 512 x 256 130 (173).
+//   Measured (us; one block per query row on the vector units in brackets): 32 heads x 333 x 80 25 (92), 32 x 512 x 80 36 (174),
+// 16 x 12 x 1024 x 128 on 2 key heads 993 (3900), 4 x 32 x 500 x 64 on 900 keys 180 (1030), 2 x 8 x 512 x 256 130 (178).  Off by
+// 1.23e-7 (1.30e-7), 1.28e-7 (1.36e-7), 1.43e-7 (1.52e-7), 1.76e-7 (1.84e-7), 1.43e-7 (1.47e-7).
 template <int D> struct F32Attn {
   static constexpr int CPR = D / 4, DT = (D + 31) / 32, TILE = 32 * D, LOADS = D / 8;   // 1 KB pieces of a tile
   static __device__ __forceinline__ int swizzle(int row) { return D == 80 ? (row >> 2) & 3 : D == 32 ? (row >> 1) & 7 : row & 15; }
 };
 
 template <int D, int KSP, bool DB>
-__global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_flash_prefill_f32(AttnArgs a) {
+__global__ void __launch_bounds__(256, D > 64 ? 1 : 2) k_flash_prefill_f32(AttnArgs a) {
   typedef F32Attn<D> F;
-  constexpr int NG = 4 / KSP, KC = D / 8, DT = F::DT, STAGE = KSP * 2 * F::TILE, LW = (F::LOADS + 3) / 4;
+  constexpr int NG = 4 / KSP, KC = D / 8, CG = D <= 128 ? 2 : 4, DT = F::DT, STAGE = KSP * 2 * F::TILE, LW = (F::LOADS + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) float af_lds[];
   typedef __attribute__((address_space(3))) void *lds_ptr;
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kh = wave % KSP;
@@ -72,6 +73,11 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_flash_prefill_f32(Attn
     k_off[j] = (uint32_t)(row * (int)a.ks[2] + 4 * (c ^ F::swizzle(row)));
     v_off[j] = (uint32_t)(row * (int)a.vs[2] + 4 * c);
   }
+  // where this lane's chunks of a row of K lie: the swizzle stays within PAT chunks, what is beyond goes into the instruction
+  constexpr int PAT = D == 80 ? 4 : D == 32 ? 8 : 16;
+  int k_lane[PAT / 2];
+#pragma unroll
+  for (int c = 0; c < PAT / 2; ++c) k_lane[c] = r * D + 4 * ((2 * c + h) ^ F::swizzle(r));
   // a tile past the end of the keys starts early: what lies before its own first key is masked
   auto fetch = [&](int base, int stage) {
 #pragma unroll
@@ -109,15 +115,15 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_flash_prefill_f32(Attn
     // (the fences keep the compiler from starting several steps' sums at once, which takes more registers than there are)
     af_f32x16 s;
 #pragma unroll
-    for (int c0 = 0; c0 < KC; c0 += 4) {
+    for (int c0 = 0; c0 < KC; c0 += CG) {
       af_f32x16 sg[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) sg[i][e] = 0.f;
 #pragma unroll
-      for (int c = c0; c < KC && c < c0 + 4; ++c) {
-        const af_f32x4 kf = *reinterpret_cast<const af_f32x4 *>(Kt + r * D + 4 * ((2 * c + h) ^ F::swizzle(r)));
+      for (int c = c0; c < KC && c < c0 + CG; ++c) {
+        const af_f32x4 kf = *reinterpret_cast<const af_f32x4 *>(Kt + k_lane[c % (PAT / 2)] + 4 * (2 * c & ~(PAT - 1)));
 #pragma unroll
         for (int j = 0; j < 4; ++j) sg[j & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j], qf[c][j], sg[j & 1], 0, 0, 0);
       }
@@ -125,11 +131,12 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_flash_prefill_f32(Attn
       for (int e = 0; e < 16; ++e) s[e] = (c0 ? s[e] : 0.f) + (sg[0][e] + sg[1][e]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    // ---- scale, cap, mask
+    // ---- scale, cap, mask (the scale, where nothing follows it, goes into the exponent's subtraction: one rounding less)
     const bool masked = k0 != kt || (a.causal && k0 + 31 > off + q0) || (a.window > 0 && k0 <= off + q0 + 31 - a.window);
     float mx = -INFINITY;
+    const float now = a.softcap > 0.f || !(a.scale > 0.f) ? a.scale : 1.f, later = now == 1.f ? a.scale : 1.f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) s[e] *= a.scale;
+    for (int e = 0; e < 16; ++e) s[e] *= now;
     if (a.softcap > 0.f) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = a.softcap * tanhf(s[e] / a.softcap);
@@ -143,14 +150,14 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_flash_prefill_f32(Attn
       }
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
+    for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e] * later);
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float m_new = fmaxf(m_run, mx), m_safe = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = expf(m_run - m_safe);
     float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      s[e] = expf(s[e] - m_safe);
+      s[e] = expf(fmaf(s[e], later, -m_safe));
       sum[e & 3] += s[e];
     }
     m_run = m_new;
@@ -170,10 +177,29 @@ __global__ void __launch_bounds__(256, D > 128 ? 1 : 2) k_flash_prefill_f32(Attn
       af_f32x16 p0, p1;
 #pragma unroll
       for (int e = 0; e < 16; ++e) p0[e] = p1[e] = 0.f;
+      if constexpr (D <= 128) {   // four chains
+        af_f32x16 q;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        p0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e], s[e], p0, 0, 0, 0);
-        p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e + 8], s[e + 8], p1, 0, 0, 0);
+        for (int half = 0; half < 2; ++half) {
+          if (half) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) { q[e] = p0[e] + p1[e]; p0[e] = p1[e] = 0.f; }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int e = 8 * half; e < 8 * half + 4; ++e) {
+            p0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e], s[e], p0, 0, 0, 0);
+            p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e + 4], s[e + 4], p1, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) p0[e] += q[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          p0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e], s[e], p0, 0, 0, 0);
+          p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e + 8], s[e + 8], p1, 0, 0, 0);
+        }
       }
 #pragma unroll
       for (int e = 0; e < 16; ++e) o[t][e] = fmaf(o[t][e], alpha, p0[e] + p1[e]);
@@ -304,9 +330,17 @@ template <int D> static int launch_f32_split(hipStream_t st, const AttnArgs &a) 
   return launch_f32<D, 1>(st, a);
 }
 
+// A block per query row (attention.hip) is done sooner where there are few rows: a tile here is a chain of some 2 us at 64
+// features (8 at 256), which takes enough rows or keys to be worth it.  Measured (us; block per row, here): 32 heads x 48 x 64
+// 7.3, 8.0, 32 x 64 x 64 9.4, 8.2; 8 x 160 x 80 12.2, 15.2, 32 x 160 x 80 28.5, 15.5; 8 x 64 on 300 x 128 20.0, 29.3, 32 x 64 on
+// 300 38.1, 29.6; 32 x 64 on 300 x 256 66, 86, 2 x 8 x 512 x 256 174, 129.  Beyond 80 features the sums of a score are longer
+// chains than a row's lanes make of them, and less exact than those until there are a few hundred keys (1.17e-7 and 1.11e-7 at 100
+// x 128, 1.67e-7 and 1.86e-7 on 300).
 bool attention_f32_serves(const AttnArgs &a) {
   if (a.dtype != RAI_F32 || a.S < 16 || a.T < 32 || a.t_dev) return false;
   if (a.D != 32 && a.D != 64 && a.D != 80 && a.D != 128 && a.D != 192 && a.D != 256) return false;
+  const int64_t rows = (int64_t)a.B * a.Hq * a.S;
+  if (rows < (a.D <= 128 ? 2048 : 8192) || (a.D <= 80 ? rows * a.T < 2048 * 64 : a.T < (a.D <= 128 ? 256 : 512))) return false;
   auto al = [](const void *p, const int64_t *s) { return (uintptr_t)p % 16 == 0 && s[0] % 4 == 0 && s[1] % 4 == 0 && s[2] % 4 == 0 && s[2] < (1 << 24); };
   return al(a.q, a.qs) && al(a.k, a.ks) && al(a.v, a.vs) && (uintptr_t)a.out % 16 == 0 && a.out_row_stride % 4 == 0 && (a.S + 31) / 32 <= 65535 && a.B <= 65535;
 }

@@ -35,7 +35,9 @@ def reference(q, k, v, scale, causal):
 
 @pytest.mark.parametrize("causal", [1, 0])
 @pytest.mark.parametrize("b,hq,hkv,s,t,d", [(1, 2, 2, 16, 32, 64), (2, 3, 1, 33, 65, 80), (1, 4, 2, 128, 128, 128), (1, 2, 1, 31, 300, 32), (1, 1, 1, 97, 129, 192),
-                                            (1, 2, 1, 64, 200, 256), (3, 24, 24, 40, 160, 64), (16, 36, 6, 64, 64, 128)])
+                                            (1, 2, 1, 64, 200, 256), (3, 24, 24, 40, 160, 64), (16, 36, 6, 64, 64, 128), (1, 64, 64, 33, 129, 80),
+                                            (1, 64, 16, 32, 65, 64), (16, 36, 6, 64, 64, 64), (2, 64, 64, 31, 80, 32), (1, 64, 8, 33, 300, 128),
+                                            (1, 64, 8, 32, 256, 128), (16, 36, 6, 33, 257, 128), (1, 32, 4, 260, 515, 192), (1, 16, 16, 520, 520, 256)])
 def test_against_64_bits(R, b, hq, hkv, s, t, d, causal):
     g = np.random.Generator(np.random.PCG64(b + s))
     q, k, v = rand(g, (b, hq, s, d), "f32"), rand(g, (b, hkv, t, d), "f32"), rand(g, (b, hkv, t, d), "f32")
@@ -44,10 +46,10 @@ def test_against_64_bits(R, b, hq, hkv, s, t, d, causal):
     assert np.all(np.abs(got - want) <= tol)
 
 
-@pytest.mark.parametrize("s,t", [(40, 70), (200, 200)])
-def test_infinite_values_reach_only_queries_that_see_them(R, s, t):
+@pytest.mark.parametrize("s,t,n", [(40, 70, 2), (200, 200, 2), (40, 70, 64), (200, 200, 16)])
+def test_infinite_values_reach_only_queries_that_see_them(R, s, t, n):
     g = np.random.Generator(np.random.PCG64(9))
-    q, k, v = rand(g, (1, 2, s, 64), "f32"), rand(g, (1, 2, t, 64), "f32"), rand(g, (1, 2, t, 64), "f32")
+    q, k, v = rand(g, (1, n, s, 64), "f32"), rand(g, (1, n, t, 64), "f32"), rand(g, (1, n, t, 64), "f32")
     clean, tol = reference(q, k, v, 0.125, 1)
     at = t - s // 2
     v[0, 0, at, 5], v[0, 0, t - 1, 7], v[0, 1, at, 63] = np.inf, np.nan, -np.inf
