@@ -513,6 +513,7 @@ static int launch_linear_bf16_rows(hipStream_t st, const LinearArgs &a) {
   if (a.M == 1) return launch_rows_r<1, 2>(st, a, whole_k);
   if (a.M == 2) return launch_rows_r<2, 2>(st, a, whole_k);
   if (a.M <= 4) return r4 ? launch_rows_r<4, 4>(st, a, whole_k) : launch_rows_r<4, 2>(st, a, whole_k);
+  if (a.M <= 6) return r4 ? launch_rows_r<6, 4>(st, a, whole_k) : launch_rows_r<6, 2>(st, a, whole_k);
   return r4 ? launch_rows_r<8, 4>(st, a, whole_k) : launch_rows_r<8, 2>(st, a, whole_k);
 }
 

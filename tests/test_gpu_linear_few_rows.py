@@ -20,7 +20,7 @@ def spread(x, w):
     return (x.shape[1] + 8) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T + 1)
 
 
-@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 6, 8])
 @pytest.mark.parametrize("k,n", [(8, 1), (8, 5), (504, 2), (520, 1031), (1024, 2049), (2048, 1026), (2056, 3), (4104, 4098), (4096, 8198), (4104, 8193), (8968, 33)])
 def test_few_rows(R, m, k, n):
     g = np.random.Generator(np.random.PCG64(m * 1000 + k))
