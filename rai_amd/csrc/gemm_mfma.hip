@@ -55,9 +55,9 @@ template <int BM, int BN, int PITCH, int WGN = 2, int WGM = 2> constexpr int gem
   return tiles > staging ? tiles : staging;
 }
 
-// LDS of the LDS-DMA tile kernels: NS stages of 32 of K, or (NS == 2) two stages of 64.
-template <int BM, int BN, int NS, int WGN, int WGM = 2> constexpr int dma_lds_bytes() {
-  return gemm_lds_bytes<BM, BN, NS == 2 ? 64 : 32 * NS / 2, WGN, WGM>();
+// LDS of the LDS-DMA tile kernels: NS stages of 32 of K, or (NS == 2, or SH == 0) of 64.
+template <int BM, int BN, int NS, int WGN, int WGM = 2, int SH = 2> constexpr int dma_lds_bytes() {
+  return gemm_lds_bytes<BM, BN, NS == 2 || SH == 0 ? 32 * NS : 32 * NS / 2, WGN, WGM>();
 }
 
 // Applies activation `act` to the elements of x[8] whose column n + e is >= from.  The switch on the
@@ -533,13 +533,14 @@ __device__ __forceinline__ void dma_tile_mainloop(const LinearArgs &a, uint16_t 
 // so every request the L1 sends to L2 is a whole 128-byte line instead of half of one (the L2s deliver 1.7x the bytes
 // per clock that way with all CUs asking, measured with the loads alone), and there is one barrier per 64 of K.  Two
 // stages (the same 128 KB for a 256 x 256 tile as four stages of 32): stage s+1 is requested when stage s-1 has been
-// left by every wave, a whole stage of multiplies before it is needed.
+// left by every wave, a whole stage of multiplies before it is needed.  A small tile multiplies a stage in less time than
+// its loads take: three or four stages (NS) keep two or three of them in flight.
 //   - 16-byte chunk c (0..7) of row r lives at chunk position c ^ ((r >> 1) & 7): the 8 lanes that fetch one row swap
 //     places within their 128-byte line, and a fragment read's 16 lanes per LDS cycle (16 rows at one chunk index; two
 //     rows span the 64 banks) land on 16 different 16-byte slots.  (Swizzling by r & 7 left rows r and r + 8 on the
 //     same banks: SQ_LDS_BANK_CONFLICT at 23 % of the kernel's cycles.)
 //   - fragment sets alternate F0 / F1 over the four K steps of a stage; the reads run one set ahead of the multiplies.
-template <int BM, int BN, int WGN, int WGM = 2>
+template <int BM, int BN, int WGN, int WGM = 2, int NS = 2>
 __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint16_t *lds, int m0, int n0, int k_begin, int KT,
                                                       int wave, int lane, f32x16 (&acc)[BM / (32 * WGM)][BN / (32 * WGN)]) {
   constexpr int BK = 64;
@@ -549,7 +550,7 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
   constexpr int LA = BM / (8 * NW), LB = BN / (8 * NW);   // loads per wave per stage (8 rows each)
   constexpr int STAGE = (BM + BN) * BK;
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "every wave loads whole groups of 8 rows");
-  static_assert(LA + LB <= 16, "the wait counts one stage of loads");
+  static_assert((LA + LB) * (NS - 1) <= 63, "the wait counts the stages' loads");
   const int wm = wave / WGN, wn = wave % WGN;
   const int lrow = lane >> 3;
   const uint16_t *gpa[LA], *gpb[LB];
@@ -586,13 +587,9 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  issue(0, 0);
-  if (KT > 1) {
-    issue(1, 1);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA + LB) : "memory");   // stage 0 has landed (this wave's part)
-  } else {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
+#pragma unroll
+  for (int st = 0; st < NS; ++st) issue(st < KT ? st : KT - 1, st);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * (LA + LB)) : "memory");   // stage 0 has landed (this wave's part)
   __builtin_amdgcn_s_barrier();
 
   const int frow = (lane & 31) * BK, sw = (lane >> 1) & 7, hi = lane >> 5;   // fragment rows start at multiples of 32
@@ -626,8 +623,9 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
   RAI_K64_READ(fa0, fb0, 0, 0);
   // Every stage but the last in one straight-line block (a branch around the multiplies would split the
   // scheduling region and leave copies of the accumulators at the join).
+  int cur = 0;
   for (int st = 0; st + 1 < KT; ++st) {
-    const int cur = st & 1;
+    const int next = NS == 2 ? cur ^ 1 : cur + 1 < NS ? cur + 1 : 0;
     RAI_K64_READ(fa1, fb1, cur, 1);
     RAI_K64_MUL(fa0, fb0);
     RAI_K64_MIX_READS();
@@ -637,12 +635,12 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
     RAI_K64_READ(fa1, fb1, cur, 3);
     RAI_K64_MUL(fa0, fb0);
     RAI_K64_MIX_READS();
-    // stage st+1 has landed (requested a stage ago) and this wave's reads of stage st are done: after the barrier
-    // stage st belongs to the loads of stage st+2 (past the end: the last stage once more, into a buffer nobody reads)
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    // stage st+1 has landed (requested NS-1 stages ago) and this wave's reads of stage st are done: after the barrier
+    // stage st belongs to the loads of stage st+NS (past the end: the last stage once more, into a buffer nobody reads)
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * (LA + LB)) : "memory");
     __builtin_amdgcn_s_barrier();
-    issue(st + 2 < KT ? st + 2 : KT - 1, cur);
-    RAI_K64_READ(fa0, fb0, cur ^ 1, 0);
+    issue(st + NS < KT ? st + NS : KT - 1, cur);
+    RAI_K64_READ(fa0, fb0, next, 0);
     RAI_K64_MUL(fa1, fb1);
 #pragma unroll
     for (int g = 0; g < MT + NT; ++g) {
@@ -652,9 +650,9 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // one LDS read
     }
     __builtin_amdgcn_sched_barrier(0);
+    cur = next;
   }
   {
-    const int cur = (KT - 1) & 1;
     RAI_K64_READ(fa1, fb1, cur, 1);
     RAI_K64_MUL(fa0, fb0);
     RAI_K64_MIX_READS();
@@ -694,13 +692,13 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArg
   const int KT = (k_end - k_begin) / BK;
 
   f32x16 acc[BM / (32 * WGM)][BN / (32 * WGN)];
-  if constexpr (NS == 2) {   // two stages of 64 (the launcher sends K % 64 == 0 and splits of whole stages here)
-    dma_tile_mainloop_k64<BM, BN, WGN, WGM>(a, lds, m0, n0, k_begin, KT / 2, wave, lane, acc);
+  if constexpr (SH == 0) {   // stages of 64 (the launcher sends K % 64 == 0 and splits of whole stages here)
+    dma_tile_mainloop_k64<BM, BN, WGN, WGM, NS>(a, lds, m0, n0, k_begin, KT / 2, wave, lane, acc);
   } else {
     static_assert(WGM == 2, "the K-32 loop is written for two waves along M");
     dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, k_begin, KT, wave, lane, acc);
   }
-  gemm_tile_epilogue<BM, BN, dma_lds_bytes<BM, BN, NS, WGN, WGM>(), WGN, WGM>(a, acc, lds, m0, n0, wave, lane, split, partial);
+  gemm_tile_epilogue<BM, BN, dma_lds_bytes<BM, BN, NS, WGN, WGM, SH>(), WGN, WGM>(a, acc, lds, m0, n0, wave, lane, split, partial);
 }
 
 // The same tile over the rows of one expert (see MoePlan): a block finds its expert and rows in the device-side table,
@@ -1101,7 +1099,7 @@ template <int BM, int BN, int BK, int SH = 0> static int launch_cfg(hipStream_t 
 
 template <int BM, int BN, int NS, int SH, int WGN = 2, int WGM = 2>
 static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
-  constexpr size_t lds = dma_lds_bytes<BM, BN, NS, WGN, WGM>();
+  constexpr size_t lds = dma_lds_bytes<BM, BN, NS, WGN, WGM, SH>();
   static bool attr_set = false;
   if (lds > 64 * 1024 && !attr_set) {
     RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_gemm_bf16_mfma_dma<BM, BN, NS, SH, WGN, WGM>,
@@ -1113,7 +1111,7 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
   int k_per_split = a.K;
   float *partial = nullptr;
   if (splits > 1) {
-    constexpr int KU = NS == 2 ? 64 : 32;   // K tile of the main loop
+    constexpr int KU = SH == 0 ? 64 : 32;   // K tile of the main loop
     const int k_tiles = a.K / KU, per = (k_tiles + splits - 1) / splits;
     splits = (k_tiles + per - 1) / per;
     k_per_split = per * KU;
@@ -1793,7 +1791,42 @@ bool linear_mfma_fuses_norm(int M, int K, int ln_kind) {
   return K <= (M <= 32 ? 8 * 8 * 32 : 8 * 4 * 32);   // one block's K span: no split over blocks
 }
 
-// Split K when the tile count alone cannot fill the GPU and a workspace was provided.
+static bool no_k64() {   // read per call: tests compare both forms in one process
+  const char *e = getenv("RAI_HIP_NO_K64");
+  return e && *e && *e != '0';
+}
+
+// Which of the tiles with K stages of 64 serves a product, and over how many parts of K.  From the kernels' measured times
+// with cold weights: a tile costs us per stage by what it draws from L2 (16, 24, 32 KB), whoever else is on its CU (0.21 for
+// 64 x 64, 0.36 for 128 x 64; 128 x 128 with four stages 0.58 alone on its CU; with two stages 0.62 alone, 0.46 each where two
+// share a CU); 4.2 us are launch and ends, a K split adds 3.2 us (a launch) and 0.4 us per MB of partial sums, and leaves
+// every part four stages.  (us, the 128 x 128 tile with two stages, which served all of these, and what this picks: 333 x
+// 512 x 512 10.4, 6.0; 72 x 2048 x 2048 11.2, 9.0; 1000 x 2048 x 2048 33.9, 15.8; 333 x 1536 x 8960 31.6, 20.2; 72 x 8192 x 2048
+// 22.6, 16; 512 x 8192 x 8960 with two stages as before, 111 against 131 with four and 140 as 64 x 64.)
+enum { kTile128 = 0, kTile128Deep, kTile128x64, kTile64 };
+struct TilePlan { int tile, splits; };
+static TilePlan tile_plan_k64(const LinearArgs &a) {
+  const int stages = a.K / 64;
+  const float part_mb = (float)a.M * a.N * 4e-6f;
+  TilePlan best = {kTile128, 1};
+  float least = 0.f;
+  for (int t = kTile128; t <= kTile64; ++t) {
+    const int64_t tiles = (int64_t)((a.M + (t == kTile64 ? 63 : 127)) / (t == kTile64 ? 64 : 128)) *
+                          ((a.N + (t >= kTile128x64 ? 63 : 127)) / (t >= kTile128x64 ? 64 : 128));
+    for (int s = 1; s <= 12; ++s) {
+      if (s > 1 && (stages / s < 4 || !a.splitk_ws || (size_t)s * a.M * a.N * sizeof(float) > a.splitk_ws_bytes)) break;
+      const int64_t per_cu = (tiles * s + kNumCU - 1) / kNumCU;
+      float stage = per_cu * (t == kTile64 ? 0.21f : t == kTile128x64 ? 0.36f : 0.58f);
+      if (t == kTile128) stage = per_cu == 1 ? 0.62f : 0.46f * per_cu + (per_cu % 2 ? 0.16f : 0.f);
+      const float cost = 4.2f + (t <= kTile128Deep ? 0.8f : 0.f) + stage * ((stages + s - 1) / s) + (s > 1 ? 3.2f + 0.4f * s * part_mb : 0.f);
+      if ((t == kTile128 && s == 1) || cost < least) { least = cost; best = {t, s}; }
+    }
+  }
+  return best;
+}
+
+// Split K when the tile count alone cannot fill the GPU and a workspace was provided (tiles of 32 of K, or a number of
+// splits that the caller asked for).
 static int tile_splits(const LinearArgs &a) {
   const int tiles = ((a.M + 127) / 128) * ((a.N + 127) / 128);
   int splits = 1;
@@ -1827,6 +1860,13 @@ static int tile_splits(const LinearArgs &a) {
   return splits;
 }
 
+// 256 x 256 tiles (or what stands in for them) once these cover a good half of the CUs, see launch_linear_bf16_mfma.
+static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 256) * ((a.N + 255) / 256)) >= 17 * kNumCU; }
+static TilePlan tile_plan(const LinearArgs &a) {
+  if (a.K % 64 || no_k64() || a.force_splits > 0 || has_huge_tiles(a)) return {kTile128, tile_splits(a)};
+  return tile_plan_k64(a);
+}
+
 template <int BM, int BN, int WGN>
 static int launch_grouped_cfg(hipStream_t st, const LinearArgs &a, int64_t w_stride, const MoePlan &plan) {
   constexpr size_t lds = dma_lds_bytes<BM, BN, 2, WGN>();
@@ -1857,12 +1897,14 @@ bool linear_fuses_post_norm(const LinearArgs &a) {
   // (RAI_HIP_NO_POST_NORM: run the norm as its own launch, for comparison)
   const char *off = getenv("RAI_HIP_NO_POST_NORM");   // read per call: the test switches it within one process
   if (off && *off) return false;
-  return a.M > 64 && post_norm_fits(a) && tile_splits(a) > 1;
+  return a.M > 64 && post_norm_fits(a) && tile_plan(a).splits > 1;
 }
 
-static bool no_k64() {   // read per call: tests compare both forms in one process
-  const char *e = getenv("RAI_HIP_NO_K64");
-  return e && *e && *e != '0';
+static int launch_tile_k64(hipStream_t st, const LinearArgs &a, TilePlan tile) {
+  if (tile.tile == kTile64) return launch_cfg_dma<64, 64, 3, 0>(st, a, tile.splits);
+  if (tile.tile == kTile128x64) return launch_cfg_dma<128, 64, 3, 0>(st, a, tile.splits);
+  if (tile.tile == kTile128Deep) return launch_cfg_dma<128, 128, 4, 0>(st, a, tile.splits);
+  return launch_cfg_dma<128, 128, 2, 0>(st, a, tile.splits);
 }
 
 int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
@@ -1880,6 +1922,13 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
               RAI_ERR_BAD_STRIDE, "linear mfma: operands must be 16-byte aligned with row strides multiple of 8");
   const bool no_skinny = getenv("RAI_HIP_NO_MFMA_SKINNY") != nullptr;
   const bool no_stream = getenv("RAI_HIP_NO_MFMA_STREAM") != nullptr;
+  // A row-major W and 9 to 64 rows: the streaming kernel reads 512-byte pieces of W's rows, at 2 to 3 TB/s; tiles with all of
+  // their loads in flight do better once there are enough of them, and split K by themselves (us, stream, tiles: 16 x 512 x
+  // 8960 11.4, 5.9; 16 x 8192 x 8960 46, 29; 64 x 8192 x 8960 78, 37; 64 x 2048 x 2048 10.4, 8.6; 16 x 8192 x 2048 16.0, 13.9; but
+  // 16 x 2048 x 2048 7.3, 8.0, 48 x 512 x 2048 5.2, 6.0, 16 x 8192 x 512 10.3, 12.1).
+  if (a.M > 8 && a.M <= 64 && !a.Wfrag && a.ln_kind < 0 && !a.f32_out && a.force_splits <= 0 && a.K % 64 == 0 && !no_k64() &&
+      !no_skinny && !no_stream && (a.N >= 4096 || (a.N >= 2048 && a.splitk_ws && a.K >= (a.M <= 16 ? 4096 : 1536))))
+    return launch_tile_k64(st, a, tile_plan_k64(a));
   if (a.M <= 64 && !no_skinny && !no_stream && (!a.f32_out || a.Wfrag)) {
     int splits = 1;
     if (a.M <= 16 && mfma_stream_fits<1, 8>(a, &splits)) return launch_mfma_stream<1, 8>(st, a, splits);
@@ -1895,7 +1944,8 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
     return launch_mfma_skinny<4>(st, a);
   }
   const int tiles = ((a.M + 127) / 128) * ((a.N + 127) / 128);
-  const int splits = tile_splits(a);
+  const TilePlan tile = tile_plan(a);
+  const int splits = tile.splits;
   // Tile choice.  The LDS-DMA kernels stream K tiles straight into LDS; the 256x128 tile halves the
   // L2 -> LDS traffic per flop for one operand and is used once there are enough tiles of that size
   // to give every CU two; smaller products keep the 128x128 tile (three blocks per CU).
@@ -1929,7 +1979,6 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
       return bk == 64 ? launch_streamk<2>(st, a, plan) : launch_streamk<4>(st, a, plan);
     }
   }
-  const int big_tiles = ((a.M + 255) / 256) * ((a.N + 127) / 128);
   const int huge_tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256);
   // 256x256 in its eight-wave form (one block per CU, 4 LDS stages, two waves per SIMD) once its tiles cover a good
   // half of the CUs: the tile with the most flops per byte drawn from L2, which is what bounds these kernels.
@@ -1937,7 +1986,7 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
   // 834, 4096 x 10240 x 2560 896 against 789, 4096 x 2560 x 10240 (160 tiles) 837 against 650, 512 x 17920 x 2560
   // (140 tiles) 689 against 621; with 128 tiles or fewer the smaller tiles win (4096 x 2048 x 2048: 618 against 760).
   // The four-wave 256x256 form is 3-9 % behind the eight-wave one everywhere.
-  if (splits == 1 && 32 * huge_tiles >= 17 * kNumCU) {
+  if (splits == 1 && has_huge_tiles(a)) {
     // K tiles of 64 (whole 128-byte lines per request) where K allows; RAI_HIP_NO_K64 keeps the tiles of 32
     const bool k64 = a.K % 64 == 0 && !no_k64();
     StreamKPlan plan;
@@ -1961,10 +2010,9 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
       return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, splits);
     return k64 ? launch_cfg_dma<256, 256, 2, 0, 4>(st, a, splits) : launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
   }
-  if (splits == 1 && big_tiles >= 2 * kNumCU) return launch_cfg_dma<256, 128, 3, 2>(st, a, splits);
   // 128 x 128 with two stages of K 64 (two blocks per CU) where K allows: 12-22 % over three stages of 32 on the
-  // prefill shapes with cold weights (512 x 10240 x 2560: 66 -> 55 us, 2048^3: 33 -> 26 us)
-  if (a.K % 64 == 0 && !no_k64()) return launch_cfg_dma<128, 128, 2, 0, 2>(st, a, splits);
+  // prefill shapes with cold weights (512 x 10240 x 2560: 66 -> 55 us)
+  if (a.K % 64 == 0 && !no_k64()) return launch_tile_k64(st, a, tile);
   return launch_cfg_dma<128, 128, 3, 2>(st, a, splits);
 }
 

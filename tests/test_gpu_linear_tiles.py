@@ -1,0 +1,52 @@
+"""bf16 Linears of more than eight rows: every tile with K stages of 64 (64 x 64, 128 x 64, 128 x 128 with two and four stages),
+one to as many stages as it keeps in flight and one more, ragged edges, K in parts, gated pairs."""
+import numpy as np
+import pytest
+
+from tests.util import down, rand, up
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def R(hip):
+    from rai_amd import ops
+
+    return ops
+
+
+def spread(x, w):
+    """K + 20 roundings of the absolute sum: any order of K f32 additions, of the parts of K and of the bias."""
+    return (x.shape[1] + 20) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T + 1)
+
+
+SIZES = [(65, 64, 8), (65, 128, 65), (97, 192, 1031), (129, 256, 257), (333, 320, 520), (72, 1536, 512), (100, 2048, 2050), (333, 2048, 72),
+         (9, 64, 4096), (16, 192, 4104), (64, 1536, 2048), (40, 2048, 4097), (15, 4096, 2056), (64, 576, 9000),
+         (1000, 512, 2048), (530, 1088, 1500), (333, 1088, 8968), (130, 2560, 8200), (600, 1152, 5000)]
+
+
+@pytest.mark.parametrize("m,k,n", SIZES)
+def test_tiles(R, m, k, n):
+    g = np.random.Generator(np.random.PCG64(m * 1000 + k))
+    x, w = rand(g, (m, k), "bf16"), rand(g, (n, k), "bf16", k ** -0.5)
+    b, r = rand(g, (n,), "bf16"), rand(g, (m, n), "bf16")
+    want, tol = x.astype(np.float64) @ w.astype(np.float64).T, spread(x, w)
+    got = down(R.linear(up(x, "bf16"), up(w, "bf16"))).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + tol)
+    z = want + b
+    full = z / (1 + np.exp(-z)) + r   # silu's slope stays below 1.1, its own error below 2^-18 of it
+    got = down(R.linear(up(x, "bf16"), up(w, "bf16"), up(b, "bf16"), "silu", up(r, "bf16"))).astype(np.float64)
+    assert np.all(np.abs(got - full) <= 2.0 ** -8 * np.abs(full) + 2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 256, 136), (300, 1536, 520), (20, 1536, 4104), (256, 2048, 2048)])
+def test_tiles_gated(R, m, k, n):
+    """act(gate) * up with gate, act(gate) and up each rounded to bf16: three roundings, and the sums' own error through a
+    product of factors below 8 in size."""
+    g = np.random.Generator(np.random.PCG64(m + n))
+    x, w = rand(g, (m, k), "bf16"), rand(g, (n, k), "bf16", k ** -0.5)
+    z = x.astype(np.float64) @ w.astype(np.float64).T
+    gate, upv = z[:, 0::2], z[:, 1::2]
+    want = gate / (1 + np.exp(-gate)) * upv
+    got = down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), act="silu", glu=True)).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 4 * 2.0 ** -8 * (np.abs(gate) + 1) * (np.abs(upv) + 1))
