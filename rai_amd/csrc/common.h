@@ -8,6 +8,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 
 #include "rai_hip.h"
 
@@ -62,9 +63,15 @@ int arg_static_scratch_init(int dev);
 // [r * splits + s] (a share of NaNs only leaves a NaN).  The caller merges the shares (reduce.hip).
 int launch_argmax_partials(hipStream_t st, int dtype, const void *in, int64_t rows, int64_t n, int splits, float *pval,
                            uint32_t *pidx);
-// Workspace that lives as long as the device context (grown on demand, never
-// shrinks); used by kernels that need partial results.  Stream-ordered reuse.
-int workspace(int dev, size_t bytes, void **out);
+// The device's scratch block, which lives as long as the device context (grown on demand, never shrinks), for kernels
+// that need partial results.  A call keeps its hold on the block until it has enqueued the last kernel or copy that uses
+// it: another thread's work then comes behind it on the device's one stream, and nobody replaces the block between the
+// call's launches.  (Without the hold two threads' kernels could be enqueued in turn and read each other's partial sums.)
+// A thread holds it once at a time.
+struct WorkspaceHold {
+  std::unique_lock<std::mutex> lock;
+};
+int workspace(int dev, size_t bytes, void **out, WorkspaceHold *hold);
 // Device counter bumped by gather kernels on an out-of-range index.
 unsigned long long *index_error_counter(int dev);
 int launch_check(const char *what);

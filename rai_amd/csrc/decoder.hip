@@ -1490,7 +1490,8 @@ int rai_hip_decoder_context_len(rai_hip_decoder *d, int32_t *len) {
 
 static int widen_to_host(rai_hip_decoder *d, hipStream_t st, const char *src, int64_t n, float *dst_host) {
   void *ws = nullptr;
-  RAI_TRY(workspace(d->dev, (size_t)n * sizeof(float), &ws));
+  WorkspaceHold hold;
+  RAI_TRY(workspace(d->dev, (size_t)n * sizeof(float), &ws, &hold));
   if (d->cfg.dtype == RAI_BF16)
     hipLaunchKernelGGL((k_to_f32<bf16_raw>), dim3(grid1d(n)), dim3(256), 0, st, (float *)ws, (const bf16_raw *)src, n);
   else
@@ -1612,8 +1613,9 @@ int rai_hip_decoder_forward(rai_hip_decoder *d, const uint32_t *ids_host, int32_
   if (logits_host) {
     // widen on device, then one synchronous copy
     void *ws = nullptr;
+    WorkspaceHold hold;
     const int64_t n = (int64_t)batch * d->V;
-    RAI_TRY(workspace(d->dev, (size_t)n * sizeof(float), &ws));
+    RAI_TRY(workspace(d->dev, (size_t)n * sizeof(float), &ws, &hold));
     if (d->cfg.dtype == RAI_BF16)
       hipLaunchKernelGGL((k_to_f32<bf16_raw>), dim3(grid1d(n)), dim3(256), 0, st, (float *)ws, (const bf16_raw *)d->logits, n);
     else

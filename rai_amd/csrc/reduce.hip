@@ -660,7 +660,8 @@ static int arg_impl(int dev, const rai_hip_tensor *in, int32_t dim, int32_t keep
       return launch_check("arg_row");
     }
     RAI_REQUIRE(!no_alloc, RAI_ERR_HIP, "argmax_static: scratch address of device %d unknown (rai_hip_init failed?)", dev);
-    RAI_TRY(workspace(dev, nparts * (sizeof(double) + sizeof(uint32_t)) + 64, &ws));
+    WorkspaceHold hold;
+    RAI_TRY(workspace(dev, nparts * (sizeof(double) + sizeof(uint32_t)) + 64, &ws, &hold));
     double *pd = (double *)ws;
     float *pf = (float *)ws;
     uint32_t *pi = (uint32_t *)((char *)ws + nparts * sizeof(double));

@@ -47,6 +47,7 @@ struct DeviceCtx {
   char *slab = nullptr;
   size_t slab_left = 0;
   std::unordered_set<void *> carved;
+  std::mutex ws_mu;                    // held by the call that uses the scratch block, see WorkspaceHold
   void *ws = nullptr;
   size_t ws_bytes = 0;
   unsigned long long *index_errors = nullptr;
@@ -157,9 +158,10 @@ unsigned long long *index_error_counter(int dev) {
   return c ? c->index_errors : nullptr;
 }
 
-int workspace(int dev, size_t bytes, void **out) {
+int workspace(int dev, size_t bytes, void **out, WorkspaceHold *hold) {
   DeviceCtx *c = ctx(dev);
   if (!c) return RAI_ERR_HIP;
+  hold->lock = std::unique_lock<std::mutex>(c->ws_mu);
   std::lock_guard<std::mutex> lk(c->mu);
   if (bytes > c->ws_bytes) {
     // The old block may still be read by enqueued kernels: drain first.

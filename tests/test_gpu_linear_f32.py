@@ -1,5 +1,7 @@
 """f32 Linears at the edges of their kernels' tiles: rows around 4, 32 and 64, K around the 32-wide tiles and the cut over
 waves and blocks, odd N, rows that are not 16-byte aligned."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -58,3 +60,28 @@ def test_f32_linear_keeps_small_and_infinite_values(R, m):
     w[7, 299], w[9, 0] = np.inf, np.nan
     got = down(R.linear(up(x, "f32"), up(w, "f32")))
     assert np.all(np.isinf(got[:, 7])) and np.all(np.isnan(got[:, 9])) and np.all(np.delete(got, [7, 9], 1) == 300)
+
+
+def test_linears_of_several_threads_share_the_scratch(R):
+    """Products that cut K leave partial sums in the device's one scratch block between two kernels: threads that launch
+    them at the same time, with sizes that make the block grow on the way, get the bits that each gets alone."""
+    sizes = [(48, 4096, 512, "f32"), (96, 4096, 1024, "f32"), (128, 8192, 512, "bf16"), (200, 8192, 2560, "f32")]
+
+    def operands(i):
+        m, k, n, dt = sizes[i]
+        g = np.random.Generator(np.random.PCG64(91 + i))
+        return up(rand(g, (m, k), dt), dt), up(rand(g, (n, k), dt, k ** -0.5), dt)
+
+    data, got = [operands(i) for i in range(len(sizes))], [[] for _ in sizes]
+
+    def work(i):
+        got[i] = [R.linear(*data[i]) for _ in range(25)]
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sizes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i, outs in enumerate(got):
+        alone = down(R.linear(*data[i]))
+        assert len(outs) == 25 and all(np.array_equal(down(y), alone) for y in outs), sizes[i]
