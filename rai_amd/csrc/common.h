@@ -72,6 +72,9 @@ struct WorkspaceHold {
   std::unique_lock<std::mutex> lock;
 };
 int workspace(int dev, size_t bytes, void **out, WorkspaceHold *hold);
+// The same for work that can do with less: up to `bytes` of the block, as many as it has where it cannot grow.  Returns
+// how many.
+size_t workspace_if_room(int dev, size_t bytes, void **out, WorkspaceHold *hold);
 // Device counter bumped by gather kernels on an out-of-range index.
 unsigned long long *index_error_counter(int dev);
 int launch_check(const char *what);

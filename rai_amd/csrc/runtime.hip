@@ -1,6 +1,7 @@
 // Device context, pooled ref-counted allocations, copies and timers.
 // Replaces the storage/device half of rai's candle backend:
 // rai-core/src/backend/candle.rs:18-68 (TensorLike), :133-195 (device cache).
+#include <cstdlib>
 #include <map>
 #include <mutex>
 #include <unordered_map>
@@ -158,26 +159,65 @@ unsigned long long *index_error_counter(int dev) {
   return c ? c->index_errors : nullptr;
 }
 
+// RAI_HIP_WORKSPACE_LIMIT (bytes, read per call): a scratch block as small as where memory has run out.
+static size_t workspace_limit() {
+  const char *e = getenv("RAI_HIP_WORKSPACE_LIMIT");
+  return e && *e ? (size_t)strtoull(e, nullptr, 10) : ~size_t(0);
+}
+static hipError_t workspace_malloc(void **p, size_t bytes) {
+  return bytes > workspace_limit() ? hipErrorOutOfMemory : hipMalloc(p, bytes);
+}
+
+// A larger block for the context, at least twice the old one's size while that is modest (a program whose products grow
+// drains the stream a few times, not once per size).
+static int workspace_grow(DeviceCtx *c, size_t bytes, bool keep_old) {
+  RAI_HIP_TRY(hipSetDevice(c->dev));
+  const size_t exact = size_class(bytes < (size_t(8) << 20) ? (size_t(8) << 20) : bytes);
+  const size_t twice = c->ws_bytes < (size_t(128) << 20) ? 2 * c->ws_bytes : 0;
+  void *fresh = nullptr;
+  size_t got = 0;
+  for (size_t want : {twice, exact})
+    if (!fresh && want >= exact && workspace_malloc(&fresh, want) == hipSuccess) got = want;
+    else if (!fresh) (void)hipGetLastError();
+  if (!fresh && keep_old) return RAI_ERR_OOM;
+  // enqueued kernels may still read the old block: drain first
+  RAI_HIP_TRY(hipStreamSynchronize(c->stream));
+  if (c->ws) RAI_HIP_TRY(hipFree(c->ws));
+  c->ws = fresh;
+  c->ws_bytes = got;
+  if (!fresh) {
+    const hipError_t e = workspace_malloc(&c->ws, exact);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      c->ws = nullptr;
+      return fail(RAI_ERR_OOM, "workspace of %zu bytes: %s", exact, hipGetErrorString(e));
+    }
+    c->ws_bytes = exact;
+  }
+  c->n_mallocs++;
+  return RAI_OK;
+}
+
 int workspace(int dev, size_t bytes, void **out, WorkspaceHold *hold) {
   DeviceCtx *c = ctx(dev);
   if (!c) return RAI_ERR_HIP;
   hold->lock = std::unique_lock<std::mutex>(c->ws_mu);
   std::lock_guard<std::mutex> lk(c->mu);
-  if (bytes > c->ws_bytes) {
-    // The old block may still be read by enqueued kernels: drain first.
-    RAI_HIP_TRY(hipSetDevice(dev));
-    RAI_HIP_TRY(hipStreamSynchronize(c->stream));
-    if (c->ws) RAI_HIP_TRY(hipFree(c->ws));
-    c->ws = nullptr;
-    c->ws_bytes = 0;
-    size_t want = size_class(bytes < (size_t(8) << 20) ? (size_t(8) << 20) : bytes);
-    hipError_t e = hipMalloc(&c->ws, want);
-    if (e != hipSuccess) return fail(RAI_ERR_OOM, "workspace of %zu bytes: %s", want, hipGetErrorString(e));
-    c->ws_bytes = want;
-    c->n_mallocs++;
-  }
+  if (bytes > c->ws_bytes) RAI_TRY(workspace_grow(c, bytes, false));
   *out = c->ws;
   return RAI_OK;
+}
+
+size_t workspace_if_room(int dev, size_t bytes, void **out, WorkspaceHold *hold) {
+  DeviceCtx *c = ctx(dev);
+  *out = nullptr;
+  if (!c) return 0;
+  hold->lock = std::unique_lock<std::mutex>(c->ws_mu);
+  std::lock_guard<std::mutex> lk(c->mu);
+  if (bytes > c->ws_bytes) (void)workspace_grow(c, bytes, true);
+  const size_t limit = workspace_limit(), room = c->ws_bytes < limit ? c->ws_bytes : limit;
+  if (room) *out = c->ws;
+  return room < bytes ? room : bytes;
 }
 
 int launch_check(const char *what) {

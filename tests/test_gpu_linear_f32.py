@@ -62,6 +62,24 @@ def test_f32_linear_keeps_small_and_infinite_values(R, m):
     assert np.all(np.isinf(got[:, 7])) and np.all(np.isnan(got[:, 9])) and np.all(np.delete(got, [7, 9], 1) == 300)
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("planes", [0, 1, 3])
+def test_linear_runs_where_the_scratch_cannot_grow(R, monkeypatch, dt, planes):
+    """A product that would cut K needs no memory of its own to run: without room for all its partial sums it runs in
+    fewer parts or in one."""
+    g = np.random.Generator(np.random.PCG64(78))
+    m, k, n = 96, 4096, 520
+    x, w = rand(g, (m, k), dt), rand(g, (n, k), dt, 0.02)
+    xd, wd = up(x, dt), up(w, dt)
+    first = down(R.linear(xd, wd))
+    monkeypatch.setenv("RAI_HIP_WORKSPACE_LIMIT", str(planes * m * n * 4))
+    got = down(R.linear(xd, wd)).astype(np.float64)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.all(np.abs(got - want) <= bound(x, w, 0.0) + (2.0 ** -8 * np.abs(want) if dt == "bf16" else 0.0))
+    monkeypatch.delenv("RAI_HIP_WORKSPACE_LIMIT")
+    assert np.array_equal(down(R.linear(xd, wd)), first)
+
+
 def test_linears_of_several_threads_share_the_scratch(R):
     """Products that cut K leave partial sums in the device's one scratch block between two kernels: threads that launch
     them at the same time, with sizes that make the block grow on the way, get the bits that each gets alone."""
