@@ -85,7 +85,11 @@ __device__ __forceinline__ void f32_finish4(const LinearArgs &a, int m, int n, f
 // units: 2700 us); 1024 rows 427 us (690); 128 x 12800 x 2560 with K cut 82 us (804); 24 x 2560 x 10240 30 us (162, and 43
 // with tiles of 64 x 64).  Tiles of 128 x 128 reach 131 TFLOP/s at 4096 rows and lose more than that to the partial round
 // at 1024 (623 us).
-//   VEC: rows 16-byte aligned and K a multiple of four (16-byte loads); otherwise element by element.
+//   Operands come in pieces of 16 bytes.  kWhole: rows 16-byte aligned and K a multiple of four.  kRagged: rows that start
+// anywhere and any K from four on: the piece that crosses the end of K is read four elements before the end and shifted, so
+// no load stands behind a branch (1024 x 8190 x 10240 in rows of 8192 1310 us, in rows of 8190 1340; element by element with
+// the ends behind branches 2318 and 2077).  kTiny: element by element.
+enum { kTiny, kRagged, kWhole };
 template <int BM, int BN>
 struct F32Tile {
   static constexpr int BK = 32, PITCH = 36;
@@ -93,20 +97,31 @@ struct F32Tile {
   static constexpr int PA = BM / 32, PB = BN / 32;  // 16-byte loads a thread makes per K tile
 };
 
-// Four consecutive k of a row.  VEC: k is a multiple of four below k_end, or clamped by the caller; otherwise element by
-// element, zeros past k_end.
-template <bool VEC>
+// Four consecutive k of a row, from k on; kTiny: those below k_end and zeros.
+template <int LOADS>
 __device__ __forceinline__ f32x4 f32_load_k(const float *row, int k, int k_end) {
-  if constexpr (VEC) return *reinterpret_cast<const f32x4 *>(row + k);
   f32x4 v;
+  if constexpr (LOADS == kTiny) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) v[j] = k + j < k_end ? row[k + j] : 0.f;
+    for (int j = 0; j < 4; ++j) v[j] = k + j < k_end ? row[k + j] : 0.f;
+  } else if constexpr (LOADS == kRagged) {
+    __builtin_memcpy(&v, row + k, 16);
+  } else {
+    v = *reinterpret_cast<const f32x4 *>(row + k);
+  }
+  return v;
+}
+// A piece that was read `past` elements ahead of its place because K ends: what lies past the end is zero.
+__device__ __forceinline__ f32x4 f32_end_of_k(f32x4 v, int past) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (past > i) v = f32x4{v[1], v[2], v[3], 0.f};
   return v;
 }
 
 // Products over [k_begin, k_end) of the tile at (m0, n0); `finish(m, n, v)` receives them, columns n .. n + 3 (n < N) of
 // row m at a time.
-template <int BM, int BN, bool VEC, class Finish>
+template <int BM, int BN, int LOADS, class Finish>
 __device__ __forceinline__ void linear_f32_tile(const LinearArgs &a, int m0, int n0, int k_begin, int k_end, float *lds, Finish finish) {
   using T = F32Tile<BM, BN>;
   constexpr int BK = T::BK, PITCH = T::PITCH;
@@ -123,18 +138,26 @@ __device__ __forceinline__ void linear_f32_tile(const LinearArgs &a, int m0, int
   for (int p = 0; p < T::PB; ++p) wrow[p] = W + (int64_t)min(n0 + lrow + 32 * p, a.N - 1) * a.ldw;
   f32x4 ra[T::PA], rb[T::PB];
   auto fetch = [&](int k0) {
-    const int k = VEC ? min(k0 + lk, k_end - 4) : k0 + lk;
+    const int k = LOADS == kTiny ? k0 + lk : min(k0 + lk, k_end - 4);
 #pragma unroll
-    for (int p = 0; p < T::PA; ++p) ra[p] = f32_load_k<VEC>(arow[p], k, k_end);
+    for (int p = 0; p < T::PA; ++p) ra[p] = f32_load_k<LOADS>(arow[p], k, k_end);
 #pragma unroll
-    for (int p = 0; p < T::PB; ++p) rb[p] = f32_load_k<VEC>(wrow[p], k, k_end);
+    for (int p = 0; p < T::PB; ++p) rb[p] = f32_load_k<LOADS>(wrow[p], k, k_end);
   };
   auto park = [&](float *st, int k0) {
-    if (VEC && k0 + BK > k_end && k0 + lk >= k_end) {   // both operands are zero past the end of K
+    // both operands are zero past the end of K
+    if (LOADS == kWhole && k0 + BK > k_end && k0 + lk >= k_end) {
 #pragma unroll
       for (int p = 0; p < T::PA; ++p) ra[p] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int p = 0; p < T::PB; ++p) rb[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (LOADS == kRagged && k0 + BK > k_end) {
+      const int past = k0 + lk - (k_end - 4);
+#pragma unroll
+      for (int p = 0; p < T::PA; ++p) ra[p] = f32_end_of_k(ra[p], past);
+#pragma unroll
+      for (int p = 0; p < T::PB; ++p) rb[p] = f32_end_of_k(rb[p], past);
     }
 #pragma unroll
     for (int p = 0; p < T::PA; ++p) *reinterpret_cast<f32x4 *>(st + (lrow + 32 * p) * PITCH + lk) = ra[p];
@@ -194,7 +217,7 @@ __device__ __forceinline__ void f32_tile_of_block(int block, int tiles_m, int ti
   tn = in / rows;
 }
 
-template <int BM, int BN, bool VEC, bool PARTIAL>
+template <int BM, int BN, int LOADS, bool PARTIAL>
 __global__ void __launch_bounds__(256, 2) k_linear_f32_tile(LinearArgs a, int k_step) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   int tm, tn;
@@ -202,9 +225,9 @@ __global__ void __launch_bounds__(256, 2) k_linear_f32_tile(LinearArgs a, int k_
   if constexpr (PARTIAL) {
     const int k0 = blockIdx.y * k_step, k1 = k0 + k_step < a.K ? k0 + k_step : a.K;
     float *part = (float *)a.splitk_ws + (int64_t)blockIdx.y * a.M * a.N;
-    linear_f32_tile<BM, BN, VEC>(a, tm * BM, tn * BN, k0, k1, lds, [&](int m, int n, f32x4 v) { f32_store_cols(part + (int64_t)m * a.N, n, a.N, v); });
+    linear_f32_tile<BM, BN, LOADS>(a, tm * BM, tn * BN, k0, k1, lds, [&](int m, int n, f32x4 v) { f32_store_cols(part + (int64_t)m * a.N, n, a.N, v); });
   } else {
-    linear_f32_tile<BM, BN, VEC>(a, tm * BM, tn * BN, 0, a.K, lds, [&](int m, int n, f32x4 v) { f32_finish4(a, m, n, v); });
+    linear_f32_tile<BM, BN, LOADS>(a, tm * BM, tn * BN, 0, a.K, lds, [&](int m, int n, f32x4 v) { f32_finish4(a, m, n, v); });
   }
 }
 
@@ -223,7 +246,7 @@ __global__ void __launch_bounds__(256) k_linear_f32_sum(LinearArgs a, int splits
 }
 
 // The 64 x 64 tile over the rows of one expert (see MoePlan): blockIdx.x = column tile, blockIdx.y = row tile.
-template <bool VEC>
+template <int LOADS>
 __global__ void __launch_bounds__(256) k_linear_f32_grouped(LinearArgs a, int64_t w_stride, const int4 *tiles, const int *n_tiles) {
   __shared__ __attribute__((aligned(16))) float lds[2 * F32Tile<64, 64>::STAGE];
   if ((int)blockIdx.y >= *n_tiles) return;
@@ -232,7 +255,7 @@ __global__ void __launch_bounds__(256) k_linear_f32_grouped(LinearArgs a, int64_
   a.W = (const float *)a.W + (int64_t)t.x * w_stride;
   a.out1 = (float *)a.out1 + (int64_t)t.y * a.ld1;
   a.M = t.z;
-  linear_f32_tile<64, 64, VEC>(a, 0, blockIdx.x * 64, 0, a.K, lds, [&](int m, int n, f32x4 v) { f32_finish4(a, m, n, v); });
+  linear_f32_tile<64, 64, LOADS>(a, 0, blockIdx.x * 64, 0, a.K, lds, [&](int m, int n, f32x4 v) { f32_finish4(a, m, n, v); });
 }
 
 // ------------------------------------------------------------------ few rows
@@ -316,17 +339,17 @@ static bool rows_aligned(const LinearArgs &a) {
   return a.K % 4 == 0 && a.lda % 4 == 0 && a.ldw % 4 == 0 && (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.W % 16 == 0;
 }
 
-template <int BM, int BN, bool VEC, bool PARTIAL>
+template <int BM, int BN, int LOADS, bool PARTIAL>
 static int launch_tile(hipStream_t st, const LinearArgs &a, int splits, int k_step) {
   constexpr size_t lds = 2 * F32Tile<BM, BN>::STAGE * sizeof(float);
   static bool attr_set = false;
   if (lds > 64 * 1024 && !attr_set) {
-    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_linear_f32_tile<BM, BN, VEC, PARTIAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_linear_f32_tile<BM, BN, LOADS, PARTIAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_set = true;
   }
   const int64_t tiles = (int64_t)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
   RAI_REQUIRE(tiles < (1LL << 31), RAI_ERR_UNSUPPORTED, "linear f32: %d x %d outputs exceed the grid", a.M, a.N);
-  hipLaunchKernelGGL((k_linear_f32_tile<BM, BN, VEC, PARTIAL>), dim3((unsigned)tiles, splits), dim3(256), lds, st, a, k_step);
+  hipLaunchKernelGGL((k_linear_f32_tile<BM, BN, LOADS, PARTIAL>), dim3((unsigned)tiles, splits), dim3(256), lds, st, a, k_step);
   return launch_check("linear_f32_tile");
 }
 
@@ -369,22 +392,25 @@ int launch_linear_f32(hipStream_t st, const LinearArgs &a) {
     int k_step = (a.K + splits - 1) / splits;
     k_step = (k_step + 31) / 32 * 32;
     splits = (a.K + k_step - 1) / k_step;
-    if (vec && a.M <= 32) RAI_TRY((launch_tile<32, 128, true, true>(st, a, splits, k_step)));
-    else RAI_TRY((vec ? launch_tile<64, 64, true, true>(st, a, splits, k_step) : launch_tile<64, 64, false, true>(st, a, splits, k_step)));
+    if (vec && a.M <= 32) RAI_TRY((launch_tile<32, 128, kWhole, true>(st, a, splits, k_step)));
+    else RAI_TRY((vec ? launch_tile<64, 64, kWhole, true>(st, a, splits, k_step) : launch_tile<64, 64, kRagged, true>(st, a, splits, k_step)));
     const int64_t blocks = ((int64_t)a.M * ((a.N + 3) / 4) + 255) / 256;
     hipLaunchKernelGGL(k_linear_f32_sum, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, st, a, splits);
     return launch_check("linear_f32_sum");
   }
-  if (vec && a.M <= 32) return launch_tile<32, 128, true, false>(st, a, 1, 0);
-  return vec ? launch_tile<64, 64, true, false>(st, a, 1, 0) : launch_tile<64, 64, false, false>(st, a, 1, 0);
+  if (vec && a.M <= 32) return launch_tile<32, 128, kWhole, false>(st, a, 1, 0);
+  if (vec) return launch_tile<64, 64, kWhole, false>(st, a, 1, 0);
+  return a.K >= 4 ? launch_tile<64, 64, kRagged, false>(st, a, 1, 0) : launch_tile<64, 64, kTiny, false>(st, a, 1, 0);
 }
 
 int launch_linear_f32_grouped(hipStream_t st, const LinearArgs &a, int64_t w_stride, const MoePlan &plan) {
   const dim3 grid((a.N + 63) / 64, plan.cap_tiles);
   if (rows_aligned(a) && w_stride % 4 == 0)
-    hipLaunchKernelGGL(k_linear_f32_grouped<true>, grid, dim3(256), 0, st, a, w_stride, plan.tiles, plan.n_tiles);
+    hipLaunchKernelGGL(k_linear_f32_grouped<kWhole>, grid, dim3(256), 0, st, a, w_stride, plan.tiles, plan.n_tiles);
+  else if (a.K >= 4)
+    hipLaunchKernelGGL(k_linear_f32_grouped<kRagged>, grid, dim3(256), 0, st, a, w_stride, plan.tiles, plan.n_tiles);
   else
-    hipLaunchKernelGGL(k_linear_f32_grouped<false>, grid, dim3(256), 0, st, a, w_stride, plan.tiles, plan.n_tiles);
+    hipLaunchKernelGGL(k_linear_f32_grouped<kTiny>, grid, dim3(256), 0, st, a, w_stride, plan.tiles, plan.n_tiles);
   return launch_check("linear_f32_grouped");
 }
 

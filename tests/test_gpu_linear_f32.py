@@ -48,6 +48,20 @@ def test_f32_linear_of_unaligned_rows(R, m):
     assert np.all(np.abs(got - xs.astype(np.float64) @ ws.astype(np.float64).T) <= bound(xs, ws, 0.0))
 
 
+@pytest.mark.parametrize("m,n", [(2, 9), (70, 66), (64, 1600)])
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 6, 7, 30, 31, 35, 66, 511, 1026])
+def test_f32_linear_where_k_ends_inside_a_piece(R, m, n, k):
+    """K of no multiple of four, rows packed, on 16-byte boundaries and off them; what stands behind a row's end, and the
+    first elements of the next row, take no part."""
+    g = np.random.Generator(np.random.PCG64(13))
+    for first, width in ((0, k), (0, (k + 3) // 4 * 4 + 4), (1, k + 3)):
+        x, w = rand(g, (m, width), "f32"), rand(g, (n, width), "f32", 0.05)
+        x[:, :first] = w[:, :first] = x[:, first + k:] = w[:, first + k:] = np.nan
+        got = down(R.linear(up(x, "f32").narrow(1, first, k), up(w, "f32").narrow(1, first, k))).astype(np.float64)
+        xs, ws = x[:, first:first + k], w[:, first:first + k]
+        assert np.all(np.abs(got - xs.astype(np.float64) @ ws.astype(np.float64).T) <= bound(xs, ws, 0.0)), (first, width)
+
+
 @pytest.mark.parametrize("m", [1, 20, 100])
 def test_f32_linear_keeps_small_and_infinite_values(R, m):
     """Denormal products are kept, and infinities and NaNs reach only the outputs that depend on them (K is no multiple
