@@ -125,9 +125,9 @@ int launch_linear_dual_row(hipStream_t st, int dev, const void *x1, int K1, cons
 int launch_gemv_group(hipStream_t st, GemvGroupArgs g);
 
 // The same NT contraction in f32 (gemm_f32.hip), and the scratch (LinearArgs::splitk_ws) with which it cuts K over blocks
-// where M x N alone leaves CUs idle; with less it cuts K less.
+// where M x N alone leaves CUs idle, of `room` bytes at most; with less it cuts K less.
 int launch_linear_f32(hipStream_t st, const LinearArgs &a);
-size_t linear_f32_workspace_bytes(int M, int N, int K);
+size_t linear_f32_workspace_bytes(const LinearArgs &a, size_t room);
 bool linear_mfma_fuses_norm(int M, int K, int ln_kind);
 
 // out[z] = A[z] B[z] (rai_hip_matmul), out contiguous.

@@ -808,15 +808,13 @@ template <typename T> static void launch_transpose_2d(hipStream_t st, T *dst, co
     hipLaunchKernelGGL(k_transpose_2d<T>, grid, dim3(256), 0, st, dst, src, K, N);
 }
 
-// Lends up to `want` bytes (at most 256 MB) of the device's scratch block to a tile GEMM that may split K, which it does
-// less or not at all with what there is; the caller keeps `hold` until the product's last kernel is enqueued.
-static void splitk_workspace(int dev, LinearArgs *la, size_t want, WorkspaceHold *hold) {
-  if (want == 0) return;
+// Lends of the device's scratch block, up to 256 MB, what a tile GEMM that may split K would take; it splits less or not at
+// all with what there is.  The caller keeps `hold` until the product's last kernel is enqueued.
+static void splitk_workspace(int dev, int dtype, LinearArgs *la, WorkspaceHold *hold) {
   const size_t cap = (size_t)256 << 20;
-  la->splitk_ws_bytes = workspace_if_room(dev, want < cap ? want : cap, &la->splitk_ws, hold);
-}
-static size_t splitk_bytes(int dtype, const LinearArgs &la) {
-  return dtype == RAI_F32 ? linear_f32_workspace_bytes(la.M, la.N, la.K) : (size_t)8 * la.M * la.N * sizeof(float);
+  size_t want = dtype == RAI_F32 ? linear_f32_workspace_bytes(*la, cap) : (size_t)8 * la->M * la->N * sizeof(float);
+  if (want > cap) want = cap;
+  if (want) la->splitk_ws_bytes = workspace_if_room(dev, want, &la->splitk_ws, hold);
 }
 
 }  // namespace rai
@@ -885,7 +883,7 @@ int rai_hip_matmul(int dev, const rai_hip_tensor *a, const rai_hip_tensor *b, co
       la.n_split = (int)N;
       if (a->dtype == RAI_BF16 && la.M > 8 && la.K % 32 != 0) goto generic;
       WorkspaceHold hold;
-      if (a->dtype == RAI_F32 || la.M > 8) splitk_workspace(dev, &la, splitk_bytes(a->dtype, la), &hold);
+      if (a->dtype == RAI_F32 || la.M > 8) splitk_workspace(dev, a->dtype, &la, &hold);
       return a->dtype == RAI_BF16 ? launch_linear_bf16(st, la) : launch_linear_f32(st, la);
     }
   }
@@ -1000,7 +998,7 @@ int rai_hip_linear(int dev, const rai_hip_tensor *x, const rai_hip_tensor *w, co
   if (x->dtype == RAI_BF16 && la.M > 8)
     RAI_REQUIRE(K % 32 == 0, RAI_ERR_UNSUPPORTED, "linear: bf16 with M > 8 needs K %% 32 == 0 (K=%lld)", (long long)K);
   WorkspaceHold hold;
-  if (x->dtype == RAI_F32 || la.M > 8) splitk_workspace(dev, &la, splitk_bytes(x->dtype, la), &hold);
+  if (x->dtype == RAI_F32 || la.M > 8) splitk_workspace(dev, x->dtype, &la, &hold);
   return x->dtype == RAI_BF16 ? launch_linear_bf16(st, la) : launch_linear_f32(st, la);
 }
 
@@ -1080,7 +1078,7 @@ int rai_hip_linear_packed(int dev, const rai_hip_tensor *x, const rai_hip_tensor
   WorkspaceHold hold;
   if (la.M > 8) {
     RAI_REQUIRE(K % 32 == 0, RAI_ERR_UNSUPPORTED, "linear_packed: M > 8 needs K %% 32 == 0 (K=%lld)", (long long)K);
-    splitk_workspace(dev, &la, splitk_bytes(RAI_BF16, la), &hold);
+    splitk_workspace(dev, RAI_BF16, &la, &hold);
   }
   return launch_linear_bf16(st, la);
 }

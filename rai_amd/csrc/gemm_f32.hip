@@ -359,46 +359,47 @@ template <int M> static int launch_rows(hipStream_t st, const LinearArgs &a) {
   return launch_check("linear_f32_rows");
 }
 
-// How many pieces of K to compute side by side, by the time the tiles and the summing pass would take: a tile of full K
-// is 0.017 us of a busy CU's time per k, a CU needs three or four blocks to be busy, the sum is a launch and a trip of
-// the partial products to memory and back.
-static int f32_splits(int M, int N, int K) {
+// How many pieces of K to compute side by side with `room` bytes for their products, by the time the tiles and the summing
+// pass would take: a tile of full K is 0.017 us of a busy CU's time per k, a CU needs three or four blocks to be busy, the
+// sum is a launch and a trip of the partial products to memory and back.
+static bool wide_tiles(const LinearArgs &a) { return a.M <= 32 && rows_aligned(a); }   // 32 x 128 instead of 64 x 64
+static int f32_splits(const LinearArgs &a, size_t room) {
   static const double busy[5] = {0, 0.45, 0.75, 0.9, 1.0};   // share of its rate a CU reaches with this many blocks
-  const int64_t tiles = M <= 32 ? (N + 127) / 128 : (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+  const int64_t tiles = wide_tiles(a) ? (a.N + 127) / 128 : (int64_t)((a.M + 63) / 64) * ((a.N + 63) / 64);
+  const size_t plane = (size_t)a.M * a.N * sizeof(float);
   int best = 1;
   double least = 0;
-  for (int s = 1; s <= 16 && (s == 1 || s * 256 <= K); ++s) {
+  for (int s = 1; s <= 16 && (s == 1 || (s * 256 <= a.K && s * plane <= room)); ++s) {
     const int64_t rounds = (tiles * s + kNumCU - 1) / kNumCU;
-    const double us = rounds * 0.017 * K / s / busy[rounds < 4 ? rounds : 4] + (s > 1 ? 3.0 + 4.0 * M * N * 2 * s / 4e6 : 0.0);
+    const double us = rounds * 0.017 * a.K / s / busy[rounds < 4 ? rounds : 4] + (s > 1 ? 3.0 + 2.0 * s * plane / 4e6 : 0.0);
     if (s == 1 || us < least) { least = us; best = s; }
   }
   return best;
 }
+static bool few_rows(const LinearArgs &a) { return a.M <= kFewRows && rows_aligned(a); }
 
-size_t linear_f32_workspace_bytes(int M, int N, int K) {
-  const int s = M <= kFewRows && K % 4 == 0 ? 1 : f32_splits(M, N, K);
-  return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+size_t linear_f32_workspace_bytes(const LinearArgs &a, size_t room) {
+  const int s = few_rows(a) ? 1 : f32_splits(a, room);
+  return s > 1 ? (size_t)s * a.M * a.N * sizeof(float) : 0;
 }
 
 int launch_linear_f32(hipStream_t st, const LinearArgs &a) {
   RAI_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0, RAI_ERR_BAD_SHAPE, "linear: empty problem");
   RAI_REQUIRE(a.ln_kind < 0, RAI_ERR_UNSUPPORTED, "linear f32: no fused norm");
-  const bool vec = rows_aligned(a);
-  if (vec && a.M <= kFewRows) return a.M == 1 ? launch_rows<1>(st, a) : a.M == 2 ? launch_rows<2>(st, a) : launch_rows<4>(st, a);
-  int splits = f32_splits(a.M, a.N, a.K);
-  const size_t plane = (size_t)a.M * a.N * sizeof(float);
-  if ((size_t)splits * plane > a.splitk_ws_bytes) splits = (int)(a.splitk_ws_bytes / plane);   // what the lent scratch holds
-  if (splits > 1 && a.splitk_ws) {
+  if (few_rows(a)) return a.M == 1 ? launch_rows<1>(st, a) : a.M == 2 ? launch_rows<2>(st, a) : launch_rows<4>(st, a);
+  const bool vec = rows_aligned(a), wide = wide_tiles(a);
+  int splits = f32_splits(a, a.splitk_ws ? a.splitk_ws_bytes : 0);
+  if (splits > 1) {
     int k_step = (a.K + splits - 1) / splits;
     k_step = (k_step + 31) / 32 * 32;
     splits = (a.K + k_step - 1) / k_step;
-    if (vec && a.M <= 32) RAI_TRY((launch_tile<32, 128, kWhole, true>(st, a, splits, k_step)));
+    if (wide) RAI_TRY((launch_tile<32, 128, kWhole, true>(st, a, splits, k_step)));
     else RAI_TRY((vec ? launch_tile<64, 64, kWhole, true>(st, a, splits, k_step) : launch_tile<64, 64, kRagged, true>(st, a, splits, k_step)));
     const int64_t blocks = ((int64_t)a.M * ((a.N + 3) / 4) + 255) / 256;
     hipLaunchKernelGGL(k_linear_f32_sum, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, st, a, splits);
     return launch_check("linear_f32_sum");
   }
-  if (vec && a.M <= 32) return launch_tile<32, 128, kWhole, false>(st, a, 1, 0);
+  if (wide) return launch_tile<32, 128, kWhole, false>(st, a, 1, 0);
   if (vec) return launch_tile<64, 64, kWhole, false>(st, a, 1, 0);
   return a.K >= 4 ? launch_tile<64, 64, kRagged, false>(st, a, 1, 0) : launch_tile<64, 64, kTiny, false>(st, a, 1, 0);
 }

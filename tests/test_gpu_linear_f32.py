@@ -62,6 +62,15 @@ def test_f32_linear_where_k_ends_inside_a_piece(R, m, n, k):
         assert np.all(np.abs(got - xs.astype(np.float64) @ ws.astype(np.float64).T) <= bound(xs, ws, 0.0)), (first, width)
 
 
+@pytest.mark.parametrize("m,k,n", [(4, 4096, 512), (32, 4096, 8192)])
+def test_unaligned_rows_are_cut_by_the_tiles_they_get(R, m, k, n):
+    """Rows off 16-byte boundaries take 64 x 64 tiles however few they are, so as few as these are cut over K like 40: the
+    same parts of K, and the same bits."""
+    g = np.random.Generator(np.random.PCG64(17))
+    x, w = up(rand(g, (40, k + 1), "f32"), "f32").narrow(1, 1, k), up(rand(g, (n, k + 1), "f32", 0.02), "f32").narrow(1, 1, k)
+    assert np.array_equal(down(R.linear(x.narrow(0, 0, m), w)), down(R.linear(x, w))[:m])
+
+
 @pytest.mark.parametrize("m", [1, 20, 100])
 def test_f32_linear_keeps_small_and_infinite_values(R, m):
     """Denormal products are kept, and infinities and NaNs reach only the outputs that depend on them (K is no multiple
