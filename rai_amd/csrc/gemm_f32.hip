@@ -376,7 +376,16 @@ static int f32_splits(const LinearArgs &a, size_t room) {
   }
   return best;
 }
-static bool few_rows(const LinearArgs &a) { return a.M <= kFewRows && rows_aligned(a); }
+// Where the few-row kernel serves.  A block's end (the sums across its lanes) is paid per two rows of W however short they
+// are: 0.36, 0.51 and 1.04 us per 1000 rows of W for one, two and four rows.  Short rows against many are done sooner by
+// the tiles, a round of which takes 3.4 us and 0.02 per k (us, this kernel, tiles, K x N; four rows 64 x 10240 13.3, 4.6; 256 x
+// 32768 36.5, 10.5; 384 x 10240 13.4, 11.0; two 128 x 16384 11.0, 6.3; one 96 x 32768 13.2, 7.7; multiply-adds on the vector units
+// 9.2, 26.6, 28.7, 11.8, 9.5).
+static bool few_rows(const LinearArgs &a) {
+  if (a.M > kFewRows || !rows_aligned(a)) return false;
+  const float per_row = a.M == 1 ? 0.36e-3f : a.M == 2 ? 0.51e-3f : 1.04e-3f;
+  return 2.f + per_row * a.N <= 3.4f + 0.02f * a.K * (float)((a.N + 16383) / 16384);
+}
 
 size_t linear_f32_workspace_bytes(const LinearArgs &a, size_t room) {
   const int s = few_rows(a) ? 1 : f32_splits(a, room);

@@ -71,6 +71,17 @@ def test_unaligned_rows_are_cut_by_the_tiles_they_get(R, m, k, n):
     assert np.array_equal(down(R.linear(x.narrow(0, 0, m), w)), down(R.linear(x, w))[:m])
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+@pytest.mark.parametrize("k,n", [(64, 10241), (256, 16385), (512, 16390), (1024, 16390)])
+def test_f32_few_rows_against_many_short_weights(R, m, k, n):
+    """Both sides of the line between the few-row kernel and the tiles."""
+    g = np.random.Generator(np.random.PCG64(19))
+    x, w, b, r = rand(g, (m, k), "f32"), rand(g, (n, k), "f32", 0.05), rand(g, (n,), "f32"), rand(g, (m, n), "f32")
+    want = x.astype(np.float64) @ w.astype(np.float64).T + b + r
+    got = down(R.linear(up(x, "f32"), up(w, "f32"), up(b, "f32"), None, up(r, "f32"))).astype(np.float64)
+    assert np.all(np.abs(got - want) <= bound(x, w, np.abs(b) + np.abs(r)))
+
+
 @pytest.mark.parametrize("m", [1, 20, 100])
 def test_f32_linear_keeps_small_and_infinite_values(R, m):
     """Denormal products are kept, and infinities and NaNs reach only the outputs that depend on them (K is no multiple
