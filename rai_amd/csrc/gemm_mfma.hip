@@ -1805,12 +1805,12 @@ static bool no_k64() {   // read per call: tests compare both forms in one proce
 // 22.6, 16; 512 x 8192 x 8960 with two stages as before, 111 against 131 with four and 140 as 64 x 64.)
 enum { kTile128 = 0, kTile128Deep, kTile128x64, kTile64 };
 struct TilePlan { int tile, splits; };
-static TilePlan tile_plan_k64(const LinearArgs &a) {
+static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int last = kTile64) {
   const int stages = a.K / 64;
   const float part_mb = (float)a.M * a.N * 4e-6f;
-  TilePlan best = {kTile128, 1};
+  TilePlan best = {first, 1};
   float least = 0.f;
-  for (int t = kTile128; t <= kTile64; ++t) {
+  for (int t = first; t <= last; ++t) {
     const int64_t tiles = (int64_t)((a.M + (t == kTile64 ? 63 : 127)) / (t == kTile64 ? 64 : 128)) *
                           ((a.N + (t >= kTile128x64 ? 63 : 127)) / (t >= kTile128x64 ? 64 : 128));
     for (int s = 1; s <= 12; ++s) {
@@ -1819,7 +1819,7 @@ static TilePlan tile_plan_k64(const LinearArgs &a) {
       float stage = per_cu * (t == kTile64 ? 0.21f : t == kTile128x64 ? 0.36f : 0.58f);
       if (t == kTile128) stage = per_cu == 1 ? 0.62f : 0.46f * per_cu + (per_cu % 2 ? 0.16f : 0.f);
       const float cost = 4.2f + (t <= kTile128Deep ? 0.8f : 0.f) + stage * ((stages + s - 1) / s) + (s > 1 ? 3.2f + 0.4f * s * part_mb : 0.f);
-      if ((t == kTile128 && s == 1) || cost < least) { least = cost; best = {t, s}; }
+      if ((t == first && s == 1) || cost < least) { least = cost; best = {t, s}; }
     }
   }
   return best;
@@ -1862,7 +1862,15 @@ static int tile_splits(const LinearArgs &a) {
 
 // 256 x 256 tiles (or what stands in for them) once these cover a good half of the CUs, see launch_linear_bf16_mfma.
 static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 256) * ((a.N + 255) / 256)) >= 17 * kNumCU; }
+// RAI_HIP_GEMM_TILE, read per call, and the names of the tiles above in it; a tile that it names gets the split of its own.
+static const char *forced_tile() { return getenv("RAI_HIP_GEMM_TILE"); }
+static const char *const kTileNames[] = {"128x128k64", "128x128deep", "128x64", "64x64"};
 static TilePlan tile_plan(const LinearArgs &a) {
+  if (const char *knob = forced_tile()) {
+    for (int t = kTile128; t <= kTile64; ++t)
+      if (!strcmp(knob, kTileNames[t])) return a.K % 64 || a.force_splits > 0 ? TilePlan{t, tile_splits(a)} : tile_plan_k64(a, t, t);
+    return {kTile128, tile_splits(a)};
+  }
   if (a.K % 64 || no_k64() || a.force_splits > 0 || has_huge_tiles(a)) return {kTile128, tile_splits(a)};
   return tile_plan_k64(a);
 }
@@ -1946,22 +1954,22 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
   const int tiles = ((a.M + 127) / 128) * ((a.N + 127) / 128);
   const TilePlan tile = tile_plan(a);
   const int splits = tile.splits;
-  // Tile choice.  The LDS-DMA kernels stream K tiles straight into LDS; the 256x128 tile halves the
-  // L2 -> LDS traffic per flop for one operand and is used once there are enough tiles of that size
-  // to give every CU two; smaller products keep the 128x128 tile (three blocks per CU).
-  // RAI_HIP_GEMM_TILE = "128x128" | "128x128k64" | "256x128" | "256x192" | "256x256" | "256x256x8w" | "256x256x8wk64" |
-  // "streamk" | "streamk64" | "classic" overrides (tuning aid; a form that does not apply to the shape is an error).
-  const char *knob = getenv("RAI_HIP_GEMM_TILE");
+  // Tile choice.  The LDS-DMA kernels stream K tiles straight into LDS: the 256 x 256 tile, 256 x 192 or stream-K over
+  // either where there are tiles enough (below); otherwise what tile_plan_k64 says, or 128 x 128 with K tiles of 32.
+  // RAI_HIP_GEMM_TILE = "64x64" | "128x64" | "128x128" | "128x128k64" | "128x128deep" | "256x128" | "256x192" | "256x256" |
+  // "256x256x8w" | "256x256x8wk64" | "streamk" | "streamk64" | "classic" overrides (tuning aid; a form that does not apply to
+  // the shape is an error).
+  const char *knob = forced_tile();
   if (knob) {
+    if (!strcmp(knob, kTileNames[tile.tile])) {
+      RAI_REQUIRE(a.K % 64 == 0, RAI_ERR_UNSUPPORTED, "linear: RAI_HIP_GEMM_TILE=%s needs K %% 64 == 0 (%dx%dx%d)", knob, a.M, a.N, a.K);
+      return launch_tile_k64(st, a, tile);
+    }
     if (!strcmp(knob, "128x128")) return launch_cfg_dma<128, 128, 3, 2>(st, a, splits);
     if (!strcmp(knob, "256x128")) return launch_cfg_dma<256, 128, 3, 2>(st, a, splits);
     if (!strcmp(knob, "256x256")) return launch_cfg_dma<256, 256, 4, 2>(st, a, splits);
     if (!strcmp(knob, "classic")) return launch_cfg<128, 128, 32>(st, a, splits);
     if (!strcmp(knob, "256x256x8w")) return launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
-    if (!strcmp(knob, "128x128k64")) {
-      RAI_REQUIRE(a.K % 64 == 0, RAI_ERR_UNSUPPORTED, "linear: RAI_HIP_GEMM_TILE=%s needs K %% 64 == 0 (%dx%dx%d)", knob, a.M, a.N, a.K);
-      return launch_cfg_dma<128, 128, 2, 0, 2>(st, a, splits);
-    }
     if (!strcmp(knob, "256x192")) {
       RAI_REQUIRE(a.K % 64 == 0, RAI_ERR_UNSUPPORTED, "linear: RAI_HIP_GEMM_TILE=%s needs K %% 64 == 0 (%dx%dx%d)", knob, a.M, a.N, a.K);
       return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, splits);

@@ -146,8 +146,8 @@ def test_argmax_64x51200(R, dt):
 
 
 # ------------------------------------------------------------------ every tile of the bf16 MFMA GEMM
-TILES = ["128x128", "128x128k64", "256x192", "256x128", "256x256", "256x256x8w", "classic"]
-K64_TILES = ("128x128k64", "256x192")      # two LDS stages of K 64: refused unless K % 64 == 0
+TILES = ["64x64", "128x64", "128x128", "128x128k64", "128x128deep", "256x192", "256x128", "256x256", "256x256x8w", "classic"]
+K64_TILES = ("64x64", "128x64", "128x128k64", "128x128deep", "256x192")      # LDS stages of K 64: refused unless K % 64 == 0
 
 
 def packed_case(g, m, n, k, scale=0.05):
@@ -301,6 +301,17 @@ def test_gemm_streamk_refuses_where_it_does_not_apply(R, monkeypatch):
     x, w = up(np.zeros((512, 64), np.float32), "bf16"), up(np.zeros((512, 64), np.float32), "bf16")
     with pytest.raises(RaiHipError):
         R.linear(x, w)      # four tiles
+
+
+def test_gemm_forced_tile_is_not_split_for_another_tile(R, monkeypatch):
+    """The dispatcher would cut this K for 128 x 128 tiles; a forced whole tile is neither cut with them nor refused."""
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", "256x256x8wk64")
+    dt, (m, n, k) = "bf16", (2100, 2048, 8192)
+    x, w, _, _, _ = packed_case(rng(123), m, n, k)
+    want = onn.linear(x, w, None, dt)
+    got = down(R.linear(up(x, dt), up(w, dt)))
+    assert_close(got, want, dt, "256x256x8wk64 alone")
+    gemm_elem_check(got, want, dt, k, "256x256x8wk64 alone")
 
 
 def test_gemm_dispatcher_picks_each_tile_by_itself(R, monkeypatch):
