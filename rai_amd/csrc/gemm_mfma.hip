@@ -1115,7 +1115,7 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
     const int k_tiles = a.K / KU, per = (k_tiles + splits - 1) / splits;
     splits = (k_tiles + per - 1) / per;
     k_per_split = per * KU;
-    partial = (float *)a.splitk_ws;
+    if (splits > 1) partial = (float *)a.splitk_ws;   // one tile of K: one part
   }
   hipLaunchKernelGGL((k_gemm_bf16_mfma_dma<BM, BN, NS, SH, WGN, WGM>), dim3(grid_x, splits), dim3(64 * WGM * WGN), lds, st, a,
                      splits, k_per_split, partial);

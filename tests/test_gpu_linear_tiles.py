@@ -39,6 +39,16 @@ def test_tiles(R, m, k, n):
     assert np.all(np.abs(got - full) <= 2.0 ** -8 * np.abs(full) + 2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)
 
 
+@pytest.mark.parametrize("k,parts", [(64, 2), (128, 3), (64, 7)])
+def test_more_parts_asked_for_than_k_has_stages(R, k, parts):
+    g = np.random.Generator(np.random.PCG64(k))
+    x, w = rand(g, (100, k), "bf16"), rand(g, (136, k), "bf16", k ** -0.5)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    down(R.linear_packed(up(-x, "bf16"), up(w, "bf16")))   # (an output that is not written may still hold its like)
+    got = down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), k_splits=parts)).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + spread(x, w))
+
+
 @pytest.mark.parametrize("m,k,n", [(70, 256, 136), (300, 1536, 520), (20, 1536, 4104), (256, 2048, 2048)])
 def test_tiles_gated(R, m, k, n):
     """act(gate) * up with gate, act(gate) and up each rounded to bf16: three roundings, and the sums' own error through a
