@@ -672,7 +672,7 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
 }
 
 template <int BM, int BN, int NS, int SH, int WGN = 2, int WGM = 2>
-__global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArgs a, int splits, int k_per_split, float *partial) {
+__global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArgs a, int longer, int k_per_split, float *partial) {
   // block = 2 x WGN waves.  WGN = 4 (eight waves, wave tile (BM/2) x (BN/4)) keeps two waves on every SIMD: one
   // multiplies while the other sits in its wait for the next tile, and twice as many waves issue loads.
   constexpr int BK = 32, PITCH = BK;
@@ -687,8 +687,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArg
   tile_coords(tile, tiles_m, tiles_n, &tile_m, &tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int split = blockIdx.y;
-  const int k_begin = split * k_per_split;
-  const int k_end = k_begin + k_per_split < a.K ? k_begin + k_per_split : a.K;
+  // the first `longer` parts of K take one stage of 64 more (parts of 32s: none does, and the last may be shorter)
+  const int k_begin = split * k_per_split + (split < longer ? split : longer) * 64;
+  const int k_span = k_per_split + (split < longer ? 64 : 0);
+  const int k_end = k_begin + k_span < a.K ? k_begin + k_span : a.K;
   const int KT = (k_end - k_begin) / BK;
 
   f32x16 acc[BM / (32 * WGM)][BN / (32 * WGN)];
@@ -1108,17 +1110,21 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
   }
   const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
   const int grid_x = ((tiles + kXcds - 1) / kXcds) * kXcds;
-  int k_per_split = a.K;
-  float *partial = nullptr;
+  int k_per_split = a.K, longer = 0;
+  if (SH == 0 && splits > a.K / 64) splits = a.K / 64;
   if (splits > 1) {
-    constexpr int KU = SH == 0 ? 64 : 32;   // K tile of the main loop
-    const int k_tiles = a.K / KU, per = (k_tiles + splits - 1) / splits;
-    splits = (k_tiles + per - 1) / per;
-    k_per_split = per * KU;
-    if (splits > 1) partial = (float *)a.splitk_ws;   // one tile of K: one part
+    if constexpr (SH == 0) {   // stages of 64, dealt out evenly
+      k_per_split = a.K / 64 / splits * 64;
+      longer = a.K / 64 % splits;
+    } else {
+      const int k_tiles = a.K / 32, per = (k_tiles + splits - 1) / splits;
+      splits = (k_tiles + per - 1) / per;
+      k_per_split = per * 32;
+    }
   }
+  float *partial = splits > 1 ? (float *)a.splitk_ws : nullptr;
   hipLaunchKernelGGL((k_gemm_bf16_mfma_dma<BM, BN, NS, SH, WGN, WGM>), dim3(grid_x, splits), dim3(64 * WGM * WGN), lds, st, a,
-                     splits, k_per_split, partial);
+                     longer, k_per_split, partial);
   RAI_TRY(launch_check("gemm_bf16_mfma_dma"));
   if (splits > 1) RAI_TRY(launch_splitk_epilogue(st, a, splits, (const float *)partial));
   return RAI_OK;

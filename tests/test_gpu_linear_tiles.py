@@ -22,7 +22,7 @@ def spread(x, w):
 
 SIZES = [(65, 64, 8), (65, 128, 65), (97, 192, 1031), (129, 256, 257), (333, 320, 520), (72, 1536, 512), (100, 2048, 2050), (333, 2048, 72),
          (9, 64, 4096), (16, 192, 4104), (64, 1536, 2048), (40, 2048, 4097), (15, 4096, 2056), (64, 576, 9000),
-         (1000, 512, 2048), (530, 1088, 1500), (333, 1088, 8968), (130, 2560, 8200), (600, 1152, 5000)]
+         (1000, 512, 2048), (530, 1088, 1500), (333, 1088, 8968), (130, 2560, 8200), (600, 1152, 5000), (65, 1664, 512), (65, 1216, 520)]
 
 
 @pytest.mark.parametrize("m,k,n", SIZES)
