@@ -687,9 +687,11 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArg
   tile_coords(tile, tiles_m, tiles_n, &tile_m, &tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int split = blockIdx.y;
-  // the first `longer` parts of K take one stage of 64 more (parts of 32s: none does, and the last may be shorter)
-  const int k_begin = split * k_per_split + (split < longer ? split : longer) * 64;
-  const int k_span = k_per_split + (split < longer ? 64 : 0);
+  int k_begin = split * k_per_split, k_span = k_per_split;
+  if constexpr (SH == 0) {   // stages of 64: the first `longer` parts take one more (parts of 32s count none: 0.5 us)
+    k_begin += (split < longer ? split : longer) * 64;
+    k_span += split < longer ? 64 : 0;
+  }
   const int k_end = k_begin + k_span < a.K ? k_begin + k_span : a.K;
   const int KT = (k_end - k_begin) / BK;
 
