@@ -1804,14 +1804,18 @@ static bool no_k64() {   // read per call: tests compare both forms in one proce
   return e && *e && *e != '0';
 }
 
-// Which of the tiles with K stages of 64 serves a product, and over how many parts of K.  From the kernels' measured times
-// with cold weights: a tile costs us per stage by what it draws from L2 (16, 24, 32 KB), whoever else is on its CU (0.21 for
-// 64 x 64, 0.36 for 128 x 64; 128 x 128 with four stages 0.58 alone on its CU; with two stages 0.62 alone, 0.46 each where two
-// share a CU); 4.2 us are launch and ends, a K split adds 3.2 us (a launch) and 0.4 us per MB of partial sums, and leaves
-// every part four stages.  (us, the 128 x 128 tile with two stages, which served all of these, and what this picks: 333 x
-// 512 x 512 10.4, 6.0; 72 x 2048 x 2048 11.2, 9.0; 1000 x 2048 x 2048 33.9, 15.8; 333 x 1536 x 8960 31.6, 20.2; 72 x 8192 x 2048
-// 22.6, 16; 512 x 8192 x 8960 with two stages as before, 111 against 131 with four and 140 as 64 x 64.)
+// Which of the tiles with K stages of 64 serves a product, and over how many parts of K, by what the kernels' own times make
+// of it (fitted to 260 products of 65 to 2100 rows, every tile, one to eight parts, weights from HBM; what is picked is within
+// 1 % of the best of them in the mean).  An XCD has 32 CUs and a run of tiles of its own, so rounds are counted there: over the
+// whole chip 36 tiles in seven parts look like one round of 256 CUs, but five tiles on an XCD are 35 blocks and two rounds (333
+// x 8960 x 1536: 38.7 us, in five parts 26.9).  Blocks share a CU: `stage` is the time of 64 of K with one, two, three of them
+// on it, `end` what a tile takes besides, to start and to write its outputs.  3 us are the launch; a K split adds 4.3 us (a
+// launch) and 0.55 us per MB of partial sums, and leaves every part four stages; partial sums in rows off 16-byte boundaries
+// cost 2.1 us per MB of outputs more.
 enum { kTile128 = 0, kTile128Deep, kTile128x64, kTile64 };
+struct TileCost { int bm, bn, share; float stage[3], end; };
+static const TileCost kTileCosts[] = {{128, 128, 2, {0.74f, 0.84f}, 2.6f},   {128, 128, 1, {0.50f}, 3.5f},
+                                      {128, 64, 2, {0.345f, 0.60f}, 1.75f},  {64, 64, 3, {0.285f, 0.415f, 0.59f}, 0.8f}};
 struct TilePlan { int tile, splits; };
 static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int last = kTile64) {
   const int stages = a.K / 64;
@@ -1819,14 +1823,15 @@ static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int las
   TilePlan best = {first, 1};
   float least = 0.f;
   for (int t = first; t <= last; ++t) {
-    const int64_t tiles = (int64_t)((a.M + (t == kTile64 ? 63 : 127)) / (t == kTile64 ? 64 : 128)) *
-                          ((a.N + (t >= kTile128x64 ? 63 : 127)) / (t >= kTile128x64 ? 64 : 128));
+    const TileCost &c = kTileCosts[t];
+    const int64_t tiles = (int64_t)((a.M + c.bm - 1) / c.bm) * ((a.N + c.bn - 1) / c.bn);
     for (int s = 1; s <= 12; ++s) {
       if (s > 1 && (stages / s < 4 || !a.splitk_ws || (size_t)s * a.M * a.N * sizeof(float) > a.splitk_ws_bytes)) break;
-      const int64_t per_cu = (tiles * s + kNumCU - 1) / kNumCU;
-      float stage = per_cu * (t == kTile64 ? 0.21f : t == kTile128x64 ? 0.36f : 0.58f);
-      if (t == kTile128) stage = per_cu == 1 ? 0.62f : 0.46f * per_cu + (per_cu % 2 ? 0.16f : 0.f);
-      const float cost = 4.2f + (t <= kTile128Deep ? 0.8f : 0.f) + stage * ((stages + s - 1) / s) + (s > 1 ? 3.2f + 0.4f * s * part_mb : 0.f);
+      const int64_t per_cu = ((tiles + kXcds - 1) / kXcds * s + kNumCU / kXcds - 1) / (kNumCU / kXcds);
+      const int left = (int)(per_cu % c.share);
+      const float stage = per_cu / c.share * c.stage[c.share - 1] + (left ? c.stage[left - 1] : 0.f);
+      const float cost = 3.f + stage * ((stages + s - 1) / s) +
+                         (s > 1 ? 4.3f + 0.55f * s * part_mb + (a.N % 4 ? 2.1f * part_mb : 0.f) : per_cu * c.end);
       if ((t == first && s == 1) || cost < least) { least = cost; best = {t, s}; }
     }
   }
