@@ -318,13 +318,17 @@ template <int D, int KSP> static int launch_f32(hipStream_t st, const AttnArgs &
   return launch_check("flash_prefill_f32");
 }
 
-// Waves to a query group: as many as keep all blocks on the chip at once (two to a CU while LDS and registers hold them), no
-// more than there are key tiles.
+// Waves to a query group.  More of them make its chain of key tiles shorter and the blocks more; measured (us, with four, two,
+// one; 32 heads, S = T, causal): 333 x 80 (352 groups; one block to a CU, so two rounds with four) 24.5, 31.9, 52.6; 512 x 80 34.7,
+// 43.1, 74.8; 700 x 80 (704 groups) 64, 58.6, 99; 1024 x 80 112, 91, 144; 512 x 64 24.5, 32.8, 59.3; 1024 x 64 67.7, 73.7, 113; 8 x 128
+// x 64 (1024 groups) 21.9, 18.4, 20.2.  So four up to 512 groups (128 features: 256), two up to 1024 (beyond 128 features: 512).
+// (Long keys of 32 or 64 features would take four further on: 700 x 64 35.5, 48.8.)  Three key tiles are enough for four waves: 75
+// x 80 on 78 keys 10.4, 15.1, 18.8, and 11.8 with a block to a row.
 template <int D> static int launch_f32_split(hipStream_t st, const AttnArgs &a) {
   const int64_t groups = (int64_t)((a.S + 31) / 32) * a.Hq * a.B;
   const int seen = a.window > 0 && a.window + 31 < a.T ? a.window + 31 : a.T, tiles = (seen + 31) / 32;
   if constexpr (D <= 128) {
-    if (groups <= (D <= 80 ? 2 : 1) * kNumCU && tiles >= 4) return launch_f32<D, 4>(st, a);
+    if (groups <= (D <= 80 ? 2 : 1) * kNumCU && tiles >= 3) return launch_f32<D, 4>(st, a);
   }
   if (groups * 2 <= (D <= 128 ? 8 : 4) * kNumCU && tiles >= 2) return launch_f32<D, 2>(st, a);
   return launch_f32<D, 1>(st, a);
