@@ -32,7 +32,9 @@ template <> __device__ __forceinline__ mm_f32x16 mm_mfma<f16_raw>(mm_chunk a, mm
 // as it lies, BK rows of ROWS elements + 16 bytes, and the fragments are put together on the way out: 16-bit elements
 // with the transposing LDS read (lane i of 16 receives element i % 4 of the 8 bytes that lanes 4j + i / 4, j = 0..3, point
 // at: with lane a pointing at row a / 4, columns 4 (a % 4), it receives column i of four rows), f32 one by one.
-// Memory is read in pieces of 16 bytes whatever their alignment.
+// Memory is read in pieces of 16 bytes whatever their alignment; where K ends inside one (KC), the last 16 bytes of the row are
+// read and moved down, or a K of less than a piece by pairs (element by element, 16-bit operands with K of 9 to 15 took up to
+// 1.1 us more than multiply-adds on the vector units: 11 x 1 x 11 x 93 in bf16 4.2 us there, 5.3, now 4.5).
 template <typename T, int ROWS, bool KC, int KB>
 struct MmOperand {
   static constexpr int V = 16 / sizeof(T), BK = KB / sizeof(T), CPR = KC ? KB / 16 : ROWS / V, P = ROWS * KB / 16 / 256;
@@ -66,6 +68,17 @@ struct MmOperand {
         reg[p] = mm_chunk{0u, 0u, 0u, 0u};
       } else if (KC ? k + V <= K : o + V <= valid) {
         __builtin_memcpy(&reg[p], at, 16);
+      } else if (KC && K >= V) {   // the piece that ends with K, moved down
+        __builtin_memcpy(&reg[p], base + (int64_t)o * stride + (K - V), 16);
+        reg[p] = end_of_k(reg[p], k + V - K);
+      } else if (KC && sizeof(T) == 2 && K > 1) {   // a shorter K, by pairs
+        const T *at_o = base + (int64_t)o * stride;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          uint32_t two;
+          __builtin_memcpy(&two, at_o + min(2 * j, K - 2), 4);
+          reg[p][j] = 2 * j < K - 1 ? two : 2 * j == K - 1 ? two >> 16 : 0u;
+        }
       } else {
         T v[V];
 #pragma unroll
@@ -78,6 +91,15 @@ struct MmOperand {
         __builtin_memcpy(&reg[p], v, 16);
       }
     }
+  }
+  // A piece that was read `past` elements (below V) ahead of its place: what lies past the end is zero.
+  static __device__ __forceinline__ mm_chunk end_of_k(mm_chunk v, int past) {
+    const int words = past * (int)sizeof(T) / 4;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (words > i) v = mm_chunk{v[1], v[2], v[3], 0u};
+    if (sizeof(T) == 2 && (past & 1)) v = mm_chunk{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+    return v;
   }
   __device__ __forceinline__ void park(char *st) const {
 #pragma unroll

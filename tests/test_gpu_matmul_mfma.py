@@ -38,6 +38,18 @@ def test_layouts_and_tile_edges(R, dt, a_t, b_t, batch, m, k, n):
     check(down(R.matmul(ad, bd)), a, b, dt)
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("k", [*range(1, 18), 31, 63, 65, 71, 97, 131])
+def test_rows_that_end_inside_a_piece(R, dt, k):
+    """K along both operands, what lies next to the rows' ends is NaN: none of it is used."""
+    g = np.random.Generator(np.random.PCG64(k))
+    for m, n, pad in [(3, 2, 1), (70, 5, 9), (33, 65, 16)]:
+        a, b = rand(g, (2, m, k + pad), dt), rand(g, (2, n, k + pad), dt)
+        a[..., k:], b[..., k:] = np.nan, np.nan
+        got = down(R.matmul(up(a, dt).narrow(2, 0, k), up(b, dt).narrow(2, 0, k).transpose(1, 2)))
+        check(got, a[..., :k], np.swapaxes(b[..., :k], 1, 2), dt)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("b_t", [0, 1])
 def test_large_tiles(R, dt, b_t):
