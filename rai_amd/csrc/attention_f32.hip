@@ -1,6 +1,8 @@
 // Prefill attention in f32 on the f32 matrix instructions (scores, probabilities and sums all in f32).
 //
 // Reference semantics: rai-models/src/llm/phi2.rs:244-262, qwen2.rs:205-221, gemma.rs:238-254 (see attention.hip).
+#include <cstdlib>
+
 #include "attention.h"
 
 namespace rai {
@@ -318,6 +320,12 @@ template <int D, int KSP> static int launch_f32(hipStream_t st, const AttnArgs &
   return launch_check("flash_prefill_f32");
 }
 
+// RAI_HIP_ATTN_F32 = 1, 2 or 4 (read per call) forces this kernel with so many waves to a group; 0: not set.
+static int forced_waves() {
+  const char *e = getenv("RAI_HIP_ATTN_F32");
+  return e ? atoi(e) : 0;
+}
+
 // Waves to a query group.  More of them make its chain of key tiles shorter and the blocks more; measured (us, with four, two,
 // one; 32 heads, S = T, causal): 333 x 80 (352 groups; one block to a CU, so two rounds with four) 24.5, 31.9, 52.6; 512 x 80 34.7,
 // 43.1, 74.8; 700 x 80 (704 groups) 64, 58.6, 99; 1024 x 80 112, 91, 144; 512 x 64 24.5, 32.8, 59.3; 1024 x 64 67.7, 73.7, 113; 8 x 128
@@ -325,6 +333,13 @@ template <int D, int KSP> static int launch_f32(hipStream_t st, const AttnArgs &
 // (Long keys of 32 or 64 features would take four further on: 700 x 64 35.5, 48.8.)  Three key tiles are enough for four waves: 75
 // x 80 on 78 keys 10.4, 15.1, 18.8, and 11.8 with a block to a row.
 template <int D> static int launch_f32_split(hipStream_t st, const AttnArgs &a) {
+  if (const int waves = forced_waves()) {
+    RAI_REQUIRE(waves == 1 || waves == 2 || (waves == 4 && D <= 128), RAI_ERR_UNSUPPORTED, "attention: RAI_HIP_ATTN_F32=%d, head size %d", waves, D);
+    if constexpr (D <= 128) {
+      if (waves == 4) return launch_f32<D, 4>(st, a);
+    }
+    return waves == 2 ? launch_f32<D, 2>(st, a) : launch_f32<D, 1>(st, a);
+  }
   const int64_t groups = (int64_t)((a.S + 31) / 32) * a.Hq * a.B;
   const int seen = a.window > 0 && a.window + 31 < a.T ? a.window + 31 : a.T, tiles = (seen + 31) / 32;
   if constexpr (D <= 128) {
@@ -334,6 +349,14 @@ template <int D> static int launch_f32_split(hipStream_t st, const AttnArgs &a) 
   return launch_f32<D, 1>(st, a);
 }
 
+// What the kernel is written for, whatever it costs.
+static bool takes(const AttnArgs &a) {
+  if (a.S < 16 || a.T < 32 || a.t_dev) return false;
+  if (a.D != 32 && a.D != 64 && a.D != 80 && a.D != 128 && a.D != 192 && a.D != 256) return false;
+  auto al = [](const void *p, const int64_t *s) { return (uintptr_t)p % 16 == 0 && s[0] % 4 == 0 && s[1] % 4 == 0 && s[2] % 4 == 0 && s[2] < (1 << 24); };
+  return al(a.q, a.qs) && al(a.k, a.ks) && al(a.v, a.vs) && (uintptr_t)a.out % 16 == 0 && a.out_row_stride % 4 == 0 && (a.S + 31) / 32 <= 65535 && a.B <= 65535;
+}
+
 // A block per query row (attention.hip) is done sooner where there are few rows: a tile here is a chain of some 2 us at 64
 // features (8 at 256), which takes enough rows or keys to be worth it.  Measured (us; block per row, here): 32 heads x 48 x 64
 // 7.3, 8.0, 32 x 64 x 64 9.4, 8.2; 8 x 160 x 80 12.2, 15.2, 32 x 160 x 80 28.5, 15.5; 8 x 64 on 300 x 128 20.0, 29.3, 32 x 64 on
@@ -341,15 +364,15 @@ template <int D> static int launch_f32_split(hipStream_t st, const AttnArgs &a) 
 // chains than a row's lanes make of them, and less exact than those until there are a few hundred keys (1.17e-7 and 1.11e-7 at 100
 // x 128, 1.67e-7 and 1.86e-7 on 300).
 bool attention_f32_serves(const AttnArgs &a) {
-  if (a.dtype != RAI_F32 || a.S < 16 || a.T < 32 || a.t_dev) return false;
-  if (a.D != 32 && a.D != 64 && a.D != 80 && a.D != 128 && a.D != 192 && a.D != 256) return false;
+  if (a.dtype != RAI_F32) return false;
+  if (forced_waves()) return true;
   const int64_t rows = (int64_t)a.B * a.Hq * a.S;
   if (rows < (a.D <= 128 ? 2048 : 8192) || (a.D <= 80 ? rows * a.T < 2048 * 64 : a.T < (a.D <= 128 ? 256 : 512))) return false;
-  auto al = [](const void *p, const int64_t *s) { return (uintptr_t)p % 16 == 0 && s[0] % 4 == 0 && s[1] % 4 == 0 && s[2] % 4 == 0 && s[2] < (1 << 24); };
-  return al(a.q, a.qs) && al(a.k, a.ks) && al(a.v, a.vs) && (uintptr_t)a.out % 16 == 0 && a.out_row_stride % 4 == 0 && (a.S + 31) / 32 <= 65535 && a.B <= 65535;
+  return takes(a);
 }
 
 int launch_attention_f32(hipStream_t st, const AttnArgs &a) {
+  RAI_REQUIRE(takes(a), RAI_ERR_UNSUPPORTED, "attention: RAI_HIP_ATTN_F32 does not apply to %d x %d x %d on %d keys", a.B, a.Hq, a.S, a.T);
   switch (a.D) {
     case 32: return launch_f32_split<32>(st, a);
     case 64: return launch_f32_split<64>(st, a);

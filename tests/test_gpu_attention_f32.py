@@ -1,8 +1,9 @@
-"""f32 prefill attention on the matrix instructions: query groups of 32, key tiles of 32, one, two or four waves to a group,
-every head size it takes."""
+"""f32 prefill attention on the matrix instructions: query groups of 32, key tiles of 32; by the size of the call (small ones
+stay with the kernel that takes a row to a block), and every head size with one, two and four waves to a group forced."""
 import numpy as np
 import pytest
 
+from rai_amd._lib import RaiHipError
 from tests.util import down, rand, up
 
 pytestmark = pytest.mark.gpu
@@ -37,7 +38,8 @@ def reference(q, k, v, scale, causal):
 @pytest.mark.parametrize("b,hq,hkv,s,t,d", [(1, 2, 2, 16, 32, 64), (2, 3, 1, 33, 65, 80), (1, 4, 2, 128, 128, 128), (1, 2, 1, 31, 300, 32), (1, 1, 1, 97, 129, 192),
                                             (1, 2, 1, 64, 200, 256), (3, 24, 24, 40, 160, 64), (16, 36, 6, 64, 64, 128), (1, 64, 64, 33, 129, 80),
                                             (1, 64, 16, 32, 65, 64), (16, 36, 6, 64, 64, 64), (2, 64, 64, 31, 80, 32), (1, 64, 8, 33, 300, 128),
-                                            (1, 64, 8, 32, 256, 128), (16, 36, 6, 33, 257, 128), (1, 32, 4, 260, 515, 192), (1, 16, 16, 520, 520, 256)])
+                                            (1, 64, 8, 32, 256, 128), (16, 36, 6, 33, 257, 128), (1, 32, 4, 260, 515, 192), (1, 16, 16, 520, 520, 256), (1, 64, 64, 33, 65, 80), (16, 36, 6, 64, 64, 80),
+                                            (8, 36, 6, 33, 257, 128), (2, 32, 4, 260, 515, 192)])
 def test_against_64_bits(R, b, hq, hkv, s, t, d, causal):
     g = np.random.Generator(np.random.PCG64(b + s))
     q, k, v = rand(g, (b, hq, s, d), "f32"), rand(g, (b, hkv, t, d), "f32"), rand(g, (b, hkv, t, d), "f32")
@@ -46,17 +48,47 @@ def test_against_64_bits(R, b, hq, hkv, s, t, d, causal):
     assert np.all(np.abs(got - want) <= tol)
 
 
+# Head sizes with the waves to a group they come with (two stages of tiles up to 128 features with one wave, one otherwise).
+FORMS = [(d, waves) for d in (32, 64, 80, 128, 192, 256) for waves in (1, 2, 4) if waves < 4 or d <= 128]
+
+
+@pytest.mark.parametrize("causal", [1, 0])
+@pytest.mark.parametrize("b,hq,hkv,s,t", [(1, 2, 1, 16, 32), (2, 3, 3, 33, 65), (1, 4, 2, 130, 161), (1, 2, 2, 200, 200)])
+@pytest.mark.parametrize("d,waves", FORMS)
+def test_every_form_against_64_bits(R, monkeypatch, d, waves, b, hq, hkv, s, t, causal):
+    monkeypatch.setenv("RAI_HIP_ATTN_F32", str(waves))   # read per call; refused where it does not apply
+    test_against_64_bits(R, b, hq, hkv, s, t, d, causal)
+
+
+def test_a_form_that_does_not_apply_is_refused(R, monkeypatch):
+    g = np.random.Generator(np.random.PCG64(3))
+    for waves, s, d in [(4, 64, 256), (3, 64, 64), (1, 15, 64), (1, 64, 48)]:
+        q = up(rand(g, (1, 2, s, d), "f32"), "f32")
+        monkeypatch.setenv("RAI_HIP_ATTN_F32", str(waves))
+        with pytest.raises(RaiHipError):
+            R.attention(q, q, q, 0.1, 1, 1)
+        monkeypatch.delenv("RAI_HIP_ATTN_F32")
+        R.attention(q, q, q, 0.1, 1, 1)
+
+
+@pytest.mark.parametrize("s,t", [(40, 70), (200, 200)])
+@pytest.mark.parametrize("d,waves", FORMS)
+def test_infinite_values_with_every_form(R, monkeypatch, d, waves, s, t):
+    monkeypatch.setenv("RAI_HIP_ATTN_F32", str(waves))
+    test_infinite_values_reach_only_queries_that_see_them(R, s, t, 2, d)
+
+
 @pytest.mark.parametrize("s,t,n", [(40, 70, 2), (200, 200, 2), (40, 70, 64), (200, 200, 16)])
-def test_infinite_values_reach_only_queries_that_see_them(R, s, t, n):
+def test_infinite_values_reach_only_queries_that_see_them(R, s, t, n, d=64):
     g = np.random.Generator(np.random.PCG64(9))
-    q, k, v = rand(g, (1, n, s, 64), "f32"), rand(g, (1, n, t, 64), "f32"), rand(g, (1, n, t, 64), "f32")
-    clean, tol = reference(q, k, v, 0.125, 1)
+    q, k, v = rand(g, (1, n, s, d), "f32"), rand(g, (1, n, t, d), "f32"), rand(g, (1, n, t, d), "f32")
+    clean, tol = reference(q, k, v, d ** -0.5, 1)
     at = t - s // 2
-    v[0, 0, at, 5], v[0, 0, t - 1, 7], v[0, 1, at, 63] = np.inf, np.nan, -np.inf
-    got = down(R.attention(up(q, "f32"), up(k, "f32"), up(v, "f32"), 0.125, 1, 1)).astype(np.float64)
+    v[0, 0, at, 5], v[0, 0, t - 1, 7], v[0, 1, at, d - 1] = np.inf, np.nan, -np.inf   # d - 1: the last feature, which 80's third tile repeats
+    got = down(R.attention(up(q, "f32"), up(k, "f32"), up(v, "f32"), d ** -0.5, 1, 1)).astype(np.float64)
     want = clean.copy()
     first = at - (t - s)   # the query at the key's own position
-    want[0, first:, 5], want[0, s - 1, 7], want[0, first:, 64 + 63] = np.inf, np.nan, -np.inf
+    want[0, first:, 5], want[0, s - 1, 7], want[0, first:, 2 * d - 1] = np.inf, np.nan, -np.inf
     same = np.isfinite(want)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~same & ~np.isnan(want)], want[~same & ~np.isnan(want)])
     assert np.all(np.abs(got - clean)[same] <= tol[same])
