@@ -48,3 +48,34 @@ def test_few_rows_gated(R, m, k, n):
     got = down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), act="silu", glu=True)).astype(np.float64)
     size = (np.abs(gate) + 1) * (np.abs(upv) + 1)
     assert np.all(np.abs(got - want) <= 4 * 2.0 ** -8 * size)
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("k,n,n1", [(520, 39, 17), (2560, 1031, 301), (4104, 8200, 4099), (8968, 40, 8)])
+def test_few_rows_two_outputs(R, m, k, n, n1):
+    """Columns [0, n1) without, the rest with an activation, into a second output; n1 odd: rows of no alignment."""
+    g = np.random.Generator(np.random.PCG64(m * 1000 + k))
+    x, w, b = rand(g, (m, k), "bf16"), rand(g, (n, k), "bf16", k ** -0.5), rand(g, (n,), "bf16")
+    z = x.astype(np.float64) @ w.astype(np.float64).T + b
+    want = np.concatenate([z[:, :n1], z[:, n1:] / (1 + np.exp(-z[:, n1:]))], 1)
+    o1, o2 = R.linear_packed(up(x, "bf16"), up(w, "bf16"), bias=up(b, "bf16"), act="silu", act_from=n1, n1=n1)
+    assert o1.shape == (m, n1) and o2.shape == (m, n - n1)
+    got = np.concatenate([down(o1), down(o2)], 1).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 2 * spread(x, w) + 2.0 ** -20)   # silu's slope stays below 1.1
+
+
+@pytest.mark.parametrize("m", [1, 2, 4, 6, 7])
+@pytest.mark.parametrize("k,n", [(504, 5), (2048, 2050), (4608, 8195)])
+def test_few_rows_two_biases(R, m, k, n):
+    """The activation from a column on within one output, two biases, a residual."""
+    g = np.random.Generator(np.random.PCG64(m + n))
+    x, w, r = rand(g, (m, k), "bf16"), rand(g, (n, k), "bf16", k ** -0.5), rand(g, (m, n), "bf16")
+    b, b2 = rand(g, (n,), "bf16"), rand(g, (n,), "bf16")
+    z = x.astype(np.float64) @ w.astype(np.float64).T + (b.astype(np.float64) + b2)
+    at = n // 2
+    z[:, at:] = z[:, at:] / (1 + np.exp(-z[:, at:]))
+    want = z + r
+    got = down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), bias=up(b, "bf16"), bias2=up(b2, "bf16"), act="silu", act_from=at, residual=up(r, "bf16")))
+    # the three additions after the sum: a rounding each of what they add
+    extra = 2.0 ** -23 * (np.abs(b) + np.abs(b2) + np.abs(z) + np.abs(r))
+    assert np.all(np.abs(got.astype(np.float64) - want) <= 2.0 ** -8 * np.abs(want) + 2 * spread(x, w) + extra + 2.0 ** -20)

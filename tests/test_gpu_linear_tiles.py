@@ -1,5 +1,6 @@
-"""bf16 Linears of more than eight rows: every tile with K stages of 64 (64 x 64, 128 x 64, 128 x 128 with two and four stages),
-one to as many stages as it keeps in flight and one more, ragged edges, K in parts, gated pairs."""
+"""bf16 Linears of more than eight rows on tiles with K stages of 64: as the sizes choose them (64 x 64 for most of these), and
+each of 64 x 64, 128 x 64 and 128 x 128 with two and four stages forced, with one to as many stages as it keeps in flight and one
+more, ragged edges, K in parts, gated pairs."""
 import numpy as np
 import pytest
 
@@ -39,6 +40,28 @@ def test_tiles(R, m, k, n):
     assert np.all(np.abs(got - full) <= 2.0 ** -8 * np.abs(full) + 2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)
 
 
+TILES = ["64x64", "128x64", "128x128k64", "128x128deep"]
+
+
+@pytest.mark.parametrize("m,k,n", [(65, 64, 8), (129, 128, 257), (200, 192, 136), (333, 256, 520), (72, 320, 1031), (65, 1664, 512), (260, 1088, 300), (130, 2560, 776)])
+@pytest.mark.parametrize("tile", TILES)
+def test_every_tile(R, monkeypatch, tile, m, k, n):
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", tile)   # read per call; K is cut as the tile's own plan says
+    test_tiles(R, m, k, n)
+
+
+@pytest.mark.parametrize("m,k,n,parts", [(65, 192, 136, 3), (65, 448, 136, 3), (130, 640, 200, 4), (97, 832, 264, 12)])
+@pytest.mark.parametrize("tile", TILES)
+def test_parts_shorter_than_the_pipeline(R, monkeypatch, tile, m, k, n, parts):
+    """Parts of one, two and three stages of K."""
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", tile)
+    g = np.random.Generator(np.random.PCG64(k))
+    x, w, b, r = rand(g, (m, k), "bf16"), rand(g, (n, k), "bf16", k ** -0.5), rand(g, (n,), "bf16"), rand(g, (m, n), "bf16")
+    want = x.astype(np.float64) @ w.astype(np.float64).T + b + r
+    got = down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), bias=up(b, "bf16"), residual=up(r, "bf16"), k_splits=parts)).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 2 * spread(x, w))
+
+
 @pytest.mark.parametrize("k,parts", [(64, 2), (128, 3), (64, 7)])
 def test_more_parts_asked_for_than_k_has_stages(R, k, parts):
     g = np.random.Generator(np.random.PCG64(k))
@@ -47,6 +70,13 @@ def test_more_parts_asked_for_than_k_has_stages(R, k, parts):
     down(R.linear_packed(up(-x, "bf16"), up(w, "bf16")))   # (an output that is not written may still hold its like)
     got = down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), k_splits=parts)).astype(np.float64)
     assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + spread(x, w))
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_every_tile_gated(R, monkeypatch, tile):
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", tile)
+    for m, k, n in [(70, 256, 136), (300, 1536, 520)]:
+        test_tiles_gated(R, m, k, n)
 
 
 @pytest.mark.parametrize("m,k,n", [(70, 256, 136), (300, 1536, 520), (20, 1536, 4104), (256, 2048, 2048)])

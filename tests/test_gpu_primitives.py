@@ -417,13 +417,16 @@ def test_linear_few_rows_k_ends_inside_a_step(R, m, k, n):
     assert_close(down(R.linear(up(x, "bf16"), up(w, "bf16"), up(b, "bf16"))), onn.linear(x, w, b, "bf16"), "bf16", f"linear {m}x{k}x{n}")
 
 
-@pytest.mark.parametrize("kernel", ["stream", "skinny", "tile"])
+@pytest.mark.parametrize("kernel", ["default", "stream", "skinny", "tile"])
 @pytest.mark.parametrize("m", [9, 16, 31, 64])
 @pytest.mark.parametrize("k,n", [(4096, 200), (1056, 2048), (16384, 64), (96, 50), (2048, 16384)])
 def test_linear_small_batch_deep_k(R, monkeypatch, m, k, n, kernel):
-    # 9..64 rows: the weight-streaming MFMA kernel by default; its two fallbacks (activations in LDS with K split over
-    # blocks, and the tile kernel) are forced through the switches the library reads at every call
-    if kernel != "stream":
+    # 9..64 rows: by default the weight-streaming MFMA kernel, or tiles with K stages of 64 where W is wide and long enough
+    # (2048 x 16384 here); the streaming kernel and its two fallbacks (activations in LDS with K split over blocks, and the
+    # tile kernel) are forced through the switches the library reads at every call
+    if kernel == "stream":
+        monkeypatch.setenv("RAI_HIP_NO_K64", "1")
+    if kernel in ("skinny", "tile"):
         monkeypatch.setenv("RAI_HIP_NO_MFMA_STREAM", "1")
     if kernel == "tile":
         monkeypatch.setenv("RAI_HIP_NO_MFMA_SKINNY", "1")
@@ -443,7 +446,8 @@ def test_linear_small_batch_deep_k(R, monkeypatch, m, k, n, kernel):
 def test_linear_k_split_summed_by_the_last_block(R, monkeypatch, m, k, n):
     """The weight-streaming kernel with K split over blocks: the block that finishes a group of weight tiles last sums
     the partial products itself.  Same bits as the separate summing pass (RAI_HIP_NO_FUSED_SPLITK=1), call after call
-    (the tickets are handed back), with and without the fused epilogue."""
+    (the tickets are handed back), with and without the fused epilogue.  (RAI_HIP_NO_K64: tiles serve the widest otherwise.)"""
+    monkeypatch.setenv("RAI_HIP_NO_K64", "1")
     g = rng(126)
     x, w, b = rand(g, (m, k), "bf16"), rand(g, (n, k), "bf16", 0.03), rand(g, (n,), "bf16")
     r = rand(g, (m, n), "bf16")
