@@ -39,7 +39,7 @@ struct LinearArgs {
   // N/2 columns are written to out1.  No residual, no output split.
   int glu;
   // Optional fused LayerNorm / RMSNorm of the rows of A before the product
-  // (skinny path only): A is normalised with ln_w / ln_b over K.
+  // (launch_linear_bf16_skinny, and the streaming kernel where linear_mfma_fuses_norm): A is normalised with ln_w / ln_b over K.
   const void *ln_w;
   const void *ln_b;
   float ln_eps;
@@ -92,11 +92,11 @@ inline LinearArgs linear_args_default() {
 size_t linear_fragment_elems(int N, int K);
 int launch_linear_fragment_layout(hipStream_t st, const void *W, int64_t ldw, int N, int K, void *Wfrag);
 
-// bf16 MFMA tile kernel (M >= 1; efficient for M >= 64).
+// bf16 on matrix instructions: streaming kernels and tiles, any M (made for 9 rows and more).
 int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a);
-// bf16 weight-streaming kernel for M <= 8 (decode): HBM-bound.
+// bf16 weight-streaming kernels for M <= 8 with a fused norm or a second product (decode): HBM-bound.
 int launch_linear_bf16_skinny(hipStream_t st, const LinearArgs &a);
-// Picks between the two.
+// Up to eight rows without either: a kernel of their own (gemm.hip); otherwise one of the two above.
 int launch_linear_bf16(hipStream_t st, const LinearArgs &a);
 
 // Up to kGemvGroupMax bf16 Linears of one activation row (M == 1, K <= 4096, a multiple of 8) in one launch: member i

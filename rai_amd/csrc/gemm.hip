@@ -1,9 +1,9 @@
 // Dense contractions.
-//   (the bf16 MFMA tile kernel lives in gemm_mfma.hip)
-//   k_linear_bf16_skinny weight-streaming kernel for M <= 8 rows (decode): each wave
-//                        streams whole weight rows with 16-byte loads; HBM-bound.
-//   (f32 Linears live in gemm_f32.hip)
+//   k_linear_bf16_rows   bf16 Linears of up to eight rows (decode): small waves, K whole or in quarters; HBM-bound.
+//   k_gemv_bf16_reg      one row with a fused norm, K <= 4096: the row in registers; _group: up to four Linears of it.
+//   k_linear_bf16_skinny up to eight rows with a fused norm, one row with a second product: the rows in LDS.
 //   k_matmul_generic     any strides / batch broadcast, f32 or f64 accumulate.
+// (More rows of bf16: gemm_mfma.hip; f32 Linears: gemm_f32.hip; other batched products: matmul_mfma.hip.)
 //
 // Reference semantics: rai-core/src/backend/candle.rs:327-443 (MatMul, stride rule),
 // rai-core/src/shape.rs:130-160 (batch broadcast), rai-nn/src/linear.rs:59-69.
@@ -16,7 +16,7 @@ namespace rai {
 
 
 // ============================================================ bf16 skinny (decode) kernel
-// M <= MROWS rows of A.  Each wave owns R consecutive weight rows at a time and
+// M <= MROWS rows of A, where a norm or a second product comes with them.  Each wave owns R consecutive weight rows at a time and
 // streams them with one 16-byte non-temporal load per lane per 512-element K
 // chunk; the (optionally normalised) activations live in LDS as bf16 and the
 // products are formed with v_dot2_f32_bf16 (two bf16 products per lane-op,
