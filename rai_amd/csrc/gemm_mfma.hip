@@ -1805,17 +1805,17 @@ static bool no_k64() {   // read per call: tests compare both forms in one proce
 }
 
 // Which of the tiles with K stages of 64 serves a product, and over how many parts of K, by what the kernels' own times make
-// of it (fitted to 260 products of 65 to 2100 rows, every tile, one to eight parts, weights from HBM; what is picked is within
-// 1 % of the best of them in the mean).  An XCD has 32 CUs and a run of tiles of its own, so rounds are counted there: over the
-// whole chip 36 tiles in seven parts look like one round of 256 CUs, but five tiles on an XCD are 35 blocks and two rounds (333
-// x 8960 x 1536: 38.7 us, in five parts 26.9).  Blocks share a CU: `stage` is the time of 64 of K with one, two, three of them
-// on it, `end` what a tile takes besides, to start and to write its outputs.  3 us are the launch; a K split adds 4.3 us (a
-// launch) and 0.55 us per MB of partial sums, and leaves every part four stages; partial sums in rows off 16-byte boundaries
-// cost 2.1 us per MB of outputs more.
+// of it (fitted to 390 products of 65 to 2100 rows, every tile, one to eight parts, weights from the caches and from HBM; what
+// is picked takes 1 % more than the best of them in the mean).  An XCD has 32 CUs and a run of tiles of its own, so rounds are
+// counted there: over the whole chip 36 tiles in seven parts look like one round of 256 CUs, but five tiles on an XCD are 35
+// blocks and two rounds (333 x 8960 x 1536: 38.7 us, in five parts 26.9).  Blocks share a CU: `stage` is the time of 64 of K with
+// one, two, three of them on it, `end` what a tile takes besides, to start and to write its outputs, `cut` the same where it
+// writes partial sums.  3 us are the launch; a K split adds 3.7 us (a launch) and 0.55 us per MB of partial sums, and leaves every
+// part four stages; partial sums in rows off 16-byte boundaries cost 2.2 us per MB of outputs more.
 enum { kTile128 = 0, kTile128Deep, kTile128x64, kTile64 };
-struct TileCost { int bm, bn, share; float stage[3], end; };
-static const TileCost kTileCosts[] = {{128, 128, 2, {0.74f, 0.84f}, 2.6f},   {128, 128, 1, {0.50f}, 3.5f},
-                                      {128, 64, 2, {0.345f, 0.60f}, 1.75f},  {64, 64, 3, {0.285f, 0.415f, 0.59f}, 0.8f}};
+struct TileCost { int bm, bn, share; float stage[3], end, cut; };
+static const TileCost kTileCosts[] = {{128, 128, 2, {0.63f, 0.775f}, 2.7f, 0.6f},  {128, 128, 1, {0.455f}, 4.0f, 2.0f},
+                                      {128, 64, 2, {0.315f, 0.535f}, 1.75f, 0.5f}, {64, 64, 3, {0.24f, 0.365f, 0.53f}, 0.8f, 0.f}};
 struct TilePlan { int tile, splits; };
 static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int last = kTile64) {
   const int stages = a.K / 64;
@@ -1831,7 +1831,7 @@ static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int las
       const int left = (int)(per_cu % c.share);
       const float stage = per_cu / c.share * c.stage[c.share - 1] + (left ? c.stage[left - 1] : 0.f);
       const float cost = 3.f + stage * ((stages + s - 1) / s) +
-                         (s > 1 ? 4.3f + 0.55f * s * part_mb + (a.N % 4 ? 2.1f * part_mb : 0.f) : per_cu * c.end);
+                         (s > 1 ? 3.7f + 0.55f * s * part_mb + (a.N % 4 ? 2.2f * part_mb : 0.f) + per_cu * c.cut : per_cu * c.end);
       if ((t == first && s == 1) || cost < least) { least = cost; best = {t, s}; }
     }
   }
