@@ -1944,10 +1944,12 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
   const bool no_skinny = getenv("RAI_HIP_NO_MFMA_SKINNY") != nullptr;
   const bool no_stream = getenv("RAI_HIP_NO_MFMA_STREAM") != nullptr;
   // A row-major W and 9 to 64 rows: the streaming kernel reads 512-byte pieces of W's rows, at 2 to 3 TB/s; tiles with all of
-  // their loads in flight do better once there are enough of them, and split K by themselves.  Where K needs no cut in the
-  // streaming kernel (2048, beyond 32 rows 1024) it takes more of them to beat it (us, stream, tiles, weights from HBM: 31 x 1728
-  // x 6016 10.6, 13.0; 26 x 2048 x 2944 8.5, 9.8; 48 x 1024 x 4736 7.8, 9.2; 17 to 32 rows x 1025 to 1535 x 4096 to 9000 in the
-  // mean 9.0, 10.6, up to 17000 12.8, 11.1; x 513 to 1024 8.6, 8.2; 49 to 64 rows there 8.2, 8.3).
+  // their loads in flight do better once there are enough of them, and split K by themselves (us, stream, tiles, weights from
+  // HBM: 16 x 512 x 8960 11.2, 6.2; 16 x 8192 x 8960 45, 35; 64 x 8192 x 8960 77, 40; 64 x 2048 x 2048 9.8, 9.2; 16 x 8192 x 2048 15.2,
+  // 14.4; but 16 x 2048 x 2048 7.1, 8.0; 48 x 512 x 2048 4.8, 5.8; 16 x 8192 x 512 9.7, 13.4).  Where K needs no cut in the streaming
+  // kernel (2048, beyond 32 rows 1024) it takes more of them (31 x 1728 x 6016 10.6, 12.9; 26 x 2048 x 2944 8.6, 10.0; 48 x 1024 x
+  // 4736 7.7, 9.3; 17 to 32 rows x 1025 to 1535 x 4096 to 9000 in the mean 9.0, 10.6, up to 17000 12.8, 11.1; x 513 to 1024 8.6, 8.2;
+  // 49 to 64 rows there 8.2, 8.3).
   const bool uncut = a.K <= (a.M <= 32 ? 2048 : 1024);
   const bool wide = a.N >= 4096 && (!uncut || a.N >= 9000 || (a.M <= 32 ? a.K <= 1024 : a.M > 48));
   const bool deep = a.N >= 2048 && !uncut && a.splitk_ws && a.K >= (a.M <= 16 ? 4096 : 1536);

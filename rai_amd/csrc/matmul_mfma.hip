@@ -147,7 +147,7 @@ template <typename T> __device__ __forceinline__ void mm_store(T *dst, const flo
 // rows are written 16 bytes at a time.  Attention-sized products are bound by a block's chain of trips (operands, LDS,
 // MFMAs, LDS, rows out), so what counts is how many blocks share a CU; long ones by the L2.
 //   Measured (us; 64 x 64 tiles of multiply-adds on the vector units before): bf16 32 x 512 x 80 x 512 (scores) 11.2 (40.5),
-// 32 x 512 x 512 x 80 (values, [K, N]) 13.4 (94.8), 64 x 1024 x 1024 x 1024 200 to 300 (2900 to 3035), one row against 32 x
+// 32 x 512 x 512 x 80 (values, [K, N]) 13.4 (94.8), 64 x 1024 x 1024 x 1024 200 to 316 (2900 to 3035), one row against 32 x
 // 777 x 128 10.4 (77.5), odd 18 x 410 x 141 x 349 10.8 (31.8); f32 32 x 512 x 80 x 512 24.4 (47.9).
 template <typename T, bool AKC, bool BKC, int F, int KB, bool ONE>
 __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T *B, MatmulArgs g, int tiles_m, int tiles_n) {
