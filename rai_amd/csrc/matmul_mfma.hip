@@ -247,7 +247,9 @@ static int launch_mm(hipStream_t st, void *out, const void *A, const void *B, co
   // 64 x 64 tiles; 16-bit operands take 128 x 128 (half the operand traffic per product) once those give every CU two and K
   // is long enough to pay for the larger prologue (64 x 1024 x 1024 x 1024: 200 to 227 against 290 us; 32 x 512 x 80 x 512:
   // 12.1 against 11.2).  Up to 256 bytes of K a tile needs no second stage: one load phase, and less LDS, so more blocks to
-  // a CU (32 x 512 x 80 x 512: 13.2 us with two stages of 128 bytes, 12.3 with one of 256, 11.2 with one of 192).
+  // a CU (us, two stages of 128 bytes, one of 256, one of 192: bf16 32 x 512 x 80 x 512 14.0, 12.0, 10.9; 32 x 512 x 96 x 512 13.5, 11.3,
+  // 10.3; 12 x 333 x 96 x 333 5.7, 5.4, 5.0; 64 x 128 x 80 x 128 4.9, 4.8, 4.6; f32 12 x 333 x 40 x 333 7.3, 6.5, 6.2; two stages and one
+  // of 256: bf16 32 x 512 x 128 x 512 13.1, 11.5; f32 32 x 512 x 64 x 512 18.4, 18.8).
   const int64_t t64 = batch * ((g.M + 63) / 64) * ((g.N + 63) / 64), tm128 = (g.M + 127) / 128, tn128 = (g.N + 127) / 128;
   const int kb = (int)(g.K * (int64_t)sizeof(T) < 512 ? g.K * sizeof(T) : 512);
   const int tm = (int)((g.M + 63) / 64), tn = (int)((g.N + 63) / 64);
