@@ -40,6 +40,7 @@ COMMON = [
 # them in the accumulation registers and copies them out and back around every rescale.
 EXTRA = {
     "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "attention_flash.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attention_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

@@ -36,6 +36,9 @@ struct AttnArgs {
 };
 
 int launch_attention(hipStream_t st, const AttnArgs &a);
+// The bf16 form on matrix instructions (attention_flash.hip) and what it takes.
+bool flash_serves(const AttnArgs &a);
+int launch_flash_prefill(hipStream_t st, const AttnArgs &a);
 // The f32 form on matrix instructions (attention_f32.hip): the head sizes and alignments it takes, from some 2000 query rows
 // of all heads on (beyond 128 features 8000) with keys enough.
 bool attention_f32_serves(const AttnArgs &a);

@@ -893,396 +893,6 @@ template <typename T> static int launch_row(hipStream_t st, const AttnArgs &a) {
   return launch_check("attention_row");
 }
 
-// ============================================================ prefill: flash attention on MFMA (bf16)
-// Block = NW waves, each owning 32 query rows; keys/values are streamed in
-// tiles of 64 through LDS and shared by the waves.  Both products run on
-// v_mfma_f32_32x32x16_bf16 in the transposed orientation
-//     S^T = K . Q^T        (rows = keys, columns = queries)
-//     O^T = V^T . P^T      (rows = head features, columns = queries)
-// so every lane owns one query column: the online-softmax statistics are
-// per-lane scalars, and the accumulator registers of S^T are, in order, exactly
-// the B-operand fragments of the second product (no cross-lane movement).
-// V is transposed while it is staged into LDS.  The score matrix never exists
-// in memory (the reference materialises [B,H,S,T]).
-typedef __attribute__((ext_vector_type(8))) __bf16 fa_bf16x8;
-typedef __attribute__((ext_vector_type(16))) float fa_f32x16;
-typedef __attribute__((ext_vector_type(4))) uint32_t fa_u32x4;
-typedef __attribute__((ext_vector_type(2))) uint32_t fa_u32x2;
-
-// KSP = 2: every 32-query group is worked on by two waves, one for the even and one for the odd key tiles, each with
-// its own running maximum, sum and output; the two are merged through LDS at the end.  For short sequences and few
-// heads, where the grid has about one block per CU and a wave's chain of key tiles is what the launch takes.
-// (Four waves per group, KSP = 4, gained another half per cent on the Phi-2 prefill: not instantiated.)
-// MODE: 0 scores rounded to bf16, 1 scores in f32, 2 scores in f32 with the cap and the sink of AttnArgs.
-template <int NW, int D, int MODE, int KSP = 1>
-__global__ void __launch_bounds__(NW * KSP * 64) k_flash_prefill_bf16(AttnArgs a) {
-  constexpr int KS = D / 16;            // K steps of the score product
-  constexpr int DT = (D + 31) / 32;     // 32-row tiles of O^T
-  constexpr int KP = D + 8;             // K tile pitch (elements)
-  constexpr int VP = 64 + 4;            // V^T tile pitch (elements)
-  constexpr int NT = NW * KSP * 64;
-  constexpr int CPR = D / 8;            // 16-byte chunks per key row
-  constexpr int KTILE = 64 * KP, VTILE = DT * 32 * VP;   // elements of one K tile / one V^T tile in LDS
-  __shared__ __attribute__((aligned(16))) uint16_t fa_smem[KSP * (KTILE + VTILE)];
-  uint16_t *const Ks = fa_smem, *const Vt = fa_smem + KSP * KTILE;   // KSP tiles each, one behind the other
-  static_assert(KSP == 1 || sizeof(float) * NW * 64 * (KSP - 1) * (2 + DT * 16) <= sizeof(uint16_t) * KSP * (KTILE + VTILE),
-                "the merge of the key halves reuses the tile memory");
-
-  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-  const int wave = (tid >> 6) / KSP, kh = (tid >> 6) % KSP;   // query group of the block, key tiles kh, kh + KSP, ...
-  const int h = blockIdx.y, b = blockIdx.z;
-  const int hk = h / (a.Hq / a.Hkv);
-  // the last query tiles see the most keys under a causal mask: they go first so that the short ones fill the tail
-  const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * (NW * 32);
-  const int off = a.T - a.S;  // absolute position of query row 0
-  const uint16_t *Kg = (const uint16_t *)a.k + b * a.ks[0] + hk * a.ks[1];
-  const uint16_t *Vg = (const uint16_t *)a.v + b * a.vs[0] + hk * a.vs[1];
-
-  const int qrow = q0 + wave * 32 + l32;
-  const int qrow_c = qrow < a.S ? qrow : a.S - 1;
-  const uint16_t *qp = (const uint16_t *)a.q + b * a.qs[0] + h * a.qs[1] + (int64_t)qrow_c * a.qs[2] + half * 8;
-  fa_bf16x8 qf[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const fa_bf16x8 *>(qp + ks * 16);
-
-  fa_f32x16 o[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
-
-  int kv_end = a.T;
-  if (a.causal) {
-    int last_q = q0 + NW * 32 < a.S ? q0 + NW * 32 : a.S;
-    kv_end = off + last_q < a.T ? off + last_q : a.T;
-  }
-  // sliding window: the block's first query sets the oldest key tile any of its queries may see
-  const int first_key = a.window > 0 ? off + q0 - a.window + 1 : 0;
-  const int kv_begin = first_key > 0 ? first_key & ~63 : 0;
-  const int wave_last_key = a.causal ? off + q0 + wave * 32 + 31 : a.T - 1;  // newest key any row of this wave may see
-  const float scale_r = round_to<bf16_raw>(a.scale);
-
-  // K/V tiles go global -> registers -> LDS; with PF the loads of tile t+1 are issued before tile t is
-  // multiplied, so their latency hides behind the MFMAs (register budget allows it for D <= 128).
-  // K: 16-byte chunks, row-major into Ks.  V: each work item is one pair of head features (d, d+1) for 8
-  // consecutive keys: eight 4-byte loads (lanes run along d, so a wave reads whole rows), repacked in
-  // registers into the two 8-key rows of V^T, which are written with 8-byte stores.
-  constexpr int CH = (KSP * 64 * CPR + NT - 1) / NT;   // 16-byte chunks of K per thread (KSP tiles per round)
-  constexpr int NP = D / 2;                            // feature pairs
-  constexpr int VI = (KSP * 8 * NP + NT - 1) / NT;     // V work items per thread
-  constexpr bool PF = D <= 128;
-  fa_u32x4 kreg[CH];
-  uint32_t vx[PF ? VI : 1][8];
-  auto load_v = [&](int i, int k0, uint32_t (&x)[8]) {
-    const int c = tid + i * NT;
-    const int pr = c % NP, g = c / NP;
-    if (c < KSP * 8 * NP) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        int t = k0 + g * 8 + j;
-        t = t < a.T ? t : a.T - 1;   // rows past the context re-read its last row (masked below)
-        x[j] = *reinterpret_cast<const uint32_t *>(Vg + (int64_t)t * a.vs[2] + 2 * pr);
-      }
-    }
-  };
-  auto store_v = [&](int i, const uint32_t (&x)[8]) {
-    const int c = tid + i * NT;
-    const int pr = c % NP, g = c / NP;
-    if (c < KSP * 8 * NP) {
-      fa_u32x2 lo0, lo1, hi0, hi1;   // feature 2*pr: keys 0-3, 4-7; feature 2*pr+1: keys 0-3, 4-7
-      lo0.x = __builtin_amdgcn_perm(x[1], x[0], 0x05040100u);
-      lo0.y = __builtin_amdgcn_perm(x[3], x[2], 0x05040100u);
-      lo1.x = __builtin_amdgcn_perm(x[5], x[4], 0x05040100u);
-      lo1.y = __builtin_amdgcn_perm(x[7], x[6], 0x05040100u);
-      hi0.x = __builtin_amdgcn_perm(x[1], x[0], 0x07060302u);
-      hi0.y = __builtin_amdgcn_perm(x[3], x[2], 0x07060302u);
-      hi1.x = __builtin_amdgcn_perm(x[5], x[4], 0x07060302u);
-      hi1.y = __builtin_amdgcn_perm(x[7], x[6], 0x07060302u);
-      uint16_t *r0 = Vt + (g / 8) * VTILE + (2 * pr) * VP + (g % 8) * 8, *r1 = r0 + VP;   // key group g: tile g / 8
-      *reinterpret_cast<fa_u32x2 *>(r0) = lo0;
-      *reinterpret_cast<fa_u32x2 *>(r0 + 4) = lo1;
-      *reinterpret_cast<fa_u32x2 *>(r1) = hi0;
-      *reinterpret_cast<fa_u32x2 *>(r1 + 4) = hi1;
-    }
-  };
-  auto load_tile = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int c = tid + i * NT;
-      const int key = c / CPR, dc = (c % CPR) * 8;
-      int t = k0 + key;
-      t = t < a.T ? t : a.T - 1;
-      if (c < KSP * 64 * CPR) kreg[i] = *reinterpret_cast<const fa_u32x4 *>(Kg + (int64_t)t * a.ks[2] + dc);
-    }
-    if constexpr (PF) {
-#pragma unroll
-      for (int i = 0; i < VI; ++i) load_v(i, k0, vx[i]);
-    }
-  };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int c = tid + i * NT;
-      const int key = c / CPR, dc = (c % CPR) * 8;
-      if (c < KSP * 64 * CPR) *reinterpret_cast<fa_u32x4 *>(Ks + key * KP + dc) = kreg[i];   // tile key / 64 follows tile 0
-    }
-    if constexpr (PF) {
-#pragma unroll
-      for (int i = 0; i < VI; ++i) store_v(i, vx[i]);
-    }
-  };
-  // without the prefetch registers the V items pass through one at a time
-  auto stage_v_direct = [&](int k0) {
-#pragma unroll 2
-    for (int i = 0; i < VI; ++i) {
-      uint32_t x[8];
-      load_v(i, k0, x);
-      store_v(i, x);
-    }
-  };
-  if (PF && kv_end > 0) load_tile(kv_begin);
-  for (int kb = kv_begin; kb < kv_end; kb += 64 * KSP) {
-    __syncthreads();
-    // ---- stage K [64][D] and V^T [D][64], KSP tiles of each
-    if (!PF) load_tile(kb);
-    store_tile();
-    if (!PF) stage_v_direct(kb);
-    __syncthreads();
-    if (PF && kb + 64 * KSP < kv_end) load_tile(kb + 64 * KSP);
-    const int k0 = kb + 64 * kh;       // this wave's tile of the round
-    // every key of this tile is masked for this wave, or the tile lies behind the block's keys (barriers stay uniform)
-    if (k0 > wave_last_key || k0 >= kv_end) continue;
-    if (a.window > 0 && k0 + 63 <= off + q0 + wave * 32 - a.window) continue;   // older than every query's window
-    const uint16_t *const Kt = Ks + kh * KTILE, *const Vw = Vt + kh * VTILE;
-
-    // ---- S^T tile: 64 keys x 32 queries
-    fa_f32x16 sc[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sc[u][r] = 0.f;
-      const uint16_t *kr = Kt + (u * 32 + l32) * KP + half * 8;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        sc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const fa_bf16x8 *>(kr + ks * 16), qf[ks], sc[u],
-                                                        0, 0, 0);
-    }
-    // ---- scale, mask, online softmax (register r of sub-tile u is key k0 + 32u + 8*(r/4) + 4*half + r%4)
-    const int q_abs = off + qrow;
-    // a tile wholly inside the context and (under a causal mask) wholly at or before this wave's first query
-    // needs no masking
-    const bool masked = k0 + 63 >= a.T || (a.causal && k0 + 63 > off + q0 + wave * 32) ||
-                        (a.window > 0 && k0 <= off + q0 + wave * 32 + 31 - a.window);
-    if constexpr (MODE >= 1) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sc[u][r] *= a.scale;
-      if (MODE == 2 && a.softcap > 0.f) {   // cap * tanh(s / cap) = cap - 2 cap / (exp(2 s / cap) + 1)
-        const float to_exp = 2.0f * 1.4426950408889634f / a.softcap;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            sc[u][r] = fmaf(-2.0f * a.softcap, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sc[u][r] * to_exp)), a.softcap);
-      }
-    } else {   // the product and its scaling are each rounded to bf16, two scores per conversion
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          uint32_t pk = pack_bf16x2(sc[u][r], sc[u][r + 1]);
-          pk = pack_bf16x2(__uint_as_float(pk << 16) * scale_r, __uint_as_float(pk & 0xffff0000u) * scale_r);
-          sc[u][r] = __uint_as_float(pk << 16);
-          sc[u][r + 1] = __uint_as_float(pk & 0xffff0000u);
-        }
-    }
-    if (masked) {
-      const int last_key = a.causal && q_abs < a.T - 1 ? q_abs : a.T - 1;   // newest key this lane's query may see
-      const int rel = last_key - k0 - 4 * half;
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sc[u][r] = u * 32 + 8 * (r >> 2) + (r & 3) > rel ? -INFINITY : sc[u][r];
-      if (a.window > 0) {
-        const int rel_lo = q_abs - a.window - k0 - 4 * half;   // newest key before this lane's window
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) sc[u][r] = u * 32 + 8 * (r >> 2) + (r & 3) <= rel_lo ? -INFINITY : sc[u][r];
-      }
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[u][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    // m_run is the exponent every p, the running sum and the output are relative to; it need not be the maximum.
-    // It is moved (and sum and output rescaled) only when some query of the wave has met a score more than kLazy
-    // above its own: after the first tiles that is rare, and the rescaling multiplies -- a third of this loop's
-    // vector instructions at D = 128 -- are skipped.  A p may then reach e^kLazy instead of 1: nothing to bf16 or f32.
-    constexpr float kLazy = 6.0f;
-    const bool move = __builtin_amdgcn_ballot_w64(mx > m_run + kLazy) != 0;   // (-inf + kLazy = -inf: the first tile moves)
-    const float m_new = move ? fmaxf(m_run, mx) : m_run;
-    const float m_safe = m_new == -INFINITY ? 0.f : m_new;  // fully masked so far: every p is exp(-inf) = 0
-    constexpr float kLog2e = 1.4426950408889634f;
-    const float ml2 = m_safe * kLog2e;
-    const float alpha = __builtin_amdgcn_exp2f(m_run * kLog2e - ml2);
-    float psum = 0.f;
-    fa_bf16x8 pf[2][2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        fa_u32x4 w;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[u][8 * s2 + 2 * j], kLog2e, -ml2));
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[u][8 * s2 + 2 * j + 1], kLog2e, -ml2));
-          psum += p0 + p1;
-          w[j] = pack_bf16x2(p0, p1);
-        }
-        pf[u][s2] = __builtin_bit_cast(fa_bf16x8, w);
-      }
-    if (move) {
-      l_run *= alpha;
-      m_run = m_new;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
-    }
-    l_run += psum;
-    // ---- O^T += V^T . P^T
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const uint16_t *vr = Vw + (dt * 32 + l32) * VP + 4 * half;
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const fa_u32x2 lo = *reinterpret_cast<const fa_u32x2 *>(vr + u * 32 + 16 * s2);
-          const fa_u32x2 hi = *reinterpret_cast<const fa_u32x2 *>(vr + u * 32 + 16 * s2 + 8);
-          const fa_u32x4 va = {lo.x, lo.y, hi.x, hi.y};
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fa_bf16x8, va), pf[u][s2], o[dt], 0, 0, 0);
-        }
-    }
-  }
-
-  if constexpr (KSP > 1) {
-    // the waves of key tiles 1 .. KSP-1 (mod KSP) hand their maximum, sum and output over; the wave of tiles 0 merges
-    // and goes on alone
-    __syncthreads();   // the tiles are no longer read
-    constexpr int MS = 2 + DT * 16;
-    float *mb = reinterpret_cast<float *>(fa_smem) + (size_t)((wave * 64 + lane) * (KSP - 1)) * MS;
-    if (kh > 0) {
-      float *mine = mb + (kh - 1) * MS;
-      mine[0] = m_run;
-      mine[1] = l_run;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mine[2 + dt * 16 + r] = o[dt][r];
-    }
-    __syncthreads();
-    if (kh > 0) return;
-    constexpr float kLog2e = 1.4426950408889634f;
-    float m = m_run;
-#pragma unroll
-    for (int j = 0; j < KSP - 1; ++j) m = fmaxf(m, mb[j * MS]);
-    const float ms = m == -INFINITY ? 0.f : m;   // nothing seen by any of them: every weight is exp(-inf) = 0
-    const float w0 = __builtin_amdgcn_exp2f((m_run - ms) * kLog2e);
-    l_run *= w0;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[dt][r] *= w0;
-#pragma unroll
-    for (int j = 0; j < KSP - 1; ++j) {
-      const float wj = __builtin_amdgcn_exp2f((mb[j * MS] - ms) * kLog2e);
-      l_run += mb[j * MS + 1] * wj;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] += mb[j * MS + 2 + dt * 16 + r] * wj;
-    }
-    m_run = ms;
-  }
-  float l_tot = l_run + __shfl_xor(l_run, 32, 64);
-  if constexpr (MODE == 2) {
-    if (a.sink) {   // relative to the running exponent, moved up to the sink's where that is larger by much
-      const float sink = sink_of<bf16_raw>(a.sink, h), m = fmaxf(m_run, sink);
-      const float w = expf(m_run - m);
-      l_tot = l_tot * w + expf(sink - m);
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] *= w;
-    }
-  }
-  if (qrow < a.S) {
-    const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-    uint16_t *op = (uint16_t *)a.out + ((int64_t)b * a.S + qrow) * a.out_row_stride + (int64_t)h * D;
-    const uint16_t *gp = a.gate ? (const uint16_t *)a.gate + ((int64_t)b * a.S + qrow) * a.gate_row_stride + (int64_t)h * D : nullptr;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = dt * 32 + 8 * g + 4 * half;
-        if (d < D) {
-          if (gp) {
-            const fa_u32x2 gv = *reinterpret_cast<const fa_u32x2 *>(gp + d);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const uint32_t wd = e < 2 ? gv.x : gv.y;
-              o[dt][4 * g + e] *= gate_sigmoid(__uint_as_float(e & 1 ? wd & 0xffff0000u : wd << 16));
-            }
-          }
-          fa_u32x2 w;
-          w.x = (uint32_t)f32_to_bf16_bits(o[dt][4 * g] * inv) | ((uint32_t)f32_to_bf16_bits(o[dt][4 * g + 1] * inv) << 16);
-          w.y = (uint32_t)f32_to_bf16_bits(o[dt][4 * g + 2] * inv) | ((uint32_t)f32_to_bf16_bits(o[dt][4 * g + 3] * inv) << 16);
-          *reinterpret_cast<fa_u32x2 *>(op + d) = w;
-        }
-      }
-  }
-}
-
-template <int D, int MODE> static int launch_flash_mode(hipStream_t st, const AttnArgs &a) {
-  const int tiles4 = (a.S + 127) / 128;
-  if ((int64_t)tiles4 * a.Hq * a.B >= kNumCU) {
-    hipLaunchKernelGGL((k_flash_prefill_bf16<4, D, MODE>), dim3(tiles4, a.Hq, a.B), dim3(256), 0, st, a);
-  } else {
-    const dim3 grid((a.S + 63) / 64, a.Hq, a.B);
-    // about one block per CU or fewer, several key tiles per block: two waves per query group, each half of the keys
-    const char *no_split = getenv("RAI_HIP_FLASH_NO_KEY_SPLIT");   // read per call: tests compare both forms
-    if constexpr (D <= 80) {
-      if ((int64_t)grid.x * grid.y * grid.z < 2 * kNumCU && a.T > 128 && !(no_split && *no_split && *no_split != '0')) {
-        hipLaunchKernelGGL((k_flash_prefill_bf16<2, D, MODE, 2>), grid, dim3(256), 0, st, a);
-        return launch_check("flash_prefill");
-      }
-    }
-    hipLaunchKernelGGL((k_flash_prefill_bf16<2, D, MODE>), grid, dim3(128), 0, st, a);
-  }
-  return launch_check("flash_prefill");
-}
-template <int D> static int launch_flash(hipStream_t st, const AttnArgs &a) {
-  if (!a.f32_scores) return launch_flash_mode<D, 0>(st, a);
-  return a.softcap > 0.f || a.sink ? launch_flash_mode<D, 2>(st, a) : launch_flash_mode<D, 1>(st, a);
-}
-
-static bool flash_eligible(const AttnArgs &a) {
-  if (a.dtype != RAI_BF16 || a.S < 16 || a.t_dev) return false;
-  if (a.D != 32 && a.D != 64 && a.D != 80 && a.D != 128 && a.D != 192 && a.D != 256) return false;
-  if (a.gate && ((uintptr_t)a.gate % 8 || a.gate_row_stride % 4)) return false;
-  auto al = [](const void *p, const int64_t *s) {
-    return (uintptr_t)p % 16 == 0 && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0;
-  };
-  return al(a.q, a.qs) && al(a.k, a.ks) && al(a.v, a.vs) && (uintptr_t)a.out % 8 == 0 && a.out_row_stride % 4 == 0 &&
-         a.Hq <= 65535 && a.B <= 65535;
-}
-
 int launch_attention(hipStream_t st, const AttnArgs &a) {
   RAI_REQUIRE(a.B > 0 && a.Hq > 0 && a.Hkv > 0 && a.S > 0 && a.T > 0 && a.D > 0, RAI_ERR_BAD_SHAPE,
               "attention: empty problem");
@@ -1290,16 +900,7 @@ int launch_attention(hipStream_t st, const AttnArgs &a) {
               a.Hkv);
   RAI_REQUIRE(a.window >= 0 && (!a.window || a.causal) && (a.f32_scores || (!a.gate && !a.sink && a.softcap <= 0.f)), RAI_ERR_BAD_ARG,
               "attention: a window needs the causal form, an output gate, a cap or a sink the f32-score form");
-  if (flash_eligible(a)) {
-    switch (a.D) {
-      case 32: return launch_flash<32>(st, a);
-      case 64: return launch_flash<64>(st, a);
-      case 80: return launch_flash<80>(st, a);
-      case 128: return launch_flash<128>(st, a);
-      case 192: return launch_flash<192>(st, a);
-      default: return launch_flash<256>(st, a);
-    }
-  }
+  if (flash_serves(a)) return launch_flash_prefill(st, a);
   if (attention_f32_serves(a)) return launch_attention_f32(st, a);
   switch (a.dtype) {
     case RAI_F32: return launch_row<float>(st, a);

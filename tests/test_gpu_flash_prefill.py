@@ -1,0 +1,77 @@
+"""bf16 prefill attention on the matrix instructions: every head size with every number of waves to a query group and both tile
+lengths, which the number of groups picks; key counts at and around the ends of tiles, strided operands, scales of any sign."""
+import numpy as np
+import pytest
+
+from oracle.dtypes import rnd
+from tests.util import down, rand, up
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def R(hip):
+    from rai_amd import ops
+
+    return ops
+
+
+def reference(q, k, v, scale, causal, f32_scores):
+    """The result in 64 bits (rounded scores rounded as the model rounds them) and how far a correct bf16 form may be off."""
+    q, k, v = (t.astype(np.float64) for t in (q, k, v))
+    n = q.shape[1] // k.shape[1]
+    k, v = np.repeat(k, n, 1), np.repeat(v, n, 1)
+    s, size = np.matmul(q, np.swapaxes(k, 2, 3)), np.matmul(np.abs(q), np.swapaxes(np.abs(k), 2, 3)).max()
+    S, T = s.shape[2:]
+    # a score's f32 sum is within D + 2 roundings of its absolute sum
+    off = (q.shape[-1] + 2) * 2.0 ** -24 * size * abs(scale)
+    if f32_scores:
+        s = s * scale
+    else:
+        s = rnd(rnd(s.astype(np.float32), "bf16") * rnd(np.float32(scale), "bf16"), "bf16").astype(np.float64)
+        off += 2 * 2.0 ** -7 * np.abs(s).max()   # which may turn either rounding to the next bf16 number
+    if causal:
+        s = np.where(np.arange(T)[None] <= np.arange(T - S, T)[:, None], s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    flat = lambda t: np.swapaxes(t, 1, 2).reshape(t.shape[0], S, -1)  # noqa: E731
+    want = flat(p @ v)
+    # scores (numerator and denominator), weights rounded to bf16 (2^-8 at most), f32 sums over the keys; the result's own rounding
+    rel = 2 * np.expm1(off) + 2.0 ** -8 + (T + 8) * 2.0 ** -23
+    return want, rel * flat(p @ np.abs(v)) * (1 + 2.0 ** -8) + 2.0 ** -8 * np.abs(want) + 1e-30
+
+
+def check(R, b, hq, hkv, s, t, d, causal, f32_scores, scale=None, transposed=False):
+    g = np.random.Generator(np.random.PCG64(b + s + d))
+    scale = d ** -0.5 if scale is None else scale
+    q, k, v = rand(g, (b, hq, s, d), "bf16"), rand(g, (b, hkv, t, d), "bf16"), rand(g, (b, hkv, t, d), "bf16")
+    lay = (lambda x: up(np.ascontiguousarray(np.swapaxes(x, 1, 2)), "bf16").transpose(1, 2)) if transposed else (lambda x: up(x, "bf16"))
+    want, tol = reference(q, k, v, scale, causal, f32_scores)
+    got = down(R.attention(lay(q), lay(k), lay(v), scale, causal, f32_scores)).astype(np.float64)
+    assert np.all(np.abs(got - want) <= tol), f"worst {np.max(np.abs(got - want) / tol):.2f} of the bound"
+
+
+# (sequences, query heads, key heads, rows, keys): up to 256 groups of 32 rows, up to 512, 1024, 1536 and beyond 1792; one tile, a last tile
+# of one key, of all but one; rows that end inside a group.
+SIZES = [(1, 2, 1, 16, 16), (1, 3, 3, 33, 65), (2, 4, 2, 64, 64), (1, 2, 2, 160, 191), (1, 8, 2, 257, 257), (2, 20, 4, 270, 285),
+         (3, 40, 40, 140, 150), (2, 64, 8, 300, 300), (7, 64, 64, 97, 129)]
+
+
+@pytest.mark.parametrize("f32_scores", [0, 1])
+@pytest.mark.parametrize("b,hq,hkv,s,t", SIZES)
+@pytest.mark.parametrize("d", [32, 64, 80, 128, 192, 256])
+def test_forms(R, d, b, hq, hkv, s, t, f32_scores):
+    check(R, b, hq, hkv, s, t, d, 1, f32_scores)
+
+
+@pytest.mark.parametrize("f32_scores", [0, 1])
+@pytest.mark.parametrize("b,hq,hkv,s,t", [(1, 3, 3, 33, 95), (3, 40, 40, 140, 150)])
+@pytest.mark.parametrize("d", [64, 80, 128, 256])
+def test_all_keys_and_strides(R, d, b, hq, hkv, s, t, f32_scores):
+    check(R, b, hq, hkv, s, t, d, 0, f32_scores, transposed=True)
+
+
+@pytest.mark.parametrize("f32_scores", [0, 1])
+@pytest.mark.parametrize("scale", [-0.125, 0.0, 0.3])
+def test_scales(R, scale, f32_scores):
+    check(R, 1, 4, 2, 70, 130, 64, 1, f32_scores, scale=scale)
