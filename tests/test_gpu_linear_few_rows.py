@@ -79,3 +79,20 @@ def test_few_rows_two_biases(R, m, k, n):
     # the three additions after the sum: a rounding each of what they add
     extra = 2.0 ** -23 * (np.abs(b) + np.abs(b2) + np.abs(z) + np.abs(r))
     assert np.all(np.abs(got.astype(np.float64) - want) <= 2.0 ** -8 * np.abs(want) + 2 * spread(x, w) + extra + 2.0 ** -20)
+
+
+@pytest.mark.parametrize("m,n", [(9, 68), (31, 132)])
+@pytest.mark.parametrize("splits", [2, 3, 5, 7, 8, 9, 13])
+def test_parts_of_k_by_batches(R, monkeypatch, splits, m, n):
+    """Nine rows and more with K cut over blocks: the last block reads the parts eight, four, two, one at a time, with the residual
+    beside them; the bits of the separate summing pass."""
+    k = 2048 * (splits - 1) + 224
+    g = np.random.Generator(np.random.PCG64(m + splits))
+    x, w = rand(g, (m, k), "bf16"), rand(g, (n, k), "bf16", k ** -0.5)
+    b, r = rand(g, (n,), "bf16"), rand(g, (m, n), "bf16")
+    args = up(x, "bf16"), up(w, "bf16"), up(b, "bf16"), None, up(r, "bf16")
+    got = down(R.linear(*args))
+    monkeypatch.setenv("RAI_HIP_NO_FUSED_SPLITK", "1")
+    np.testing.assert_array_equal(got, down(R.linear(*args)))
+    full = x.astype(np.float64) @ w.astype(np.float64).T + b + r
+    assert np.all(np.abs(got - full) <= 2.0 ** -8 * np.abs(full) + spread(x, w))
