@@ -1830,36 +1830,52 @@ static bool no_k64() {   // read per call: tests compare both forms in one proce
   return e && *e && *e != '0';
 }
 
+// 256 x 256 tiles cover a good half of the CUs.
+static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 256) * ((a.N + 255) / 256)) >= 17 * kNumCU; }
+
 // Which of the tiles with K stages of 64 serves a product, and over how many parts of K, by what the kernels' own times make
-// of it (fitted to 390 products of 65 to 2100 rows, every tile, one to eight parts, weights from the caches and from HBM; what
-// is picked takes 1 % more than the best of them in the mean).  An XCD has 32 CUs and a run of tiles of its own, so rounds are
+// of it (fitted to 170 products of 9 to 16384 rows, every tile, one to eight parts, weights from the caches and from HBM; what
+// is picked takes 2 % more than the best of them in the mean).  An XCD has 32 CUs and a run of tiles of its own, so rounds are
 // counted there: over the whole chip 36 tiles in seven parts look like one round of 256 CUs, but five tiles on an XCD are 35
 // blocks and two rounds (333 x 8960 x 1536: 38.7 us, in five parts 26.9).  Blocks share a CU: `stage` is the time of 64 of K with
 // one, two, three of them on it, `end` what a tile takes besides, to start and to write its outputs, `cut` the same where it
-// writes partial sums.  3 us are the launch; a K split adds 3.7 us (a launch) and 0.55 us per MB of partial sums, and leaves every
-// part four stages; partial sums in rows off 16-byte boundaries cost 2.2 us per MB of outputs more.
-enum { kTile128 = 0, kTile128Deep, kTile128x64, kTile64 };
+// writes partial sums.  3 us are the launch; a K split adds 3.5 us (a launch) and 0.53 us per MB of partial sums, and leaves every
+// part four stages; partial sums in rows off 16-byte boundaries cost 2.2 us per MB of outputs more.  A norm of the finished rows rides on
+// the pass that sums the parts and is a launch of 5 us without one.
+// 128 x 128 with eight waves (4 x 2, 32 x 64 each, two to a SIMD) took the place of four waves in two and four stages: 333 x 8960 x 1536
+// 20.5 to 18.9 us, 2000 x 2048 x 2048 22.7 to 21.1.  128 x 256 and 192 x 256 (eight waves, three and two stages) serve where 256 x 256
+// leaves a last round nearly empty: 1200 x 16384 x 2048 108 to 97 us, 3000 x 4096 x 4096 105 to 88, 777 x 22528 x 2048 114 to 91.
+enum { kTile128 = 0, kTile128x64, kTile64, kTile128x256, kTile256x192, kTile192x256, kTile256, kTileStreamK };
 struct TileCost { int bm, bn, share; float stage[3], end, cut; };
-static const TileCost kTileCosts[] = {{128, 128, 2, {0.63f, 0.775f}, 2.7f, 0.6f},  {128, 128, 1, {0.455f}, 4.0f, 2.0f},
-                                      {128, 64, 2, {0.315f, 0.535f}, 1.75f, 0.5f}, {64, 64, 3, {0.24f, 0.365f, 0.53f}, 0.8f, 0.f}};
+static const TileCost kTileCosts[] = {{128, 128, 1, {0.45f}, 2.9f, 1.5f},       {128, 64, 2, {0.32f, 0.56f}, 2.15f, 1.0f}, {64, 64, 3, {0.256f, 0.406f, 0.626f}, 0.67f, 0.46f},
+                                      {128, 256, 1, {0.77f}, 6.2f, 2.9f}, {256, 192, 1, {1.16f}, 8.2f, 0.f},       {192, 256, 1, {1.02f}, 8.9f, 4.8f},
+                                      {256, 256, 1, {1.29f}, 11.3f, 3.7f}};
 struct TilePlan { int tile, splits; };
-static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int last = kTile64) {
+static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int last = kTileStreamK) {
   const int stages = a.K / 64;
   const float part_mb = (float)a.M * a.N * 4e-6f;
   TilePlan best = {first, 1};
   float least = 0.f;
-  for (int t = first; t <= last; ++t) {
+  for (int t = first; t <= last && t < kTileStreamK; ++t) {
     const TileCost &c = kTileCosts[t];
     const int64_t tiles = (int64_t)((a.M + c.bm - 1) / c.bm) * ((a.N + c.bn - 1) / c.bn);
     for (int s = 1; s <= 12; ++s) {
-      if (s > 1 && (stages / s < 4 || !a.splitk_ws || (size_t)s * a.M * a.N * sizeof(float) > a.splitk_ws_bytes)) break;
+      if (s > 1 && (a.force_splits == 1 || stages / s < 4 || !a.splitk_ws || (size_t)s * a.M * a.N * sizeof(float) > a.splitk_ws_bytes)) break;
       const int64_t per_cu = ((tiles + kXcds - 1) / kXcds * s + kNumCU / kXcds - 1) / (kNumCU / kXcds);
       const int left = (int)(per_cu % c.share);
       const float stage = per_cu / c.share * c.stage[c.share - 1] + (left ? c.stage[left - 1] : 0.f);
       const float cost = 3.f + stage * ((stages + s - 1) / s) +
-                         (s > 1 ? 3.7f + 0.55f * s * part_mb + (a.N % 4 ? 2.2f * part_mb : 0.f) + per_cu * c.cut : per_cu * c.end);
+                         (s > 1 ? 3.5f + 0.53f * s * part_mb + (a.N % 4 ? 2.2f * part_mb : 0.f) + per_cu * c.cut : per_cu * c.end + (a.post_ln_out ? 5.f : 0.f));
       if ((t == first && s == 1) || cost < least) { least = cost; best = {t, s}; }
     }
+  }
+  // Stream-K over 256 x 256 tiles: no round is left empty, for an exchange of the shares: 21 us with two of them to a tile, 94 with three
+  // (4096 x 10240 x 2560 in 215 us for 222 of whole tiles, 16384 x 1536 x 8960 366 for 411 of 256 x 192).
+  StreamKPlan sk;
+  if (last == kTileStreamK && has_huge_tiles(a) && streamk_applies(a, 64, &sk)) {
+    const TileCost &c = kTileCosts[kTile256];
+    const float rounds = (float)(((a.M + 255) / 256) * ((a.N + 255) / 256)) / kNumCU;
+    if (3.f + rounds * (c.end + c.stage[0] * stages) + (sk.k.max_parts <= 2 ? 21.f : 94.f) < least) best = {kTileStreamK, 1};
   }
   return best;
 }
@@ -1899,18 +1915,22 @@ static int tile_splits(const LinearArgs &a) {
   return splits;
 }
 
-// 256 x 256 tiles (or what stands in for them) once these cover a good half of the CUs, see launch_linear_bf16_mfma.
-static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 256) * ((a.N + 255) / 256)) >= 17 * kNumCU; }
 // RAI_HIP_GEMM_TILE, read per call, and the names of the tiles above in it; a tile that it names gets the split of its own.
 static const char *forced_tile() { return getenv("RAI_HIP_GEMM_TILE"); }
-static const char *const kTileNames[] = {"128x128k64", "128x128deep", "128x64", "64x64"};
+static const struct { const char *name; int tile; } kTileNames[] = {{"128x128k64", kTile128}, {"128x128deep", kTile128}, {"128x64", kTile128x64},
+                                                                   {"64x64", kTile64},        {"128x256", kTile128x256}, {"192x256", kTile192x256}};
+static int named_tile(const char *knob) {   // -1: none of them
+  for (const auto &t : kTileNames)
+    if (!strcmp(knob, t.name)) return t.tile;
+  return -1;
+}
 static TilePlan tile_plan(const LinearArgs &a) {
   if (const char *knob = forced_tile()) {
-    for (int t = kTile128; t <= kTile64; ++t)
-      if (!strcmp(knob, kTileNames[t])) return a.K % 64 || a.force_splits > 0 ? TilePlan{t, tile_splits(a)} : tile_plan_k64(a, t, t);
+    const int t = named_tile(knob);
+    if (t >= 0) return a.K % 64 || a.force_splits > 0 ? TilePlan{t, tile_splits(a)} : tile_plan_k64(a, t, t);
     return {kTile128, tile_splits(a)};
   }
-  if (a.K % 64 || no_k64() || a.force_splits > 0 || has_huge_tiles(a)) return {kTile128, tile_splits(a)};
+  if (a.K % 64 || no_k64() || a.force_splits > 1) return {kTile128, tile_splits(a)};
   return tile_plan_k64(a);
 }
 
@@ -1948,10 +1968,20 @@ bool linear_fuses_post_norm(const LinearArgs &a) {
 }
 
 static int launch_tile_k64(hipStream_t st, const LinearArgs &a, TilePlan tile) {
-  if (tile.tile == kTile64) return launch_cfg_dma<64, 64, 3, 0>(st, a, tile.splits);
-  if (tile.tile == kTile128x64) return launch_cfg_dma<128, 64, 3, 0>(st, a, tile.splits);
-  if (tile.tile == kTile128Deep) return launch_cfg_dma<128, 128, 4, 0>(st, a, tile.splits);
-  return launch_cfg_dma<128, 128, 2, 0>(st, a, tile.splits);
+  switch (tile.tile) {
+    case kTile64: return launch_cfg_dma<64, 64, 3, 0>(st, a, tile.splits);
+    case kTile128x64: return launch_cfg_dma<128, 64, 3, 0>(st, a, tile.splits);
+    case kTile128x256: return launch_cfg_dma<128, 256, 3, 0, 4, 2>(st, a, tile.splits);
+    case kTile256x192: return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, tile.splits);
+    case kTile192x256: return launch_cfg_dma<192, 256, 2, 0, 4, 2>(st, a, tile.splits);
+    case kTile256: return launch_cfg_dma<256, 256, 2, 0, 4>(st, a, tile.splits);
+    case kTileStreamK: {
+      StreamKPlan plan;
+      RAI_REQUIRE(streamk_applies(a, 64, &plan), RAI_ERR_UNSUPPORTED, "linear: stream-K does not apply to %dx%dx%d", a.M, a.N, a.K);
+      return launch_streamk<2>(st, a, plan);
+    }
+    default: return launch_cfg_dma<128, 128, 4, 0, 2, 4>(st, a, tile.splits);
+  }
 }
 
 int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
@@ -1996,17 +2026,17 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
     if (mt == 3) return launch_mfma_skinny<3>(st, a);
     return launch_mfma_skinny<4>(st, a);
   }
-  const int tiles = ((a.M + 127) / 128) * ((a.N + 127) / 128);
   const TilePlan tile = tile_plan(a);
   const int splits = tile.splits;
-  // Tile choice.  The LDS-DMA kernels stream K tiles straight into LDS: the 256 x 256 tile, 256 x 192 or stream-K over
-  // either where there are tiles enough (below); otherwise what tile_plan_k64 says, or 128 x 128 with K tiles of 32.
-  // RAI_HIP_GEMM_TILE = "64x64" | "128x64" | "128x128" | "128x128k64" | "128x128deep" | "256x128" | "256x192" | "256x256" |
-  // "256x256x8w" | "256x256x8wk64" | "streamk" | "streamk64" | "classic" overrides (tuning aid; a form that does not apply to
-  // the shape is an error).
+  // Tile choice.  The LDS-DMA kernels stream K tiles straight into LDS, with stages of 64 where K allows (whole 128-byte lines per request;
+  // RAI_HIP_NO_K64: never): what tile_plan_k64 says.  Other K: 256 x 256 in its eight-wave form (one block per CU, 4 LDS stages of 32, two
+  // waves per SIMD) or stream-K over it once its tiles cover a good half of the CUs, 128 x 128 with three stages below that.
+  // RAI_HIP_GEMM_TILE = "64x64" | "128x64" | "128x128" | "128x128k64" | "128x128deep" (the same) | "128x256" | "192x256" | "256x128" |
+  // "256x192" | "256x256" | "256x256x8w" | "256x256x8wk64" | "streamk" | "streamk64" | "classic" overrides (tuning aid; a form that does
+  // not apply to the shape is an error).
   const char *knob = forced_tile();
   if (knob) {
-    if (!strcmp(knob, kTileNames[tile.tile])) {
+    if (named_tile(knob) >= 0) {
       RAI_REQUIRE(a.K % 64 == 0, RAI_ERR_UNSUPPORTED, "linear: RAI_HIP_GEMM_TILE=%s needs K %% 64 == 0 (%dx%dx%d)", knob, a.M, a.N, a.K);
       return launch_tile_k64(st, a, tile);
     }
@@ -2032,40 +2062,9 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
       return bk == 64 ? launch_streamk<2>(st, a, plan) : launch_streamk<4>(st, a, plan);
     }
   }
-  const int huge_tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256);
-  // 256x256 in its eight-wave form (one block per CU, 4 LDS stages, two waves per SIMD) once its tiles cover a good
-  // half of the CUs: the tile with the most flops per byte drawn from L2, which is what bounds these kernels.
-  // Measured against the smaller tiles: 16384 x 8960 x 1536 845 against 736 TFLOP/s, 16384 x 2048 x 1536 983 against
-  // 834, 4096 x 10240 x 2560 896 against 789, 4096 x 2560 x 10240 (160 tiles) 837 against 650, 512 x 17920 x 2560
-  // (140 tiles) 689 against 621; with 128 tiles or fewer the smaller tiles win (4096 x 2048 x 2048: 618 against 760).
-  // The four-wave 256x256 form is 3-9 % behind the eight-wave one everywhere.
-  if (splits == 1 && has_huge_tiles(a)) {
-    // K tiles of 64 (whole 128-byte lines per request) where K allows; RAI_HIP_NO_K64 keeps the tiles of 32
-    const bool k64 = a.K % 64 == 0 && !no_k64();
-    StreamKPlan plan;
-    const int tiles_192 = ((a.M + 255) / 256) * ((a.N + 191) / 192);
-    const int rounds_192 = (tiles_192 + kNumCU - 1) / kNumCU;
-    if (streamk_applies(a, k64 ? 64 : 32, &plan)) {
-      // Whole rounds of 256 x 192 tiles against stream-K over 256 x 256 ones, in us per tile from the two kernels'
-      // measured times (K = 1536 and 8960, all CUs busy): short K makes the exchange of the shares expensive next
-      // to the tiles themselves (16384 x 1536 x 1536: 512 tiles of 256 x 192 in 80 us, stream-K over 384 in 90 us;
-      // at K = 8960 stream-K wins, 433 against 456 us).
-      const float st64 = (float)(a.K / 64);
-      const float t256 = 5.8f + 1.69f * st64, t192 = 1.1f + 1.62f * st64;
-      const float est_sk = (float)huge_tiles / kNumCU * t256 + (plan.k.max_parts <= 2 ? 18.f : 39.f);
-      if (k64 && rounds_192 * t192 < 0.95f * est_sk) return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, splits);
-      return k64 ? launch_streamk<2>(st, a, plan) : launch_streamk<4>(st, a, plan);
-    }
-    // 256 x 192 (eight waves as 4 x 2, 64 x 96 each) where its tiles need no more rounds over the CUs than the
-    // 256 x 256 ones: the same round then holds three quarters of the work per CU, spread over more of them
-    // (512 x 17920 x 2560 with cold weights: 188 tiles in 64.7 us against 140 tiles in 71.2 us)
-    if (k64 && rounds_192 <= (huge_tiles + kNumCU - 1) / kNumCU)
-      return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, splits);
-    return k64 ? launch_cfg_dma<256, 256, 2, 0, 4>(st, a, splits) : launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
-  }
-  // 128 x 128 with two stages of K 64 (two blocks per CU) where K allows: 12-22 % over three stages of 32 on the
-  // prefill shapes with cold weights (512 x 10240 x 2560: 66 -> 55 us)
   if (a.K % 64 == 0 && !no_k64()) return launch_tile_k64(st, a, tile);
+  StreamKPlan plan;
+  if (splits == 1 && has_huge_tiles(a)) return streamk_applies(a, 32, &plan) ? launch_streamk<4>(st, a, plan) : launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
   return launch_cfg_dma<128, 128, 3, 2>(st, a, splits);
 }
 

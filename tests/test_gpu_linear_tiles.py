@@ -90,3 +90,18 @@ def test_tiles_gated(R, m, k, n):
     want = gate / (1 + np.exp(-gate)) * upv
     got = down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), act="silu", glu=True)).astype(np.float64)
     assert np.all(np.abs(got - want) <= 4 * 2.0 ** -8 * (np.abs(gate) + 1) * (np.abs(upv) + 1))
+
+
+# The eight-wave tiles of 256 columns: short K (stages fewer than the pipeline), ragged rows and columns, parts of K.
+@pytest.mark.parametrize("m,k,n", [(65, 64, 8), (129, 128, 257), (193, 192, 520), (383, 256, 1031), (385, 1088, 264), (130, 2560, 776)])
+@pytest.mark.parametrize("tile", ["128x256", "192x256"])
+def test_wide_tiles(R, monkeypatch, tile, m, k, n):
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", tile)
+    test_tiles(R, m, k, n)
+    test_tiles_gated(R, m, k, 8 * (n // 8))
+
+
+# What the rule picks by itself: small tiles cut over K, 128 x 128, 128 x 256, 192 x 256, 256 x 192, 256 x 256, stream-K.
+@pytest.mark.parametrize("m,k,n", [(100, 4096, 1024), (333, 512, 8960), (777, 256, 8192), (777, 192, 22528), (2048, 320, 4096), (4096, 128, 10240)])
+def test_what_the_rule_picks(R, m, k, n):
+    test_tiles(R, m, k, n)
