@@ -917,16 +917,26 @@ __global__ void __launch_bounds__(256) k_splitk_epilogue(LinearArgs a, int split
 // ITEMS columns).  The sums over the partial products, bias / activation / residual and the bf16 store are element
 // by element, so they are shared out: every wave takes a quarter of the row's 16-byte packs (512 rows are then eight
 // waves per CU with one round of loads each, instead of two waves with two rounds).  The stored (rounded) row goes
-// through LDS to the first wave, which runs LayerNorm on it with the arithmetic of the stand-alone norm kernel -- same
-// per-lane order, same wave reductions -- so fusing changes no bit (rai-nn/src/layer_norm.rs:32-42).
+// through LDS to the block, which runs LayerNorm on it with the arithmetic of the stand-alone norm kernel's block form -- same
+// order in a thread, same reductions -- so fusing changes no bit (rai-nn/src/layer_norm.rs:32-42) as long as that form serves the rows.
 template <int ITEMS>
 __global__ void __launch_bounds__(256) k_splitk_epilogue_ln(LinearArgs a, int splits, const float *partial) {
   constexpr int NWV = 4;                                 // waves per row
   constexpr int JT = (ITEMS * 64 / NWV + 63) / 64;       // packs per lane in the summing part
+  constexpr int NI = (ITEMS + 3) / 4;                    // packs per thread in the norm
   __shared__ u32x4 rowbuf[64 * ITEMS];
+  __shared__ float sums[2][4];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int row = blockIdx.x;
   const int packs = a.N / 8;
+  const uint16_t *lw = (const uint16_t *)a.post_ln_w, *lb = (const uint16_t *)a.post_ln_b;
+  u32x4 lwr[NI], lbr[NI];   // the norm's weights, asked for with everything else
+#pragma unroll
+  for (int it = 0; it < NI; ++it) {
+    const int p = threadIdx.x + it * 256 < packs ? threadIdx.x + it * 256 : 0;
+    if (lw) lwr[it] = *reinterpret_cast<const u32x4 *>(lw + p * 8);
+    if (lb) lbr[it] = *reinterpret_cast<const u32x4 *>(lb + p * 8);
+  }
   const int quarter = (packs + NWV - 1) / NWV;
   const int64_t total = (int64_t)a.M * a.N;
   const uint16_t *bias = (const uint16_t *)a.bias, *bias2 = (const uint16_t *)a.bias2;
@@ -1000,54 +1010,51 @@ __global__ void __launch_bounds__(256) k_splitk_epilogue_ln(LinearArgs a, int sp
     }
   }
   __syncthreads();
-  if (wv != 0) return;
-  // ---- LayerNorm of the stored row, one wave, pack p = lane + 64 it
-  float v[ITEMS][8];
-  float s = 0.f;
+  // ---- LayerNorm of the stored row: thread t has packs t, t + 256, ..
+  float v[NI][8], s = 0.f;
 #pragma unroll
-  for (int it = 0; it < ITEMS; ++it) {
-    const int p = lane + it * 64;
-    if (p < packs) {
-      unpack8(rowbuf[p], v[it]);
+  for (int it = 0; it < NI; ++it) {
+    const int p = threadIdx.x + it * 256;
+    if (p < packs) unpack8(rowbuf[p], v[it]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s += v[it][e];
+    for (int e = 0; e < 8; ++e) {
+      if (p >= packs) v[it][e] = 0.f;
+      s += v[it][e];
     }
   }
-  s = wave_sum(s);
-  const float mean = s / (float)a.N;
-  float q = 0.f;
+  auto block_sum = [&](float x, float (&part)[4]) {
+    x = wave_sum(x);
+    if (lane == 0) part[wv] = x;
+    __syncthreads();
+    return (part[0] + part[1]) + (part[2] + part[3]);
+  };
+  const float mean = block_sum(s, sums[0]) / (float)a.N;
+  s = 0.f;
 #pragma unroll
-  for (int it = 0; it < ITEMS; ++it) {
-    const int p = lane + it * 64;
-    if (p < packs) {
+  for (int it = 0; it < NI; ++it)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float d = v[it][e] - mean;
-        q += d * d;
-      }
+    for (int e = 0; e < 8; ++e) {
+      const float d = threadIdx.x + it * 256 < packs ? v[it][e] - mean : 0.f;
+      s += d * d;
     }
-  }
-  q = wave_sum(q);
-  const float scale = 1.0f / sqrtf(q / (float)a.N + a.post_ln_eps);
-  const uint16_t *lw = (const uint16_t *)a.post_ln_w, *lb = (const uint16_t *)a.post_ln_b;
+  const float scale = 1.0f / sqrtf(block_sum(s, sums[1]) / (float)a.N + a.post_ln_eps);
 #pragma unroll
-  for (int it = 0; it < ITEMS; ++it) {
-    const int p = lane + it * 64;
+  for (int it = 0; it < NI; ++it) {
+    const int p = threadIdx.x + it * 256;
     if (p < packs) {
-      const int n = p * 8;
-      float wv[8], bv[8];
-      if (lw) unpack8(*reinterpret_cast<const u32x4 *>(lw + n), wv);
-      if (lb) unpack8(*reinterpret_cast<const u32x4 *>(lb + n), bv);
+      float wf[8], bf[8];
+      if (lw) unpack8(lwr[it], wf);
+      if (lb) unpack8(lbr[it], bf);
       uint32_t h[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         float y = (v[it][e] - mean) * scale;
-        if (lw) y *= wv[e];
-        if (lb) y += bv[e];
+        if (lw) y *= wf[e];
+        if (lb) y += bf[e];
         h[e] = f32_to_bf16_bits(y);
       }
       u32x4 o = {h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
-      *reinterpret_cast<u32x4 *>((uint16_t *)a.post_ln_out + (int64_t)row * a.N + n) = o;
+      *reinterpret_cast<u32x4 *>((uint16_t *)a.post_ln_out + (int64_t)row * a.N + p * 8) = o;
     }
   }
 }

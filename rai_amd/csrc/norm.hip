@@ -83,6 +83,71 @@ k_norm_wave(T *out, const T *x, const T *w, const T *b, int64_t rows, int64_t n,
   }
 }
 
+// A block to a row, x, w and b asked for together: the wave form above holds a long row in one wave's registers and asks for w and b when
+// it has the row's statistics, one more trip to memory, which many rows hide and few do not.  Bound by the launch and two trips
+// up to a thousand rows, by HBM beyond.  Measured (us, wave, block): f32 layer norm of 2560 columns, 1 row 5.8, 3.9, 256 rows 7.0, 4.0,
+// 8192 rows 29.0, 25.4; 4096 columns, 256 rows 9.5, 4.0; bf16 rms norm 1536, 1 row 4.3, 4.0, 4096 columns 16384 rows 57.6, 40.2.
+template <typename T, int V, int ITEMS>
+__global__ void __launch_bounds__(256) k_norm_row(T *out, const T *x, const T *w, const T *b, int64_t n, int64_t x_row_stride, float eps, int kind) {
+  __shared__ float sh[2][4];
+  const int tid = threadIdx.x, packs = (int)(n / V);
+  const T *xr = x + blockIdx.x * x_row_stride;
+  T *yr = out + blockIdx.x * n;
+  NPack<T, V> xk[ITEMS], wk[ITEMS], bk[ITEMS];
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it)
+    if (const int p = tid + it * 256; p < packs) {
+      xk[it] = *reinterpret_cast<const NPack<T, V> *>(xr + p * V);
+      if (w) wk[it] = *reinterpret_cast<const NPack<T, V> *>(w + p * V);
+      if (b) bk[it] = *reinterpret_cast<const NPack<T, V> *>(b + p * V);
+    }
+  auto block_sum = [&](float v, float (&part)[4]) {
+    v = wave_sum(v);
+    if ((tid & 63) == 0) part[tid >> 6] = v;
+    __syncthreads();
+    return (part[0] + part[1]) + (part[2] + part[3]);
+  };
+  float v[ITEMS][V], s = 0.f, mean = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it)
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      v[it][j] = tid + it * 256 < packs ? (float)Scalar<T>::load(&xk[it].v[j]) : 0.f;
+      s += kind == kLayerNorm ? v[it][j] : v[it][j] * v[it][j];
+    }
+  s = block_sum(s, sh[0]);
+  if (kind == kLayerNorm) {
+    mean = s / (float)n;
+    s = 0.f;
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it)
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        const float d = tid + it * 256 < packs ? v[it][j] - mean : 0.f;
+        s += d * d;
+      }
+    s = block_sum(s, sh[1]);
+  }
+  const float scale = 1.0f / sqrtf(s / (float)n + eps);
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int p = tid + it * 256;
+    if (p >= packs) continue;
+    NPack<T, V> ok;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      float y = (v[it][j] - mean) * scale;
+      if (w) {
+        const float wf = (float)Scalar<T>::load(&wk[it].v[j]);
+        y *= kind == kRmsNormAddOne ? 1.0f + wf : wf;
+      }
+      if (b) y += (float)Scalar<T>::load(&bk[it].v[j]);
+      Scalar<T>::store(&ok.v[j], y);
+    }
+    *reinterpret_cast<NPack<T, V> *>(yr + p * V) = ok;
+  }
+}
+
 // Fallback for rows that do not fit the register budget or are unaligned: one
 // block per row, the row is re-read from L2 for each pass.
 template <typename T>
@@ -410,6 +475,28 @@ static int norm_impl(int dev, const rai_hip_tensor *x, const rai_hip_tensor *w, 
   bool aligned = (n % v == 0) && (row_stride % v == 0) && al(x) && al(out) && al(w) && al(b);
   const int64_t packs = n / v;
   if (aligned && x->dtype != RAI_F64 && packs <= 64 * 16) {
+    // 16-bit rows beyond 2048 of them go to the wave form unless they fill three quarters of a block's threads (us, wave, block, 8192
+    // rows: bf16 layer norm 2560 19.8, 21.4, 800 8.8, 11.7, rms norm 1024 7.8, 9.3; 2048 15.4, 13.1, 4096 30.4, 21.6); f32 rows never.
+    if (x->dtype == RAI_F32 || rows <= 8 * kNumCU || 4 * packs > 3 * ((packs + 255) / 256 * 256)) {
+      RAI_REQUIRE(rows <= 0x7fffffff, RAI_ERR_UNSUPPORTED, "%s: too many rows", what);
+#define NORM_ROW(T, V, ITEMS)                                                                                          \
+  hipLaunchKernelGGL((k_norm_row<T, V, ITEMS>), dim3((unsigned)rows), dim3(256), 0, st, (T *)base_ptr(out),            \
+                     (const T *)base_ptr(x), w ? (const T *)base_ptr(w) : nullptr,                                     \
+                     b ? (const T *)base_ptr(b) : nullptr, n, row_stride, (float)eps, kind)
+#define NORM_ROW_ITEMS(T, V)                   \
+  do {                                         \
+    if (packs <= 256) NORM_ROW(T, V, 1);       \
+    else if (packs <= 512) NORM_ROW(T, V, 2);  \
+    else if (packs <= 768) NORM_ROW(T, V, 3);  \
+    else NORM_ROW(T, V, 4);                    \
+  } while (0)
+      if (x->dtype == RAI_F32) NORM_ROW_ITEMS(float, 4);
+      else if (x->dtype == RAI_BF16) NORM_ROW_ITEMS(bf16_raw, 8);
+      else NORM_ROW_ITEMS(f16_raw, 8);
+#undef NORM_ROW_ITEMS
+#undef NORM_ROW
+      return launch_check(what);
+    }
     int64_t blocks = (rows + 3) / 4;
     int grid = (int)(blocks < kNumCU * 32 ? blocks : kNumCU * 32);
 #define NORM_LAUNCH(T, V, ITEMS)                                                                                  \
@@ -423,8 +510,7 @@ static int norm_impl(int dev, const rai_hip_tensor *x, const rai_hip_tensor *w, 
     else if (packs <= 64 * 10) NORM_LAUNCH(T, V, 10); \
     else NORM_LAUNCH(T, V, 16);                    \
   } while (0)
-    if (x->dtype == RAI_F32) NORM_BY_ITEMS(float, 4);
-    else if (x->dtype == RAI_BF16) NORM_BY_ITEMS(bf16_raw, 8);
+    if (x->dtype == RAI_BF16) NORM_BY_ITEMS(bf16_raw, 8);
     else NORM_BY_ITEMS(f16_raw, 8);
 #undef NORM_BY_ITEMS
 #undef NORM_LAUNCH

@@ -1,0 +1,35 @@
+"""Norms around the sizes where a row goes from a block to a wave and a thread from one 16-byte piece to the next."""
+import numpy as np
+import pytest
+
+from tests.util import down, rand, up
+
+pytestmark = pytest.mark.gpu
+U = {"f32": 2.0 ** -24, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}
+
+
+@pytest.mark.parametrize("rows,n", [(1, 8), (3, 1016), (2, 2048), (5, 2056), (1, 4104), (2, 8192), (2048, 264), (2049, 264), (2049, 1536), (2051, 1544), (2050, 2048)])
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+def test_rows(hip, dt, rows, n):
+    from rai_amd import ops as R
+
+    if dt == "f32":
+        n //= 2   # the same number of 16-byte pieces
+    g = np.random.Generator(np.random.PCG64(rows + n))
+    x, w, b = rand(g, (rows, n), dt, 2.0), rand(g, (n,), dt), rand(g, (n,), dt)
+    d = x.astype(np.float64)
+
+    def check(got, mean, scale, w, b):
+        y = (d - mean) * scale
+        want = y * w + b
+        # the statistics' sums are within n + 8 roundings of n (terms of one sign, or below 2 in the mean), halved by the root; a
+        # handful of roundings of the factors; the result's own
+        tol = (n + 16) * 2.0 ** -24 * (np.abs(y) + 2) * np.abs(w) + 4 * 2.0 ** -24 * np.abs(b) + 2 * U[dt] * np.abs(want) + 2.0 ** -24
+        assert np.all(np.abs(down(got).astype(np.float64) - want) <= tol)
+
+    ms = (d * d).mean(-1, keepdims=True)
+    check(R.rms_norm(up(x, dt), up(w, dt), 1e-6), 0.0, 1 / np.sqrt(ms + 1e-6), w, 0.0)
+    check(R.rms_norm(up(x, dt), up(w, dt), 1e-6, True), 0.0, 1 / np.sqrt(ms + 1e-6), 1.0 + w, 0.0)
+    mean, var = d.mean(-1, keepdims=True), d.var(-1, keepdims=True)
+    check(R.layer_norm(up(x, dt), up(w, dt), up(b, dt), 1e-5), mean, 1 / np.sqrt(var + 1e-5), w, b)
+    check(R.layer_norm(up(x, dt), None, None, 1e-5), mean, 1 / np.sqrt(var + 1e-5), 1.0, 0.0)
