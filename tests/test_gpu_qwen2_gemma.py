@@ -148,3 +148,19 @@ def test_grouped_query_decode_attention_long_context(hip, name, splits, keys, mo
         check_tokens(tok, want, "bf16")
         nxt = np.argmax(want, -1).astype(np.uint32).reshape(3, 1)
     dec.close()
+
+
+@pytest.mark.parametrize("heads,kv,dim,context", [(4, 1, 64, 64), (8, 2, 64, 65), (8, 1, 128, 96), (12, 2, 128, 97), (16, 1, 64, 128), (8, 1, 256, 33),
+                                                  (8, 1, 256, 83), (4, 1, 256, 128), (8, 1, 128, 129)])
+def test_decode_attention_of_short_contexts(hip, heads, kv, dim, context):
+    """Up to 128 keys one block of 64, 96 or 128 keys writes a sequence's result itself; beyond, two are merged.  The cache is filled to its
+    last place."""
+    cfg = qwen2.Config("qwen2", 300, 192, 256, 1, heads, kv, "silu", max_position_embeddings=256, head_dim=dim)
+    dec, ref = make(cfg, "bf16", max_batch=3, max_context=context)
+    ids = np.random.Generator(np.random.PCG64(context)).integers(0, cfg.vocab_size, (3, context - 2)).astype(np.uint32)
+    for step in range(3):
+        logits, _ = dec.forward(ids)
+        want = ref.fwd(ids)
+        assert_close(logits, want, "bf16", f"step {step}")
+        ids = np.argmax(want, -1).astype(np.uint32).reshape(3, 1)
+    dec.close()
