@@ -369,20 +369,67 @@ __global__ void __launch_bounds__(256) k_delta_out_wide(DeltaArgs a) {
 // anything is computed.  Both sums over the state's rows are formed from the decayed state before the write,
 //   S^T q after the write = (g S)^T q + (k . q) u,
 // so one exchange through LDS serves v's correction and the read-out.
+// Latency and what one CU can ask for bound it: a head's block moves 128 KiB of state and 64 KiB of factors, and there are only `heads` blocks.
+// 16 heads of 128 x 128, ranks 128, bf16: 11.1 us with the inputs asked for where they are used, 9.7 us all at once.
 constexpr int kStepThreads = 512;
-template <typename T> __device__ __forceinline__ float factor_row(const T *w, const T *x, int rank, int part) {
-  constexpr int V = 16 / sizeof(T);
+// A quarter (`part`) of the dot product of two rows, summed over four lanes.  The first kAhead pieces are asked for by fetch(), which needs
+// nothing that is computed here.
+template <typename T> struct FactorRow {
+  static constexpr int V = 16 / sizeof(T), kAhead = 4;
   struct alignas(16) Pack { T v[V]; };
-  float acc = 0.f;
-  for (int k = part * V; k < rank; k += 4 * V) {
-    const Pack p = *reinterpret_cast<const Pack *>(w + k), y = *reinterpret_cast<const Pack *>(x + k);
+  Pack p[kAhead], y[kAhead];
+  __device__ __forceinline__ void fetch(const T *w, const T *x, int rank, int part) {   // (pieces past the end re-read the first)
 #pragma unroll
-    for (int e = 0; e < V; ++e) acc = fmaf((float)Scalar<T>::load(&p.v[e]), (float)Scalar<T>::load(&y.v[e]), acc);
+    for (int i = 0; i < kAhead; ++i) {
+      const int k = part * V + i * 4 * V, at = k < rank ? k : part * V < rank ? part * V : 0;
+      p[i] = *reinterpret_cast<const Pack *>(w + at);
+      y[i] = *reinterpret_cast<const Pack *>(x + at);
+    }
   }
-  acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), 0xB1, 0xf, 0xf, true));
-  acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), 0x4E, 0xf, 0xf, true));
-  return acc;
-}
+  __device__ __forceinline__ float sum(const T *w, const T *x, int rank, int part) const {
+    float acc = 0.f;
+    auto add = [&](const Pack &a, const Pack &b) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) acc = fmaf((float)Scalar<T>::load(&a.v[e]), (float)Scalar<T>::load(&b.v[e]), acc);
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i)
+      if (part * V + i * 4 * V < rank) add(p[i], y[i]);
+    for (int k = part * V + kAhead * 4 * V; k < rank; k += 4 * V) add(*reinterpret_cast<const Pack *>(w + k), *reinterpret_cast<const Pack *>(x + k));
+    acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), 0xB1, 0xf, 0xf, true));
+    acc += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), 0x4E, 0xf, 0xf, true));
+    return acc;
+  }
+};
+
+// conv_silu for one token and up to kAhead taps, in its order.  All of the ring's places are asked for, so that no place waits for the
+// position; the place that this token's input goes to is among them, possibly while another head's block writes it, and is not used.
+template <typename T> struct ConvStep {
+  static constexpr int kAhead = 4;
+  float w[kAhead], r0, r1, r2, r3, x;
+  __device__ __forceinline__ void fetch(const DeltaArgs &a, int b, int c) {
+    const int taps = a.s.taps;
+    auto ring = [&](int at) { return ld<T>(a.ring, ((int64_t)b * taps + (at < taps ? at : 0)) * a.s.channels + c); };
+    x = ld<T>(a.dn, b * a.s.ldn + c);
+    r0 = ring(0); r1 = ring(1); r2 = ring(2); r3 = ring(3);
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) w[j] = ld<T>(a.conv, (int64_t)c * taps + (j < taps ? j : 0));
+  }
+  __device__ __forceinline__ float silu(int taps, int pos0) const {
+    const float p0 = r0, p1 = r1, p2 = r2, p3 = r3;   // (by value: chosen as addresses they would go through scratch memory)
+    float y = 0.f;
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int t = j - (taps - 1), at = (pos0 + t) % taps;
+      float old = p0;
+      old = at == 1 ? p1 : old;
+      old = at == 2 ? p2 : old;
+      old = at == 3 ? p3 : old;
+      if (j < taps) y = fmaf(t == 0 ? x : pos0 + t >= 0 ? old : 0.f, w[j], y);
+    }
+    return y * dl_sigmoid(y);
+  }
+};
 
 template <typename T, int NI, bool FACTORS>
 __global__ void __launch_bounds__(kStepThreads) k_delta_step(DeltaArgs a) {
@@ -393,41 +440,75 @@ __global__ void __launch_bounds__(kStepThreads) k_delta_step(DeltaArgs a) {
   const int CQ = z.Vp / 4, RG = kStepThreads / CQ, cq = tid % CQ, rg = tid / CQ;
   float *qs = st_lds, *ks = qs + z.Dk, *gs = ks + z.Dk, *vs = gs + z.Dk, *zs = vs + z.Vp, *us = zs + z.Vp, *red = us + z.Vp;   // red[2][RG][Vp]
   __shared__ float sums[4], part[kStepThreads / 64];
-  const int pos0 = a.state->pos;
+  // Everything whose place does not depend on the position is asked for along with it: the convolution's inputs, the low-rank factors' rows
+  // (tap by tap, row by row and piece by piece they were a dozen trips to memory one after the other), the state, the head's scalars.
+  const int inputs = 2 * z.Dk + z.Vp;
+  auto channel = [&](int i) { return i < z.Dk ? kv * z.Dk + i : i < 2 * z.Dk ? kd + kv * z.Dk + i - z.Dk : 2 * kd + h * z.Vp + i - 2 * z.Dk; };
+  const bool conv_ahead = z.taps <= ConvStep<T>::kAhead;
+  ConvStep<T> conv{};
+  if (conv_ahead) conv.fetch(a, b, channel(min(tid, inputs - 1)));
+  const int *pos_at = &a.state->pos;
+  FactorRow<T> rows[2];
+  const T *fw[2], *fx[2];
+  float bias[2];
+  if constexpr (FACTORS) {
+    const T *a1 = (const T *)a.dn + b * z.ldn + z.off_a1, *g1 = (const T *)a.dn + b * z.ldn + z.off_g1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = min((tid >> 2) + i * (kStepThreads / 4), z.Dk + z.Vp - 1);
+      const bool dec = r < z.Dk;
+      fw[i] = dec ? (const T *)a.a2 + (int64_t)(h * z.Dk + r) * a.a_rank : (const T *)a.g2 + (int64_t)(h * z.Vp + r - z.Dk) * a.g_rank;
+      fx[i] = dec ? a1 : g1;
+      rows[i].fetch(fw[i], fx[i], dec ? a.a_rank : a.g_rank, tid & 3);
+      bias[i] = dec ? ld<T>(a.dt_bias, h * z.Dk + r) : 0.f;
+    }
+  }
+  const float a_log = ld<T>(a.A_log, h), beta_in = ld<T>(a.dn, b * z.ldn + z.off_b + h), out_w = tid < z.Vp ? ld<T>(a.norm_w, tid) : 0.f;
   float *st = a.carried + ((int64_t)b * z.heads + h) * z.Dk * z.Vp;
   float4 S[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int r = rg + i * RG;
-    S[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (rg < RG && r < z.Dk && pos0 > 0) S[i] = *reinterpret_cast<const float4 *>(st + (int64_t)r * z.Vp + cq * 4);
+    S[i] = *reinterpret_cast<const float4 *>(st + (int64_t)(rg < RG && r < z.Dk ? r : 0) * z.Vp + cq * 4);
   }
+  const int pos0 = *pos_at;
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+    if (rg >= RG || rg + i * RG >= z.Dk || pos0 == 0) S[i] = make_float4(0.f, 0.f, 0.f, 0.f);   // (the first token's state has no value yet)
   // ---- convolutions; the ring's free place takes this token's inputs
-  for (int i = tid; i < 2 * z.Dk + z.Vp; i += kStepThreads) {
-    const int c = i < z.Dk ? kv * z.Dk + i : i < 2 * z.Dk ? kd + kv * z.Dk + i - z.Dk : 2 * kd + h * z.Vp + i - 2 * z.Dk;
-    (i < 2 * z.Dk ? qs : vs - 2 * z.Dk)[i] = conv_silu<T>(a, b, 0, pos0, c);   // ks follows qs
+  for (int i = tid; i < inputs; i += kStepThreads) {
+    const int c = channel(i);
+    (i < 2 * z.Dk ? qs : vs - 2 * z.Dk)[i] = conv_ahead && i == tid ? conv.silu(z.taps, pos0) : conv_silu<T>(a, b, 0, pos0, c);   // ks follows qs
     if (i >= 2 * z.Dk || h % rep == 0) ((T *)a.ring)[((int64_t)b * z.taps + pos0 % z.taps) * z.channels + c] = ((const T *)a.dn)[b * z.ldn + c];
   }
   // ---- decays and gate
-  const float rate = -expf(ld<T>(a.A_log, h));
+  const float rate = -expf(a_log);
   if constexpr (FACTORS) {
-    const T *a1 = (const T *)a.dn + b * z.ldn + z.off_a1, *g1 = (const T *)a.dn + b * z.ldn + z.off_g1;
-    for (int r = tid >> 2; r < z.Dk + z.Vp; r += kStepThreads / 4) {
+    auto row = [&](int r, float y, float dt) {
+      if ((tid & 3) != 0) return;
+      if (r < z.Dk) gs[r] = expf(rate * dl_softplus(y + dt));
+      else zs[r - z.Dk] = dl_sigmoid(y);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = (tid >> 2) + i * (kStepThreads / 4);
+      if (r < z.Dk + z.Vp) row(r, rows[i].sum(fw[i], fx[i], r < z.Dk ? a.a_rank : a.g_rank, tid & 3), bias[i]);
+    }
+    for (int r = (tid >> 2) + 2 * (kStepThreads / 4); r < z.Dk + z.Vp; r += kStepThreads / 4) {
       const bool dec = r < z.Dk;
-      const int n = dec ? h * z.Dk + r : h * z.Vp + r - z.Dk;
-      const float y = dec ? factor_row<T>((const T *)a.a2 + (int64_t)n * a.a_rank, a1, a.a_rank, tid & 3)
-                          : factor_row<T>((const T *)a.g2 + (int64_t)n * a.g_rank, g1, a.g_rank, tid & 3);
-      if ((tid & 3) == 0) {
-        if (dec) gs[r] = expf(rate * dl_softplus(y + ld<T>(a.dt_bias, n)));
-        else zs[r - z.Dk] = dl_sigmoid(y);
-      }
+      const T *w = dec ? (const T *)a.a2 + (int64_t)(h * z.Dk + r) * a.a_rank : (const T *)a.g2 + (int64_t)(h * z.Vp + r - z.Dk) * a.g_rank;
+      const T *x = (const T *)a.dn + b * z.ldn + (dec ? z.off_a1 : z.off_g1);
+      const int rank = dec ? a.a_rank : a.g_rank;
+      FactorRow<T> f;
+      f.fetch(w, x, rank, tid & 3);
+      row(r, f.sum(w, x, rank, tid & 3), dec ? ld<T>(a.dt_bias, h * z.Dk + r) : 0.f);
     }
   } else {
     for (int r = tid; r < z.Dk; r += kStepThreads)
       gs[r] = expf(rate * dl_softplus(a.decay[((int64_t)b * z.heads + h) * z.Dk + r] + ld<T>(a.dt_bias, h * z.Dk + r)));
     for (int c = tid; c < z.Vp; c += kStepThreads) zs[c] = dl_sigmoid(ld<T>(a.gate, ((int64_t)b * z.heads + h) * z.Vp + c));
   }
-  const float beta = dl_sigmoid(ld<T>(a.dn, b * z.ldn + z.off_b + h));
+  const float beta = dl_sigmoid(beta_in);
   __syncthreads();
   if (wave < 3) {   // |q|^2, |k|^2, k . q
     const float *x = wave == 0 ? qs : ks, *y = wave == 1 ? ks : qs;
@@ -456,6 +537,7 @@ __global__ void __launch_bounds__(kStepThreads) k_delta_step(DeltaArgs a) {
   float o = 0.f;
   if (tid < z.Vp) {
     float x = 0.f, y = 0.f;
+#pragma unroll 8
     for (int g = 0; g < RG; ++g) {
       x += red[g * z.Vp + tid];
       y += red[(RG + g) * z.Vp + tid];
@@ -481,7 +563,7 @@ __global__ void __launch_bounds__(kStepThreads) k_delta_step(DeltaArgs a) {
     float t = 0.f;
     for (int w = 0; w < kStepThreads / 64; ++w) t += part[w];
     const float r = 1.0f / sqrtf(t / (float)z.vdim + a.eps);
-    Scalar<T>::store((T *)a.out + b * a.ldo + h * z.Vp + tid, o * r * ld<T>(a.norm_w, tid) * zs[tid]);
+    Scalar<T>::store((T *)a.out + b * a.ldo + h * z.Vp + tid, o * r * out_w * zs[tid]);
   }
 }
 

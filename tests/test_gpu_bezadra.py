@@ -357,6 +357,21 @@ def test_trace_runner(hip, tmp_path):
             deep_close(np.fromfile(out / f"{k}.f32", "<f4").reshape(w.shape), w, dt, f"{name} step {k}")
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("conv,rank,dim,vdim", [(1, 64, 20, 36), (2, 65, 64, 64), (3, 128, 128, 128), (4, 129, 96, 40), (4, 300, 200, 120), (5, 200, 128, 128),
+                                                (9, 1, 300, 500)])
+def test_steps_of_one_token(hip, dt, conv, rank, dim, vdim):
+    """Token by token, twice through one state: convolutions of as many taps as are asked for ahead and of more, ranks of fewer and of more
+    pieces than that, more channels and rows than a block has threads for."""
+    cfg = bm.config([bm.delta(heads=4, kv_heads=2, dim=dim, vdim=vdim, conv=conv, ff=None)], width=128)
+    p = bezadra.random_params(cfg, dt, 31, a_rank=rank, g_rank=rank + 7)
+    ref, dec = bezadra.Model(cfg, p), bm.build(cfg, p, dt)
+    for n, seed in ((14, 1), (6, 2)):
+        ids = tokens(cfg, n, seed)
+        deep_close(bm.run_portions(dec, ids, [1])[0], ref.logits(ids), dt, f"{conv} taps, rank {rank}, sequence of {n}")
+    dec.close()
+
+
 def test_errors(hip):
     from rai_amd._lib import RaiHipError
     from rai_amd.config import decoder_from_config
