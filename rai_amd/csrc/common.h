@@ -58,11 +58,6 @@ int streamk_counters_reset(int dev, hipStream_t st);
 // Looks up this device's address of the fixed scratch array of the allocation-free argmax (reduce.hip); called once
 // per device, with that device current, while its context is created.
 int arg_static_scratch_init(int dev);
-// First stage of an argmax over the last axis of contiguous [rows, n] (bf16, f16 or f32): the axis is cut into `splits`
-// shares, and share s of row r leaves its best (value, index) under rai_hip_argmax's ordering in pval / pidx
-// [r * splits + s] (a share of NaNs only leaves a NaN).  The caller merges the shares (reduce.hip).
-int launch_argmax_partials(hipStream_t st, int dtype, const void *in, int64_t rows, int64_t n, int splits, float *pval,
-                           uint32_t *pidx);
 // The device's scratch block, which lives as long as the device context (grown on demand, never shrinks), for kernels
 // that need partial results.  A call keeps its hold on the block until it has enqueued the last kernel or copy that uses
 // it: another thread's work then comes behind it on the device's one stream, and nobody replaces the block between the

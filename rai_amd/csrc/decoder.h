@@ -167,6 +167,7 @@ struct rai_hip_decoder {
   int token_log_cap;
   float *choice_val;          // [max_batch][kChoiceMaxSplits]: best value of each share of a wide logits row
   uint32_t *choice_idx;       // and its index
+  uint32_t *choice_tickets;   // [max_batch]: shares of a row that have been scanned, zero between launches
   unsigned long long *head_best;   // one (value, row) word per block of the head kernel that also chooses the token
   char *hidden_copy;          // [max_rows, H]: the residual stream after the last layer, kept when a caller asks for it
   bool want_hidden;           // the running forward copies its final residual stream to hidden_copy

@@ -21,7 +21,7 @@
 
 namespace rai {
 
-constexpr int kChoiceMaxSplits = 64;  // shares a logits row is scanned in before the token choice
+constexpr int kChoiceMaxSplits = 64;  // shares a logits row is scanned in for the token choice
 constexpr int kGraphSteps = 8;  // single-token steps recorded in the multi-step decode graph
 
 // ------------------------------------------------------------------ small kernels
@@ -164,69 +164,86 @@ __global__ void k_set_state(DevState *st, int pos, int step) {
   st->done = 0;
 }
 
-// Tail of the token-selection kernels (every thread of the block calls it with the block's chosen token):
-// the token's embedding row becomes the next step's input x[b], and the last block to finish advances the
-// device-side context length / step counters and the exchange epoch of the persistent decode kernel.
+// Tail of the token-selection kernels (every thread of the block calls it with the row's chosen token; the threads that need the
+// state's `step` or `pos` have read it before a barrier that precedes the call): the token's embedding row becomes the next step's
+// input x[b], and the block that finishes the last row advances the device-side context length / step counters and the exchange
+// epoch of the persistent decode kernel.
 template <typename T>
 __device__ __forceinline__ void publish_token(uint32_t chosen, int b, DevState *state, int B, int dpos, int dstep,
                                               const T *embed, T *x_next, int H, float embed_scale) {
-  if (x_next) {
-    const T *row = embed + (int64_t)chosen * H;
-    for (int c = threadIdx.x; c < H; c += blockDim.x) {
-      if (embed_scale != 1.0f)
-        Scalar<T>::store(x_next + (int64_t)b * H + c, (typename Scalar<T>::compute)((float)Scalar<T>::load(row + c) * embed_scale));
-      else
-        x_next[(int64_t)b * H + c] = row[c];
+  if (threadIdx.x == 0) {
+    // no fence: `step` was read (and used for an address) before this point, and what this block writes is
+    // consumed by later kernels only
+    if (B == 1 || atomicAdd(&state->done, 1) == B - 1) {  // every row's block has read `step`
+      const unsigned epoch = state->epoch;
+      const int pos = state->pos, step = state->step;
+      state->epoch = epoch + 1u;   // the next launch of the decode kernel tags its packets differently
+      state->done = 0;
+      state->pos = pos + dpos;
+      state->step = step + dstep;
     }
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    // no fence: `step` was read (and used for an address) before this point, and what this block wrote is
-    // consumed by later kernels only
-    int prev = atomicAdd(&state->done, 1);
-    if (prev == B - 1) {  // every block has read `step` and written its outputs
-      state->epoch += 1u;   // the next launch of the decode kernel tags its packets differently
-      state->done = 0;
-      state->pos += dpos;
-      state->step += dstep;
+  if (x_next) {
+    constexpr int VEC = 16 / sizeof(T);
+    struct alignas(16) Pack { T v[VEC]; };
+    const T *row = embed + (int64_t)chosen * H;
+    T *out = x_next + (int64_t)b * H;
+    auto scaled = [&](T v) {
+      if (embed_scale != 1.0f) Scalar<T>::store(&v, (typename Scalar<T>::compute)((float)Scalar<T>::load(&v) * embed_scale));
+      return v;
+    };
+    const int packs = (((uintptr_t)row | (uintptr_t)out) & 15) == 0 ? H / VEC : 0;
+    for (int c = threadIdx.x; c < packs; c += blockDim.x) {
+      Pack p = reinterpret_cast<const Pack *>(row)[c];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) p.v[j] = scaled(p.v[j]);
+      reinterpret_cast<Pack *>(out)[c] = p;
     }
+    for (int c = packs * VEC + threadIdx.x; c < H; c += blockDim.x) out[c] = scaled(row[c]);
   }
 }
 
-// Greedy token selection for every sequence, one 1024-thread block per row of
-// logits: argmax (first maximum wins; NaN never wins except at index 0), the
-// token goes to tokens[b] and to history[step][b], the token's embedding row
-// becomes the next step's input x[b], and the last block to finish advances the
-// device-side context length / step counters.  Everything the next
-// single-token step needs is then on the device.
+// Greedy token selection: `splits` blocks to a sequence's row of logits, each the argmax of its share (first maximum wins; NaN never
+// wins except at index 0).  The block of a row that arrives last chooses among the shares' results: the token goes to tokens[b] and to
+// history[step][b] and is published.  Everything the next single-token step needs is then on the device.
+//
+// Launch and trips to memory bound it (a row is 0.1 - 1 MB).  The shares' results cross blocks, and so XCDs, as device-scope relaxed
+// atomics; the ticket is drawn only after they have completed, and the last block puts the counter back to zero for the next launch.
+// One row of 32768, shares and choice as two launches -> one: bf16 4.9 + 7.1 -> 6.5 us, f32 4.9 + 5.2 -> 7.2 us; 24 rows in bf16: 5.2 + 7.0 -> 8.5 us.
+struct Best {
+  float v = -INFINITY;
+  uint32_t i = 0xffffffffu;   // none yet
+  __device__ __forceinline__ void offer(float ov, uint32_t oi) {   // (a value that is NaN is not offered)
+    if (oi != 0xffffffffu && (i == 0xffffffffu || ov > v || (ov == v && oi < i))) { v = ov; i = oi; }
+  }
+  __device__ __forceinline__ void of_wave() {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) offer(__shfl_xor(v, o, 64), (uint32_t)__shfl_xor((int)i, o, 64));
+  }
+};
 template <typename T>
 __global__ void __launch_bounds__(1024)
 k_select_token(const T *logits, int64_t n, uint32_t *tokens, uint32_t *history, DevState *state, int B, int dpos,
-               int dstep, const T *embed, T *x_next, int H, float embed_scale, const float *pval, const uint32_t *pidx,
-               int splits) {
+               int dstep, const T *embed, T *x_next, int H, float embed_scale, float *share_val, uint32_t *share_idx,
+               uint32_t *tickets, int splits) {
   __shared__ float sv[16];
   __shared__ uint32_t si[16];
   __shared__ uint32_t chosen;
-  const int b = blockIdx.x;
-  const int step = state->step;
+  const int b = blockIdx.x / splits, share = blockIdx.x % splits;
   const T *x = logits + (int64_t)b * n;
-  float bv = -INFINITY;
-  uint32_t bi = 0xffffffffu;
   constexpr int VEC = 16 / sizeof(T);
-  if (splits > 0) {
-    // wide rows: launch_argmax_partials has scanned the row in `splits` shares spread over the GPU; what is left is
-    // the choice among their (value, index) pairs (a share of NaNs only offers nothing)
-    for (int sp = threadIdx.x; sp < splits; sp += blockDim.x) {
-      const float v = pval[(int64_t)b * splits + sp];
-      const uint32_t i = pidx[(int64_t)b * splits + sp];
-      if (v == v && (bi == 0xffffffffu || v > bv || (v == bv && i < bi))) { bv = v; bi = i; }
-    }
-  } else if (n % VEC == 0 && ((uintptr_t)x & 15) == 0) {
-    // 16-byte loads, four per thread in flight; every thread still visits its elements in
-    // increasing index order, so the first maximum wins exactly as in the scalar scan
+  const int64_t len = ((n + splits - 1) / splits + VEC - 1) / VEC * VEC;
+  const int64_t lo = share * len < n ? share * len : n, hi = lo + len < n ? lo + len : n;
+  const int step = state->step;
+  const float first = (float)Scalar<T>::load(x);
+  Best best;
+  auto visit = [&](float v, uint32_t i) {   // in increasing index order within a thread: the first maximum stays
+    if (v > best.v || (best.i == 0xffffffffu && v == v)) { best.v = v; best.i = i; }
+  };
+  if (((uintptr_t)x & 15) == 0) {   // 16-byte loads, four per thread in flight
     struct alignas(16) Pack { T v[VEC]; };
-    const Pack *xp = reinterpret_cast<const Pack *>(x);
-    const int64_t chunks = n / VEC;
+    const Pack *xp = reinterpret_cast<const Pack *>(x + lo);
+    const int64_t chunks = (hi - lo) / VEC;
     for (int64_t c0 = threadIdx.x; c0 < chunks; c0 += (int64_t)blockDim.x * 4) {
       Pack pk[4];
 #pragma unroll
@@ -239,40 +256,52 @@ k_select_token(const T *logits, int64_t n, uint32_t *tokens, uint32_t *history, 
         const int64_t c = c0 + (int64_t)u * blockDim.x;
         if (c < chunks) {
 #pragma unroll
-          for (int j = 0; j < VEC; ++j) {
-            const float v = (float)Scalar<T>::load(&pk[u].v[j]);
-            if (v > bv || (bi == 0xffffffffu && v == v)) { bv = v; bi = (uint32_t)(c * VEC + j); }
-          }
+          for (int j = 0; j < VEC; ++j) visit((float)Scalar<T>::load(&pk[u].v[j]), (uint32_t)(lo + c * VEC + j));
         }
       }
     }
+    for (int64_t i = lo + chunks * VEC + threadIdx.x; i < hi; i += blockDim.x) visit((float)Scalar<T>::load(x + i), (uint32_t)i);
   } else {
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-      float v = (float)Scalar<T>::load(x + i);
-      if (v > bv || (bi == 0xffffffffu && v == v)) { bv = v; bi = (uint32_t)i; }
+    for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) visit((float)Scalar<T>::load(x + i), (uint32_t)i);
+  }
+  best.of_wave();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  if (lane == 0) { sv[wave] = best.v; si[wave] = best.i; }
+  __syncthreads();
+  if (wave == 0) {
+    best = Best();
+    if (lane < waves) best.offer(sv[lane], si[lane]);
+    best.of_wave();
+    int last = 1;
+    if (splits > 1) {
+      if (lane == 0) {
+        __hip_atomic_store(&share_val[blockIdx.x], best.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&share_idx[blockIdx.x], best.i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        last = atomicAdd(&tickets[b], 1u) == (uint32_t)splits - 1u;
+      }
+      last = __shfl(last, 0, 64);
+      if (last) {
+        best = Best();
+        for (int i = lane; i < splits; i += 64)
+          best.offer(__hip_atomic_load(&share_val[(int64_t)b * splits + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                     __hip_atomic_load(&share_idx[(int64_t)b * splits + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        best.of_wave();
+        if (lane == 0) __hip_atomic_store(&tickets[b], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    if (lane == 0) {
+      uint32_t token = 0xffffffffu;   // not this block's to choose
+      if (last) {
+        token = best.i == 0xffffffffu || first != first ? 0u : best.i;
+        tokens[b] = token;
+        if (history) history[(int64_t)step * B + b] = token;
+      }
+      chosen = token;
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(bv, o, 64);
-    uint32_t oi = (uint32_t)__shfl_xor((int)bi, o, 64);
-    if (oi != 0xffffffffu && (bi == 0xffffffffu || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; }
-  }
-  if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = bv; si[threadIdx.x >> 6] = bi; }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) {
-      float ov = sv[w];
-      uint32_t oi = si[w];
-      if (oi != 0xffffffffu && (bi == 0xffffffffu || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; }
-    }
-    float first = (float)Scalar<T>::load(x);
-    if (bi == 0xffffffffu || first != first) bi = 0;
-    tokens[b] = bi;
-    if (history) history[(int64_t)step * B + b] = bi;
-    chosen = bi;
-  }
-  __syncthreads();
+  if (chosen == 0xffffffffu) return;
   publish_token<T>(chosen, b, state, B, dpos, dstep, embed, x_next, H, embed_scale);
 }
 
@@ -738,23 +767,22 @@ int launch_token_choice(rai_hip_decoder *d, hipStream_t st, int B, int S, bool a
                          d->H, d->embed_scale, d->token_log, d->token_log_cap, d->sample_penalty, d->sample_last_n);
     return launch_check("sample_token");
   }
-  // A wide vocabulary is scanned by many blocks first (one block per row would fetch its 100 KB - 500 KB in several
-  // dependent rounds of loads: 35 us for 32 rows of 256000); the choice kernel then merges the shares' results.
-  int splits = 0;
-  if (d->V >= 32768 && !getenv("RAI_HIP_NO_SPLIT_CHOICE")) {
-    splits = 1;
-    while (B * splits < kNumCU && splits < kChoiceMaxSplits && d->V / (splits * 2) >= 8192) splits *= 2;
-    RAI_TRY(launch_argmax_partials(st, dt, d->logits, B, d->V, splits, d->choice_val, d->choice_idx));
-  }
-  const int threads = splits > 0 ? 256 : 1024;
+  // A wide vocabulary is scanned by several blocks a row (one would fetch its 100 KB - 500 KB in several dependent rounds of loads: 35 us
+  // for 32 rows of 256000).  Shares of 8192 and more while there are CUs for them; few rows get shares down to 2048 (one row of 32768 in
+  // bf16: 16 shares 6.5 us, 4 shares 7.6 us), many don't, as every share costs a ticket (24 rows: 4 shares 8.5 us, 16 shares 9.7 us).
+  int splits = 1;
+  if (d->V >= 32768 && !getenv("RAI_HIP_NO_SPLIT_CHOICE"))
+    while (splits < kChoiceMaxSplits && ((B * splits < kNumCU && d->V / (splits * 2) >= 8192) || (B * splits < 16 && d->V / (splits * 2) >= 2048)))
+      splits *= 2;
+  const int threads = d->V / splits >= 8192 ? 1024 : 256;
   if (dt == RAI_BF16)
-    hipLaunchKernelGGL((k_select_token<bf16_raw>), dim3(B), dim3(threads), 0, st, (const bf16_raw *)d->logits,
+    hipLaunchKernelGGL((k_select_token<bf16_raw>), dim3(B * splits), dim3(threads), 0, st, (const bf16_raw *)d->logits,
                        (int64_t)d->V, d->tokens, hist, d->state, B, S, dstep, (const bf16_raw *)d->embed,
-                       (bf16_raw *)d->x, d->H, d->embed_scale, d->choice_val, d->choice_idx, splits);
+                       (bf16_raw *)d->x, d->H, d->embed_scale, d->choice_val, d->choice_idx, d->choice_tickets, splits);
   else
-    hipLaunchKernelGGL((k_select_token<float>), dim3(B), dim3(threads), 0, st, (const float *)d->logits, (int64_t)d->V,
+    hipLaunchKernelGGL((k_select_token<float>), dim3(B * splits), dim3(threads), 0, st, (const float *)d->logits, (int64_t)d->V,
                        d->tokens, hist, d->state, B, S, dstep, (const float *)d->embed, (float *)d->x, d->H,
-                       d->embed_scale, d->choice_val, d->choice_idx, splits);
+                       d->embed_scale, d->choice_val, d->choice_idx, d->choice_tickets, splits);
   return launch_check("select_token");
 }
 
@@ -1259,7 +1287,7 @@ void decoder_init_fields(rai_hip_decoder *d, int dev, const rai_hip_decoder_conf
   d->graph_sampled = false; d->graph_penalty = 0.f; d->graph_last_n = 0;
   d->head_f = nullptr; d->frag_ready = false;
   d->hidden_copy = nullptr; d->want_hidden = false;
-  d->choice_val = nullptr; d->choice_idx = nullptr; d->head_best = nullptr;
+  d->choice_val = nullptr; d->choice_idx = nullptr; d->choice_tickets = nullptr; d->head_best = nullptr;
   d->mega_layers = nullptr;
   d->mega_ok = false;
   d->mega_prof = nullptr;
@@ -1298,6 +1326,9 @@ int decoder_alloc_common(rai_hip_decoder *d) {
   d->choice_val = (float *)tmp;
   RAI_TRY(dalloc(d, (size_t)cfg->max_batch * kChoiceMaxSplits * sizeof(uint32_t), &tmp));
   d->choice_idx = (uint32_t *)tmp;
+  RAI_TRY(dalloc(d, (size_t)cfg->max_batch * sizeof(uint32_t), &tmp));
+  d->choice_tickets = (uint32_t *)tmp;
+  RAI_HIP_TRY(hipMemset(d->choice_tickets, 0, (size_t)cfg->max_batch * sizeof(uint32_t)));
   RAI_TRY(dalloc(d, (size_t)cfg->max_batch * d->V * d->es, &d->logits));
   RAI_HIP_TRY(hipMemset(d->state, 0, sizeof(DevState)));
   return RAI_OK;

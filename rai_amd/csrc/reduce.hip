@@ -688,21 +688,6 @@ static int arg_impl(int dev, const rai_hip_tensor *in, int32_t dim, int32_t keep
   return launch_check("arg_thread");
 }
 
-int launch_argmax_partials(hipStream_t st, int dtype, const void *in, int64_t rows, int64_t n, int splits, float *pval,
-                           uint32_t *pidx) {
-  RAI_REQUIRE(rows > 0 && n > 0 && splits >= 1 && in && pval && pidx, RAI_ERR_BAD_ARG, "argmax partials: bad arguments");
-  RAI_REQUIRE(dtype == RAI_BF16 || dtype == RAI_F16 || dtype == RAI_F32, RAI_ERR_BAD_DTYPE, "argmax partials: dtype %s",
-              dtype_name(dtype));
-  const int threads = n / splits >= 8192 ? 1024 : 256;
-  RAI_DISPATCH_FLOAT(dtype, T, {
-    if constexpr (sizeof(T) <= 4)
-      hipLaunchKernelGGL((k_arg_row_partial<T, true>), dim3((unsigned)(rows * splits)), dim3(threads), 0, st, (const T *)in,
-                         rows, n, n, (int64_t)1, splits, pval, (double *)nullptr, pidx, (uint32_t *)nullptr,
-                         (uint32_t *)nullptr);
-  });
-  return launch_check("argmax_partials");
-}
-
 }  // namespace rai
 
 using namespace rai;

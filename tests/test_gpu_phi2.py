@@ -247,3 +247,29 @@ def test_decoder_errors(hip):
     with pytest.raises(RaiHipError):
         dec.load_param("model.layers.0.nope", np.zeros(4, np.float32))
     dec.close()
+
+
+@pytest.mark.parametrize("dt,vocab,batch", [("f32", 1000, 3), ("bf16", 1000, 1), ("bf16", 32767, 2), ("f32", 32768, 1), ("bf16", 51200, 4),
+                                            ("f32", 65541, 3), ("bf16", 65541, 33)])
+def test_token_choice_in_shares(hip, dt, vocab, batch):
+    """Logits that are the head's bias and nothing else: the first of equal maxima, wherever the shares of a row end; NaN only at index 0;
+    the same choice launch after launch, replayed ones included (a counter that is not put back would show)."""
+    cfg = small_cfg(vocab_size=vocab)
+    dec, _ = make(cfg, dt, hip, max_batch=batch, max_context=64)
+    dec.load_param("lm_head.weight", to_storage(np.zeros((vocab, cfg.hidden_size), np.float32), dt))
+    rng = np.random.Generator(np.random.PCG64(vocab + batch))
+    ids = rng.integers(0, vocab, (batch, 5)).astype(np.uint32)
+    low = -rng.integers(1, 100, vocab).astype(np.float32)
+    half, last = vocab // 2, vocab - 1
+    for want, at in ((last, {last: 1.0}), (half - 1, {half - 1: 1.0, half: 1.0, last: 1.0}), (half, {half: 2.0, half + 1: 2.0, 0: 1.0}),
+                     (2, {1: np.nan, 2: 1.0, last: np.nan}), (last, {**{i: np.nan for i in range(1, half + 9)}, 0: -200.0, last: 3.0}),
+                     (0, {0: np.nan, last: 5.0}), (3, {3: np.inf, last: np.inf}), (0, {i: -np.inf for i in range(vocab)})):
+        bias = low.copy()
+        bias[list(at)] = list(at.values())
+        dec.load_param("lm_head.bias", to_storage(bias, dt))
+        dec.clear_kv_cache()
+        assert (dec.forward(ids)[1] == want).all()
+        dec.clear_kv_cache()
+        toks, _, _ = dec.generate(ids, 6)
+        assert (toks == want).all()
+    dec.close()
