@@ -229,4 +229,14 @@ __device__ __forceinline__ float wave_max(float v) {
 constexpr int kWave = 64;
 constexpr int kNumCU = 256;
 
+// A grid of at least `blocks` blocks: HIP launches no dimension of 2^32 threads or more, so blocks beyond 2^31 threads go to a second
+// one.  A kernel's block is blockIdx.y * gridDim.x + blockIdx.x (blocks go to the XCDs in that order, as gridDim.x is a multiple
+// of 8 there), and those past the last one leave.
+inline int grid_of_blocks(int64_t blocks, int threads, dim3 *grid) {
+  const int64_t most = (1ll << 31) / threads / 8 * 8, x = blocks < most ? blocks : most, y = (blocks + x - 1) / x;
+  RAI_REQUIRE(y <= 65535, RAI_ERR_UNSUPPORTED, "%lld blocks in one launch", (long long)blocks);
+  *grid = dim3((unsigned)x, (unsigned)y);
+  return RAI_OK;
+}
+
 }  // namespace rai

@@ -87,12 +87,16 @@ k_norm_wave(T *out, const T *x, const T *w, const T *b, int64_t rows, int64_t n,
 // it has the row's statistics, one more trip to memory, which many rows hide and few do not.  Bound by the launch and two trips
 // up to a thousand rows, by HBM beyond.  Measured (us, wave, block): f32 layer norm of 2560 columns, 1 row 5.8, 3.9, 256 rows 7.0, 4.0,
 // 8192 rows 29.0, 25.4; 4096 columns, 256 rows 9.5, 4.0; bf16 rms norm 1536, 1 row 4.3, 4.0, 4096 columns 16384 rows 57.6, 40.2.
+// Rows beyond 2^23 are blocks of a second grid dimension.
 template <typename T, int V, int ITEMS>
-__global__ void __launch_bounds__(256) k_norm_row(T *out, const T *x, const T *w, const T *b, int64_t n, int64_t x_row_stride, float eps, int kind) {
+__global__ void __launch_bounds__(256)
+k_norm_row(T *out, const T *x, const T *w, const T *b, int64_t rows, int64_t n, int64_t x_row_stride, float eps, int kind) {
   __shared__ float sh[2][4];
   const int tid = threadIdx.x, packs = (int)(n / V);
-  const T *xr = x + blockIdx.x * x_row_stride;
-  T *yr = out + blockIdx.x * n;
+  const int64_t row = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;   // (the whole block leaves)
+  if (row >= rows) return;
+  const T *xr = x + row * x_row_stride;
+  T *yr = out + row * n;
   NPack<T, V> xk[ITEMS], wk[ITEMS], bk[ITEMS];
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it)
@@ -478,11 +482,12 @@ static int norm_impl(int dev, const rai_hip_tensor *x, const rai_hip_tensor *w, 
     // 16-bit rows beyond 2048 of them go to the wave form unless they fill three quarters of a block's threads (us, wave, block, 8192
     // rows: bf16 layer norm 2560 19.8, 21.4, 800 8.8, 11.7, rms norm 1024 7.8, 9.3; 2048 15.4, 13.1, 4096 30.4, 21.6); f32 rows never.
     if (x->dtype == RAI_F32 || rows <= 8 * kNumCU || 4 * packs > 3 * ((packs + 255) / 256 * 256)) {
-      RAI_REQUIRE(rows <= 0x7fffffff, RAI_ERR_UNSUPPORTED, "%s: too many rows", what);
+      dim3 grid;
+      RAI_TRY(grid_of_blocks(rows, 256, &grid));
 #define NORM_ROW(T, V, ITEMS)                                                                                          \
-  hipLaunchKernelGGL((k_norm_row<T, V, ITEMS>), dim3((unsigned)rows), dim3(256), 0, st, (T *)base_ptr(out),            \
+  hipLaunchKernelGGL((k_norm_row<T, V, ITEMS>), grid, dim3(256), 0, st, (T *)base_ptr(out),                              \
                      (const T *)base_ptr(x), w ? (const T *)base_ptr(w) : nullptr,                                     \
-                     b ? (const T *)base_ptr(b) : nullptr, n, row_stride, (float)eps, kind)
+                     b ? (const T *)base_ptr(b) : nullptr, rows, n, row_stride, (float)eps, kind)
 #define NORM_ROW_ITEMS(T, V)                   \
   do {                                         \
     if (packs <= 256) NORM_ROW(T, V, 1);       \

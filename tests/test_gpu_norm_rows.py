@@ -33,3 +33,24 @@ def test_rows(hip, dt, rows, n):
     mean, var = d.mean(-1, keepdims=True), d.var(-1, keepdims=True)
     check(R.layer_norm(up(x, dt), up(w, dt), up(b, dt), 1e-5), mean, 1 / np.sqrt(var + 1e-5), w, b)
     check(R.layer_norm(up(x, dt), None, None, 1e-5), mean, 1 / np.sqrt(var + 1e-5), 1.0, 0.0)
+
+
+@pytest.mark.parametrize("dt,n", [("f32", 4), ("f32", 1028), ("bf16", 1544)])
+def test_more_rows_than_one_grid_dimension_holds(hip, dt, n):
+    """2^24 rows and a few: 2^32 threads where a block of 256 has a row.  Equal rows, read with a stride of zero; the output (up to
+    69 GB) is looked at around every power of two that a count of rows or threads could be cut off at."""
+    from rai_amd import ops as R
+    from rai_amd._lib import call
+
+    rows = (1 << 24) + 5
+    g = np.random.Generator(np.random.PCG64(n))
+    x, w, b = rand(g, (n,), dt, 2.0), rand(g, (n,), dt), rand(g, (n,), dt)
+    many = up(x, dt).broadcast_to((rows, n))
+    for fn in (lambda t: R.rms_norm(t, up(w, dt), 1e-6), lambda t: R.layer_norm(t, up(w, dt), up(b, dt), 1e-5)):
+        want, got = down(fn(up(x[None], dt))), fn(many)
+        for at in (0, (1 << 22) - 2, (1 << 23) - 2, (1 << 24) - 2, rows - 4):
+            part = down(got.narrow(0, at, 4)).astype(np.float64)
+            # one row and many may be served by different kernels: both are within an f32 norm's roundings and one of dt
+            assert np.all(np.abs(part - want) <= (n + 16) * 2.0 ** -23 * (np.abs(want) + 4 * np.abs(w) + np.abs(b)) + 2 * U[dt] * np.abs(want)), at
+        del got
+        call("rai_hip_trim", 0)
