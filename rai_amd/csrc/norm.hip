@@ -152,6 +152,21 @@ k_norm_row(T *out, const T *x, const T *w, const T *b, int64_t rows, int64_t n, 
   }
 }
 
+// Whether a block takes a row (else a wave does), rows of `packs` 16-byte pieces.  The block has the shorter way to memory while the CUs hold
+// all rows at once, and wherever its threads are filled; a wave costs no barriers and leaves no thread idle.  Measured, us, wave / block:
+//   f32, 64 columns, layer norm, 2048 rows 3.8 / 3.8, 4096 3.8 / 4.8, 65536 16.1 / 44.5; 512 columns 4096 rows 4.7 / 5.8, 65536 40 / 55;
+//   768 columns 3072 rows 5.2 / 5.6, 40000 37 / 42; 1100 columns 3072 rows 6.8 / 6.7, 40000 74 / 67; 2560 columns 8192 rows 29.3 / 25.3;
+//   a block's layer norm of little more than one piece a thread, with a barrier more than the other norms': f32 1024 columns 6144 rows
+//   9.8 / 10.3, 8192 rows 13.6 / 12.6; bf16 2048 columns 2048 rows 6.3 / 5.5, 4096 8.3 / 8.7, 5120 12.5 / 10.9;
+//   16-bit rows that leave a quarter of the threads idle: layer norm 2560 columns, 1536 rows 6.7 / 5.7, 2048 7.0 / 7.3, 8192 19.8 / 21.4;
+//   rms norm 1024 columns, 8192 rows 7.8 / 9.3; rows that fill them: rms norm 2048 columns 8192 rows 15.4 / 13.1, 4096 30.4 / 21.6.
+static bool norm_row_serves(int dtype, int kind, int64_t rows, int64_t packs) {
+  const bool f32 = dtype == RAI_F32, filled = 4 * packs > 3 * ((packs + 255) / 256 * 256);
+  if (rows <= (f32 || filled ? 8 : 6) * kNumCU) return true;
+  if (f32 ? packs <= 192 : !filled) return false;
+  return !(kind == kLayerNorm && packs <= 288 && rows <= (f32 ? 24 : 16) * kNumCU);
+}
+
 // Fallback for rows that do not fit the register budget or are unaligned: one
 // block per row, the row is re-read from L2 for each pass.
 template <typename T>
@@ -479,9 +494,7 @@ static int norm_impl(int dev, const rai_hip_tensor *x, const rai_hip_tensor *w, 
   bool aligned = (n % v == 0) && (row_stride % v == 0) && al(x) && al(out) && al(w) && al(b);
   const int64_t packs = n / v;
   if (aligned && x->dtype != RAI_F64 && packs <= 64 * 16) {
-    // 16-bit rows beyond 2048 of them go to the wave form unless they fill three quarters of a block's threads (us, wave, block, 8192
-    // rows: bf16 layer norm 2560 19.8, 21.4, 800 8.8, 11.7, rms norm 1024 7.8, 9.3; 2048 15.4, 13.1, 4096 30.4, 21.6); f32 rows never.
-    if (x->dtype == RAI_F32 || rows <= 8 * kNumCU || 4 * packs > 3 * ((packs + 255) / 256 * 256)) {
+    if (norm_row_serves(x->dtype, kind, rows, packs)) {
       dim3 grid;
       RAI_TRY(grid_of_blocks(rows, 256, &grid));
 #define NORM_ROW(T, V, ITEMS)                                                                                          \
@@ -508,15 +521,19 @@ static int norm_impl(int dev, const rai_hip_tensor *x, const rai_hip_tensor *w, 
   hipLaunchKernelGGL((k_norm_wave<T, V, ITEMS>), dim3(grid), dim3(256), 0, st, (T *)base_ptr(out),                \
                      (const T *)base_ptr(x), w ? (const T *)base_ptr(w) : nullptr,                                \
                      b ? (const T *)base_ptr(b) : nullptr, rows, n, row_stride, (float)eps, kind)
-#define NORM_BY_ITEMS(T, V)                        \
-  do {                                             \
-    if (packs <= 64 * 2) NORM_LAUNCH(T, V, 2);     \
-    else if (packs <= 64 * 5) NORM_LAUNCH(T, V, 5); \
-    else if (packs <= 64 * 10) NORM_LAUNCH(T, V, 10); \
-    else NORM_LAUNCH(T, V, 16);                    \
+    if (x->dtype == RAI_F32) {   // (up to 288 pieces)
+      if (packs <= 64 * 2) NORM_LAUNCH(float, 4, 2);
+      else NORM_LAUNCH(float, 4, 5);
+    } else {                     // (up to 576)
+#define NORM_BY_ITEMS(T)                            \
+  do {                                              \
+    if (packs <= 64 * 2) NORM_LAUNCH(T, 8, 2);      \
+    else if (packs <= 64 * 5) NORM_LAUNCH(T, 8, 5); \
+    else NORM_LAUNCH(T, 8, 9);                      \
   } while (0)
-    if (x->dtype == RAI_BF16) NORM_BY_ITEMS(bf16_raw, 8);
-    else NORM_BY_ITEMS(f16_raw, 8);
+      if (x->dtype == RAI_BF16) NORM_BY_ITEMS(bf16_raw);
+      else NORM_BY_ITEMS(f16_raw);
+    }
 #undef NORM_BY_ITEMS
 #undef NORM_LAUNCH
     return launch_check(what);

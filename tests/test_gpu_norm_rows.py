@@ -8,7 +8,12 @@ pytestmark = pytest.mark.gpu
 U = {"f32": 2.0 ** -24, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}
 
 
-@pytest.mark.parametrize("rows,n", [(1, 8), (3, 1016), (2, 2048), (5, 2056), (1, 4104), (2, 8192), (2048, 264), (2049, 264), (2049, 1536), (2051, 1544), (2050, 2048)])
+# Columns by 16-byte pieces of 16-bit elements: a wave's two, five and nine pieces a lane at both ends, a block's one to four a thread; rows on
+# both sides of 1536, 2048, 4096 and 6144, beyond which the other form may serve.
+@pytest.mark.parametrize("rows,n", [(1, 8), (3, 1016), (2, 2048), (5, 2056), (1, 4104), (2, 8192), (1536, 264), (1537, 264), (2048, 264), (2049, 264),
+                                    (2049, 1024), (2049, 1032), (2049, 1536), (2051, 1544), (2050, 2048), (4096, 1800), (4097, 1800), (2049, 2304),
+                                    (2049, 2312), (6144, 2304), (6145, 2304), (2049, 2560), (2049, 2568), (2049, 3072), (2050, 3080), (2050, 4104),
+                                    (2050, 4608), (2050, 4616)])
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
 def test_rows(hip, dt, rows, n):
     from rai_amd import ops as R
