@@ -62,7 +62,8 @@ __global__ void __launch_bounds__(NW * KSP * 64, D <= 128 ? 2 : 1) k_flash_prefi
   const int wave = w / KSP, kh = w % KSP;   // query group of the block, key tiles kh, kh + KSP, ...
   // Under a causal mask the last query tiles see the most keys: those of all heads go first, so that the short ones fill the
   // tail.  Blocks go to the XCDs in turn, so an XCD takes a run of heads, whose keys then are in its L2 alone.
-  const int heads = a.Hq * a.B, tiles = gridDim.x / heads, id = blockIdx.x;
+  const int heads = a.Hq * a.B, tiles = (a.S + NW * 32 - 1) / (NW * 32), id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  if (id >= tiles * heads) return;
   int hb, qt;
   if (heads % 8 == 0) {
     const int per = heads / 8, slot = id / 8;
@@ -435,8 +436,10 @@ template <int NW, int D, int MODE, int KSP, int TK> static int launch_flash_cfg(
     attr_set = true;
   }
   const int64_t blocks = (int64_t)((a.S + 32 * NW - 1) / (32 * NW)) * a.Hq * a.B;
-  RAI_REQUIRE(blocks <= 0x7fffffff, RAI_ERR_UNSUPPORTED, "attention: grid too large");
-  hipLaunchKernelGGL((k_flash_prefill_bf16<NW, D, MODE, KSP, TK>), dim3((unsigned)blocks), dim3(NW * KSP * 64), lds, st, a);
+  RAI_REQUIRE(blocks < 1 << 30, RAI_ERR_UNSUPPORTED, "attention: grid too large");   // (the output alone would be a terabyte)
+  dim3 grid;
+  RAI_TRY(grid_of_blocks(blocks, NW * KSP * 64, &grid));
+  hipLaunchKernelGGL((k_flash_prefill_bf16<NW, D, MODE, KSP, TK>), grid, dim3(NW * KSP * 64), lds, st, a);
   return launch_check("flash_prefill");
 }
 

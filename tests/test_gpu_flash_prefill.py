@@ -75,3 +75,19 @@ def test_all_keys_and_strides(R, d, b, hq, hkv, s, t, f32_scores):
 @pytest.mark.parametrize("scale", [-0.125, 0.0, 0.3])
 def test_scales(R, scale, f32_scores):
     check(R, 1, 4, 2, 70, 130, 64, 1, f32_scores, scale=scale)
+
+
+def test_more_blocks_than_one_grid_dimension_holds(R):
+    """257 x 65528 heads of one block of 256 threads: more than 2^32 threads (the output is 17 GB; whole sequences of it are looked at,
+    among them those on both sides of block 2^23 and of block 2^24)."""
+    from rai_amd._lib import call
+
+    b, hq, s, d = 257, 65528, 16, 32
+    g = np.random.Generator(np.random.PCG64(2))
+    q, k, v = rand(g, (1, hq, s, d), "bf16"), rand(g, (b, 1, s, d), "bf16"), rand(g, (b, 1, s, d), "bf16")
+    got = R.attention(up(q, "bf16").broadcast_to((b, hq, s, d)), up(k, "bf16"), up(v, "bf16"), d ** -0.5, 1, 1)
+    for i in (0, 127, 128, 129, 255, 256):
+        want, tol = reference(q, k[i:i + 1], v[i:i + 1], d ** -0.5, 1, 1)
+        assert np.all(np.abs(down(got.narrow(0, i, 1)).astype(np.float64) - want) <= tol), i
+    del got
+    call("rai_hip_trim", 0)
