@@ -137,17 +137,18 @@ __global__ void __launch_bounds__(NW * KSP * 64, D <= 128 ? 2 : 1) k_flash_prefi
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
-  // Scaling keeps the order of scores (a negative scale's sign goes to the queries, and a scale of zero), so the maximum is taken
-  // of the products as they are, and scaled alone.
+  // Scaling keeps the order of scores (a negative scale's sign goes to the queries, and a scale of zero: a score of 0 x infinity or NaN
+  // stays NaN), so the maximum is taken of the products as they are, and scaled alone.
   float scale = MODE == 0 ? fa_round(a.scale) : a.scale;
   if (scale <= 0.f) {
-    const uint32_t keep = scale < 0.f ? ~0u : 0u, flip = scale < 0.f ? 0x80008000u : 0u;
-    scale = scale < 0.f ? -scale : 1.f;
+    const bool zero = scale == 0.f;
+    scale = zero ? 1.f : -scale;
+    auto turned = [&](uint32_t x) { return zero ? ((x & 0x7f80u) == 0x7f80u ? 0x7fc0u : 0u) : x ^ 0x8000u; };   // of one bf16
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       fa_u32x4 v = __builtin_bit_cast(fa_u32x4, qf[ks]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = (v[j] & keep) ^ flip;
+      for (int j = 0; j < 4; ++j) v[j] = turned(v[j] & 0xffffu) | turned(v[j] >> 16) << 16;
       qf[ks] = __builtin_bit_cast(fa_bf16x8, v);
     }
   }

@@ -77,6 +77,30 @@ def test_scales(R, scale, f32_scores):
     check(R, 1, 4, 2, 70, 130, 64, 1, f32_scores, scale=scale)
 
 
+@pytest.mark.parametrize("f32_scores", [0, 1])
+@pytest.mark.parametrize("scale", [0.0, -0.125, 0.25])
+def test_scales_keep_what_is_not_a_number(R, scale, f32_scores):
+    """Queries and keys with an infinity or a NaN in them: the rows that see one, and no others, are not numbers, at a scale of zero too."""
+    g = np.random.Generator(np.random.PCG64(4))
+    q, k, v = rand(g, (1, 2, 96, 64), "bf16"), rand(g, (1, 2, 96, 64), "bf16"), rand(g, (1, 2, 96, 64), "bf16")
+    q[0, 0, 7, 3], q[0, 0, 40, 63] = np.inf, np.nan
+    k[0, 1, 70, 5] = np.nan
+    k[0, 1, 80, 6] = np.inf
+    got = down(R.attention(up(q, "bf16"), up(k, "bf16"), up(v, "bf16"), scale, 1, f32_scores)).reshape(96, 2, 64)
+    lost = np.zeros((96, 2), bool)
+    lost[[7, 40], 0] = True
+    lost[70:, 1] = True
+    if scale:   # a row's infinite scores are of either sign: above all others its weights are not numbers, below them they are zero
+        lost[7, 0] = bool((np.sign(k[0, 0, :8, 3]) * np.sign(scale) > 0).any())
+    np.testing.assert_array_equal(np.isnan(got).any(-1), lost)
+    if scale == 0:
+        mean = np.cumsum(v[0].astype(np.float64), 1) / np.arange(1, 97)[:, None]
+        keep = ~lost
+        want = np.swapaxes(mean, 0, 1)[keep]
+        bound = np.swapaxes(np.cumsum(np.abs(v[0].astype(np.float64)), 1) / np.arange(1, 97)[:, None], 0, 1)[keep]
+        assert np.all(np.abs(got[keep] - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -15 * bound)   # weights of 1: f32 sums, one rounding
+
+
 def test_more_blocks_than_one_grid_dimension_holds(R):
     """257 x 65528 heads of one block of 256 threads: more than 2^32 threads (the output is 17 GB; whole sequences of it are looked at,
     among them those on both sides of block 2^23 and of block 2^24)."""
