@@ -1569,6 +1569,11 @@ __global__ void __launch_bounds__(512) k_linear_bf16_mfma_stream(LinearArgs a, i
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(xf[mt][ks]));
     __syncthreads();
+    if (k0 + KS * 32 > a.K) {   // an infinite weight, read in their place, would make the zeros beyond K NaN
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        if (k0 + ks * 32 >= a.K) wv[ks] = bf16x8{};
+    }
     float scale[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {

@@ -164,3 +164,20 @@ def test_decode_attention_of_short_contexts(hip, heads, kv, dim, context):
         assert_close(logits, want, "bf16", f"step {step}")
         ids = np.argmax(want, -1).astype(np.uint32).reshape(3, 1)
     dec.close()
+
+
+@pytest.mark.parametrize("batch", [9, 17, 33, 49])
+def test_infinite_norm_weight(hip, batch):
+    """The last norm has an infinite weight among the first 32: every logit is infinite, of its own sign, also where the product's
+    kernel norms the rows itself and spans more columns than there are."""
+    cfg = CFGS["qwen2"]()
+    dec, ref = make(cfg, "bf16", max_batch=batch, max_context=4)
+    ids = np.random.Generator(np.random.PCG64(batch)).integers(0, cfg.vocab_size, (batch, 1)).astype(np.uint32)
+    weight = np.array(ref.p["model.norm.weight"])
+    weight[3] = np.inf
+    dec.load_param("model.norm.weight", to_storage(weight, "bf16"))
+    hidden = dec.forward_hidden(ids)[0][:, 0, 3]
+    dec.clear_kv_cache()
+    logits, _ = dec.forward(ids)
+    np.testing.assert_array_equal(logits, np.inf * np.sign(hidden)[:, None] * np.sign(ref.p["lm_head.weight"][:, 3])[None])
+    dec.close()
