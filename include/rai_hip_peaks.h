@@ -1,9 +1,10 @@
-/* Measurement aid of librai_hip.so: the ceilings of the GPU it runs on, measured with loops that have no workload
- * around them.  No counterpart in the reference (cksac/rai measures nothing of the kind); not used by any product
- * path.  `python bench.py --workload peaks` prints every figure. */
+/* Measurement aids of librai_hip.so: the ceilings of the GPU it runs on, measured with loops that have no workload
+ * around them (`python bench.py --workload peaks` prints every figure), and which kernel serves a product.  No counterpart in
+ * the reference (cksac/rai measures nothing of the kind); not used by any product path. */
 #ifndef RAI_HIP_PEAKS_H
 #define RAI_HIP_PEAKS_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
@@ -30,6 +31,12 @@ typedef enum rai_hip_peak_kind {
  * time of a launch and the work one launch does (flops or bytes, see above).  Allocates and frees its own buffers. */
 int rai_hip_measure_peak(int dev, int32_t kind, int64_t bytes, int32_t launches, double *seconds_per_launch,
                          double *work_per_launch);
+
+/* The tile that a bf16 Linear of m > 64 rows, n columns and k % 64 == 0 takes on `dev` with `scratch_bytes` of scratch lent to it, under
+ * the name that RAI_HIP_GEMM_TILE has for it, and the parts that K is cut into.  rai_hip_linear lends 32 m n bytes, at
+ * most 256 MiB.  Launches nothing. */
+int rai_hip_linear_plan(int dev, int32_t m, int32_t k, int32_t n, size_t scratch_bytes, char *tile, size_t tile_len,
+                        int32_t *k_parts);
 
 #ifdef __cplusplus
 }

@@ -182,6 +182,7 @@ _I32P = C.POINTER(_i32)
 # include/rai_hip_peaks.h (measurement aid)
 PEAK_PROTOTYPES = {
     "rai_hip_measure_peak": [C.c_int, C.c_int32, C.c_int64, C.c_int32, C.POINTER(C.c_double), C.POINTER(C.c_double)],
+    "rai_hip_linear_plan": [C.c_int, _i32, _i32, _i32, C.c_size_t, C.c_char_p, C.c_size_t, C.POINTER(_i32)],
 }
 PEAK_KINDS = {"mfma_bf16": 0, "mfma_bf16_lds": 1, "lds_read": 2, "hbm_read": 3, "hbm_copy": 4, "stage_dma": 5, "stage_vgpr": 6, "gemm_loop": 7}
 

@@ -19,6 +19,7 @@
 
 #include "gemm.h"
 #include "latent.h"
+#include "rai_hip_peaks.h"
 
 namespace rai {
 
@@ -1929,8 +1930,9 @@ static int tile_splits(const LinearArgs &a) {
 
 // RAI_HIP_GEMM_TILE, read per call, and the names of the tiles above in it; a tile that it names gets the split of its own.
 static const char *forced_tile() { return getenv("RAI_HIP_GEMM_TILE"); }
-static const struct { const char *name; int tile; } kTileNames[] = {{"128x128k64", kTile128}, {"128x128deep", kTile128}, {"128x64", kTile128x64},
-                                                                   {"64x64", kTile64},        {"128x256", kTile128x256}, {"192x256", kTile192x256}};
+static const struct { const char *name; int tile; } kTileNames[] = {{"128x128k64", kTile128},   {"128x128deep", kTile128},  {"128x64", kTile128x64},
+                                                                   {"64x64", kTile64},         {"128x256", kTile128x256},  {"192x256", kTile192x256},
+                                                                   {"256x192", kTile256x192}, {"256x256k64", kTile256}};
 static int named_tile(const char *knob) {   // -1: none of them
   for (const auto &t : kTileNames)
     if (!strcmp(knob, t.name)) return t.tile;
@@ -2044,8 +2046,8 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
   // RAI_HIP_NO_K64: never): what tile_plan_k64 says.  Other K: 256 x 256 in its eight-wave form (one block per CU, 4 LDS stages of 32, two
   // waves per SIMD) or stream-K over it once its tiles cover a good half of the CUs, 128 x 128 with three stages below that.
   // RAI_HIP_GEMM_TILE = "64x64" | "128x64" | "128x128" | "128x128k64" | "128x128deep" (the same) | "128x256" | "192x256" | "256x128" |
-  // "256x192" | "256x256" | "256x256x8w" | "256x256x8wk64" | "streamk" | "streamk64" | "classic" overrides (tuning aid; a form that does
-  // not apply to the shape is an error).
+  // "256x192" | "256x256" | "256x256k64" | "256x256x8w" | "256x256x8wk64" (256x256k64, K never cut) | "streamk" | "streamk64" | "classic"
+  // overrides (tuning aid; a form that does not apply to the shape is an error).
   const char *knob = forced_tile();
   if (knob) {
     if (named_tile(knob) >= 0) {
@@ -2057,10 +2059,6 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
     if (!strcmp(knob, "256x256")) return launch_cfg_dma<256, 256, 4, 2>(st, a, splits);
     if (!strcmp(knob, "classic")) return launch_cfg<128, 128, 32>(st, a, splits);
     if (!strcmp(knob, "256x256x8w")) return launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
-    if (!strcmp(knob, "256x192")) {
-      RAI_REQUIRE(a.K % 64 == 0, RAI_ERR_UNSUPPORTED, "linear: RAI_HIP_GEMM_TILE=%s needs K %% 64 == 0 (%dx%dx%d)", knob, a.M, a.N, a.K);
-      return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, splits);
-    }
     if (!strcmp(knob, "256x256x8wk64")) {
       RAI_REQUIRE(splits == 1 && a.K % 64 == 0, RAI_ERR_UNSUPPORTED,
                   "linear: RAI_HIP_GEMM_TILE=256x256x8wk64 needs K %% 64 == 0 and no K split (%dx%dx%d)", a.M, a.N, a.K);
@@ -2081,3 +2079,20 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
 }
 
 }  // namespace rai
+
+extern "C" int rai_hip_linear_plan(int dev, int32_t m, int32_t k, int32_t n, size_t scratch_bytes, char *tile, size_t tile_len, int32_t *k_parts) {
+  using namespace rai;
+  RAI_REQUIRE(tile && tile_len && k_parts && n > 0, RAI_ERR_BAD_ARG, "linear_plan: null argument");
+  RAI_REQUIRE(m > 64 && k > 0 && k % 64 == 0, RAI_ERR_UNSUPPORTED, "linear_plan: %dx%dx%d is not served by one rule", m, n, k);
+  LinearArgs a = linear_args_default();
+  a.M = m; a.N = n; a.K = k; a.dev = dev;
+  a.splitk_ws = scratch_bytes ? (void *)16 : nullptr;   // (looked at, not into)
+  a.splitk_ws_bytes = scratch_bytes;
+  const TilePlan plan = tile_plan_k64(a);
+  const char *name = "streamk64";
+  for (const auto &t : kTileNames)
+    if (t.tile == plan.tile) { name = t.name; break; }
+  snprintf(tile, tile_len, "%s", name);
+  *k_parts = plan.splits;
+  return RAI_OK;
+}

@@ -146,8 +146,9 @@ def test_argmax_64x51200(R, dt):
 
 
 # ------------------------------------------------------------------ every tile of the bf16 MFMA GEMM
-TILES = ["64x64", "128x64", "128x128", "128x128k64", "128x128deep", "256x192", "256x128", "256x256", "256x256x8w", "classic"]
-K64_TILES = ("64x64", "128x64", "128x128k64", "128x128deep", "256x192")      # LDS stages of K 64: refused unless K % 64 == 0
+# LDS stages of K 64 (refused unless K % 64 == 0); 128x128k64 and 128x128deep are two names of one kernel
+K64_TILES = ("64x64", "128x64", "128x128k64", "128x128deep", "256x192", "128x256", "192x256", "256x256k64")
+TILES = [*K64_TILES, "128x128", "256x128", "256x256", "256x256x8w", "classic"]
 
 
 def packed_case(g, m, n, k, scale=0.05):
@@ -315,8 +316,7 @@ def test_gemm_forced_tile_is_not_split_for_another_tile(R, monkeypatch):
 
 
 def test_gemm_dispatcher_picks_each_tile_by_itself(R, monkeypatch):
-    # no override: 3072 x 3072 gives 144 tiles of 256 x 256 (the eight-wave tile), 4096 x 2048 gives 512 of 256 x 128,
-    # 600 x 520 stays on 128 x 128; K = 64 is shorter than the prefetch depth of every one of them
+    # no override: K of 64 and 96, shorter than the prefetch depth of every tile, with stages of 64 and of 32, and 3000 x 3100 x 2560
     monkeypatch.delenv("RAI_HIP_GEMM_TILE", raising=False)
     dt = "bf16"
     for m, n, k in [(3072, 3072, 64), (4096, 2048, 96), (600, 520, 64), (3000, 3100, 2560)]:

@@ -1,6 +1,8 @@
-"""bf16 Linears of more than eight rows on tiles with K stages of 64: as the sizes choose them (64 x 64 for most of these), and
-each of 64 x 64, 128 x 64 and 128 x 128 with two and four stages forced, with one to as many stages as it keeps in flight and one
-more, ragged edges, K in parts, gated pairs."""
+"""bf16 Linears of more than eight rows on tiles with K stages of 64: as the sizes choose them (64 x 64 for most of these; the
+rule's pick of every tile, cut over K and whole, is asked for and asserted below), and each tile forced, with one to as many stages
+as it keeps in flight and one more, ragged edges, K in parts, gated pairs."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -40,7 +42,7 @@ def test_tiles(R, m, k, n):
     assert np.all(np.abs(got - full) <= 2.0 ** -8 * np.abs(full) + 2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)
 
 
-TILES = ["64x64", "128x64", "128x128k64", "128x128deep"]
+TILES = ["64x64", "128x64", "128x128k64", "128x128deep", "128x256", "192x256", "256x192", "256x256k64"]   # (128x128k64 and 128x128deep: one kernel)
 
 
 @pytest.mark.parametrize("m,k,n", [(65, 64, 8), (129, 128, 257), (200, 192, 136), (333, 256, 520), (72, 320, 1031), (65, 1664, 512), (260, 1088, 300), (130, 2560, 776)])
@@ -94,14 +96,50 @@ def test_tiles_gated(R, m, k, n):
 
 # The eight-wave tiles of 256 columns: short K (stages fewer than the pipeline), ragged rows and columns, parts of K.
 @pytest.mark.parametrize("m,k,n", [(65, 64, 8), (129, 128, 257), (193, 192, 520), (383, 256, 1031), (385, 1088, 264), (130, 2560, 776)])
-@pytest.mark.parametrize("tile", ["128x256", "192x256"])
+@pytest.mark.parametrize("tile", ["128x256", "192x256", "256x192", "256x256k64"])
 def test_wide_tiles(R, monkeypatch, tile, m, k, n):
     monkeypatch.setenv("RAI_HIP_GEMM_TILE", tile)
     test_tiles(R, m, k, n)
     test_tiles_gated(R, m, k, 8 * (n // 8))
 
 
-# What the rule picks by itself: small tiles cut over K, 128 x 128, 128 x 256, 192 x 256, 256 x 192, 256 x 256, stream-K.
-@pytest.mark.parametrize("m,k,n", [(100, 4096, 1024), (333, 512, 8960), (777, 256, 8192), (777, 192, 22528), (2048, 320, 4096), (4096, 128, 10240)])
-def test_what_the_rule_picks(R, m, k, n):
-    test_tiles(R, m, k, n)
+def plan(m, k, n):
+    """(tile, parts of K) that the rule gives R.linear."""
+    from rai_amd._lib import call
+
+    name, parts = C.create_string_buffer(32), C.c_int32()
+    call("rai_hip_linear_plan", 0, m, k, n, min(32 * m * n, 256 << 20), name, 32, C.byref(parts))
+    return name.value.decode(), parts.value
+
+
+# What the rule picks by itself: every tile whole and, where it is ever the best, cut over K.
+@pytest.mark.parametrize("m,k,n,tile,cut", [
+    (87, 320, 312, "64x64", False), (68, 2176, 288, "64x64", True), (524, 704, 2112, "128x64", False), (69, 3840, 3376, "128x64", True),
+    (1450, 448, 1552, "128x128k64", False), (277, 4096, 1808, "128x128k64", True), (393, 320, 12728, "128x256", False), (819, 6784, 2512, "128x256", True),
+    (3692, 448, 2232, "192x256", False), (809, 5888, 6352, "192x256", True), (1446, 256, 7848, "256x192", False), (8352, 384, 1552, "256x256k64", False),
+    (409, 5760, 8416, "256x256k64", True), (8383, 1536, 2048, "streamk64", False)])
+def test_what_the_rule_picks(R, m, k, n, tile, cut):
+    picked, parts = plan(m, k, n)
+    assert (picked, parts > 1) == (tile, cut), (picked, parts)
+    g = np.random.Generator(np.random.PCG64(m * 1000 + k))
+    x, w, b, r = rand(g, (m, k), "bf16"), rand(g, (n, k), "bf16", k ** -0.5), rand(g, (n,), "bf16"), rand(g, (m, n), "bf16")
+    xd, wd = up(x, "bf16"), up(w, "bf16")
+    want = x @ w.T   # in f32: both sides' sums are within the spread of the exact ones
+    tol = 2 * (k + 20) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T + 1)
+    assert np.all(np.abs(down(R.linear(xd, wd)) - want) <= 2.0 ** -8 * np.abs(want) + tol)
+    z = want + b
+    full = z / (1 + np.exp(-z)) + r   # silu's slope stays below 1.1, its own error below 2^-18 of it
+    got = down(R.linear(xd, wd, up(b, "bf16"), "silu", up(r, "bf16")))
+    assert np.all(np.abs(got - full) <= 2.0 ** -8 * np.abs(full) + 2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)
+
+
+def test_plan_is_what_runs(R, monkeypatch):
+    """A product whose sums differ by tile and parts: the rule's name and parts, forced, give the bits of the call that is not."""
+    m, k, n = 277, 4096, 1808
+    g = np.random.Generator(np.random.PCG64(3))
+    x, w = up(rand(g, (m, k), "bf16"), "bf16"), up(rand(g, (n, k), "bf16"), "bf16")
+    tile, parts = plan(m, k, n)
+    free = down(R.linear(x, w))
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", tile)
+    np.testing.assert_array_equal(free, down(R.linear_packed(x, w, k_splits=parts)))
+    assert not np.array_equal(free, down(R.linear_packed(x, w, k_splits=parts + 1)))
