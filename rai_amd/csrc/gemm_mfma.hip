@@ -1144,12 +1144,12 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
 static __device__ int g_streamk_counters[4 * kNumCU];
 
 // How the stream-K kernel would share out an M x N x K product: false when it does not apply (tile count a multiple
-// of the CU count, too few tiles, or a tile would be the work of more than three blocks).
+// of the CU count, too few tiles, or a tile would be the work of more than three blocks).  Whether it pays: streamk_us.
 struct StreamKPlan {
   StreamKArgs k;
   size_t ws_bytes;
 };
-static bool streamk_plan(int M, int N, int K, int bk, StreamKPlan *plan, bool forced = false) {
+static bool streamk_plan(int M, int N, int K, int bk, StreamKPlan *plan) {
   const int P = kNumCU, KT = K / bk;
   const int T = ((M + 255) / 256) * ((N + 255) / 256);
   const int full = T / P, left = T % P;
@@ -1175,25 +1175,12 @@ static bool streamk_plan(int M, int N, int K, int bk, StreamKPlan *plan, bool fo
     if (parts > max_parts) max_parts = parts;
   }
   if (max_parts > 3 || sk_tiles > 2 * kNumCU) return false;
-  // Worth it when the CU time saved exceeds what the exchange of the shares costs.  Measured with cold weights, bias
-  // and gelu_new: 4096 x 10240 x 2560 (two shares per tile, 40 K tiles of a round saved) 237 -> 215 us, i.e. ~18 us
-  // for the exchange; 512 x 17920 x 2560 (three shares, 36 saved) 81 -> 84 us, i.e. ~39 us: every block ends on a
-  // read of the other shares plus the epilogue, with nothing left to hide them behind.  One K tile of a 256 x 256
-  // tile takes ~1 us with all CUs busy.
-  const float saved_us = (float)(P - left) / P * (K / 32) * 1.0f;
-  const float exchange_us = max_parts <= 2 ? 18.f : 39.f;
-  if (!forced && saved_us < 1.3f * exchange_us) return false;
   k.max_parts = max_parts;
   k.ws = nullptr;
   k.counters = nullptr;
   plan->k = k;
   plan->ws_bytes = (size_t)sk_tiles * max_parts * 256 * 256 * sizeof(float);
   return true;
-}
-
-size_t linear_streamk_workspace_bytes(int M, int N, int K) {
-  StreamKPlan plan;
-  return streamk_plan(M, N, K, 32, &plan) ? plan.ws_bytes : 0;
 }
 
 static int linear_device(const LinearArgs &a, int *dev) {
@@ -1203,15 +1190,15 @@ static int linear_device(const LinearArgs &a, int *dev) {
   return RAI_OK;
 }
 
-// True when the stream-K kernel serves this Linear (plain tile epilogue, workspace large enough, not switched off).
-static bool streamk_applies(const LinearArgs &a, int bk, StreamKPlan *plan, bool forced = false) {
+// True when the stream-K kernel can serve this Linear (plain tile epilogue, workspace large enough, not switched off).
+static bool streamk_applies(const LinearArgs &a, int bk, StreamKPlan *plan) {
   const char *off = getenv("RAI_HIP_NO_STREAMK");   // read per call: tests compare both forms in one process
   if (off && *off && *off != '0') return false;
   if (!a.splitk_ws || ((uintptr_t)a.splitk_ws & 15) || a.post_ln_out) return false;
   // one block per CU of a 256-CU part: the plan, the counter array and the XCD order are laid out for that grid
   int dev = -1;
   if (linear_device(a, &dev) != RAI_OK || device_cu_count(dev) != kNumCU) return false;
-  return a.K % bk == 0 && streamk_plan(a.M, a.N, a.K, bk, plan, forced) && plan->ws_bytes <= a.splitk_ws_bytes;
+  return a.K % bk == 0 && streamk_plan(a.M, a.N, a.K, bk, plan) && plan->ws_bytes <= a.splitk_ws_bytes;
 }
 
 // every GPU holds its own copy of a __device__ array at its own address: looked up once per device
@@ -1847,22 +1834,41 @@ static bool no_k64() {   // read per call: tests compare both forms in one proce
 static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 256) * ((a.N + 255) / 256)) >= 17 * kNumCU; }
 
 // Which of the tiles with K stages of 64 serves a product, and over how many parts of K, by what the kernels' own times make
-// of it (fitted to 170 products of 9 to 16384 rows, every tile, one to eight parts, weights from the caches and from HBM; what
-// is picked takes 2 % more than the best of them in the mean).  An XCD has 32 CUs and a run of tiles of its own, so rounds are
-// counted there: over the whole chip 36 tiles in seven parts look like one round of 256 CUs, but five tiles on an XCD are 35
-// blocks and two rounds (333 x 8960 x 1536: 38.7 us, in five parts 26.9).  Blocks share a CU: `stage` is the time of 64 of K with
-// one, two, three of them on it, `end` what a tile takes besides, to start and to write its outputs, `cut` the same where it
-// writes partial sums.  3 us are the launch; a K split adds 3.5 us (a launch) and 0.53 us per MB of partial sums, and leaves every
-// part four stages; partial sums in rows off 16-byte boundaries cost 2.2 us per MB of outputs more.  A norm of the finished rows rides on
-// the pass that sums the parts and is a launch of 5 us without one.
+// of it.  The constants are fitted to 1276 products (random ones of 9 to 16384 rows, and the widths of the decoders' layers by twelve
+// numbers of rows; every tile, one to twelve parts, weights from the caches and from HBM); over 654 others what is picked takes 0.7 %
+// more than the best of them in the mean, over a twentieth more at 34 and over a tenth at 9 (200 of another day: 0.9 %).  The worst of all: 1221 x 328 x 3776 (18.8 us
+// for 14.8), 512 x 1536 x 8960 (five parts 37.3, four 31.8), 6863 x 2368 x 2176 (102.5 for 87.3 by stream-K, see below).
+// An XCD has 32 CUs and a run of tiles of its own, so rounds are counted there: over the whole chip 36 tiles in seven parts look like one
+// round of 256 CUs, but five tiles on an XCD are 35 blocks and two rounds (333 x 8960 x 1536: 38.7 us, in five parts 26.9).  Blocks
+// share a CU: `stage` is the time of 64 of K with one, two, three of them on it, `end` what a tile takes besides, to start and to write
+// its outputs, `cut` the same where it writes partial sums.  A K split adds a launch and the partial sums' own time, and leaves every
+// part four stages; of more than 80 MB of partial sums none was the best (beyond 160 MB they took 0.15 us a MB more than counted
+// here); partial sums in rows off 16-byte boundaries cost 2.2 us per MB of outputs more.  A norm of the finished rows rides on the pass
+// that sums the parts and is a launch of 5 us without one.
 // 128 x 128 with eight waves (4 x 2, 32 x 64 each, two to a SIMD) took the place of four waves in two and four stages: 333 x 8960 x 1536
 // 20.5 to 18.9 us, 2000 x 2048 x 2048 22.7 to 21.1.  128 x 256 and 192 x 256 (eight waves, three and two stages) serve where 256 x 256
 // leaves a last round nearly empty: 1200 x 16384 x 2048 108 to 97 us, 3000 x 4096 x 4096 105 to 88, 777 x 22528 x 2048 114 to 91.
 enum { kTile128 = 0, kTile128x64, kTile64, kTile128x256, kTile256x192, kTile192x256, kTile256, kTileStreamK };
 struct TileCost { int bm, bn, share; float stage[3], end, cut; };
-static const TileCost kTileCosts[] = {{128, 128, 1, {0.45f}, 2.9f, 1.5f},       {128, 64, 2, {0.32f, 0.56f}, 2.15f, 1.0f}, {64, 64, 3, {0.256f, 0.406f, 0.626f}, 0.67f, 0.46f},
-                                      {128, 256, 1, {0.77f}, 6.2f, 2.9f}, {256, 192, 1, {1.16f}, 8.2f, 0.f},       {192, 256, 1, {1.02f}, 8.9f, 4.8f},
-                                      {256, 256, 1, {1.29f}, 11.3f, 3.7f}};
+static const TileCost kTileCosts[] = {{128, 128, 1, {0.482f}, 3.24f, 1.46f}, {128, 64, 2, {0.36f, 0.568f}, 2.02f, 0.929f}, {64, 64, 3, {0.256f, 0.382f, 0.614f}, 0.81f, 0.428f},
+                                      {128, 256, 1, {0.785f}, 6.77f, 2.27f}, {256, 192, 1, {1.21f}, 7.82f, 0.293f},        {192, 256, 1, {1.16f}, 7.58f, 0.472f},
+                                      {256, 256, 1, {1.33f}, 10.1f, 0.493f}};
+constexpr float kLaunchUs = 2.43f, kCutUs = 4.04f, kPartUsPerMB = 0.555f, kMostPartMB = 80.f, kShareUs = 20.9f;
+
+// Stream-K over 256 x 256 tiles, where its last round is exactly half full and so each of that round's tiles the work of two CUs, a half of
+// K each: no CU is left idle, for an exchange of the halves (us, stream-K, the best whole tiles: 4096 x 10240 x 2560 200, 212; 16384 x
+// 1536 x 8960 374, 419; 1200 x 32768 x 2048 168, 174).  Shares that begin anywhere in K lose more in the L2s, where blocks no longer read
+// the same columns together, than they win in idle CUs: of 168 such products with 40 stages and more the median took 1.14 times the best
+// whole tiles' time (7770 x 2560 x 10240 476 us for 369, 7443 x 2560 x 2560 133 for 104), three less than 0.96 of it (14476 x 1536 x 8960
+// 344 for 388).  0: does not pay or does not apply.
+static float streamk_us(const LinearArgs &a, int bk) {
+  const int tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256);
+  StreamKPlan plan;
+  if (!has_huge_tiles(a) || tiles % kNumCU != kNumCU / 2 || a.K / bk % 2 || !streamk_applies(a, bk, &plan)) return 0.f;
+  const float tile = kTileCosts[kTile256].end + kTileCosts[kTile256].stage[0] * ((float)a.K / 64), shared = tile * ((float)tiles / kNumCU) + kShareUs;
+  return shared < tile * ((tiles + kNumCU - 1) / kNumCU) ? kLaunchUs + shared : 0.f;
+}
+
 struct TilePlan { int tile, splits; };
 static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int last = kTileStreamK) {
   const int stages = a.K / 64;
@@ -1873,23 +1879,17 @@ static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int las
     const TileCost &c = kTileCosts[t];
     const int64_t tiles = (int64_t)((a.M + c.bm - 1) / c.bm) * ((a.N + c.bn - 1) / c.bn);
     for (int s = 1; s <= 12; ++s) {
-      if (s > 1 && (a.force_splits == 1 || stages / s < 4 || !a.splitk_ws || (size_t)s * a.M * a.N * sizeof(float) > a.splitk_ws_bytes)) break;
+      if (s > 1 && (a.force_splits == 1 || stages / s < 4 || s * part_mb > kMostPartMB || !a.splitk_ws || (size_t)s * a.M * a.N * sizeof(float) > a.splitk_ws_bytes)) break;
       const int64_t per_cu = ((tiles + kXcds - 1) / kXcds * s + kNumCU / kXcds - 1) / (kNumCU / kXcds);
       const int left = (int)(per_cu % c.share);
       const float stage = per_cu / c.share * c.stage[c.share - 1] + (left ? c.stage[left - 1] : 0.f);
-      const float cost = 3.f + stage * ((stages + s - 1) / s) +
-                         (s > 1 ? 3.5f + 0.53f * s * part_mb + (a.N % 4 ? 2.2f * part_mb : 0.f) + per_cu * c.cut : per_cu * c.end + (a.post_ln_out ? 5.f : 0.f));
+      const float cost = kLaunchUs + stage * ((stages + s - 1) / s) +
+                         (s > 1 ? kCutUs + kPartUsPerMB * s * part_mb + (a.N % 4 ? 2.2f * part_mb : 0.f) + per_cu * c.cut : per_cu * c.end + (a.post_ln_out ? 5.f : 0.f));
       if ((t == first && s == 1) || cost < least) { least = cost; best = {t, s}; }
     }
   }
-  // Stream-K over 256 x 256 tiles: no round is left empty, for an exchange of the shares: 21 us with two of them to a tile, 94 with three
-  // (4096 x 10240 x 2560 in 215 us for 222 of whole tiles, 16384 x 1536 x 8960 366 for 411 of 256 x 192).
-  StreamKPlan sk;
-  if (last == kTileStreamK && has_huge_tiles(a) && streamk_applies(a, 64, &sk)) {
-    const TileCost &c = kTileCosts[kTile256];
-    const float rounds = (float)(((a.M + 255) / 256) * ((a.N + 255) / 256)) / kNumCU;
-    if (3.f + rounds * (c.end + c.stage[0] * stages) + (sk.k.max_parts <= 2 ? 21.f : 94.f) < least) best = {kTileStreamK, 1};
-  }
+  if (last == kTileStreamK)
+    if (const float us = streamk_us(a, 64); us > 0.f && us < least) best = {kTileStreamK, 1};
   return best;
 }
 
@@ -2067,14 +2067,17 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
     if (!strcmp(knob, "streamk") || !strcmp(knob, "streamk64")) {
       const int bk = knob[7] ? 64 : 32;
       StreamKPlan plan;
-      RAI_REQUIRE(splits == 1 && streamk_applies(a, bk, &plan, true), RAI_ERR_UNSUPPORTED,
+      RAI_REQUIRE(splits == 1 && streamk_applies(a, bk, &plan), RAI_ERR_UNSUPPORTED,
                   "linear: RAI_HIP_GEMM_TILE=%s does not apply to %dx%dx%d", knob, a.M, a.N, a.K);
       return bk == 64 ? launch_streamk<2>(st, a, plan) : launch_streamk<4>(st, a, plan);
     }
   }
   if (a.K % 64 == 0 && !no_k64()) return launch_tile_k64(st, a, tile);
-  StreamKPlan plan;
-  if (splits == 1 && has_huge_tiles(a)) return streamk_applies(a, 32, &plan) ? launch_streamk<4>(st, a, plan) : launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
+  if (splits == 1 && has_huge_tiles(a)) {
+    StreamKPlan plan;
+    if (streamk_us(a, 32) > 0.f && streamk_applies(a, 32, &plan)) return launch_streamk<4>(st, a, plan);
+    return launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
+  }
   return launch_cfg_dma<128, 128, 3, 2>(st, a, splits);
 }
 

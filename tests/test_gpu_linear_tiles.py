@@ -114,10 +114,10 @@ def plan(m, k, n):
 
 # What the rule picks by itself: every tile whole and, where it is ever the best, cut over K.
 @pytest.mark.parametrize("m,k,n,tile,cut", [
-    (87, 320, 312, "64x64", False), (68, 2176, 288, "64x64", True), (524, 704, 2112, "128x64", False), (69, 3840, 3376, "128x64", True),
-    (1450, 448, 1552, "128x128k64", False), (277, 4096, 1808, "128x128k64", True), (393, 320, 12728, "128x256", False), (819, 6784, 2512, "128x256", True),
-    (3692, 448, 2232, "192x256", False), (809, 5888, 6352, "192x256", True), (1446, 256, 7848, "256x192", False), (8352, 384, 1552, "256x256k64", False),
-    (409, 5760, 8416, "256x256k64", True), (8383, 1536, 2048, "streamk64", False)])
+    (87, 320, 312, "64x64", False), (68, 2176, 288, "64x64", True), (675, 192, 5432, "128x64", False), (69, 3840, 3376, "128x64", True),
+    (1450, 448, 1552, "128x128k64", False), (65, 5632, 3424, "128x128k64", True), (393, 320, 12728, "128x256", False), (130, 6400, 5560, "128x256", True),
+    (3692, 448, 2232, "192x256", False), (259, 3520, 11096, "192x256", True), (4843, 192, 2312, "256x192", False), (8352, 384, 1552, "256x256k64", False),
+    (409, 5760, 8416, "256x256k64", True), (4000, 2560, 10200, "streamk64", False)])
 def test_what_the_rule_picks(R, m, k, n, tile, cut):
     picked, parts = plan(m, k, n)
     assert (picked, parts > 1) == (tile, cut), (picked, parts)
@@ -135,7 +135,7 @@ def test_what_the_rule_picks(R, m, k, n, tile, cut):
 
 def test_plan_is_what_runs(R, monkeypatch):
     """A product whose sums differ by tile and parts: the rule's name and parts, forced, give the bits of the call that is not."""
-    m, k, n = 277, 4096, 1808
+    m, k, n = 409, 5760, 8416
     g = np.random.Generator(np.random.PCG64(3))
     x, w = up(rand(g, (m, k), "bf16"), "bf16"), up(rand(g, (n, k), "bf16"), "bf16")
     tile, parts = plan(m, k, n)
