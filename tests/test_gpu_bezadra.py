@@ -265,6 +265,20 @@ def test_sink(hip, dt, sink):
         dec.close()
 
 
+@pytest.mark.parametrize("batch", [1, 8, 16, 24])
+@pytest.mark.parametrize("dim,softcap", [(64, 2.5), (64, 0.0), (128, 2.5), (256, 2.5)])
+def test_capped_attention_by_number_of_groups(hip, dim, softcap, batch):
+    """The prefill attention with cap, sink and gate in bf16, at 80, 640, 1280 and 1920 groups of 32 queries: each head size with every number
+    of waves to a group and both lengths of key tiles."""
+    cfg = bm.config([bm.attention(heads=16, kv_heads=4, dim=dim, vdim=dim, dims=32, scale=dim ** -0.5, softcap=softcap, ff=None)])
+    p = bezadra.random_params(cfg, "bf16", 30)
+    dec, ids = bm.build(cfg, p, "bf16", max_batch=batch, max_context=160), tokens(cfg, (batch, 150), 31)
+    ref, got = bezadra.Model(cfg, p), bm.run_portions(dec, ids, [150])
+    for b in sorted({0, batch // 2, batch - 1}):
+        assert_close(got[b], ref.logits(ids[b]), "bf16", f"row {b} of {batch}")
+    dec.close()
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 def test_long_prompt(hip, dt):
     """Positions far beyond the frequency scaling's original length, more rows than the largest product tile."""

@@ -16,20 +16,30 @@ def R(hip):
     return ops
 
 
-def reference(q, k, v, scale, causal, f32_scores):
-    """The result in 64 bits (rounded scores rounded as the model rounds them) and how far a correct bf16 form may be off."""
+def whole(g, shape, step=1.0):
+    """Whole multiples of a power of two: sums of their products are exact in f32, in any order."""
+    return (g.integers(-4, 5, shape) * step).astype(np.float32)
+
+
+def reference(q, k, v, scale, causal, f32_scores, rounded=True):
+    """The result in 64 bits (scores rounded as the model rounds them) and how far a correct bf16 form may be off.  Scores that are
+    rounded are those of whole(): either rounding could turn on the last bit of a sum, and a turned score is far more than the
+    arithmetic's own error."""
     q, k, v = (t.astype(np.float64) for t in (q, k, v))
     n = q.shape[1] // k.shape[1]
     k, v = np.repeat(k, n, 1), np.repeat(v, n, 1)
     s, size = np.matmul(q, np.swapaxes(k, 2, 3)), np.matmul(np.abs(q), np.swapaxes(np.abs(k), 2, 3)).max()
     S, T = s.shape[2:]
-    # a score's f32 sum is within D + 2 roundings of its absolute sum
-    off = (q.shape[-1] + 2) * 2.0 ** -24 * size * abs(scale)
-    if f32_scores:
+    if f32_scores:   # a score's f32 sum is within D + 2 roundings of its absolute sum
+        off = (q.shape[-1] + 2) * 2.0 ** -24 * size * abs(scale)
         s = s * scale
     else:
-        s = rnd(rnd(s.astype(np.float32), "bf16") * rnd(np.float32(scale), "bf16"), "bf16").astype(np.float64)
-        off += 2 * 2.0 ** -7 * np.abs(s).max()   # which may turn either rounding to the next bf16 number
+        assert size < 2 ** 20 and np.array_equal(s * 4, np.rint(s * 4))
+        if rounded:
+            s = rnd(rnd(s.astype(np.float32), "bf16") * rnd(np.float32(scale), "bf16"), "bf16").astype(np.float64)
+        else:
+            s = s * scale
+        off = (2 * np.abs(s).max() + 8) * 2.0 ** -24   # the exponent's product with log2(e) and the exponential
     if causal:
         s = np.where(np.arange(T)[None] <= np.arange(T - S, T)[:, None], s, -np.inf)
     p = np.exp(s - s.max(-1, keepdims=True))
@@ -41,14 +51,24 @@ def reference(q, k, v, scale, causal, f32_scores):
     return want, rel * flat(p @ np.abs(v)) * (1 + 2.0 ** -8) + 2.0 ** -8 * np.abs(want) + 1e-30
 
 
+def operands(g, b, hq, hkv, s, t, d, f32_scores):
+    if f32_scores:
+        return rand(g, (b, hq, s, d), "bf16"), rand(g, (b, hkv, t, d), "bf16"), rand(g, (b, hkv, t, d), "bf16")
+    return whole(g, (b, hq, s, d)), whole(g, (b, hkv, t, d), 0.25), rand(g, (b, hkv, t, d), "bf16")
+
+
 def check(R, b, hq, hkv, s, t, d, causal, f32_scores, scale=None, transposed=False):
     g = np.random.Generator(np.random.PCG64(b + s + d))
-    scale = d ** -0.5 if scale is None else scale
-    q, k, v = rand(g, (b, hq, s, d), "bf16"), rand(g, (b, hkv, t, d), "bf16"), rand(g, (b, hkv, t, d), "bf16")
+    plain, scale = scale is None, (1 if f32_scores else 3) * d ** -0.5 if scale is None else scale
+    q, k, v = operands(g, b, hq, hkv, s, t, d, f32_scores)
     lay = (lambda x: up(np.ascontiguousarray(np.swapaxes(x, 1, 2)), "bf16").transpose(1, 2)) if transposed else (lambda x: up(x, "bf16"))
     want, tol = reference(q, k, v, scale, causal, f32_scores)
     got = down(R.attention(lay(q), lay(k), lay(v), scale, causal, f32_scores)).astype(np.float64)
     assert np.all(np.abs(got - want) <= tol), f"worst {np.max(np.abs(got - want) / tol):.2f} of the bound"
+    if plain and t > 16:   # the bound tells scores that are a fiftieth off, and ones that are not rounded, from these
+        others = [reference(q, k, v, 1.02 * scale, causal, f32_scores)] + ([] if f32_scores else [reference(q, k, v, scale, causal, 0, False)])
+        for other, _ in others:
+            assert np.any(np.abs(other - want) > 2 * tol)
 
 
 # (sequences, query heads, key heads, rows, keys): up to 256 groups of 32 rows, up to 512, 1024, 1536 and beyond 1792; one tile, a last tile

@@ -139,6 +139,20 @@ def test_batch_against_each_alone(hip, dt, batch):
     dec.close()
 
 
+@pytest.mark.parametrize("batch", [1, 8, 16, 24])
+@pytest.mark.parametrize("dim,window", [(64, 20), (64, 60), (128, 34), (128, 100), (256, 40), (64, None)])
+def test_windowed_attention_by_number_of_groups(hip, dim, window, batch):
+    """The prefill attention with window and gate in bf16, at 80, 640, 1280 and 1920 groups of 32 queries: each head size with every number
+    of waves to a group and both lengths of key tiles; windows within a tile of keys and over several."""
+    cfg = lm.config([lm.layer(heads=16, dim=dim, vdim=dim, window=window, scale=dim ** -0.5, mlp=None)])
+    p = lm.random_params(cfg, "bf16", 30)
+    dec, ids = lm.build(cfg, p, "bf16", max_batch=batch, max_context=160), tokens(cfg, (batch, 150), 31)
+    ref, got = lelitar.Model(cfg, p), lm.run_portions(dec, ids, [150])
+    for b in sorted({0, batch // 2, batch - 1}):
+        assert_close(got[b], ref.logits(ids[b]), "bf16", f"row {b} of {batch}")
+    dec.close()
+
+
 def edge_cases():
     return [(w, mlp) for w in (2, 9, 64, 65, 100) for mlp in (None, "moe")]
 
