@@ -793,8 +793,10 @@ __global__ void __launch_bounds__(256) k_attn_decode_merge_bf16(AttnDecodeArgs a
   ((bf16_raw *)a.out + (int64_t)b * a.out_row_stride + (int64_t)h * D + d)->bits = f32_to_bf16_bits(O * gate);
 }
 
-// Splits of the context over blocks of `ch` keys.  One that holds the longest context writes the result itself, without the launch that
-// merges: 24 sequences on 51 to 83 keys (8 heads of 256 on one) 11.7 us for 8.9 + 4.7 in two blocks a sequence.
+// Splits of the context over blocks of `ch` keys.  A block that holds the longest context the cache has room for (the context itself is the
+// device's to know) writes the result itself, without the launch that merges: 24 sequences on 51 to 83 keys (8 heads of 256 on one) 11.7 us
+// for 8.9 + 4.7 in two blocks a sequence.  One to 32 sequences of 52 to 122 keys decoded so, against two blocks each: 128 features 0.2 to
+// 3 % sooner, 256 features 0.3 to 2 % up to 96 keys and within 1 % either way beyond.
 static int mfma_decode_splits(const AttnDecodeArgs &a, int ch) {
   if (a.Tmax <= ch && !getenv("RAI_HIP_ATTN_SPLITS")) return 1;
   const int ns = decode_splits(a, a.Hkv), need = (a.Tmax + ch - 1) / ch;
