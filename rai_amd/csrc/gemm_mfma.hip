@@ -1144,7 +1144,8 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
 static __device__ int g_streamk_counters[4 * kNumCU];
 
 // How the stream-K kernel would share out an M x N x K product: false when it does not apply (tile count a multiple
-// of the CU count, too few tiles, or a tile would be the work of more than three blocks).  Whether it pays: streamk_us.
+// of the CU count, too few tiles, or a tile would be the work of more than three blocks).  Whether it pays: streamk_us,
+// streamk_pays_k32.
 struct StreamKPlan {
   StreamKArgs k;
   size_t ws_bytes;
@@ -1836,8 +1837,9 @@ static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 25
 // Which of the tiles with K stages of 64 serves a product, and over how many parts of K, by what the kernels' own times make
 // of it.  The constants are fitted to 1276 products (random ones of 9 to 16384 rows, and the widths of the decoders' layers by twelve
 // numbers of rows; every tile, one to twelve parts, weights from the caches and from HBM); over 654 others what is picked takes 0.7 %
-// more than the best of them in the mean, over a twentieth more at 34 and over a tenth at 9 (200 of another day: 0.9 %).  The worst of all: 1221 x 328 x 3776 (18.8 us
-// for 14.8), 512 x 1536 x 8960 (five parts 37.3, four 31.8), 6863 x 2368 x 2176 (102.5 for 87.3 by stream-K, see below).
+// more than the best of them in the mean, over a twentieth more at 34 and over a tenth at 9 (600 of other days: 0.8 to 0.9 %).  The
+// worst of all: 1221 x 328 x 3776 (18.8 us for 14.8), 1226 x 536 x 8128 (41.6 for 33.8), 512 x 1536 x 8960 (five parts 37.3, four 31.8),
+// 6863 x 2368 x 2176 (102.5 for 87.3 by stream-K, see below).
 // An XCD has 32 CUs and a run of tiles of its own, so rounds are counted there: over the whole chip 36 tiles in seven parts look like one
 // round of 256 CUs, but five tiles on an XCD are 35 blocks and two rounds (333 x 8960 x 1536: 38.7 us, in five parts 26.9).  Blocks
 // share a CU: `stage` is the time of 64 of K with one, two, three of them on it, `end` what a tile takes besides, to start and to write
@@ -1861,12 +1863,20 @@ constexpr float kLaunchUs = 2.43f, kCutUs = 4.04f, kPartUsPerMB = 0.555f, kMostP
 // the same columns together, than they win in idle CUs: of 168 such products with 40 stages and more the median took 1.14 times the best
 // whole tiles' time (7770 x 2560 x 10240 476 us for 369, 7443 x 2560 x 2560 133 for 104), three less than 0.96 of it (14476 x 1536 x 8960
 // 344 for 388).  0: does not pay or does not apply.
-static float streamk_us(const LinearArgs &a, int bk) {
+static float streamk_us(const LinearArgs &a) {
   const int tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256);
   StreamKPlan plan;
-  if (!has_huge_tiles(a) || tiles % kNumCU != kNumCU / 2 || a.K / bk % 2 || !streamk_applies(a, bk, &plan)) return 0.f;
+  if (!has_huge_tiles(a) || tiles % kNumCU != kNumCU / 2 || a.K / 64 % 2 || !streamk_applies(a, 64, &plan)) return 0.f;
   const float tile = kTileCosts[kTile256].end + kTileCosts[kTile256].stage[0] * ((float)a.K / 64), shared = tile * ((float)tiles / kNumCU) + kShareUs;
   return shared < tile * ((tiles + kNumCU - 1) / kNumCU) ? kLaunchUs + shared : 0.f;
+}
+// With K stages of 32 (K no multiple of 64) whole 256 x 256 tiles are all there is beside it, and any shares pay where the CU time saved
+// exceeds the exchange of two or three to a tile; a K tile of 32 takes some 1 us with all CUs busy (us, stream-K, whole tiles: 16384 x
+// 1536 x 8928 464, 586; 8192 x 2560 x 5152 235, 306; 7770 x 2560 x 10272 475, 495; 4096 x 2560 x 10272 235, 286).
+static bool streamk_pays_k32(const LinearArgs &a, StreamKPlan *plan) {
+  if (!streamk_applies(a, 32, plan)) return false;
+  const int left = ((a.M + 255) / 256) * ((a.N + 255) / 256) % kNumCU;
+  return (float)(kNumCU - left) / kNumCU * (a.K / 32) >= 1.3f * (plan->k.max_parts <= 2 ? 18.f : 39.f);
 }
 
 struct TilePlan { int tile, splits; };
@@ -1889,7 +1899,7 @@ static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int las
     }
   }
   if (last == kTileStreamK)
-    if (const float us = streamk_us(a, 64); us > 0.f && us < least) best = {kTileStreamK, 1};
+    if (const float us = streamk_us(a); us > 0.f && us < least) best = {kTileStreamK, 1};
   return best;
 }
 
@@ -2075,8 +2085,7 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
   if (a.K % 64 == 0 && !no_k64()) return launch_tile_k64(st, a, tile);
   if (splits == 1 && has_huge_tiles(a)) {
     StreamKPlan plan;
-    if (streamk_us(a, 32) > 0.f && streamk_applies(a, 32, &plan)) return launch_streamk<4>(st, a, plan);
-    return launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
+    return streamk_pays_k32(a, &plan) ? launch_streamk<4>(st, a, plan) : launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
   }
   return launch_cfg_dma<128, 128, 3, 2>(st, a, splits);
 }

@@ -316,10 +316,11 @@ def test_gemm_forced_tile_is_not_split_for_another_tile(R, monkeypatch):
 
 
 def test_gemm_dispatcher_picks_each_tile_by_itself(R, monkeypatch):
-    # no override: K of 64 and 96, shorter than the prefetch depth of every tile, with stages of 64 and of 32, and 3000 x 3100 x 2560
+    # no override: K of 64 and 96, shorter than the prefetch depth of every tile, with stages of 64 and of 32; 3000 x 3100 x 2560; and
+    # stream-K with stages of 32 (144 tiles on 256 CUs, K no multiple of 64)
     monkeypatch.delenv("RAI_HIP_GEMM_TILE", raising=False)
     dt = "bf16"
-    for m, n, k in [(3072, 3072, 64), (4096, 2048, 96), (600, 520, 64), (3000, 3100, 2560)]:
+    for m, n, k in [(3072, 3072, 64), (4096, 2048, 96), (600, 520, 64), (3000, 3100, 2560), (3000, 3070, 3744)]:
         g = rng(114)
         x, w = rand(g, (m, k), dt), rand(g, (n, k), dt, 0.05)
         want = onn.linear(x, w, None, dt)
