@@ -17,38 +17,11 @@
 #include <cstring>
 #include <type_traits>
 
-#include "gemm.h"
+#include "gemm_device.h"
 #include "latent.h"
 #include "rai_hip_peaks.h"
 
 namespace rai {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
-constexpr int kXcds = 8;
-
-// Tile order inside an XCD's run: bands of kGroupM tile rows swept across all tile columns, so the
-// ~100 tiles that are resident on an XCD at any moment form a block of about kGroupM x 12 tiles and
-// share their A and B panels through that XCD's L2 (a column-by-column order re-reads all of A from
-// memory for every tile column).
-constexpr int kGroupM = 8;
-__device__ __forceinline__ void tile_coords(int tile, int tiles_m, int tiles_n, int *tile_m, int *tile_n) {
-  const int band = tile / (kGroupM * tiles_n);
-  const int first_m = band * kGroupM;
-  const int height = tiles_m - first_m < kGroupM ? tiles_m - first_m : kGroupM;
-  const int in_band = tile - band * kGroupM * tiles_n;
-  *tile_m = first_m + in_band % height;
-  *tile_n = in_band / height;
-}
-
-__device__ __forceinline__ int xcd_remap(int bid, int total) {
-  // blocks bid, bid+8, bid+16, ... run on the same XCD; give them consecutive tiles
-  const int per = (total + kXcds - 1) / kXcds;
-  return (bid % kXcds) * per + bid / kXcds;
-}
 
 // LDS a tile kernel needs: two stages of A and B tiles, or the epilogue staging area if that is larger.
 template <int BM, int BN, int PITCH, int WGN = 2, int WGM = 2> constexpr int gemm_lds_bytes() {
@@ -59,42 +32,6 @@ template <int BM, int BN, int PITCH, int WGN = 2, int WGM = 2> constexpr int gem
 // LDS of the LDS-DMA tile kernels: NS stages of 32 of K, or (NS == 2, or SH == 0) of 64.
 template <int BM, int BN, int NS, int WGN, int WGM = 2, int SH = 2> constexpr int dma_lds_bytes() {
   return gemm_lds_bytes<BM, BN, NS == 2 || SH == 0 ? 32 * NS : 32 * NS / 2, WGN, WGM>();
-}
-
-// Applies activation `act` to the elements of x[8] whose column n + e is >= from.  The switch on the
-// (block-uniform) activation sits outside the element loop, so only one activation's code runs.
-// The results are rounded to bf16 (relative step 2^-8), so tanh-GELU and SiLU are evaluated through the hardware
-// exponential and reciprocal (relative error ~1e-6) instead of the library tanhf / expf and a division:
-// 0.5 x (1 + tanh u) = x / (1 + exp(-2u)).  The f32 Linear keeps the library functions (act_eval).
-__device__ __forceinline__ float act_eval_bf16_out(int act, float x) {
-  if (act == RAI_UN_NEW_GELU) {
-    const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-2.0f * 1.4426950408889634f * u));
-  }
-  if (act == RAI_UN_SILU) return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
-  return act_eval(act, x);
-}
-template <int N>
-__device__ __forceinline__ void act_n(int act, float (&x)[N], int n, int from) {
-#define RAI_ACT_CASE(K)                                     \
-  case K:                                                   \
-    _Pragma("unroll") for (int e = 0; e < N; ++e)           \
-      if (n + e >= from) x[e] = act_eval_bf16_out(K, x[e]); \
-    break;
-  switch (act) {
-    RAI_ACT_CASE(RAI_UN_GELU)
-    RAI_ACT_CASE(RAI_UN_NEW_GELU)
-    RAI_ACT_CASE(RAI_UN_SILU)
-    RAI_ACT_CASE(RAI_UN_RELU)
-    RAI_ACT_CASE(RAI_UN_TANH)
-    default: break;
-  }
-#undef RAI_ACT_CASE
-}
-__device__ __forceinline__ void act8(int act, float (&x)[8], int n, int from) { act_n<8>(act, x, n, from); }
-__device__ __forceinline__ void unpack8(const u32x4 &p, float (&f)[8]) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) f[e] = bf16_bits_to_f32((uint16_t)(p[e >> 1] >> (16 * (e & 1))));
 }
 
 // Tile epilogue shared by the tile kernels: every wave stages 32 x WN accumulators at a time in
@@ -117,41 +54,15 @@ __device__ __forceinline__ void gemm_tile_epilogue(const LinearArgs &a, f32x16 (
   // rows (CG = 12, the 96-column wave tile, leaves 16 of the 64 lanes idle)
   constexpr int RP = 64 / CG >= 16 ? 16 : 64 / CG >= 8 ? 8 : 64 / CG >= 4 ? 4 : 2;
   constexpr int ITEMS = 32 / RP;             // passes
-  const uint16_t *bias = (const uint16_t *)a.bias;
-  const uint16_t *bias2 = (const uint16_t *)a.bias2;
-  const uint16_t *res = (const uint16_t *)a.residual;
-  const bool vec_out = (a.ld1 % 8 == 0) && (a.n_split % 8 == 0) && (a.n_split == a.N || a.ld2 % 8 == 0) &&
-                       ((uintptr_t)a.out1 % 16 == 0) && (a.n_split == a.N || (uintptr_t)a.out2 % 16 == 0) &&
-                       (!res || (a.ldr % 8 == 0 && (uintptr_t)res % 16 == 0)) && a.N % 8 == 0;
+  const bool vec_out = rows_store_16(a);
   // A lane serves the same 8 columns in every pass: their bias values are fetched once, ahead of the passes, not
   // inside each of them, where the load's latency (about a microsecond under load) sat between the LDS read and the
   // store of every pass.
   static_assert(RP * CG <= 64 && 32 % RP == 0, "a pass is RP whole rows of CG column groups");
   const int n = n0 + wn * WN + (lane % CG) * 8;
   const bool whole = n + 8 <= a.N;
-  float bv[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) bv[e] = 0.f;
-  if (bias && !partial && n < a.N) {
-    if (whole && ((uintptr_t)(bias + n) & 15) == 0) unpack8(*reinterpret_cast<const u32x4 *>(bias + n), bv);
-    else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (n + e < a.N) bv[e] = bf16_bits_to_f32(bias[n + e]);
-    }
-  }
-  if (bias2 && !partial && n < a.N) {
-    float b2[8];
-    if (whole && ((uintptr_t)(bias2 + n) & 15) == 0) {
-      unpack8(*reinterpret_cast<const u32x4 *>(bias2 + n), b2);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) bv[e] += b2[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (n + e < a.N) bv[e] += bf16_bits_to_f32(bias2[n + e]);
-    }
-  }
+  float bv[8] = {};
+  if (!partial) load_bias8(a, n, bv);
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     // accumulator register r of lane l is C[8*(r/4) + 4*(l/32) + r%4][l%32]
@@ -181,92 +92,7 @@ __device__ __forceinline__ void gemm_tile_epilogue(const LinearArgs &a, f32x16 (
         }
         continue;
       }
-      if (a.glu) {  // columns n..n+7 are four (gate, up) pairs -> four outputs at column n/2
-        uint16_t *dst = (uint16_t *)a.out1 + (int64_t)m * a.ld1 + (n >> 1);
-        float gr[8], ga[4], gl[4];
-        if (a.act == kActClampedGlu) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) gl[e] = glu_clamped_bf16_out(v[2 * e] + bv[2 * e], v[2 * e + 1] + bv[2 * e + 1], a.act_limit, a.act_alpha);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) gr[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e] + bv[e]));  // gate / up rounded to bf16 as the reference does
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ga[e] = gr[2 * e];
-          act_n<4>(a.act, ga, 0, 0);   // the four gates
-#pragma unroll
-          for (int e = 0; e < 4; ++e) gl[e] = bf16_bits_to_f32(f32_to_bf16_bits(ga[e])) * gr[2 * e + 1];
-        }
-        if (whole && a.ld1 % 4 == 0 && (uintptr_t)a.out1 % 8 == 0) {
-          typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
-          u32x2 o = {pack_bf16x2(gl[0], gl[1]), pack_bf16x2(gl[2], gl[3])};
-          *reinterpret_cast<u32x2 *>(dst) = o;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + 2 * e + 1 < a.N) dst[e] = f32_to_bf16_bits(gl[e]);
-        }
-        continue;
-      }
-      // compile-time element indices throughout: a loop bounded by a run-time count would index v[]
-      // dynamically, which the compiler lowers to a chain of selects per access
-      const int lim = a.N - n < 8 ? a.N - n : 8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] += bv[e];
-      if (a.act >= 0) act8(a.act, v, n, a.act_from);
-      if (a.f32_out) {
-        float *dst = (float *)a.out1 + (int64_t)m * a.ld1 + n;
-        const float *rsrc = res ? (const float *)a.residual + (int64_t)m * a.ldr + n : nullptr;
-        if (whole && a.ld1 % 4 == 0 && (!res || a.ldr % 4 == 0) && (((uintptr_t)a.out1 | (uintptr_t)a.residual) & 15) == 0) {
-          f32x4 r0 = {0.f, 0.f, 0.f, 0.f}, r1 = r0;
-          if (rsrc) {
-            r0 = *reinterpret_cast<const f32x4 *>(rsrc);
-            r1 = *reinterpret_cast<const f32x4 *>(rsrc + 4);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            r0[e] = fmaf(a.out_scale, v[e], r0[e]);
-            r1[e] = fmaf(a.out_scale, v[4 + e], r1[e]);
-          }
-          *reinterpret_cast<f32x4 *>(dst) = r0;
-          *reinterpret_cast<f32x4 *>(dst + 4) = r1;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (e < lim) dst[e] = fmaf(a.out_scale, v[e], rsrc ? rsrc[e] : 0.f);
-        }
-        continue;
-      }
-      if (res) {
-        if (vec_out) {
-          float rv[8];
-          unpack8(*reinterpret_cast<const u32x4 *>(res + (int64_t)m * a.ldr + n), rv);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] += rv[e];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (e < lim) v[e] += bf16_bits_to_f32(res[(int64_t)m * a.ldr + n + e]);
-        }
-      }
-      if (vec_out) {
-        u32x4 o;
-        o.x = (uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16);
-        o.y = (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16);
-        o.z = (uint32_t)f32_to_bf16_bits(v[4]) | ((uint32_t)f32_to_bf16_bits(v[5]) << 16);
-        o.w = (uint32_t)f32_to_bf16_bits(v[6]) | ((uint32_t)f32_to_bf16_bits(v[7]) << 16);
-        uint16_t *dst = n < a.n_split ? (uint16_t *)a.out1 + (int64_t)m * a.ld1 + n
-                                      : (uint16_t *)a.out2 + (int64_t)m * a.ld2 + (n - a.n_split);
-        *reinterpret_cast<u32x4 *>(dst) = o;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          if (e < lim) {
-            const int nn = n + e;
-            if (nn < a.n_split) ((uint16_t *)a.out1)[(int64_t)m * a.ld1 + nn] = f32_to_bf16_bits(v[e]);
-            else ((uint16_t *)a.out2)[(int64_t)m * a.ld2 + (nn - a.n_split)] = f32_to_bf16_bits(v[e]);
-          }
-        }
-      }
+      store_row8(a, v, bv, m, n, whole, vec_out);
     }
   }
 }
@@ -739,26 +565,9 @@ __global__ void __launch_bounds__(128 * WGN) k_gemm_bf16_mfma_grouped(LinearArgs
 // with device-scope stores and counts itself in; the block that arrives
 // last adds the slots in slot order (so the sum does not depend on who was last) and runs the epilogue.  Nobody
 // waits for anybody.  The remaining tiles follow in whole rounds, one tile per block as before.
-struct StreamKArgs {
-  int sk_tiles;   // tiles 0 .. sk_tiles-1 are shared out by K tile; the rest run whole
-  int q, rem;     // units per block: blocks 0 .. rem-1 take q + 1, the others q
-  int max_parts;  // slots per tile in the workspace
-  float *ws;      // [sk_tiles][max_parts][BM * BN] f32
-  int *counters;  // [sk_tiles][2] (tickets, stored shares), zero between launches
-  int *fault;     // host-visible word: RAI_FAULT_STREAMK is stored here when a wait for shares expires
-  int spin_limit; // polls of the stored-shares counter before the wait is given up
-  int drop_tile;  // test hook: the stored shares of this tile are never counted (-1: none), so its wait must expire
-};
-
-__device__ __forceinline__ int sk_start(const StreamKArgs &k, int p) { return p * k.q + (p < k.rem ? p : k.rem); }
-__device__ __forceinline__ int sk_block_of(const StreamKArgs &k, int u) {
-  const int big = k.rem * (k.q + 1);
-  return u < big ? u / (k.q + 1) : k.rem + (u - big) / k.q;
-}
-
 template <int BM, int BN, int NS, int SH, int WGN>
 __global__ void __launch_bounds__(128 * WGN) k_gemm_bf16_mfma_dma_streamk(LinearArgs a, StreamKArgs sk) {
-  constexpr int BK = NS == 2 ? 64 : 32;   // the unit of sharing is one K tile of the main loop
+  constexpr int BK = 32;   // the unit of sharing is one K tile of the main loop
   constexpr int MT = BM / 64, NT = BN / (32 * WGN);
   constexpr int LDS_BYTES = dma_lds_bytes<BM, BN, NS, WGN>();
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -796,11 +605,7 @@ __global__ void __launch_bounds__(128 * WGN) k_gemm_bf16_mfma_dma_streamk(Linear
     tile_coords(tile, tiles_m, tiles_n, &tile_m, &tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     __syncthreads();   // the previous segment's epilogue staging is done with the LDS
-    if constexpr (NS == 2) {
-      dma_tile_mainloop_k64<BM, BN, WGN>(a, lds, m0, n0, kt0 * BK, kt1 - kt0, wave, lane, acc);
-    } else {
-      dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, kt0 * BK, kt1 - kt0, wave, lane, acc);
-    }
+    dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, kt0 * BK, kt1 - kt0, wave, lane, acc);
     if (kt1 - kt0 != KT) {
       // a share of the tile: which slot is ours, and how many there are
       const int first = sk_block_of(sk, tile * KT), last = sk_block_of(sk, tile * KT + KT - 1);
@@ -1195,7 +1000,7 @@ static int linear_device(const LinearArgs &a, int *dev) {
 static bool streamk_applies(const LinearArgs &a, int bk, StreamKPlan *plan) {
   const char *off = getenv("RAI_HIP_NO_STREAMK");   // read per call: tests compare both forms in one process
   if (off && *off && *off != '0') return false;
-  if (!a.splitk_ws || ((uintptr_t)a.splitk_ws & 15) || a.post_ln_out) return false;
+  if (!a.splitk_ws || ((uintptr_t)a.splitk_ws & 15) || a.post_ln_out || (bk == 64 && !gemm_persist_serves(a))) return false;
   // one block per CU of a 256-CU part: the plan, the counter array and the XCD order are laid out for that grid
   int dev = -1;
   if (linear_device(a, &dev) != RAI_OK || device_cu_count(dev) != kNumCU) return false;
@@ -1236,9 +1041,8 @@ int streamk_counters_reset(int dev, hipStream_t st) {
   return RAI_OK;
 }
 
-template <int NS>
-static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan) {
-  constexpr int BM = 256, BN = 256, SH = 2, WGN = 4;
+static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan, int bk) {
+  constexpr int BM = 256, BN = 256, NS = 4, SH = 2, WGN = 4;
   constexpr size_t lds = dma_lds_bytes<BM, BN, NS, WGN>();
   int dev = 0;
   RAI_TRY(linear_device(a, &dev));
@@ -1260,6 +1064,7 @@ static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan)
     int lim = 0, tile = -1;
     if (sscanf(t, "%d,%d", &lim, &tile) == 2 && lim > 0) { plan.k.spin_limit = lim; plan.k.drop_tile = tile; }
   }
+  if (bk == 64) return launch_gemm_bf16_persist(st, a, plan.k);
   hipLaunchKernelGGL((k_gemm_bf16_mfma_dma_streamk<BM, BN, NS, SH, WGN>), dim3(kNumCU), dim3(128 * WGN), lds, st, a, plan.k);
   return launch_check("gemm_bf16_mfma_dma_streamk");
 }
@@ -1850,16 +1655,19 @@ static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 25
 // 128 x 128 with eight waves (4 x 2, 32 x 64 each, two to a SIMD) took the place of four waves in two and four stages: 333 x 8960 x 1536
 // 20.5 to 18.9 us, 2000 x 2048 x 2048 22.7 to 21.1.  128 x 256 and 192 x 256 (eight waves, three and two stages) serve where 256 x 256
 // leaves a last round nearly empty: 1200 x 16384 x 2048 108 to 97 us, 3000 x 4096 x 4096 105 to 88, 777 x 22528 x 2048 114 to 91.
+// Whole 256 x 256 tiles run on one block per CU that keeps its pipeline full from tile to tile (gemm_persist.hip): `end` is what each
+// then costs besides (10.1 us when every tile was a block; over 320 products with 100 such tiles and more what is picked takes 0.4 %
+// more than the best in the mean, 1.2 % by the old figure).  Their K parts are blocks of their own as before.
 enum { kTile128 = 0, kTile128x64, kTile64, kTile128x256, kTile256x192, kTile192x256, kTile256, kTileStreamK };
 struct TileCost { int bm, bn, share; float stage[3], end, cut; };
 static const TileCost kTileCosts[] = {{128, 128, 1, {0.482f}, 3.24f, 1.46f}, {128, 64, 2, {0.36f, 0.568f}, 2.02f, 0.929f}, {64, 64, 3, {0.256f, 0.382f, 0.614f}, 0.81f, 0.428f},
                                       {128, 256, 1, {0.785f}, 6.77f, 2.27f}, {256, 192, 1, {1.21f}, 7.82f, 0.293f},        {192, 256, 1, {1.16f}, 7.58f, 0.472f},
-                                      {256, 256, 1, {1.33f}, 10.1f, 0.493f}};
+                                      {256, 256, 1, {1.33f}, 8.f, 0.493f}};
 constexpr float kLaunchUs = 2.43f, kCutUs = 4.04f, kPartUsPerMB = 0.555f, kMostPartMB = 80.f, kShareUs = 20.9f;
 
 // Stream-K over 256 x 256 tiles, where its last round is exactly half full and so each of that round's tiles the work of two CUs, a half of
-// K each: no CU is left idle, for an exchange of the halves (us, stream-K, the best whole tiles: 4096 x 10240 x 2560 200, 212; 16384 x
-// 1536 x 8960 374, 419; 1200 x 32768 x 2048 168, 174).  Shares that begin anywhere in K lose more in the L2s, where blocks no longer read
+// K each: no CU is left idle, for an exchange of the halves (us, stream-K, the best whole tiles when both were blocks of a tile each: 4096 x 10240 x 2560 200,
+// 212; 16384 x 1536 x 8960 374, 419; 1200 x 32768 x 2048 168, 174; so 186, 386, 152).  Shares that begin anywhere in K lose more in the L2s, where blocks no longer read
 // the same columns together, than they win in idle CUs: of 168 such products with 40 stages and more the median took 1.14 times the best
 // whole tiles' time (7770 x 2560 x 10240 476 us for 369, 7443 x 2560 x 2560 133 for 104), three less than 0.96 of it (14476 x 1536 x 8960
 // 344 for 388).  0: does not pay or does not apply.
@@ -1998,11 +1806,13 @@ static int launch_tile_k64(hipStream_t st, const LinearArgs &a, TilePlan tile) {
     case kTile128x256: return launch_cfg_dma<128, 256, 3, 0, 4, 2>(st, a, tile.splits);
     case kTile256x192: return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, tile.splits);
     case kTile192x256: return launch_cfg_dma<192, 256, 2, 0, 4, 2>(st, a, tile.splits);
-    case kTile256: return launch_cfg_dma<256, 256, 2, 0, 4>(st, a, tile.splits);
+    case kTile256:
+      if (tile.splits == 1 && gemm_persist_serves(a)) return launch_gemm_bf16_persist(st, a, StreamKArgs{});
+      return launch_cfg_dma<256, 256, 2, 0, 4>(st, a, tile.splits);
     case kTileStreamK: {
       StreamKPlan plan;
       RAI_REQUIRE(streamk_applies(a, 64, &plan), RAI_ERR_UNSUPPORTED, "linear: stream-K does not apply to %dx%dx%d", a.M, a.N, a.K);
-      return launch_streamk<2>(st, a, plan);
+      return launch_streamk(st, a, plan, 64);
     }
     default: return launch_cfg_dma<128, 128, 4, 0, 2, 4>(st, a, tile.splits);
   }
@@ -2072,20 +1882,20 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
     if (!strcmp(knob, "256x256x8wk64")) {
       RAI_REQUIRE(splits == 1 && a.K % 64 == 0, RAI_ERR_UNSUPPORTED,
                   "linear: RAI_HIP_GEMM_TILE=256x256x8wk64 needs K %% 64 == 0 and no K split (%dx%dx%d)", a.M, a.N, a.K);
-      return launch_cfg_dma<256, 256, 2, 0, 4>(st, a, splits);
+      return launch_tile_k64(st, a, {kTile256, 1});
     }
     if (!strcmp(knob, "streamk") || !strcmp(knob, "streamk64")) {
       const int bk = knob[7] ? 64 : 32;
       StreamKPlan plan;
       RAI_REQUIRE(splits == 1 && streamk_applies(a, bk, &plan), RAI_ERR_UNSUPPORTED,
                   "linear: RAI_HIP_GEMM_TILE=%s does not apply to %dx%dx%d", knob, a.M, a.N, a.K);
-      return bk == 64 ? launch_streamk<2>(st, a, plan) : launch_streamk<4>(st, a, plan);
+      return launch_streamk(st, a, plan, bk);
     }
   }
   if (a.K % 64 == 0 && !no_k64()) return launch_tile_k64(st, a, tile);
   if (splits == 1 && has_huge_tiles(a)) {
     StreamKPlan plan;
-    return streamk_pays_k32(a, &plan) ? launch_streamk<4>(st, a, plan) : launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
+    return streamk_pays_k32(a, &plan) ? launch_streamk(st, a, plan, 32) : launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
   }
   return launch_cfg_dma<128, 128, 3, 2>(st, a, splits);
 }
