@@ -430,13 +430,23 @@ static int single_row_runs(rai_hip_decoder *d, hipStream_t st) {
       in.W2 = y.Wgu; in.N2 = 2 * y.Fp; in.gated2 = 1; in.out2 = hm.cat + (size_t)y.QD * es;
       in.act = kActClampedGlu; in.act_limit = (float)y.c.mlp_limit; in.act_alpha = (float)y.c.mlp_alpha;
     }
-    RAI_TRY(launch_latent_in(st, in));
     if (y.c.mixer == RAI_MIXER_ATTENTION) {
+      RAI_TRY(launch_latent_in(st, in));
       RAI_TRY(launch_attention_decode(st, decode_attention_args(d, y, r, 1)));
     } else {
       DeltaArgs a = delta_args(d, y, r, 1, 1);
       a.a2 = y.a2; a.g2 = y.g2; a.a_rank = y.a_rank; a.g_rank = y.g_rank;
-      RAI_TRY(launch_delta_step(st, d->cfg.dtype, a));
+      // the MLP's first half waits for the norm only: beside the step, whose blocks are few
+      LatentInArgs beside = in;
+      if (in.N2 && delta_step_beside_serves(y.delta, in.K)) {
+        in.N2 = 0;
+        beside.N1 = 0;
+        RAI_TRY(launch_latent_in(st, in));
+        RAI_TRY(launch_delta_step_beside(st, a, beside));
+      } else {
+        RAI_TRY(launch_latent_in(st, in));
+        RAI_TRY(launch_delta_step(st, d->cfg.dtype, a));
+      }
     }
     LatentDownArgs dn;
     memset(&dn, 0, sizeof(dn));

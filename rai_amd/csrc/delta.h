@@ -55,5 +55,10 @@ int launch_delta_tokens(hipStream_t st, int dtype, const DeltaArgs &a);
 // One token per sequence in one launch, where it serves the head sizes.
 bool delta_step_serves(const DeltaShape &s);
 int launch_delta_step(hipStream_t st, int dtype, const DeltaArgs &a);
+// The same for one bf16 row with both factors folded in, and beside it, on the CUs that the heads leave idle, Linears that do
+// not wait for it.
+struct LatentInArgs;
+bool delta_step_beside_serves(const DeltaShape &s, int K);
+int launch_delta_step_beside(hipStream_t st, const DeltaArgs &a, const LatentInArgs &beside);
 
 }  // namespace rai

@@ -9,6 +9,7 @@
 
 #include "delta.h"
 #include "delta_device.h"
+#include "latent_device.h"
 
 namespace rai {
 
@@ -431,9 +432,7 @@ template <typename T> struct ConvStep {
   }
 };
 
-template <typename T, int NI, bool FACTORS>
-__global__ void __launch_bounds__(kStepThreads) k_delta_step(DeltaArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float st_lds[];
+template <typename T, int NI, bool FACTORS> __device__ __forceinline__ void delta_step_head(const DeltaArgs &a, float *st_lds) {
   const DeltaShape &z = a.s;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int h = blockIdx.x, b = blockIdx.y, rep = z.heads / z.kv_heads, kv = h / rep, kd = z.kv_heads * z.Dk;
@@ -567,6 +566,20 @@ __global__ void __launch_bounds__(kStepThreads) k_delta_step(DeltaArgs a) {
   }
 }
 
+template <typename T, int NI, bool FACTORS>
+__global__ void __launch_bounds__(kStepThreads) k_delta_step(DeltaArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float st_lds[];
+  delta_step_head<T, NI, FACTORS>(a, st_lds);
+}
+// One row: a block to a head, and behind them blocks for the Linears, each with a CU to itself (by the LDS it asks for): a
+// head's block moves 192 KB, and beside others' streams on its own CU it took as long as both one after the other (16 heads of 128 x 128
+// and 16384 gated rows of 2048: 9.7 + 13.2 us one after the other, 20.2 with shared CUs, 14.6 so).
+template <int NI, int KC> __global__ void __launch_bounds__(kStepThreads) k_delta_step_beside(DeltaArgs a, LatentInArgs in) {
+  extern __shared__ __attribute__((aligned(16))) float st_lds[];
+  if ((int)blockIdx.x < a.s.heads) delta_step_head<bf16_raw, NI, true>(a, st_lds);
+  else latent_in_block<KC>(in, blockIdx.x - a.s.heads, gridDim.x - a.s.heads, reinterpret_cast<char *>(st_lds));
+}
+
 // ---------------------------------------------------------------- launchers
 static int check_delta(const DeltaArgs &a) {
   const DeltaShape &z = a.s;
@@ -649,11 +662,10 @@ bool delta_step_serves(const DeltaShape &z) {
   return z.Dk % 32 == 0 && z.Vp % 32 == 0 && z.Dk <= kDeltaMaxHead && z.Vp <= kDeltaMaxHead && step_rows(z) <= 32;
 }
 
+static size_t step_lds(const DeltaShape &z) { return (size_t)(3 * z.Dk + 3 * z.Vp + 2 * (kStepThreads / (z.Vp / 4)) * z.Vp) * sizeof(float); }   // at most 28 KB
 template <typename T, int NI> static int launch_step_n(hipStream_t st, const DeltaArgs &a) {
-  const DeltaShape &z = a.s;
-  const int RG = kStepThreads / (z.Vp / 4);
-  const size_t lds = (size_t)(3 * z.Dk + 3 * z.Vp + 2 * RG * z.Vp) * sizeof(float);   // at most 28 KB
-  const dim3 grid(z.heads, a.B), block(kStepThreads);
+  const size_t lds = step_lds(a.s);
+  const dim3 grid(a.s.heads, a.B), block(kStepThreads);
   if (a.a2) hipLaunchKernelGGL((k_delta_step<T, NI, true>), grid, block, lds, st, a);
   else hipLaunchKernelGGL((k_delta_step<T, NI, false>), grid, block, lds, st, a);
   return launch_check("delta_step");
@@ -671,6 +683,35 @@ int launch_delta_step(hipStream_t st, int dtype, const DeltaArgs &a) {
   RAI_REQUIRE(a.S == 1 && delta_step_serves(a.s) && (a.a2 == nullptr) == (a.g2 == nullptr) && (!a.a2 || (a.a_rank % 8 == 0 && a.g_rank % 8 == 0)),
               RAI_ERR_BAD_ARG, "delta step: not served");
   return dtype == RAI_BF16 ? launch_step_t<bf16_raw>(st, a) : launch_step_t<float>(st, a);
+}
+
+constexpr size_t kWholeCu = 84 * 1024;   // of LDS: more than half of what a CU has
+template <int NI, int KC> static int launch_beside_nk(hipStream_t st, const DeltaArgs &a, const LatentInArgs &in) {
+  static bool attr_set[64];
+  int dev = 0;
+  RAI_HIP_TRY(hipGetDevice(&dev));
+  RAI_REQUIRE(dev >= 0 && dev < 64, RAI_ERR_BAD_ARG, "device %d out of range", dev);
+  if (!attr_set[dev]) {
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_delta_step_beside<NI, KC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWholeCu));
+    attr_set[dev] = true;
+  }
+  const dim3 grid(a.s.heads + latent_in_blocks(in, kNumCU - a.s.heads)), block(kStepThreads);
+  hipLaunchKernelGGL((k_delta_step_beside<NI, KC>), grid, block, kWholeCu, st, a, in);
+  return launch_check("delta_step_beside");
+}
+template <int NI> static int launch_beside_n(hipStream_t st, const DeltaArgs &a, const LatentInArgs &in) {
+  if (in.K <= 512) return launch_beside_nk<NI, 1>(st, a, in);
+  if (in.K <= 1024) return launch_beside_nk<NI, 2>(st, a, in);
+  return in.K <= 2048 ? launch_beside_nk<NI, 4>(st, a, in) : launch_beside_nk<NI, 8>(st, a, in);
+}
+// (larger states take registers from the rows)
+bool delta_step_beside_serves(const DeltaShape &z, int K) { return delta_step_serves(z) && step_rows(z) <= 8 && K <= 4096 && z.heads <= kNumCU / 4; }
+int launch_delta_step_beside(hipStream_t st, const DeltaArgs &a, const LatentInArgs &in) {
+  RAI_TRY(check_delta(a));
+  RAI_REQUIRE(a.S == 1 && a.B == 1 && delta_step_beside_serves(a.s, in.K) && a.a2 && a.g2 && a.a_rank % 8 == 0 && a.g_rank % 8 == 0, RAI_ERR_BAD_ARG,
+              "delta step beside Linears: not served");
+  const int n = step_rows(a.s);
+  return n <= 2 ? launch_beside_n<2>(st, a, in) : n <= 4 ? launch_beside_n<4>(st, a, in) : launch_beside_n<8>(st, a, in);
 }
 
 }  // namespace rai

@@ -97,9 +97,9 @@ struct LatentInArgs {
   const void *bias2;
   void *out2;
   void *h2;                     // the second norm's output, for the experts; null: not kept
-  int waves1, rows_per_wave;    // filled in by the launcher
 };
-int launch_latent_in(hipStream_t st, LatentInArgs a);
+int latent_in_blocks(const LatentInArgs &a, int cus);   // of eight waves, on `cus` CUs
+int launch_latent_in(hipStream_t st, const LatentInArgs &a);
 struct LatentMidArgs {
   const void *dn;               // [query latent (Qp) | latent (Rp) | gate]
   int q_rank, Qp, kv_rank, Rp;

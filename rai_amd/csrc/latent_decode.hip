@@ -6,174 +6,22 @@
 //                  chosen experts' gated products on the scaled input
 //   k_latent_down  o and down (or the chosen experts' downs) as one contraction per stream element, residual added in f32
 // A wave streams R weight rows at a time with the activation vector in registers (as k_gemv_bf16_reg does), lane l
-// holding positions l * 8 + 512 u; every wave prepares its activation vector itself while its first weights fly.
+// holding positions l * 8 + 512 u.  k_latent_in's blocks (a CU each) prepare that vector once for their eight waves while the
+// first weights fly, k_latent_mid's waves each by themselves.
+// Bound by the weights' stream behind a start of some 3 us (launch, activations, norm).  Width 2048, us, with a block of four waves that
+// each formed the norm and waited for the weights first (loads under masks are waited for where the mask ends) / so: 6464 rows
+// 9.9, 8.0; 16384 gated 15.1, 13.2; 22848 18.2, 17.2; a head of 32768 24.0, 22.7; [o | down] of 2048 x 10240 11.1, 9.9.
 #include <cstdlib>
 
-#include "latent.h"
+#include "latent_device.h"
 #include "moe.h"
 
 namespace rai {
 
-typedef __attribute__((ext_vector_type(2))) __bf16 ld_bf16x2;
-typedef __attribute__((ext_vector_type(4))) uint32_t ld_u32x4;
-typedef __attribute__((ext_vector_type(4))) float ld_f32x4;
-
-__device__ __forceinline__ float ld_dot8(ld_u32x4 a, ld_u32x4 b, float c) {
-  // elements named one by one: see dot2_bf16 in gemm.hip
-  auto dot2 = [](uint32_t x, uint32_t y, float z) {
-    ld_bf16x2 p, q;
-    __builtin_memcpy(&p, &x, 4);
-    __builtin_memcpy(&q, &y, 4);
-    return __builtin_amdgcn_fdot2_f32_bf16(p, q, z, false);
-  };
-  c = dot2(a.x, b.x, c);
-  c = dot2(a.y, b.y, c);
-  c = dot2(a.z, b.z, c);
-  return dot2(a.w, b.w, c);
-}
-__device__ __forceinline__ float lo_f32(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float hi_f32(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-__device__ __forceinline__ float gated(int act, float g, float u) { return act_eval(act, g) * u; }
-__device__ __forceinline__ float gated(const LatentInArgs &a, float g, float u) {
-  return a.act == kActClampedGlu ? glu_clamped_bf16_out(g, u, a.act_limit, a.act_alpha) : gated(a.act, g, u);
-}
-
-// R rows of W in flight, rows n .. n + R - 1 clamped to n_last.
-template <int KC, int R> struct RowSet {
-  ld_u32x4 w[R][KC];
-  __device__ __forceinline__ void load(const uint16_t *W, int64_t ldw, int n, int n_last, int K, int lane) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const uint16_t *p = W + (int64_t)(n + r < n_last ? n + r : n_last) * ldw + lane * 8;
-#pragma unroll
-      for (int u = 0; u < KC; ++u)
-        w[r][u] = lane * 8 + u * 512 < K ? __builtin_nontemporal_load(reinterpret_cast<const ld_u32x4 *>(p + u * 512)) : ld_u32x4{0u, 0u, 0u, 0u};
-    }
-  }
-};
-
-// Rows [n0, n1) against the activation vector x, R at a time, the next set requested before the current one's sums are
-// reduced; store(n, value of row n, value of row n + 1 or 0) runs on lane 0 for the first row of each pair (R == 2).
-template <int KC, typename Store>
-__device__ __forceinline__ void stream_rows(RowSet<KC, 2> &rs, const ld_u32x4 (&x)[KC], const uint16_t *W, int64_t ldw, int n0, int n1, int K,
-                                            int lane, Store store) {
-  for (int n = n0; n < n1; n += 2) {
-    float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-    for (int u = 0; u < KC; ++u) {
-      a0 = ld_dot8(rs.w[0][u], x[u], a0);
-      a1 = ld_dot8(rs.w[1][u], x[u], a1);
-    }
-    if (n + 2 < n1) rs.load(W, ldw, n + 2, n1 - 1, K, lane);
-    a0 = wave_sum(a0);
-    a1 = wave_sum(a1);
-    if (lane == 0) store(n, a0, a1);
-  }
-}
-
 template <int KC>
-__global__ void __launch_bounds__(256) k_latent_in(LatentInArgs a) {
-  const int lane = threadIdx.x & 63;
-  int gw = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  const bool second = gw >= a.waves1;
-  if (second) gw -= a.waves1;
-  const int N = second ? a.N2 : a.N1;
-  const int n0 = gw * a.rows_per_wave, n1 = n0 + a.rows_per_wave < N ? n0 + a.rows_per_wave : N;
-  if (n0 >= N) return;
-  const uint16_t *W = (const uint16_t *)(second ? a.W2 : a.W1), *nw = (const uint16_t *)(second ? a.n2 : a.n1) + lane * 8;
-  // the small, L2-resident vectors first (loads return in order), then the first weights
-  float x[KC][8];
-  ld_u32x4 wn[KC];
-#pragma unroll
-  for (int u = 0; u < KC; ++u) {
-    const int k = lane * 8 + u * 512;
-    wn[u] = ld_u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[u][e] = 0.f;
-    if (k < a.H) {
-      if (a.kind != kStreamCopy) wn[u] = *reinterpret_cast<const ld_u32x4 *>(nw + u * 512);
-      if (a.src_f32) {
-        const ld_f32x4 v0 = *reinterpret_cast<const ld_f32x4 *>((const float *)a.src + k), v1 = *reinterpret_cast<const ld_f32x4 *>((const float *)a.src + k + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { x[u][e] = v0[e]; x[u][4 + e] = v1[e]; }
-      } else {
-        const ld_u32x4 v = *reinterpret_cast<const ld_u32x4 *>((const uint16_t *)a.src + k);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { x[u][2 * e] = lo_f32(v[e]); x[u][2 * e + 1] = hi_f32(v[e]); }
-      }
-    }
-  }
-  RowSet<KC, 2> rs;
-  rs.load(W, a.ldw, n0, n1 - 1, a.K, lane);
-  if (a.src_scale != 0.f) {
-#pragma unroll
-    for (int u = 0; u < KC; ++u)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[u][e] *= a.src_scale;
-  }
-  if (a.kind == kStreamLayerNorm) {
-    float s = 0.f;
-#pragma unroll
-    for (int u = 0; u < KC; ++u)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s += x[u][e];
-    const float mean = wave_sum(s) / (float)a.H;
-#pragma unroll
-    for (int u = 0; u < KC; ++u)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[u][e] = lane * 8 + u * 512 < a.H ? x[u][e] - mean : 0.f;
-  }
-  const int gsize = a.H / a.groups;
-  const float h_scale = a.h_scale != 0.f ? a.h_scale : 1.0f;
-  float q[KC], sc[KC];
-  int grp[KC];
-#pragma unroll
-  for (int u = 0; u < KC; ++u) {
-    q[u] = sc[u] = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) q[u] = fmaf(x[u][e], x[u][e], q[u]);
-    grp[u] = (lane * 8 + u * 512) / gsize;
-  }
-  for (int g = 0; g < a.groups; ++g) {
-    float s = 0.f;
-#pragma unroll
-    for (int u = 0; u < KC; ++u) s += grp[u] == g ? q[u] : 0.f;
-    s = h_scale / sqrtf(wave_sum(s) / (float)gsize + a.eps);
-#pragma unroll
-    for (int u = 0; u < KC; ++u) sc[u] = grp[u] == g ? s : sc[u];
-  }
-  ld_u32x4 xv[KC];
-  if (a.kind == kStreamCopy) {
-#pragma unroll
-    for (int u = 0; u < KC; ++u) {
-      sc[u] = h_scale;
-      wn[u] = ld_u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};   // ones
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < KC; ++u)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) xv[u][e] = pack_bf16x2(x[u][2 * e] * sc[u] * lo_f32(wn[u][e]), x[u][2 * e + 1] * sc[u] * hi_f32(wn[u][e]));
-  if (second && a.h2 && n0 == 0) {
-#pragma unroll
-    for (int u = 0; u < KC; ++u)
-      if (lane * 8 + u * 512 < a.K) *reinterpret_cast<ld_u32x4 *>((uint16_t *)a.h2 + lane * 8 + u * 512) = xv[u];
-  }
-  stream_rows<KC>(rs, xv, W, a.ldw, n0, n1, a.K, lane, [&](int n, float v0, float v1) {
-    if (!second) {
-      uint16_t *o = (uint16_t *)a.out1 + n;
-      o[0] = f32_to_bf16_bits(v0);
-      if (n + 1 < n1) o[1] = f32_to_bf16_bits(v1);
-    } else if (a.gated2) {
-      ((uint16_t *)a.out2)[n >> 1] = f32_to_bf16_bits(gated(a, v0, v1));
-    } else {
-      float *o = (float *)a.out2 + n;
-      if (a.add2) { v0 += a.add2[n]; if (n + 1 < n1) v1 += a.add2[n + 1]; }
-      if (a.bias2) { v0 += bf16_bits_to_f32(((const uint16_t *)a.bias2)[n]); if (n + 1 < n1) v1 += bf16_bits_to_f32(((const uint16_t *)a.bias2)[n + 1]); }
-      o[0] = v0;
-      if (n + 1 < n1) o[1] = v1;
-    }
-  });
+__global__ void __launch_bounds__(kRowThreads) k_latent_in(LatentInArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char in_lds[];
+  latent_in_block<KC>(a, blockIdx.x, gridDim.x, in_lds);
 }
 
 // The expert of rank j among the logits, and its score (the choice of k_moe_route_ranked).
@@ -301,61 +149,73 @@ struct DownChunk {
 };
 
 // A block of eight waves shares one copy of the activations; a wave owns one output row and has Q chunks in flight, each
-// replaced by the chunk Q places on as soon as it has been multiplied.
+// replaced by the chunk Q places on as soon as it has been multiplied.  Without experts (EX false) a row is one run of K0 columns and
+// needs no table.  Every lane and every place in flight asks for something, where there is nothing for the row's first piece: a load
+// under a mask is waited for where the mask ends, and loads that may not have been made cannot be counted.
 constexpr int kDownWaves = 8, kDownThreads = kDownWaves * 64;
-template <int Q>
+template <int Q, bool EX>
 __global__ void __launch_bounds__(kDownThreads) k_latent_down(LatentDownArgs a) {
   extern __shared__ __attribute__((aligned(16))) char dn_lds[];
+  typedef const __attribute__((address_space(1))) ld_u32x4 *weights;   // (a pointer out of LDS would be a flat one)
   const int tid = threadIdx.x, lane = tid & 63;
   {   // this block's row
     const int64_t m = blockIdx.y;
     a.x0 = (const uint16_t *)a.x0 + m * a.K0;
     a.x1 = (const uint16_t *)a.x1 + m * a.top * a.K1;
-    if (a.top) a.choice += m * a.top;
+    if (EX) a.choice += m * a.top;
     a.res = a.res_f32 ? (const void *)((const float *)a.res + m * a.N) : (const void *)((const uint16_t *)a.res + m * a.H);
     a.out += m * a.N;
   }
-  const int c0 = (a.K0 + 511) / 512, c1 = (a.K1 + 511) / 512, chunks = c0 + a.top * c1;
-  const int Kt = a.K0 + a.top * a.K1;
+  const int c0 = (a.K0 + 511) / 512, c1 = EX ? (a.K1 + 511) / 512 : 0, chunks = EX ? c0 + a.top * c1 : c0;
+  const int Kt = EX ? a.K0 + a.top * a.K1 : a.K0;
   DownChunk *table = reinterpret_cast<DownChunk *>(dn_lds);
-  uint16_t *xs = reinterpret_cast<uint16_t *>(table + chunks);
-  const int n = blockIdx.x * kDownWaves + (tid >> 6);
-  float res = 0.f;
-  if (n < a.H) res = a.res_f32 ? ((const float *)a.res)[n] : bf16_bits_to_f32(((const uint16_t *)a.res)[n]);
-  if (a.res_scale != 0.f) res *= a.res_scale;
-  for (int c = tid; c < chunks; c += kDownThreads) {
-    DownChunk d;
-    if (c < c0) {
-      d.w = (const uint16_t *)a.W0 + c * 512;
-      d.ld = a.K0;
-      d.meta = (c * 512) | ((a.K0 - c * 512 < 512 ? a.K0 - c * 512 : 512) << 20);
-    } else {
-      const int j = (c - c0) / c1, i = (c - c0) - j * c1;
-      d.w = (const uint16_t *)a.W1 + (int64_t)a.choice[j] * a.stride1 + i * 512;
-      d.ld = a.K1;
-      d.meta = (a.K0 + j * a.K1 + i * 512) | ((a.K1 - i * 512 < 512 ? a.K1 - i * 512 : 512) << 20);
+  uint16_t *xs = reinterpret_cast<uint16_t *>(table + (EX ? chunks : 0));
+  const int n = __builtin_amdgcn_readfirstlane(blockIdx.x * kDownWaves + (tid >> 6));
+  const int64_t row = n < a.N ? n : a.N - 1;
+  if constexpr (EX) {
+    for (int c = tid; c < chunks; c += kDownThreads) {
+      DownChunk d;
+      if (c < c0) {
+        d.w = (const uint16_t *)a.W0 + c * 512;
+        d.ld = a.K0;
+        d.meta = (c * 512) | ((a.K0 - c * 512 < 512 ? a.K0 - c * 512 : 512) << 20);
+      } else {
+        const int j = (c - c0) / c1, i = (c - c0) - j * c1;
+        d.w = (const uint16_t *)a.W1 + (int64_t)a.choice[j] * a.stride1 + i * 512;
+        d.ld = a.K1;
+        d.meta = (a.K0 + j * a.K1 + i * 512) | ((a.K1 - i * 512 < 512 ? a.K1 - i * 512 : 512) << 20);
+      }
+      table[c] = d;
     }
-    table[c] = d;
+    __syncthreads();
   }
-  __syncthreads();
+  // rows start where chunks do: each wave begins its own at another, so that together they ask all of the HBM's channels
+  const int turn = n % chunks;
+  auto place = [&](int c) { return (c + turn < chunks ? c + turn : c + turn - chunks) * 512; };
   ld_u32x4 w[Q];
   auto request = [&](ld_u32x4 &dst, int c) {
-    if (c < chunks) {
-      const DownChunk d = table[c];
-      if (lane * 8 < (d.meta >> 20) && n < a.N) dst = __builtin_nontemporal_load(reinterpret_cast<const ld_u32x4 *>(d.w + (int64_t)n * d.ld + lane * 8));
+    if constexpr (EX) {
+      const DownChunk d = table[c < chunks ? c : 0];
+      dst = __builtin_nontemporal_load((weights)(d.w + row * d.ld + (c < chunks && lane * 8 < (d.meta >> 20) ? lane * 8 : 0)));
+    } else {
+      const int at = place(c);
+      dst = __builtin_nontemporal_load((weights)((const uint16_t *)a.W0 + row * a.K0 + (c < chunks && at + lane * 8 < a.K0 ? at + lane * 8 : 0)));
     }
   };
-  // the activations come from the L2 and are asked for first; they reach LDS while the weights are on their way
+  // the residual and the activations come from the L2 and are asked for first; the latter reach LDS while the weights are on their way
+  const int64_t rat = n < a.H ? n : 0;
+  uint32_t rraw;
+  if (a.res_f32) rraw = ((const uint32_t *)a.res)[rat];
+  else rraw = ((const uint16_t *)a.res)[rat];
   constexpr int XP = 3;
   ld_u32x4 xp[XP];
-  auto x_at = [&](int k) { return *reinterpret_cast<const ld_u32x4 *>(k < a.K0 ? (const uint16_t *)a.x0 + k : (const uint16_t *)a.x1 + (k - a.K0)); };
+  auto x_at = [&](int k) { return *reinterpret_cast<const ld_u32x4 *>(!EX || k < a.K0 ? (const uint16_t *)a.x0 + k : (const uint16_t *)a.x1 + (k - a.K0)); };
 #pragma unroll
-  for (int i = 0; i < XP; ++i)
-    if ((tid + i * kDownThreads) * 8 < Kt) xp[i] = x_at((tid + i * kDownThreads) * 8);
+  for (int i = 0; i < XP; ++i) xp[i] = x_at((tid + i * kDownThreads) * 8 < Kt ? (tid + i * kDownThreads) * 8 : 0);
 #pragma unroll
   for (int u = 0; u < Q; ++u) {
-    w[u] = ld_u32x4{0u, 0u, 0u, 0u};
     request(w[u], u);
+    if (EX && u % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // (with everything at hand at once registers run out)
   }
 #pragma unroll
   for (int i = 0; i < XP; ++i)
@@ -363,18 +223,34 @@ __global__ void __launch_bounds__(kDownThreads) k_latent_down(LatentDownArgs a) 
   for (int k = (tid + XP * kDownThreads) * 8; k < Kt; k += kDownThreads * 8) *reinterpret_cast<ld_u32x4 *>(xs + k) = x_at(k);
   __syncthreads();
   float acc = 0.f;
-  for (int first = 0; first < chunks; first += Q) {
+  auto multiply = [&](const ld_u32x4 &w, int c) {   // (a chunk's last lanes may have nothing)
+    int at = place(c), cols = a.K0 - at;
+    if constexpr (EX) {
+      const int meta = table[c < chunks ? c : 0].meta;
+      at = meta & 0xfffff;
+      cols = meta >> 20;
+    }
+    const bool some = c < chunks && lane * 8 < cols;
+    const ld_u32x4 x = *reinterpret_cast<const ld_u32x4 *>(xs + (some ? at + lane * 8 : 0)), zero = {0u, 0u, 0u, 0u};
+    acc = ld_dot8(some ? w : zero, some ? x : zero, acc);
+  };
+  int first = 0;
+  for (; first + Q < chunks; first += Q) {
 #pragma unroll
     for (int u = 0; u < Q; ++u) {
-      const int c = first + u;
-      if (c < chunks) {
-        const int meta = table[c].meta;
-        if (lane * 8 < (meta >> 20)) acc = ld_dot8(w[u], *reinterpret_cast<const ld_u32x4 *>(xs + (meta & 0xfffff) + lane * 8), acc);
-        request(w[u], c + Q);
-      }
+      multiply(w[u], first + u);
+      request(w[u], first + Q + u);
+      if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
   }
+#pragma unroll
+  for (int u = 0; u < Q; ++u) {
+    multiply(w[u], first + u);
+    if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  }
   acc = wave_sum(acc);
+  float res = a.res_f32 ? __uint_as_float(rraw) : __uint_as_float(rraw << 16);
+  if (a.res_scale != 0.f) res *= a.res_scale;
   if (lane == 0 && n < a.N) a.out[n] = n < a.H ? fmaf(a.mult, acc, res) : 0.f;
 }
 
@@ -385,19 +261,19 @@ bool latent_single_row_serves(int width, int groups, int max_rank, int max_exper
   return width % 8 == 0 && width <= 4096 && groups <= 16 && (width / groups) % 8 == 0 && max_rank <= 4096 && max_experts <= kRankedExperts && down_columns * 2 + 16 * 1024 <= 150 * 1024;
 }
 
-int launch_latent_in(hipStream_t st, LatentInArgs a) {
-  const int rows = a.N1 + a.N2;
-  // about eight waves per CU at least, whole pairs of rows
-  int rpw = (rows + kNumCU * 16 - 1) / (kNumCU * 16);
-  a.rows_per_wave = rpw < 2 ? 2 : (rpw + 1) / 2 * 2;
-  a.waves1 = (a.N1 + a.rows_per_wave - 1) / a.rows_per_wave;
-  const int waves = a.waves1 + (a.N2 + a.rows_per_wave - 1) / a.rows_per_wave;
-  const dim3 grid((waves + 3) / 4), block(256);
-  if (a.K <= 512) hipLaunchKernelGGL(k_latent_in<1>, grid, block, 0, st, a);
-  else if (a.K <= 1024) hipLaunchKernelGGL(k_latent_in<2>, grid, block, 0, st, a);
-  else if (a.K <= 2048) hipLaunchKernelGGL(k_latent_in<4>, grid, block, 0, st, a);
-  else if (a.K <= 2560) hipLaunchKernelGGL(k_latent_in<5>, grid, block, 0, st, a);
-  else hipLaunchKernelGGL(k_latent_in<8>, grid, block, 0, st, a);
+int latent_in_blocks(const LatentInArgs &a, int cus) {
+  const int pairs = (a.N1 + 1) / 2 + (a.N2 + 1) / 2, blocks = (pairs + kRowWaves - 1) / kRowWaves;
+  return blocks < cus ? blocks : cus;
+}
+int launch_latent_in(hipStream_t st, const LatentInArgs &a) {
+  RAI_REQUIRE(a.groups <= kRowGroups && a.K <= 8 * kRowThreads, RAI_ERR_UNSUPPORTED, "latent in: %d groups, %d columns", a.groups, a.K);
+  const dim3 grid(latent_in_blocks(a, kNumCU)), block(kRowThreads);
+  const size_t lds = latent_in_lds(a);
+  if (a.K <= 512) hipLaunchKernelGGL(k_latent_in<1>, grid, block, lds, st, a);
+  else if (a.K <= 1024) hipLaunchKernelGGL(k_latent_in<2>, grid, block, lds, st, a);
+  else if (a.K <= 2048) hipLaunchKernelGGL(k_latent_in<4>, grid, block, lds, st, a);
+  else if (a.K <= 2560) hipLaunchKernelGGL(k_latent_in<5>, grid, block, lds, st, a);
+  else hipLaunchKernelGGL(k_latent_in<8>, grid, block, lds, st, a);
   return launch_check("latent_in");
 }
 
@@ -438,23 +314,26 @@ int launch_moe_slots(hipStream_t st, MoeSlotsArgs a) {
   return launch_check("moe_slots");
 }
 
-template <int Q> static int launch_latent_down_q(hipStream_t st, const LatentDownArgs &a, size_t lds) {
+template <int Q, bool EX> static int launch_latent_down_q(hipStream_t st, const LatentDownArgs &a, size_t lds) {
   static bool attr_set = false;
   if (!attr_set) {
-    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_latent_down<Q>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_latent_down<Q, EX>, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
     attr_set = true;
   }
-  hipLaunchKernelGGL(k_latent_down<Q>, dim3((a.N + kDownWaves - 1) / kDownWaves, a.rows), dim3(kDownThreads), lds, st, a);
+  hipLaunchKernelGGL((k_latent_down<Q, EX>), dim3((a.N + kDownWaves - 1) / kDownWaves, a.rows), dim3(kDownThreads), lds, st, a);
   return launch_check("latent_down");
+}
+template <bool EX> static int launch_latent_down_e(hipStream_t st, const LatentDownArgs &a, int chunks, size_t lds) {
+  if (chunks <= 8) return launch_latent_down_q<8, EX>(st, a, lds);
+  if (chunks <= 16) return launch_latent_down_q<16, EX>(st, a, lds);
+  if (!EX && chunks <= 20) return launch_latent_down_q<20, false>(st, a, lds);   // (24, and 20 with the table, spill)
+  return launch_latent_down_q<16, EX>(st, a, lds);
 }
 int launch_latent_down(hipStream_t st, const LatentDownArgs &a) {
   const int chunks = (a.K0 + 511) / 512 + a.top * ((a.K1 + 511) / 512);
   const size_t lds = (size_t)chunks * sizeof(DownChunk) + ((size_t)a.K0 + (size_t)a.top * a.K1) * 2;
   RAI_REQUIRE(lds <= 150 * 1024 && a.K0 % 8 == 0 && a.K1 % 8 == 0, RAI_ERR_UNSUPPORTED, "latent down: %d + %d x %d columns", a.K0, a.top, a.K1);
-  if (chunks <= 8) return launch_latent_down_q<8>(st, a, lds);
-  if (chunks <= 16) return launch_latent_down_q<16>(st, a, lds);
-  if (chunks > 16 && chunks <= 24) return launch_latent_down_q<24>(st, a, lds);
-  return launch_latent_down_q<16>(st, a, lds);
+  return a.top ? launch_latent_down_e<true>(st, a, chunks, lds) : launch_latent_down_e<false>(st, a, chunks, lds);
 }
 
 }  // namespace rai
