@@ -92,3 +92,17 @@ def test_infinite_values_reach_only_queries_that_see_them(R, s, t, n, d=64):
     same = np.isfinite(want)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~same & ~np.isnan(want)], want[~same & ~np.isnan(want)])
     assert np.all(np.abs(got - clean)[same] <= tol[same])
+
+
+@pytest.mark.parametrize("causal", [1, 0])
+@pytest.mark.parametrize("b,hq,hkv,s,t,d", [(1, 64, 8, 16, 63, 80), (1, 65, 13, 16, 63, 80), (1, 1, 1, 16, 64, 64), (2, 3, 1, 17, 95, 32), (1, 4, 2, 16, 1000, 80), (1, 32, 8, 33, 40, 64),
+                                            (1, 48, 6, 256, 256, 64), (1, 49, 7, 256, 256, 32), (8, 32, 8, 64, 64, 80), (7, 32, 8, 64, 65, 80), (16, 16, 4, 63, 160, 32)])
+def test_around_the_lines_of_the_dispatch(R, b, hq, hkv, s, t, d, causal):
+    """A block to a row or tiles; four, two or one wave to a group of 16 rows."""
+    test_against_64_bits(R, b, hq, hkv, s, t, d, causal)
+
+
+def test_few_rows_of_more_keys_than_a_block_holds_are_refused(R):
+    q, k = up(np.zeros((1, 1, 16, 32), np.float32), "f32"), up(np.zeros((1, 1, 40000, 32), np.float32), "f32")
+    with pytest.raises(RaiHipError):
+        R.attention(q, k, k, 0.1, 1, 1)
