@@ -249,6 +249,14 @@ def test_decays_from_none_to_all(hip, dt, bias, rate, dim):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("dim", [32, 64, 128])
+@pytest.mark.parametrize("bias,rate", [(3.5, 0.0), (4.0, 0.0), (2.0, 1.5), (14.8, 0.0), (15.2, 0.0)])
+def test_decays_around_the_steps_of_a_diagonal_block(hip, dt, bias, rate, dim):
+    """Sixteen tokens just within e^-60 and beyond, four tokens just within and beyond: one product, rows in fours, pairs."""
+    test_decays_from_none_to_all(hip, dt, bias, rate, dim)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("sink", [-8.0, 3.0, 40.0])
 def test_sink(hip, dt, sink):
     """Sinks far below, among and far above the capped scores, for every head and for some of them."""
