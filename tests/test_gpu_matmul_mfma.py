@@ -61,6 +61,31 @@ def test_large_tiles(R, dt, b_t):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("a_t,b_t", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("batch,m,n", [(3, 70, 61), (130, 255, 241)])
+@pytest.mark.parametrize("k", [4, 9, 32, 40, 41, 63, 64, 65, 80, 95, 96, 97, 128, 129, 160, 161, 193])
+def test_every_length_of_k_that_changes_the_form(R, dt, a_t, b_t, batch, m, n, k):
+    """K up to each size of a single stage and one beyond, in 64 x 64 and in 128 x 128 tiles; what lies around the operands is NaN."""
+    g = np.random.Generator(np.random.PCG64(k))
+    a, b = rand(g, (3, m, k), dt), rand(g, (3, k, n), dt)
+    pad = lambda x: np.pad(x, ((0, 0), (1, 1), (3, 3)), constant_values=np.nan)  # noqa: E731
+    some = np.arange(batch) % 3   # the same few products over and over: the batch's strides are checked, the oracle stays small
+    A, B = pad(np.swapaxes(a, 1, 2) if a_t else a)[some], pad(np.swapaxes(b, 1, 2) if b_t else b)[some]
+    ad = up(A, dt).narrow(1, 1, A.shape[1] - 2).narrow(2, 3, A.shape[2] - 6)
+    bd = up(B, dt).narrow(1, 1, B.shape[1] - 2).narrow(2, 3, B.shape[2] - 6)
+    got = down(R.matmul(ad.transpose(1, 2) if a_t else ad, bd.transpose(1, 2) if b_t else bd))
+    check(got[:3], a, b, dt)
+    assert all(np.array_equal(got[i], got[i % 3]) for i in range(3, batch))
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("a_t,b_t", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,k,n", [(5, 3, 70), (3, 300, 5), (70, 200, 7), (2, 2, 2), (67, 130, 66)])
+def test_operands_of_less_than_a_piece(R, dt, a_t, b_t, m, k, n):
+    test_layouts_and_tile_edges(R, dt, a_t, b_t, 2, m, k, n)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
 def test_views_broadcasts_and_general_strides(R, dt):
     g = np.random.Generator(np.random.PCG64(7))
     # heads of a [B, S, H, D] tensor, first feature dropped: strided batches, rows off any alignment
