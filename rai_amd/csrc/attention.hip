@@ -161,6 +161,42 @@ __device__ __forceinline__ float rope_feature(const T *head, int d, int rot, con
   return round_to<T>(round_to<T>(v * c) + round_to<T>(other * s));
 }
 
+// The same in two steps, so that what it reads is asked for before anything waits: no request stands under a condition (what
+// such a load returns is waited for where the condition ends).  A table's element is read as the aligned word around it.
+template <typename T> struct RopeRaw {
+  T v, other;
+  uint32_t c, s, half_c, half_s;
+};
+template <typename T> __device__ __forceinline__ void rope_request_row(RopeRaw<T> &x, const T *head, int d, int rot) {
+  const int half = rot >> 1;
+  x.v = head[d];
+  x.other = head[d < half ? d + half : d < rot ? d - half : d];
+}
+template <typename T>
+__device__ __forceinline__ void rope_request_tables(RopeRaw<T> &x, int d, int rot, const void *cos_t, const void *sin_t, const void *any, int pos, int tab_f32) {
+  const uint32_t size = tab_f32 ? 4 : sizeof(T);
+  const int64_t at = rot ? ((int64_t)pos * rot + (d < rot ? d : 0)) * size : 0;   // (rot 0: no tables)
+  const uintptr_t c = (uintptr_t)(rot ? cos_t : any) + at, s = (uintptr_t)(rot ? sin_t : any) + at;
+  typedef const __attribute__((address_space(1))) uint32_t *word;
+  x.c = *(word)(c & ~(uintptr_t)3);
+  x.s = *(word)(s & ~(uintptr_t)3);
+  x.half_c = (uint32_t)(c & 2) * 8;
+  x.half_s = (uint32_t)(s & 2) * 8;
+}
+template <typename T> __device__ __forceinline__ float table_value(uint32_t word, uint32_t shift) {
+  if constexpr (sizeof(T) == 4) return __uint_as_float(word);
+  else {
+    const T t = {(uint16_t)(word >> shift)};
+    return (float)Scalar<T>::load(&t);
+  }
+}
+template <typename T> __device__ __forceinline__ float rope_finish(const RopeRaw<T> &x, int d, int rot, int tab_f32) {
+  const float v = (float)Scalar<T>::load(&x.v), o = (float)Scalar<T>::load(&x.other), other = d < (rot >> 1) ? -o : o;
+  const float f = round_to<T>(fmaf(v, __uint_as_float(x.c), other * __uint_as_float(x.s)));
+  const float t = round_to<T>(round_to<T>(v * table_value<T>(x.c, x.half_c)) + round_to<T>(other * table_value<T>(x.s, x.half_s)));
+  return d >= rot ? v : tab_f32 ? f : t;
+}
+
 // Decode attention, split over the context ("flash decoding"): block
 // (split, kv-head group, batch) handles ceil((pos+1)/NS) consecutive keys for
 // the R query heads that share one KV head, so the cached K and V are read once
@@ -172,6 +208,10 @@ __device__ __forceinline__ float rope_feature(const T *head, int d, int rot, con
 // merges the NS partials and writes the output row.  The new token's rotated
 // key and value are appended to the cache by the block that owns position pos
 // and are used from LDS.  Probabilities stay in f32 until the product with V.
+//   What bounds it is the chain of trips: the position, everything that is read, the partials, the counter, the merge.  So nothing is
+// asked for under a condition, and the tables come before the keys, whose arrival the rotation need not wait for: one head of 128
+// a block, 777 keys over 33 splits 16.3 -> 10.8 us (masked loads: seven trips before the first score), the form below with 24 blocks of
+// 96 keys x 256 features 11.7 -> 10.4.
 constexpr int kDecodeThreads = 256;
 constexpr int kDecodeMaxSplits = 64;
 constexpr int kDecodeCounterStride = 32;
@@ -192,13 +232,13 @@ __device__ __forceinline__ float load_device(const float *p) {
 // counts itself in; the last block of the head group to arrive merges the NS
 // partials of the R query heads starting at hq0 and writes their output rows.
 // wbuf is block-shared scratch of 2 * R * NS floats that no wave uses any more.
-// The merge is a chain of dependent memory round trips, so it is kept short: one
-// for all (m, l) statistics, then the per-split weights exp(m_s - M) / L are
-// computed once per head, and every thread has 64 partial-output loads in flight.
-template <typename T>
+// The merge is a chain of dependent memory round trips, so it is kept short: one for the (m, l) statistics, the sinks, the gate and
+// the first SB splits' outputs alike (EU features a thread; up to 64 loads in flight), then the per-split weights
+// exp(m_s - M) / L are computed once per head.  EU R: the features of a block's heads for up to 256 of them a head.
+template <typename T, int EU>
 __device__ __forceinline__ void decode_merge_last(const AttnDecodeArgs &a, int b, int hq0, int R, int *sh_last,
                                                   float *wbuf) {
-  constexpr int NT = kDecodeThreads;
+  constexpr int NT = kDecodeThreads, SB = EU == 1 ? 32 : 64 / EU;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, NS = a.ns, D = a.D, PW = D + 2;
   // every thread's write-through stores have completed before the block's arrival is counted
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -209,51 +249,77 @@ __device__ __forceinline__ void decode_merge_last(const AttnDecodeArgs &a, int b
   if (!*sh_last) return;
   const float *all = a.ws + ((int64_t)b * a.Hq + hq0) * NS * PW;
   float *wm = wbuf, *wl = wbuf + R * NS;
-  for (int i = tid; i < R * NS; i += NT) {
-    const float *st = all + (int64_t)i * PW;   // (head r, split s) at index r*NS + s
+  const float *po[EU];
+  int hr[EU], hd[EU];
+  float ov[EU][SB], gate[EU];
+  auto features = [&](int e0) {   // this thread's features from e0 on
+#pragma unroll
+    for (int i = 0; i < EU; ++i) {
+      const int e = e0 + i * NT < R * D ? e0 + i * NT : R * D - 1;
+      hr[i] = e / D;
+      hd[i] = e - hr[i] * D;
+      po[i] = all + (int64_t)hr[i] * NS * PW + 2 + hd[i];
+    }
+  };
+  auto outputs = [&](int s0) {
+#pragma unroll
+    for (int i = 0; i < EU; ++i)
+#pragma unroll
+      for (int j = 0; j < SB; ++j) ov[i][j] = load_device(po[i] + (s0 + j < NS ? s0 + j : NS - 1) * PW);
+  };
+  const float first_m = load_device(all + (int64_t)min(tid, R * NS - 1) * PW), first_l = load_device(all + (int64_t)min(tid, R * NS - 1) * PW + 1);
+  const float sink0 = sink_of<T>(a.sink, hq0 + min(wave, R - 1));
+  features(tid);
+  if (a.gate) {
+#pragma unroll
+    for (int i = 0; i < EU; ++i)
+      gate[i] = (float)Scalar<T>::load((const T *)a.gate + (int64_t)b * a.gate_row_stride + (int64_t)(hq0 + hr[i]) * D + hd[i]);
+  }
+  outputs(0);
+  if (tid < R * NS) {   // (head r, split s) at index r*NS + s
+    wm[tid] = first_m;
+    wl[tid] = first_l;
+  }
+  for (int i = tid + NT; i < R * NS; i += NT) {
+    const float *st = all + (int64_t)i * PW;
     wm[i] = load_device(st);
     wl[i] = load_device(st + 1);
   }
   __syncthreads();
   for (int r = wave; r < R; r += NT / 64) {      // NS <= 64: one split per lane
     const float m = lane < NS ? wm[r * NS + lane] : -INFINITY;
-    const float sink = sink_of<T>(a.sink, hq0 + r);
+    const float sink = r == wave ? sink0 : sink_of<T>(a.sink, hq0 + r);
     const float M = fmaxf(wave_max(m), sink);    // split 0 always holds a key, so M is finite
     const float e = lane < NS ? expf(m - M) : 0.f;  // an empty split has m = -inf: weight 0
     const float L = wave_sum(lane < NS ? e * wl[r * NS + lane] : 0.f) + (a.sink ? expf(sink - M) : 0.f);
     if (lane < NS) wm[r * NS + lane] = e / L;
   }
   __syncthreads();
-  constexpr int EU = 8, SB = 8;
-  for (int e0 = tid; e0 < R * D; e0 += NT * EU) {
-    const float *po[EU];
-    int hr[EU], hd[EU];
-    float O[EU];
-#pragma unroll
-    for (int i = 0; i < EU; ++i) {
-      const int e = e0 + i * NT < R * D ? e0 + i * NT : e0;
-      hr[i] = e / D;
-      hd[i] = e - hr[i] * D;
-      po[i] = all + (int64_t)hr[i] * NS * PW + 2 + hd[i];
-      O[i] = 0.f;
-    }
-    for (int s0 = 0; s0 < NS; s0 += SB) {
-      float ov[EU][SB];
+  for (int e0 = tid; e0 - tid < R * D; e0 += NT * EU) {
+    if (e0 != tid) {   // (more than 256 features a head)
+      features(e0);
 #pragma unroll
       for (int i = 0; i < EU; ++i)
+        if (a.gate) gate[i] = (float)Scalar<T>::load((const T *)a.gate + (int64_t)b * a.gate_row_stride + (int64_t)(hq0 + hr[i]) * D + hd[i]);
+      outputs(0);
+    }
+    float O[EU];
 #pragma unroll
-        for (int j = 0; j < SB; ++j) ov[i][j] = load_device(po[i] + (s0 + j < NS ? s0 + j : NS - 1) * PW);
+    for (int i = 0; i < EU; ++i) O[i] = 0.f;
+    for (int s0 = 0;;) {
 #pragma unroll
       for (int i = 0; i < EU; ++i)
 #pragma unroll
         for (int j = 0; j < SB; ++j)
           if (s0 + j < NS) O[i] = fmaf(wm[hr[i] * NS + s0 + j], ov[i][j], O[i]);
+      s0 += SB;
+      if (s0 >= NS) break;
+      outputs(s0);
     }
 #pragma unroll
     for (int i = 0; i < EU; ++i)
       if (e0 + i * NT < R * D) {
-        if (a.gate)
-          O[i] *= gate_sigmoid((float)Scalar<T>::load((const T *)a.gate + (int64_t)b * a.gate_row_stride + (int64_t)(hq0 + hr[i]) * D + hd[i]));
+        if (a.gate) O[i] *= gate_sigmoid(gate[i]);
         Scalar<T>::store((T *)a.out + (int64_t)b * a.out_row_stride + (int64_t)(hq0 + hr[i]) * D + hd[i],
                          (typename Scalar<T>::compute)O[i]);
       }
@@ -282,6 +348,23 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_split(AttnDecode
   const int n_rep = a.Hq / a.Hkv, hk = hq0 / n_rep;
   const bool writer = hq0 % n_rep == 0;     // one block per KV head appends the new token
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int QD = a.Hq * D, KD = a.Hkv * D;
+  // the new token's rows: one packed [q | k | v] row per sequence, or three separate ones
+  const T *qrow = (const T *)a.qkv + (int64_t)b * (a.k_new ? a.q_row_stride : (int64_t)(QD + 2 * KD));
+  const T *krow = (a.k_new ? (const T *)a.k_new + (int64_t)b * a.k_row_stride : qrow + QD) + hk * D;
+  const T *vrow = (a.k_new ? (const T *)a.v_new + (int64_t)b * a.v_row_stride : qrow + QD + KD) + hk * D;
+  // asked for before the position is here: the query rows (up to 256 features a head; what is beyond, further down), the new key and value
+  RopeRaw<T> qx[R], kx;
+  int qd[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int e = min(tid + i * NT, R * D - 1), r = e / D;
+    qd[i] = e - r * D;
+    rope_request_row(qx[i], qrow + (hq0 + r) * D, qd[i], a.rot);
+  }
+  const int kd = min(tid, D - 1);
+  rope_request_row(kx, krow, kd, a.rot);
+  const T v_new = vrow[kd];
   int pos = a.pos_dev ? *a.pos_dev : a.pos_host;
   if (pos > a.Tmax - 1) pos = a.Tmax - 1;   // capacity is checked on the host; never write past the cache
   const int cnt = pos + 1;
@@ -293,42 +376,46 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_split(AttnDecode
   const bool has_new = pos >= t0 && pos < t1;
   const int t1c = has_new ? pos : t1;       // cached keys are [t0, t1c)
 
-  const int QD = a.Hq * D, KD = a.Hkv * D;
-  // the new token's rows: one packed [q | k | v] row per sequence, or three separate ones
-  const T *qrow = (const T *)a.qkv + (int64_t)b * (a.k_new ? a.q_row_stride : (int64_t)(QD + 2 * KD));
-  const T *krow = a.k_new ? (const T *)a.k_new + (int64_t)b * a.k_row_stride : qrow + QD;
-  const T *vrow = a.k_new ? (const T *)a.v_new + (int64_t)b * a.v_row_stride : qrow + QD + KD;
   T *Kc = (T *)a.kcache + ((int64_t)b * a.Hkv + hk) * a.Tmax * D;
   T *Vc = (T *)a.vcache + ((int64_t)b * a.Hkv + hk) * a.Tmax * D;
   const T *cos_t = (const T *)a.cos_t, *sin_t = (const T *)a.sin_t;
   const int g = tid >> 4, gl = tid & 15;
   const int col = tid % ncol, grp = tid / ncol;
 
-  // ---- first round of K and V loads
+  // ---- tables, then the first round of K and V: every load whole (keys past the end: the last one, never used)
+#pragma unroll
+  for (int i = 0; i < R; ++i) rope_request_tables(qx[i], qd[i], a.rot, cos_t, sin_t, qrow, pos, a.tab_f32);
+  rope_request_tables(kx, kd, a.rot, cos_t, sin_t, qrow, pos, a.tab_f32);
   APack<T, V> kreg[UK][CC], vreg[UV];
+  const int last = max(t1c - 1, 0);
+  auto ask_k = [&](int tb) __attribute__((always_inline)) {
 #pragma unroll
-  for (int u = 0; u < UK; ++u) {
-    const int t = t0 + g + 16 * u;
+    for (int u = 0; u < UK; ++u)
 #pragma unroll
-    for (int cc = 0; cc < CC; ++cc) {
-      const int c = gl + 16 * cc;
-      if (t < t1c && c < ncol) kreg[u][cc] = *reinterpret_cast<const APack<T, V> *>(Kc + (int64_t)t * D + c * V);
-    }
-  }
+      for (int cc = 0; cc < CC; ++cc)
+        kreg[u][cc] = *reinterpret_cast<const APack<T, V> *>(Kc + (int64_t)min(tb + 16 * u, last) * D + min(gl + 16 * cc, ncol - 1) * V);
+  };
+  auto ask_v = [&](int tb) __attribute__((always_inline)) {
 #pragma unroll
-  for (int u = 0; u < UV; ++u) {
-    const int t = t0 + grp + u * groups;
-    if (grp < groups && t < t1c) vreg[u] = *reinterpret_cast<const APack<T, V> *>(Vc + (int64_t)t * D + col * V);
-  }
+    for (int u = 0; u < UV; ++u) vreg[u] = *reinterpret_cast<const APack<T, V> *>(Vc + (int64_t)min(tb + u * groups, last) * D + col * V);
+  };
+  ask_k(t0 + g);
+  ask_v(t0 + grp);
   // ---- rotary embedding of the R query rows (and of the new key where it is needed)
-  for (int e = tid; e < R * D; e += NT) {
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const float x = rope_finish(qx[i], qd[i], a.rot, a.tab_f32);
+    if (tid + i * NT < R * D) qf[tid + i * NT] = x;
+  }
+  for (int e = tid + R * NT; e < R * D; e += NT) {
     const int r = e / D, d = e - r * D;
     qf[e] = rope_feature<T>(qrow + (hq0 + r) * D, d, a.rot, cos_t, sin_t, pos, a.tab_f32);
   }
   if (has_new) {
     for (int d = tid; d < D; d += NT) {
-      const float kr = rope_feature<T>(krow + hk * D, d, a.rot, cos_t, sin_t, pos, a.tab_f32);
-      const float vr = (float)Scalar<T>::load(vrow + hk * D + d);
+      const float kr = d == tid ? rope_finish(kx, kd, a.rot, a.tab_f32) : rope_feature<T>(krow, d, a.rot, cos_t, sin_t, pos, a.tab_f32);
+      const T vt = d == tid ? v_new : vrow[d];
+      const float vr = (float)Scalar<T>::load(&vt);
       knew[d] = kr;
       vnew[d] = vr;
       if (writer) {
@@ -343,27 +430,20 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_split(AttnDecode
     if (a.f32_scores) return cap_score(acc * a.scale, a.softcap);
     return round_to<T>(round_to<T>(acc) * round_to<T>(a.scale));
   };
-  // ---- scores against the cached keys: 16 lanes per key row, round 0 from the prefetched registers
-  for (int tb = t0 + g; tb < t1c; tb += 16 * UK) {
-    if (tb != t0 + g) {
+  // ---- scores against the cached keys: 16 lanes per key row, each round's keys asked for a round ahead
+  for (int base = t0; base < t1c; base += 16 * UK) {
+    const int tb = base + g;
+    float kf[UK][CC][V];
 #pragma unroll
-      for (int u = 0; u < UK; ++u) {
-        const int t = tb + 16 * u;
-#pragma unroll
-        for (int cc = 0; cc < CC; ++cc) {
-          const int c = gl + 16 * cc;
-          if (t < t1c && c < ncol) kreg[u][cc] = *reinterpret_cast<const APack<T, V> *>(Kc + (int64_t)t * D + c * V);
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UK; ++u) {
-      const int t = tb + 16 * u;
-      float kf[CC][V];
+    for (int u = 0; u < UK; ++u)
 #pragma unroll
       for (int cc = 0; cc < CC; ++cc)
 #pragma unroll
-        for (int j = 0; j < V; ++j) kf[cc][j] = (float)Scalar<T>::load(&kreg[u][cc].v[j]);
+        for (int j = 0; j < V; ++j) kf[u][cc][j] = (float)Scalar<T>::load(&kreg[u][cc].v[j]);
+    if (base + 16 * UK < t1c) ask_k(tb + 16 * UK);
+#pragma unroll
+    for (int u = 0; u < UK; ++u) {
+      const int t = tb + 16 * u;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         float acc = 0.f;
@@ -372,7 +452,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_split(AttnDecode
           const int c = gl + 16 * cc;
           if (t < t1c && c < ncol) {
 #pragma unroll
-            for (int j = 0; j < V; ++j) acc = fmaf(qf[r * D + c * V + j], kf[cc][j], acc);
+            for (int j = 0; j < V; ++j) acc = fmaf(qf[r * D + c * V + j], kf[u][cc][j], acc);
           }
         }
         acc += __shfl_xor(acc, 8, 64);
@@ -414,19 +494,14 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_split(AttnDecode
     for (int r = 0; r < R; ++r)
 #pragma unroll
       for (int j = 0; j < V; ++j) acc[r][j] = 0.f;
-    if (grp < groups) {
-      for (int tb = t0 + grp; tb < t1c; tb += UV * groups) {
-        if (tb != t0 + grp) {
-#pragma unroll
-          for (int u = 0; u < UV; ++u) {
-            const int t = tb + u * groups;
-            if (t < t1c) vreg[u] = *reinterpret_cast<const APack<T, V> *>(Vc + (int64_t)t * D + col * V);
-          }
-        }
+    {
+      for (int base = t0; base < t1c; base += UV * groups) {
+        const int tb = base + grp;
+        if (base != t0) ask_v(tb);
 #pragma unroll
         for (int u = 0; u < UV; ++u) {
           const int t = tb + u * groups;
-          if (t < t1c) {
+          if (t < t1c && grp < groups) {
             float vf[V];
 #pragma unroll
             for (int j = 0; j < V; ++j) vf[j] = (float)Scalar<T>::load(&vreg[u].v[j]);
@@ -439,10 +514,12 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_split(AttnDecode
           }
         }
       }
+      if (grp < groups) {
 #pragma unroll
-      for (int r = 0; r < R; ++r)
+        for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int j = 0; j < V; ++j) red[(grp * R + r) * D + col * V + j] = acc[r][j];
+          for (int j = 0; j < V; ++j) red[(grp * R + r) * D + col * V + j] = acc[r][j];
+      }
     }
   }
   __syncthreads();
@@ -459,7 +536,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_split(AttnDecode
     store_device(part + (int64_t)tid * NS * PW, sh_m[tid]);
     store_device(part + (int64_t)tid * NS * PW + 1, sh_l[tid]);
   }
-  decode_merge_last<T>(a, b, hq0, R, &sh_last, smem);
+  decode_merge_last<T, R>(a, b, hq0, R, &sh_last, smem);
 }
 
 // Number of context splits: enough blocks to fill the chip, bounded so that a
@@ -526,6 +603,28 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, lq = lane >> 4;
   const int NS = a.ns;
+  const int QD = a.Hq * D, KD = a.Hkv * D;
+  // the new token's rows: one packed [q | k | v] row per sequence, or three separate ones
+  const T *qrow = (const T *)a.qkv + (int64_t)b * (a.k_new ? a.q_row_stride : (int64_t)(QD + 2 * KD));
+  const T *krow = (a.k_new ? (const T *)a.k_new + (int64_t)b * a.k_row_stride : qrow + QD) + hk * D;
+  const T *vrow = (a.k_new ? (const T *)a.v_new + (int64_t)b * a.v_row_stride : qrow + QD + KD) + hk * D;
+  // ---- asked for before the position is here, every load whole: feature tid of the new token's key and value, the query rows
+  // (eight features per item; `by8`: a rotary half is whole items)
+  static_assert(D <= kDecodeThreads, "a thread per feature");
+  constexpr int QI = (16 * CPR + kDecodeThreads - 1) / kDecodeThreads;
+  const bool by8 = a.rot % 16 == 0;
+  const int rot8 = by8 ? a.rot : 0, half = rot8 >> 1, kd = tid < D ? tid : D - 1;
+  RopeRaw<T> kx;
+  rope_request_row(kx, krow, kd, a.rot);
+  const T new_v = vrow[kd];
+  ad_u32x4 qx[QI], qo[QI], qc[QI][2], qn[QI][2];
+#pragma unroll
+  for (int i = 0; i < QI; ++i) {
+    const int item = tid + i * kDecodeThreads, r = item / CPR, d = (item - r * CPR) * 8;
+    const T *row = qrow + (hq0 + min(r, R - 1)) * D;
+    qx[i] = *reinterpret_cast<const ad_u32x4 *>(row + d);
+    qo[i] = *reinterpret_cast<const ad_u32x4 *>(row + (d < half ? d + half : d < rot8 ? d - half : d));
+  }
   int pos = a.pos_dev ? *a.pos_dev : a.pos_host;
   if (pos > a.Tmax - 1) pos = a.Tmax - 1;   // capacity is checked on the host; never write past the cache
   const int cnt = pos + 1;
@@ -538,79 +637,45 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
   const int t1c = has_new ? pos : t1;       // cached keys are [t0, t1c)
   const int new_row = pos - t0;
 
-  const int QD = a.Hq * D, KD = a.Hkv * D;
-  // the new token's rows: one packed [q | k | v] row per sequence, or three separate ones
-  const T *qrow = (const T *)a.qkv + (int64_t)b * (a.k_new ? a.q_row_stride : (int64_t)(QD + 2 * KD));
-  const T *krow = a.k_new ? (const T *)a.k_new + (int64_t)b * a.k_row_stride : qrow + QD;
-  const T *vrow = a.k_new ? (const T *)a.v_new + (int64_t)b * a.v_row_stride : qrow + QD + KD;
   T *Kc = (T *)a.kcache + ((int64_t)b * a.Hkv + hk) * a.Tmax * D;
   T *Vc = (T *)a.vcache + ((int64_t)b * a.Hkv + hk) * a.Tmax * D;
   const T *cos_t = (const T *)a.cos_t, *sin_t = (const T *)a.sin_t;
 
-  // ---- all K and V loads of the block
+  // ---- the tables (eight values are 16 or 32 bytes), then all K and V loads of the block (past the end: the last key once more)
+#pragma unroll
+  for (int i = 0; i < QI; ++i) {
+    const int item = tid + i * kDecodeThreads, d = item % CPR * 8, size = a.tab_f32 ? 4 : 2;
+    const int64_t at = ((int64_t)pos * rot8 + (d < rot8 ? d : 0)) * size;
+    const char *c = by8 && rot8 ? (const char *)a.cos_t + at : (const char *)qrow, *sn = by8 && rot8 ? (const char *)a.sin_t + at : (const char *)qrow;
+    const int second = a.tab_f32 && by8 && rot8 ? 16 : 0;
+    __builtin_memcpy(&qc[i][0], c, 16);
+    __builtin_memcpy(&qc[i][1], c + second, 16);
+    __builtin_memcpy(&qn[i][0], sn, 16);
+    __builtin_memcpy(&qn[i][1], sn + second, 16);
+  }
+  rope_request_tables(kx, kd, a.rot, cos_t, sin_t, qrow, pos, a.tab_f32);
+  const int last = max(t1c - 1, 0);
   ad_bf16x8 kreg[KT][KS];
 #pragma unroll
-  for (int i = 0; i < KT; ++i) {
-    const int t = t0 + (wave + 4 * i) * 16 + lrow;
-    const bool tile_ok = (wave + 4 * i) * 16 < CH;
+  for (int i = 0; i < KT; ++i)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      ad_bf16x8 z = {};
-      if (tile_ok && t < t1c) z = *reinterpret_cast<const ad_bf16x8 *>(Kc + (int64_t)t * D + ks * 32 + lq * 8);
-      kreg[i][ks] = z;
-    }
-  }
+    for (int ks = 0; ks < KS; ++ks)
+      kreg[i][ks] = *reinterpret_cast<const ad_bf16x8 *>(Kc + (int64_t)min(t0 + (wave + 4 * i) * 16 + lrow, last) * D + ks * 32 + lq * 8);
   ad_u32x4 vreg[VL];
 #pragma unroll
   for (int j = 0; j < VL; ++j) {
     const int c = tid + j * kDecodeThreads, r = c / CPR, c8 = c - r * CPR;
-    ad_u32x4 z = {0u, 0u, 0u, 0u};
-    if (t0 + r < t1c) z = *reinterpret_cast<const ad_u32x4 *>(Vc + (int64_t)(t0 + r) * D + c8 * 8);
-    vreg[j] = z;
+    vreg[j] = *reinterpret_cast<const ad_u32x4 *>(Vc + (int64_t)min(t0 + r, last) * D + c8 * 8);
   }
-  // ---- feature tid of the new token's key and value, asked for with the rest
-  static_assert(D <= kDecodeThreads, "a thread per feature");
-  T new_x{}, new_o{}, new_v{};
-  float new_c = 0.f, new_s = 0.f;
-  if (has_new && tid < D) {
-    new_x = krow[hk * D + tid];
-    new_v = vrow[hk * D + tid];
-    if (tid < a.rot) {
-      const int half = a.rot >> 1;
-      const int64_t e = (int64_t)pos * a.rot + tid;
-      new_o = krow[hk * D + (tid < half ? tid + half : tid - half)];
-      new_c = a.tab_f32 ? ((const float *)cos_t)[e] : (float)Scalar<T>::load(cos_t + e);
-      new_s = a.tab_f32 ? ((const float *)sin_t)[e] : (float)Scalar<T>::load(sin_t + e);
-    }
-  }
-  // ---- rotated queries (rows >= R are zero).  Eight features per item, all loads of a thread in
-  //      flight together: one memory round trip instead of one per feature.
-  if (a.rot % 16 == 0) {
-    constexpr int QI = (16 * CPR + kDecodeThreads - 1) / kDecodeThreads;
-    const int half = a.rot >> 1;
-    ad_u32x4 qx[QI], qo[QI], qc[QI], qn[QI];
-#pragma unroll
-    for (int i = 0; i < QI; ++i) {
-      const int item = tid + i * kDecodeThreads, r = item / CPR, d = (item - r * CPR) * 8;
-      qx[i] = qo[i] = qc[i] = qn[i] = ad_u32x4{0u, 0u, 0u, 0u};
-      if (item < 16 * CPR && r < R) {
-        const T *head = qrow + (hq0 + r) * D;
-        qx[i] = *reinterpret_cast<const ad_u32x4 *>(head + d);
-        if (d < a.rot) qo[i] = *reinterpret_cast<const ad_u32x4 *>(head + (d < half ? d + half : d - half));
-        if (d < a.rot && !a.tab_f32) {
-          qc[i] = *reinterpret_cast<const ad_u32x4 *>(cos_t + (int64_t)pos * a.rot + d);
-          qn[i] = *reinterpret_cast<const ad_u32x4 *>(sin_t + (int64_t)pos * a.rot + d);
-        }
-      }
-    }
+  // ---- rotated queries (rows >= R are zero)
+  if (by8) {
 #pragma unroll
     for (int i = 0; i < QI; ++i) {
       const int item = tid + i * kDecodeThreads, r = item / CPR, d = (item - r * CPR) * 8;
       if (item >= 16 * CPR) continue;
-      ad_u32x4 out = qx[i];
+      ad_u32x4 out = r < R ? qx[i] : ad_u32x4{0u, 0u, 0u, 0u};
       if (r < R && d < a.rot && a.tab_f32) {   // f32 tables: products and sum in f32, one rounding
         const float sign = d < half ? -1.f : 1.f;
-        const float *cp = (const float *)cos_t + (int64_t)pos * a.rot + d, *sp = (const float *)sin_t + (int64_t)pos * a.rot + d;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           float res[2];
@@ -618,7 +683,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
           for (int hbit = 0; hbit < 2; ++hbit) {
             const int sh = 16 * hbit;
             const float x = bf16_bits_to_f32((uint16_t)(qx[i][w] >> sh)), o = sign * bf16_bits_to_f32((uint16_t)(qo[i][w] >> sh));
-            res[hbit] = fmaf(x, cp[2 * w + hbit], o * sp[2 * w + hbit]);
+            res[hbit] = fmaf(x, __uint_as_float(qc[i][w >> 1][(2 * w + hbit) & 3]), o * __uint_as_float(qn[i][w >> 1][(2 * w + hbit) & 3]));
           }
           out[w] = pack_bf16x2(res[0], res[1]);
         }
@@ -631,7 +696,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
           for (int hbit = 0; hbit < 2; ++hbit) {
             const int sh = 16 * hbit;
             const float x = bf16_bits_to_f32((uint16_t)(qx[i][w] >> sh)), o = sign * bf16_bits_to_f32((uint16_t)(qo[i][w] >> sh));
-            const float c = bf16_bits_to_f32((uint16_t)(qc[i][w] >> sh)), sn = bf16_bits_to_f32((uint16_t)(qn[i][w] >> sh));
+            const float c = bf16_bits_to_f32((uint16_t)(qc[i][0][w] >> sh)), sn = bf16_bits_to_f32((uint16_t)(qn[i][0][w] >> sh));
             // three roundings, as rope_feature
             const float res = round_to<T>(round_to<T>(x * c) + round_to<T>(o * sn));
             packed |= (uint32_t)f32_to_bf16_bits(res) << sh;
@@ -649,13 +714,8 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
     }
   }
   for (int e = tid; e < 16 * PP; e += kDecodeThreads) ps[e] = 0;
-  if (has_new && tid < D) {   // as rope_feature does it
-    float key = bf16_bits_to_f32(new_x.bits);
-    if (tid < a.rot) {
-      const float other = tid < (a.rot >> 1) ? -bf16_bits_to_f32(new_o.bits) : bf16_bits_to_f32(new_o.bits);
-      key = a.tab_f32 ? round_to<T>(fmaf(key, new_c, other * new_s)) : round_to<T>(round_to<T>(key * new_c) + round_to<T>(other * new_s));
-    }
-    const uint16_t kr = f32_to_bf16_bits(key);
+  if (has_new && tid < D) {
+    const uint16_t kr = f32_to_bf16_bits(rope_finish(kx, kd, a.rot, a.tab_f32));
     knew[tid] = kr;
     vnew[tid] = new_v.bits;
     (Kc + (int64_t)pos * D + tid)->bits = kr;
@@ -693,7 +753,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
 #pragma unroll
   for (int j = 0; j < VL; ++j) {
     const int c = tid + j * kDecodeThreads, r = c / CPR, c8 = c - r * CPR;
-    ad_u32x4 v = vreg[j];
+    ad_u32x4 v = t0 + r < t1c ? vreg[j] : ad_u32x4{0u, 0u, 0u, 0u};
     if (has_new && r == new_row) v = *reinterpret_cast<const ad_u32x4 *>(vnew + c8 * 8);
     *reinterpret_cast<ad_u32x4 *>(Vs + r * VP + c8 * 8) = v;
   }
@@ -794,8 +854,8 @@ __global__ void __launch_bounds__(256) k_attn_decode_merge_bf16(AttnDecodeArgs a
 }
 
 // Splits of the context over blocks of `ch` keys.  A block that holds the longest context the cache has room for (the context itself is the
-// device's to know) writes the result itself, without the launch that merges: 24 sequences on 51 to 83 keys (8 heads of 256 on one) 11.7 us
-// for 8.9 + 4.7 in two blocks a sequence.  One to 32 sequences of 52 to 122 keys decoded so, against two blocks each: 128 features 0.2 to
+// device's to know) writes the result itself, without the launch that merges: 24 sequences on 51 to 83 keys (8 heads of 256 on one) 10.4 us
+// for 7.2 + 4.7 in two blocks a sequence.  One to 32 sequences of 52 to 122 keys decoded so, against two blocks each: 128 features 0.2 to
 // 3 % sooner, 256 features 0.3 to 2 % up to 96 keys and within 1 % either way beyond.
 static int mfma_decode_splits(const AttnDecodeArgs &a, int ch) {
   if (a.Tmax <= ch && !getenv("RAI_HIP_ATTN_SPLITS")) return 1;
