@@ -9,6 +9,7 @@
 // (scores, scale and softmax rounded to the model dtype), repeat_kv
 // gemma.rs:191-201 (query head h reads kv head h / (Hq/Hkv)).
 #include <cstdlib>
+#include <type_traits>
 
 #include "attention.h"
 
@@ -64,28 +65,57 @@ __global__ void __launch_bounds__(256) k_attn_row(AttnArgs a) {
   for (int d = tid; d < D; d += 256) qf[d] = (float)Scalar<T>::load(q + d);
   __syncthreads();
 
+  // A pass over the keys is a chain of trips to memory, so U rows of each group are on their way together, every load whole (past the
+  // last key, that one again): a load under a mask is waited for where the mask ends.  Measured (us, one row of a group at a time before):
+  // 2 x 32 heads x 4 x 256 on 689 keys in bf16 74 -> 31, 8 x 15 x 128 on 1500 84 -> 34, 8 x 32 x 12 x 64 on 64 14.6 -> 12.9, f32 32 x 2 x 128 on 900
+  // 78 -> 26; eight rows: 31.5, 34, 16.8, 25.
+  // kAll: every group has U keys; kSome: some have; kFew: none has, and what no group needs is not asked for.
+  constexpr int U = 4;
+  enum { kAll, kSome, kFew };
   // ---- scores: 16 lanes cooperate on one key row
   {
     const int g = tid >> 4, gl = tid & 15;
-    for (int t = t_begin + g; t < t_end; t += 16) {
-      const T *kr = K + (int64_t)t * a.ks[2];
-      float acc = 0.f;
-      for (int c = gl; c < ncol; c += 16) {
-        APack<T, V> pk = *reinterpret_cast<const APack<T, V> *>(kr + c * V);
+    auto round = [&](int base, auto keys) __attribute__((always_inline)) {
+      float acc[U];
 #pragma unroll
-        for (int j = 0; j < V; ++j) acc = fmaf(qf[c * V + j], (float)Scalar<T>::load(&pk.v[j]), acc);
+      for (int u = 0; u < U; ++u) acc[u] = 0.f;
+      for (int c0 = 0; c0 < ncol; c0 += 16) {
+        const int c = min(c0 + gl, ncol - 1);
+        APack<T, V> pk[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (keys() != kFew || base + 16 * u < t_end)
+            pk[u] = *reinterpret_cast<const APack<T, V> *>(K + (int64_t)(keys() == kAll ? base + g + 16 * u : min(base + g + 16 * u, t_end - 1)) * a.ks[2] + c * V);
+        const bool mine = c0 + gl < ncol;
+        float qv[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) qv[j] = qf[c * V + j];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float sum = acc[u];
+#pragma unroll
+          for (int j = 0; j < V; ++j) sum = fmaf(qv[j], (float)Scalar<T>::load(&pk[u].v[j]), sum);
+          acc[u] = mine ? sum : acc[u];
+        }
       }
-      acc += __shfl_xor(acc, 8, 64);
-      acc += __shfl_xor(acc, 4, 64);
-      acc += __shfl_xor(acc, 2, 64);
-      acc += __shfl_xor(acc, 1, 64);
-      if (gl == 0) {
+      float sum = 0.f;   // lane gl finishes the group's key gl
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float all = row_sum(acc[u]);
+        sum = gl == u ? all : sum;
+      }
+      const int t = base + g + 16 * gl;
+      if (gl < U && (keys() == kAll || t < t_end)) {
         float sc;
-        if (a.f32_scores) sc = cap_score(acc * a.scale, a.softcap);
-        else sc = round_to<T>(round_to<T>(acc) * round_to<T>(a.scale));
+        if (a.f32_scores) sc = cap_score(sum * a.scale, a.softcap);
+        else sc = round_to<T>(round_to<T>(sum) * round_to<T>(a.scale));
         scores[t - t_begin] = sc;
       }
-    }
+    };
+    int base = t_begin;
+    for (; base + 16 * U <= t_end; base += 16 * U) round(base, std::integral_constant<int, kAll>());
+    if (base + 16 * (U - 1) < t_end) round(base, std::integral_constant<int, kSome>());
+    else if (base < t_end) round(base, std::integral_constant<int, kFew>());
   }
   __syncthreads();
 
@@ -120,14 +150,31 @@ __global__ void __launch_bounds__(256) k_attn_row(AttnArgs a) {
     float acc[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[j] = 0.f;
-    if (grp < groups) {
-      for (int t = grp; t < n_seen; t += groups) {
-        // the reference rounds the normalised probabilities to V's dtype
-        const float p = a.f32_scores ? round_to<T>(scores[t] * inv) : round_to<T>(scores[t] / sum);
-        APack<T, V> pk = *reinterpret_cast<const APack<T, V> *>(Vp + (int64_t)(t_begin + t) * a.vs[2] + col * V);
+    auto round = [&](int base, auto keys) __attribute__((always_inline)) {
+      APack<T, V> pk[U];
 #pragma unroll
-        for (int j = 0; j < V; ++j) acc[j] = fmaf(p, (float)Scalar<T>::load(&pk.v[j]), acc[j]);
+      for (int u = 0; u < U; ++u)
+        if (keys() != kFew || base + groups * u < n_seen)
+          pk[u] = *reinterpret_cast<const APack<T, V> *>(Vp + (int64_t)(t_begin + min(base + grp + groups * u, n_seen - 1)) * a.vs[2] + col * V);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (keys() == kFew && base + groups * u >= n_seen) break;
+        const int t = base + grp + groups * u;
+        const float e = scores[min(t, n_seen - 1)];
+        // the reference rounds the normalised probabilities to V's dtype
+        const float p = a.f32_scores ? round_to<T>(e * inv) : round_to<T>(e / sum);
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          const float with = fmaf(p, (float)Scalar<T>::load(&pk[u].v[j]), acc[j]);
+          acc[j] = keys() == kAll || t < n_seen ? with : acc[j];
+        }
       }
+    };
+    int base = 0;
+    for (; base + groups * U <= n_seen; base += groups * U) round(base, std::integral_constant<int, kAll>());
+    if (base + groups * (U - 1) < n_seen) round(base, std::integral_constant<int, kSome>());
+    else if (base < n_seen) round(base, std::integral_constant<int, kFew>());
+    if (grp < groups) {
 #pragma unroll
       for (int j = 0; j < V; ++j) red[grp * D + col * V + j] = acc[j];
     }
@@ -455,10 +502,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_split(AttnDecode
             for (int j = 0; j < V; ++j) acc = fmaf(qf[r * D + c * V + j], kf[u][cc][j], acc);
           }
         }
-        acc += __shfl_xor(acc, 8, 64);
-        acc += __shfl_xor(acc, 4, 64);
-        acc += __shfl_xor(acc, 2, 64);
-        acc += __shfl_xor(acc, 1, 64);
+        acc = row_sum(acc);
         if (gl == 0 && t < t1c) scores[r * CH + (t - t0)] = finish_score(acc);
       }
     }

@@ -211,16 +211,8 @@ template <> struct Scalar<int64_t> {
   }
 
 // ---------------------------------------------------------------- wave helpers (wave64)
-// op(v of lane l, v of lane l ^ 32), then ^ 16, 8, 4, 2, 1, in every lane, by swaps of half and quarter waves and by DPP: some
-// twenty vector instructions, where each of the six __shfl_xor is a trip through the LDS pipeline (bits as with those).
-template <typename Op> __device__ __forceinline__ float wave_fold(float v, Op op) {
-  typedef __attribute__((ext_vector_type(2))) unsigned pair;
-  auto swap32 = [](float x) { return __builtin_bit_cast(pair, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false)); };
-  auto swap16 = [](float x) { return __builtin_bit_cast(pair, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)); };
-  pair p = swap32(v);
-  v = op(__uint_as_float(p.x), __uint_as_float(p.y));
-  p = swap16(v);
-  v = op(__uint_as_float(p.x), __uint_as_float(p.y));
+// op(v of lane l, v of lane l ^ 8), then ^ 4, 2, 1, in every lane, by DPP: over the 16 lanes of a row.
+template <typename Op> __device__ __forceinline__ float row_fold(float v, Op op) {
   const auto dpp = [](int old, float x, auto ctrl, auto banks) { return __builtin_amdgcn_update_dpp(old, __float_as_int(x), decltype(ctrl)::value, 0xf, decltype(banks)::value, false); };
   using std::integral_constant;
   typedef integral_constant<int, 0xf> all;
@@ -230,6 +222,18 @@ template <typename Op> __device__ __forceinline__ float wave_fold(float v, Op op
   v = op(v, __int_as_float(four));
   v = op(v, __int_as_float(dpp(0, v, integral_constant<int, 0x4e>{}, all{})));   // quad_perm [2, 3, 0, 1]
   return op(v, __int_as_float(dpp(0, v, integral_constant<int, 0xb1>{}, all{})));   // quad_perm [1, 0, 3, 2]
+}
+__device__ __forceinline__ float row_sum(float v) { return row_fold(v, [](float a, float b) { return a + b; }); }
+// ^ 32 and ^ 16 before that: swaps of half and quarter waves.  Some twenty vector instructions in all, where each of the six __shfl_xor
+// is a trip through the LDS pipeline (bits as with those).
+template <typename Op> __device__ __forceinline__ float wave_fold(float v, Op op) {
+  typedef __attribute__((ext_vector_type(2))) unsigned pair;
+  auto swap32 = [](float x) { return __builtin_bit_cast(pair, __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false)); };
+  auto swap16 = [](float x) { return __builtin_bit_cast(pair, __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)); };
+  pair p = swap32(v);
+  v = op(__uint_as_float(p.x), __uint_as_float(p.y));
+  p = swap16(v);
+  return row_fold(op(__uint_as_float(p.x), __uint_as_float(p.y)), op);
 }
 __device__ __forceinline__ float wave_sum(float v) { return wave_fold(v, [](float a, float b) { return a + b; }); }
 __device__ __forceinline__ double wave_sum(double v) {
