@@ -367,9 +367,12 @@ __device__ __forceinline__ void dma_tile_mainloop(const LinearArgs &a, uint16_t 
 //     rows span the 64 banks) land on 16 different 16-byte slots.  (Swizzling by r & 7 left rows r and r + 8 on the
 //     same banks: SQ_LDS_BANK_CONFLICT at 23 % of the kernel's cycles.)
 //   - fragment sets alternate F0 / F1 over the four K steps of a stage; the reads run one set ahead of the multiplies.
+//   - `half`: stage 0 begins 32 before the operands' rows do, and reads zeros there (K of an odd number of 32s).  The first stage and
+//     not the last: it is asked for outside the loop, which then is the same.
+static __device__ uint4 g_k_zeros[1];   // (sixteen bytes that nobody writes)
 template <int BM, int BN, int WGN, int WGM = 2, int NS = 2>
 __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint16_t *lds, int m0, int n0, int k_begin, int KT,
-                                                      int wave, int lane, f32x16 (&acc)[BM / (32 * WGM)][BN / (32 * WGN)]) {
+                                                      int wave, int lane, f32x16 (&acc)[BM / (32 * WGM)][BN / (32 * WGN)], bool half = false) {
   constexpr int BK = 64;
   constexpr int WM = BM / WGM, WN = BN / WGN;
   constexpr int MT = WM / 32, NT = WN / 32;
@@ -414,8 +417,16 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
+  {
+    uint16_t *sa = lds + wave * LA * 8 * BK, *sb = lds + BM * BK + wave * LB * 8 * BK;
+    auto source = [&](const uint16_t *p, int r) { return half && ((lane & 7) ^ ((r >> 1) & 7)) < 4 ? (const uint16_t *)g_k_zeros : p; };
 #pragma unroll
-  for (int st = 0; st < NS; ++st) issue(st < KT ? st : KT - 1, st);
+    for (int j = 0; j < LA; ++j) __builtin_amdgcn_global_load_lds((const void *)source(gpa[j], (wave * LA + j) * 8 + lrow), (lds_ptr)(sa + j * 8 * BK), 16, 0, 0);
+#pragma unroll
+    for (int j = 0; j < LB; ++j) __builtin_amdgcn_global_load_lds((const void *)source(gpb[j], (wave * LB + j) * 8 + lrow), (lds_ptr)(sb + j * 8 * BK), 16, 0, 0);
+  }
+#pragma unroll
+  for (int st = 1; st < NS; ++st) issue(st < KT ? st : KT - 1, st);   // (half: two stages or more)
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * (LA + LB)) : "memory");   // stage 0 has landed (this wave's part)
   __builtin_amdgcn_s_barrier();
 
@@ -519,12 +530,14 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArg
     k_begin += (split < longer ? split : longer) * 64;
     k_span += split < longer ? 64 : 0;
   }
-  const int k_end = k_begin + k_span < a.K ? k_begin + k_span : a.K;
+  // (stages of 64: K in whole stages, of which the first may begin 32 before it)
+  const int early = SH == 0 ? a.K & 32 : 0;
+  const int k_end = k_begin + k_span < a.K + early ? k_begin + k_span : a.K + early;
   const int KT = (k_end - k_begin) / BK;
 
   f32x16 acc[BM / (32 * WGM)][BN / (32 * WGN)];
-  if constexpr (SH == 0) {   // stages of 64 (the launcher sends K % 64 == 0 and splits of whole stages here)
-    dma_tile_mainloop_k64<BM, BN, WGN, WGM, NS>(a, lds, m0, n0, k_begin, KT / 2, wave, lane, acc);
+  if constexpr (SH == 0) {   // stages of 64 (the launcher sends splits of whole stages here)
+    dma_tile_mainloop_k64<BM, BN, WGN, WGM, NS>(a, lds, m0, n0, k_begin - early, KT / 2, wave, lane, acc, early && split == 0);
   } else {
     static_assert(WGM == 2, "the K-32 loop is written for two waves along M");
     dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, k_begin, KT, wave, lane, acc);
@@ -925,12 +938,13 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
   }
   const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
   const int grid_x = ((tiles + kXcds - 1) / kXcds) * kXcds;
-  int k_per_split = a.K, longer = 0;
-  if (SH == 0 && splits > a.K / 64) splits = a.K / 64;
+  const int stages = (a.K + 32) / 64;
+  int k_per_split = SH == 0 ? stages * 64 : a.K, longer = 0;
+  if (SH == 0 && splits > stages) splits = stages;
   if (splits > 1) {
     if constexpr (SH == 0) {   // stages of 64, dealt out evenly
-      k_per_split = a.K / 64 / splits * 64;
-      longer = a.K / 64 % splits;
+      k_per_split = stages / splits * 64;
+      longer = stages % splits;
     } else {
       const int k_tiles = a.K / 32, per = (k_tiles + splits - 1) / splits;
       splits = (k_tiles + per - 1) / per;
@@ -1689,7 +1703,7 @@ static bool streamk_pays_k32(const LinearArgs &a, StreamKPlan *plan) {
 
 struct TilePlan { int tile, splits; };
 static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int last = kTileStreamK) {
-  const int stages = a.K / 64;
+  const int stages = (a.K + 32) / 64;
   const float part_mb = (float)a.M * a.N * 4e-6f;
   TilePlan best = {first, 1};
   float least = 0.f;
@@ -1706,7 +1720,7 @@ static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int las
       if ((t == first && s == 1) || cost < least) { least = cost; best = {t, s}; }
     }
   }
-  if (last == kTileStreamK)
+  if (last == kTileStreamK && a.K % 64 == 0)
     if (const float us = streamk_us(a); us > 0.f && us < least) best = {kTileStreamK, 1};
   return best;
 }
@@ -1756,13 +1770,28 @@ static int named_tile(const char *knob) {   // -1: none of them
     if (!strcmp(knob, t.name)) return t.tile;
   return -1;
 }
+// Stages of 64 also where K is an odd number of 32s: half of the first stage is zeros.  Over 280 such products they took 0.75 times the
+// time of stages of 32 in the mean (us, stages of 32, of 64: 646 x 608 x 2456 20.9, 8.0; 1024 x 2080 x 2048 35.9, 17.7; 277 x 1376 x 600 11.8,
+// 8.9; 16384 x 1504 x 8960 479, 434; 5105 x 672 x 9608 105, 101).  Stages of 32 stay where a short K meets one to two rounds of 128 x 128 tiles,
+// which then share CUs (3574 x 160 x 1728 9.7, 11.5; 2405 x 608 x 1744 14.6, 15.9; with 10 stages and more even), and where stream-K saves
+// much of a long one (6061 x 9504 x 13584 1501, 1551; but 4096 x 2592 x 10240, with `saved` at 40, 212, 208).
+static bool stages_of_64(const LinearArgs &a) {
+  if (a.K < 64 || no_k64()) return false;
+  if (a.K % 64 == 0) return true;
+  const int64_t tiles = (int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128);
+  if (a.K <= 12 * 64 && tiles > 224 && tiles <= 2 * kNumCU) return false;
+  StreamKPlan plan;
+  const int left = (int)((int64_t)((a.M + 255) / 256) * ((a.N + 255) / 256) % kNumCU);
+  const float saved = (float)(kNumCU - left) / kNumCU * (a.K / 32);
+  return !(saved >= 100.f && has_huge_tiles(a) && streamk_applies(a, 32, &plan));
+}
 static TilePlan tile_plan(const LinearArgs &a) {
   if (const char *knob = forced_tile()) {
     const int t = named_tile(knob);
     if (t >= 0) return a.K % 64 || a.force_splits > 0 ? TilePlan{t, tile_splits(a)} : tile_plan_k64(a, t, t);
     return {kTile128, tile_splits(a)};
   }
-  if (a.K % 64 || no_k64() || a.force_splits > 1) return {kTile128, tile_splits(a)};
+  if (!stages_of_64(a) || a.force_splits > 1) return {kTile128, tile_splits(a)};
   return tile_plan_k64(a);
 }
 
@@ -1807,7 +1836,7 @@ static int launch_tile_k64(hipStream_t st, const LinearArgs &a, TilePlan tile) {
     case kTile256x192: return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, tile.splits);
     case kTile192x256: return launch_cfg_dma<192, 256, 2, 0, 4, 2>(st, a, tile.splits);
     case kTile256:
-      if (tile.splits == 1 && gemm_persist_serves(a)) return launch_gemm_bf16_persist(st, a, StreamKArgs{});
+      if (tile.splits == 1 && a.K % 64 == 0 && gemm_persist_serves(a)) return launch_gemm_bf16_persist(st, a, StreamKArgs{});
       return launch_cfg_dma<256, 256, 2, 0, 4>(st, a, tile.splits);
     case kTileStreamK: {
       StreamKPlan plan;
@@ -1862,8 +1891,8 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
   }
   const TilePlan tile = tile_plan(a);
   const int splits = tile.splits;
-  // Tile choice.  The LDS-DMA kernels stream K tiles straight into LDS, with stages of 64 where K allows (whole 128-byte lines per request;
-  // RAI_HIP_NO_K64: never): what tile_plan_k64 says.  Other K: 256 x 256 in its eight-wave form (one block per CU, 4 LDS stages of 32, two
+  // Tile choice.  The LDS-DMA kernels stream K tiles straight into LDS, with stages of 64 where that pays (whole 128-byte lines per request;
+  // RAI_HIP_NO_K64: never; stages_of_64): what tile_plan_k64 says.  Else 256 x 256 in its eight-wave form (one block per CU, 4 LDS stages of 32, two
   // waves per SIMD) or stream-K over it once its tiles cover a good half of the CUs, 128 x 128 with three stages below that.
   // RAI_HIP_GEMM_TILE = "64x64" | "128x64" | "128x128" | "128x128k64" | "128x128deep" (the same) | "128x256" | "192x256" | "256x128" |
   // "256x192" | "256x256" | "256x256k64" | "256x256x8w" | "256x256x8wk64" (256x256k64, K never cut) | "streamk" | "streamk64" | "classic"
@@ -1892,7 +1921,7 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
       return launch_streamk(st, a, plan, bk);
     }
   }
-  if (a.K % 64 == 0 && !no_k64()) return launch_tile_k64(st, a, tile);
+  if (stages_of_64(a)) return launch_tile_k64(st, a, tile);
   if (splits == 1 && has_huge_tiles(a)) {
     StreamKPlan plan;
     return streamk_pays_k32(a, &plan) ? launch_streamk(st, a, plan, 32) : launch_cfg_dma<256, 256, 4, 2, 4>(st, a, splits);
