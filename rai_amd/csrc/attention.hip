@@ -92,6 +92,7 @@ __global__ void __launch_bounds__(256) k_attn_row(AttnArgs a) {
         for (int j = 0; j < V; ++j) qv[j] = qf[c * V + j];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+          if (keys() == kFew && base + 16 * u >= t_end) break;
           float sum = acc[u];
 #pragma unroll
           for (int j = 0; j < V; ++j) sum = fmaf(qv[j], (float)Scalar<T>::load(&pk[u].v[j]), sum);
@@ -101,6 +102,7 @@ __global__ void __launch_bounds__(256) k_attn_row(AttnArgs a) {
       float sum = 0.f;   // lane gl finishes the group's key gl
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        if (keys() == kFew && base + 16 * u >= t_end) break;
         const float all = row_sum(acc[u]);
         sum = gl == u ? all : sum;
       }
