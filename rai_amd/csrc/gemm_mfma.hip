@@ -940,7 +940,8 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
   const int grid_x = ((tiles + kXcds - 1) / kXcds) * kXcds;
   const int stages = (a.K + 32) / 64;
   int k_per_split = SH == 0 ? stages * 64 : a.K, longer = 0;
-  if (SH == 0 && splits > stages) splits = stages;
+  const int most = stages - (a.K % 64 != 0);   // the part whose first stage begins before the rows has a second one
+  if (SH == 0 && splits > most) splits = most;
   if (splits > 1) {
     if constexpr (SH == 0) {   // stages of 64, dealt out evenly
       k_per_split = stages / splits * 64;

@@ -24,3 +24,13 @@ def test_nothing_before_the_rows(R, m, k, n):  # noqa: F811
     near(down(R.linear(up(x, "bf16"), up(w, "bf16"), residual=up(r, "bf16"))), want + r, tol)
     z = want + b
     near(down(R.linear(xd, wd, up(b, "bf16"), "silu")), silu(z), 2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)
+
+
+@pytest.mark.parametrize("k", [96, 160, 608])
+def test_more_parts_than_stages(R, k):  # noqa: F811
+    """The first part always has a second stage: what it asks for again past its last one would begin before the rows."""
+    g = np.random.Generator(np.random.PCG64(k))
+    x, w = rand(g, (130, k), "bf16"), rand(g, (264, k), "bf16", k ** -0.5)
+    tol = 2 * (k + 20) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T + 1)
+    for parts in (1, 2, 3, 5, 9, 40):
+        near(down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), k_splits=parts)), x @ w.T, tol)
