@@ -417,9 +417,11 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  {
+  if (!half) {
+    issue(0, 0);
+  } else {
     uint16_t *sa = lds + wave * LA * 8 * BK, *sb = lds + BM * BK + wave * LB * 8 * BK;
-    auto source = [&](const uint16_t *p, int r) { return half && ((lane & 7) ^ ((r >> 1) & 7)) < 4 ? (const uint16_t *)g_k_zeros : p; };
+    auto source = [&](const uint16_t *p, int r) { return ((lane & 7) ^ ((r >> 1) & 7)) < 4 ? (const uint16_t *)g_k_zeros : p; };
 #pragma unroll
     for (int j = 0; j < LA; ++j) __builtin_amdgcn_global_load_lds((const void *)source(gpa[j], (wave * LA + j) * 8 + lrow), (lds_ptr)(sa + j * 8 * BK), 16, 0, 0);
 #pragma unroll
