@@ -70,6 +70,9 @@ __device__ __forceinline__ void stream_rows(RowSet<KC, 2> &rs, const ld_u32x4 (&
 // (8 blocks)-th pair of rows and keeps two pairs on their way, the first two from the block's first instructions on.
 constexpr int kRowWaves = 8, kRowThreads = 64 * kRowWaves, kRowGroups = 16;
 inline size_t latent_in_lds(const LatentInArgs &a) { return ((size_t)a.K * ((a.N1 > 0) + (a.N2 > 0)) * 2 + 15) / 16 * 16 + (kRowWaves * (1 + kRowGroups)) * sizeof(float); }
+// Whether the wave at pair `at` takes the second product's vector, which lies K elements behind the first one's if both are there.  A
+// wave behind the last pair takes one as well, and only those that are there.
+__host__ __device__ __forceinline__ bool latent_in_second(const LatentInArgs &a, int at) { return a.N2 > 0 && at >= (a.N1 + 1) / 2; }
 template <int KC> __device__ __forceinline__ void latent_in_block(const LatentInArgs &a, int block, int blocks, char *lds) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int pairs1 = (a.N1 + 1) / 2, pairs = pairs1 + (a.N2 + 1) / 2, stride = blocks * kRowWaves;
@@ -161,10 +164,10 @@ template <int KC> __device__ __forceinline__ void latent_in_block(const LatentIn
     for (int u = 0; u < KC; ++u)
       xv[u] = lane * 8 + u * 512 < a.K ? *reinterpret_cast<const ld_u32x4 *>((second ? xs2 : xs1) + lane * 8 + u * 512) : ld_u32x4{0u, 0u, 0u, 0u};
   };
-  bool second = at >= pairs1;
+  bool second = latent_in_second(a, at);
   take(second);
   auto finish = [&](RowSet<KC, 2> &r) {
-    if (!second && at >= pairs1) take(second = true);
+    if (!second && latent_in_second(a, at)) take(second = true);
     float v0 = 0.f, v1 = 0.f;
 #pragma unroll
     for (int u = 0; u < KC; ++u) {
