@@ -198,8 +198,8 @@ __device__ __forceinline__ int sk_block_of(const StreamKArgs &k, int u) {
 
 // The 256 x 256 tiles of a product on one block per CU, the next tile's loads under way while the last one's outputs are
 // written (gemm_persist.hip); sk: which of them are shared out by K tile (sk_tiles == 0: none).
-// It addresses the rows of a tile by 32-bit offsets.
-inline bool gemm_persist_serves(const LinearArgs &a) { return a.lda < (1 << 22) && a.ldw < (1 << 22); }
+// It addresses the rows of a tile by 32-bit offsets: of bytes in the operands, 256 rows, and of elements in the outputs, 16 rows.
+inline bool gemm_persist_serves(const LinearArgs &a) { return a.lda < (1 << 22) && a.ldw < (1 << 22) && a.ld1 < (1 << 28) && a.ld2 < (1 << 28); }
 int launch_gemm_bf16_persist(hipStream_t st, const LinearArgs &a, const StreamKArgs &sk);
 
 }  // namespace rai

@@ -41,3 +41,26 @@ int main() {{
   puts("done");
 }}""")
     assert lines == ["done"]
+
+
+def test_offsets_of_tile_rows_fit_32_bits(tmp_path):
+    """The 256 x 256 tiles of one block per CU: whatever row strides they take, a row's offset in 32 bits is the one in 64."""
+    lines = run(tmp_path, """
+#include "gemm_device.h"
+using namespace rai;
+int main() {
+  LinearArgs a;
+  memset(&a, 0, sizeof(a));
+  const int64_t usual[4] = {64, 64, 64, 64};
+  for (int which = 0; which < 4; ++which)
+    for (int64_t ld = 64; ld < 1ll << 34; ld += ld < 4096 ? 8 : ld / 64 * 8) {
+      int64_t l[4];
+      for (int i = 0; i < 4; ++i) l[i] = i == which ? ld : usual[i];
+      a.lda = l[0]; a.ldw = l[1]; a.ld1 = l[2]; a.ld2 = l[3];
+      const bool fits = which < 2 ? 255 * 2 * ld + 7 * 16 < 1ll << 32 : 15 * ld + 7 * 8 < 1ll << 32;
+      if (gemm_persist_serves(a) && !fits) { printf("stride %d of %lld\\n", which, (long long)ld); break; }
+      if (ld <= 1 << 20 && !gemm_persist_serves(a)) printf("stride %d of %lld refused\\n", which, (long long)ld);
+    }
+  puts("done");
+}""")
+    assert lines == ["done"]
