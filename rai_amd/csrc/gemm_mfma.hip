@@ -1058,6 +1058,9 @@ int streamk_counters_reset(int dev, hipStream_t st) {
   return RAI_OK;
 }
 
+// Whether whole 256 x 256 tiles of stages of 64 are those of one block per CU (gemm_persist.hip); otherwise a block has one tile.
+static bool persists(const LinearArgs &a) { return a.K % 64 == 0 && gemm_persist_serves(a); }
+
 static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan, int bk) {
   constexpr int BM = 256, BN = 256, NS = 4, SH = 2, WGN = 4;
   constexpr size_t lds = dma_lds_bytes<BM, BN, NS, WGN>();
@@ -1672,15 +1675,15 @@ static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 25
 // 128 x 128 with eight waves (4 x 2, 32 x 64 each, two to a SIMD) took the place of four waves in two and four stages: 333 x 8960 x 1536
 // 20.5 to 18.9 us, 2000 x 2048 x 2048 22.7 to 21.1.  128 x 256 and 192 x 256 (eight waves, three and two stages) serve where 256 x 256
 // leaves a last round nearly empty: 1200 x 16384 x 2048 108 to 97 us, 3000 x 4096 x 4096 105 to 88, 777 x 22528 x 2048 114 to 91.
-// Whole 256 x 256 tiles run on one block per CU that keeps its pipeline full from tile to tile (gemm_persist.hip): `end` is what each
-// then costs besides (10.1 us when every tile was a block; over 320 products with 100 such tiles and more what is picked takes 0.4 %
-// more than the best in the mean, 1.2 % by the old figure).  Their K parts are blocks of their own as before.
+// Whole 256 x 256 tiles on one block per CU that keeps its pipeline full from tile to tile (gemm_persist.hip; persists()) cost kPersistEnd
+// besides (over 320 products with 100 such tiles and more what is picked takes 0.4 % more than the best in the mean, 1.2 % by the
+// figure of a block per tile).  K of an odd number of 32s and K parts are blocks' work.
 enum { kTile128 = 0, kTile128x64, kTile64, kTile128x256, kTile256x192, kTile192x256, kTile256, kTileStreamK };
 struct TileCost { int bm, bn, share; float stage[3], end, cut; };
 static const TileCost kTileCosts[] = {{128, 128, 1, {0.482f}, 3.24f, 1.46f}, {128, 64, 2, {0.36f, 0.568f}, 2.02f, 0.929f}, {64, 64, 3, {0.256f, 0.382f, 0.614f}, 0.81f, 0.428f},
                                       {128, 256, 1, {0.785f}, 6.77f, 2.27f}, {256, 192, 1, {1.21f}, 7.82f, 0.293f},        {192, 256, 1, {1.16f}, 7.58f, 0.472f},
-                                      {256, 256, 1, {1.33f}, 8.f, 0.493f}};
-constexpr float kLaunchUs = 2.43f, kCutUs = 4.04f, kPartUsPerMB = 0.555f, kMostPartMB = 80.f, kShareUs = 20.9f;
+                                      {256, 256, 1, {1.33f}, 10.1f, 0.493f}};
+constexpr float kPersistEnd = 8.f, kLaunchUs = 2.43f, kCutUs = 4.04f, kPartUsPerMB = 0.555f, kMostPartMB = 80.f, kShareUs = 20.9f;
 
 // Stream-K over 256 x 256 tiles, where its last round is exactly half full and so each of that round's tiles the work of two CUs, a half of
 // K each: no CU is left idle, for an exchange of the halves (us, stream-K, the best whole tiles when both were blocks of a tile each: 4096 x 10240 x 2560 200,
@@ -1692,7 +1695,7 @@ static float streamk_us(const LinearArgs &a) {
   const int tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256);
   StreamKPlan plan;
   if (!has_huge_tiles(a) || tiles % kNumCU != kNumCU / 2 || a.K / 64 % 2 || !streamk_applies(a, 64, &plan)) return 0.f;
-  const float tile = kTileCosts[kTile256].end + kTileCosts[kTile256].stage[0] * ((float)a.K / 64), shared = tile * ((float)tiles / kNumCU) + kShareUs;
+  const float tile = kPersistEnd + kTileCosts[kTile256].stage[0] * ((float)a.K / 64), shared = tile * ((float)tiles / kNumCU) + kShareUs;
   return shared < tile * ((tiles + kNumCU - 1) / kNumCU) ? kLaunchUs + shared : 0.f;
 }
 // With K stages of 32 (K no multiple of 64) whole 256 x 256 tiles are all there is beside it, and any shares pay where the CU time saved
@@ -1718,8 +1721,9 @@ static TilePlan tile_plan_k64(const LinearArgs &a, int first = kTile128, int las
       const int64_t per_cu = ((tiles + kXcds - 1) / kXcds * s + kNumCU / kXcds - 1) / (kNumCU / kXcds);
       const int left = (int)(per_cu % c.share);
       const float stage = per_cu / c.share * c.stage[c.share - 1] + (left ? c.stage[left - 1] : 0.f);
+      const float end = t == kTile256 && persists(a) ? kPersistEnd : c.end;
       const float cost = kLaunchUs + stage * ((stages + s - 1) / s) +
-                         (s > 1 ? kCutUs + kPartUsPerMB * s * part_mb + (a.N % 4 ? 2.2f * part_mb : 0.f) + per_cu * c.cut : per_cu * c.end + (a.post_ln_out ? 5.f : 0.f));
+                         (s > 1 ? kCutUs + kPartUsPerMB * s * part_mb + (a.N % 4 ? 2.2f * part_mb : 0.f) + per_cu * c.cut : per_cu * end + (a.post_ln_out ? 5.f : 0.f));
       if ((t == first && s == 1) || cost < least) { least = cost; best = {t, s}; }
     }
   }
@@ -1839,7 +1843,7 @@ static int launch_tile_k64(hipStream_t st, const LinearArgs &a, TilePlan tile) {
     case kTile256x192: return launch_cfg_dma<256, 192, 2, 0, 2, 4>(st, a, tile.splits);
     case kTile192x256: return launch_cfg_dma<192, 256, 2, 0, 4, 2>(st, a, tile.splits);
     case kTile256:
-      if (tile.splits == 1 && a.K % 64 == 0 && gemm_persist_serves(a)) return launch_gemm_bf16_persist(st, a, StreamKArgs{});
+      if (tile.splits == 1 && persists(a)) return launch_gemm_bf16_persist(st, a, StreamKArgs{});
       return launch_cfg_dma<256, 256, 2, 0, 4>(st, a, tile.splits);
     case kTileStreamK: {
       StreamKPlan plan;

@@ -64,3 +64,42 @@ int main() {
   puts("done");
 }""")
     assert lines == ["done"]
+
+
+RULES = """
+#include "gemm_mfma.hip"
+namespace rai { int device_cu_count(int) { return 256; } }
+using namespace rai;
+static LinearArgs product(int m, int n, int k) {
+  LinearArgs a = linear_args_default();
+  a.M = m; a.N = n; a.K = k; a.dev = 0;
+  a.lda = a.ldw = k; a.ld1 = n;
+  a.splitk_ws = (void *)16; a.splitk_ws_bytes = 256 << 20;
+  return a;
+}
+static const char *tile(int m, int n, int k) {
+  const int t = tile_plan(product(m, n, k)).tile;
+  for (const auto &x : kTileNames) if (x.tile == t) return x.name;
+  return t == kTileStreamK ? "streamk64" : "?";
+}
+"""
+
+
+def test_which_256_tiles_go_from_tile_to_tile(tmp_path):
+    lines = run(tmp_path, RULES + """
+int main() {
+  LinearArgs a = product(4096, 4096, 4096);
+  printf("%d ", persists(a));
+  a.K = 4064; printf("%d ", persists(a));
+  a.K = 4096; a.lda = 1 << 22; printf("%d ", persists(a));
+  a.lda = 4096; a.ld1 = 1ll << 28; printf("%d ", persists(a));
+  puts("");
+}""")
+    assert lines == ["1 0 0 0 "]
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    # K an odd number of 32s: 256 x 256 tiles are a block's each and cost as much
+    (4397, 19664, 288, "192x256"), (14470, 5768, 224, "192x256"), (16384, 8960, 1504, "256x256k64")])
+def test_tile_of_a_product(tmp_path, m, n, k, want):
+    assert run(tmp_path, RULES + f'int main() {{ puts(tile({m}, {n}, {k})); }}') == [want]
