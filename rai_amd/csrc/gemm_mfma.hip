@@ -578,11 +578,12 @@ __global__ void __launch_bounds__(128 * WGN) k_gemm_bf16_mfma_grouped(LinearArgs
 // of the sk_tiles * KT (tile, K tile) units, i.e. the tail of one tile and the head of the next.  A tile is then the
 // work of two or three blocks: each stores its f32 accumulators to its slot of the workspace in register order
 // with device-scope stores and counts itself in; the block that arrives
-// last adds the slots in slot order (so the sum does not depend on who was last) and runs the epilogue.  Nobody
-// waits for anybody.  The remaining tiles follow in whole rounds, one tile per block as before.
-template <int BM, int BN, int NS, int SH, int WGN>
-__global__ void __launch_bounds__(128 * WGN) k_gemm_bf16_mfma_dma_streamk(LinearArgs a, StreamKArgs sk) {
-  constexpr int BK = 32;   // the unit of sharing is one K tile of the main loop
+// last adds the slots in slot order (so the sum does not depend on who was last) and runs the epilogue.  It alone
+// waits, for stores under way, and not for ever.  The remaining tiles follow in whole rounds, one tile per block as before.
+//   With stages of 64 this is the form for operands that stay in no cache (persists() below), else gemm_persist.hip's.
+template <int NS>   // four stages of 32, two of 64
+__global__ void __launch_bounds__(512) k_gemm_bf16_mfma_dma_streamk(LinearArgs a, StreamKArgs sk) {
+  constexpr int BM = 256, BN = 256, SH = 2, WGN = 4, BK = NS == 2 ? 64 : 32;   // the unit of sharing is one K tile of the main loop
   constexpr int MT = BM / 64, NT = BN / (32 * WGN);
   constexpr int LDS_BYTES = dma_lds_bytes<BM, BN, NS, WGN>();
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -620,7 +621,8 @@ __global__ void __launch_bounds__(128 * WGN) k_gemm_bf16_mfma_dma_streamk(Linear
     tile_coords(tile, tiles_m, tiles_n, &tile_m, &tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     __syncthreads();   // the previous segment's epilogue staging is done with the LDS
-    dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, kt0 * BK, kt1 - kt0, wave, lane, acc);
+    if constexpr (NS == 2) dma_tile_mainloop_k64<BM, BN, WGN>(a, lds, m0, n0, kt0 * BK, kt1 - kt0, wave, lane, acc);
+    else dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, kt0 * BK, kt1 - kt0, wave, lane, acc);
     if (kt1 - kt0 != KT) {
       // a share of the tile: which slot is ours, and how many there are
       const int first = sk_block_of(sk, tile * KT), last = sk_block_of(sk, tile * KT + KT - 1);
@@ -1017,7 +1019,7 @@ static int linear_device(const LinearArgs &a, int *dev) {
 static bool streamk_applies(const LinearArgs &a, int bk, StreamKPlan *plan) {
   const char *off = getenv("RAI_HIP_NO_STREAMK");   // read per call: tests compare both forms in one process
   if (off && *off && *off != '0') return false;
-  if (!a.splitk_ws || ((uintptr_t)a.splitk_ws & 15) || a.post_ln_out || (bk == 64 && !gemm_persist_serves(a))) return false;
+  if (!a.splitk_ws || ((uintptr_t)a.splitk_ws & 15) || a.post_ln_out) return false;
   // one block per CU of a 256-CU part: the plan, the counter array and the XCD order are laid out for that grid
   int dev = -1;
   if (linear_device(a, &dev) != RAI_OK || device_cu_count(dev) != kNumCU) return false;
@@ -1058,20 +1060,29 @@ int streamk_counters_reset(int dev, hipStream_t st) {
   return RAI_OK;
 }
 
-// Whether whole 256 x 256 tiles of stages of 64 are those of one block per CU (gemm_persist.hip); otherwise a block has one tile.
-static bool persists(const LinearArgs &a) { return a.K % 64 == 0 && gemm_persist_serves(a); }
-
-static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan, int bk) {
-  constexpr int BM = 256, BN = 256, NS = 4, SH = 2, WGN = 4;
-  constexpr size_t lds = dma_lds_bytes<BM, BN, NS, WGN>();
-  int dev = 0;
-  RAI_TRY(linear_device(a, &dev));
+template <int NS> static int launch_streamk_blocks(hipStream_t st, const LinearArgs &a, const StreamKArgs &sk, int dev) {
+  constexpr size_t lds = dma_lds_bytes<256, 256, NS, 4>();
   static bool attr_set[64];
   if (!attr_set[dev]) {
-    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_gemm_bf16_mfma_dma_streamk<BM, BN, NS, SH, WGN>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_gemm_bf16_mfma_dma_streamk<NS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_set[dev] = true;
   }
+  hipLaunchKernelGGL(k_gemm_bf16_mfma_dma_streamk<NS>, dim3(kNumCU), dim3(512), lds, st, a, sk);
+  return launch_check("gemm_bf16_mfma_dma_streamk");
+}
+
+// Whether the 256 x 256 tiles of stages of 64 are those of one block per CU (gemm_persist.hip); otherwise a block has one tile, or stream-K's
+// shares.  Those ask for a stage as soon as the one before the last is let go, all waves at once, and that is worth more where the operands
+// outgrow the memory-side cache of 256 MB and come from HBM again and again.  Measured (us, blocks / one per CU): stream-K 16384 x 1536 x 8960
+// (321 MB) 372, 382, 8032 x 8984 x 8832 (300 MB) 1033, 1065; whole 4318 x 16496 x 10432 (434 MB) 1279, 1324, 3784 x 15064 x 7680 (290 MB) 751, 773,
+// 4426 x 6392 x 12544 (271 MB) 608, 620.  From 200 MB on either may be ahead (8803 x 5064 x 7744, 215 MB, 560, 543; 16384 x 1536 x 6144, 220 MB, by
+// stream-K 260, 267), below one per CU is (4096 x 4096 x 12288 312, 289; 8192 x 7168 x 4096 397, 370).
+constexpr int64_t kPersistBytes = 256 << 20;
+static bool persists(const LinearArgs &a) { return a.K % 64 == 0 && gemm_persist_serves(a) && ((int64_t)a.M + a.N) * a.K * 2 <= kPersistBytes; }
+
+static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan, int bk) {
+  int dev = 0;
+  RAI_TRY(linear_device(a, &dev));
   plan.k.ws = (float *)a.splitk_ws;
   plan.k.counters = streamk_counters_of(dev);
   plan.k.fault = kernel_fault_word(dev);
@@ -1084,9 +1095,8 @@ static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan,
     int lim = 0, tile = -1;
     if (sscanf(t, "%d,%d", &lim, &tile) == 2 && lim > 0) { plan.k.spin_limit = lim; plan.k.drop_tile = tile; }
   }
-  if (bk == 64) return launch_gemm_bf16_persist(st, a, plan.k);
-  hipLaunchKernelGGL((k_gemm_bf16_mfma_dma_streamk<BM, BN, NS, SH, WGN>), dim3(kNumCU), dim3(128 * WGN), lds, st, a, plan.k);
-  return launch_check("gemm_bf16_mfma_dma_streamk");
+  if (bk == 32) return launch_streamk_blocks<4>(st, a, plan.k, dev);
+  return persists(a) ? launch_gemm_bf16_persist(st, a, plan.k) : launch_streamk_blocks<2>(st, a, plan.k, dev);
 }
 
 // ---- small M (9..64 rows): weight streaming through 16x16x32 MFMA -----------------------
@@ -1677,26 +1687,30 @@ static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 25
 // leaves a last round nearly empty: 1200 x 16384 x 2048 108 to 97 us, 3000 x 4096 x 4096 105 to 88, 777 x 22528 x 2048 114 to 91.
 // Whole 256 x 256 tiles on one block per CU that keeps its pipeline full from tile to tile (gemm_persist.hip; persists()) cost kPersistEnd
 // besides (over 320 products with 100 such tiles and more what is picked takes 0.4 % more than the best in the mean, 1.2 % by the
-// figure of a block per tile).  K of an odd number of 32s and K parts are blocks' work.
+// figure of a block per tile).  K of an odd number of 32s, K parts and operands that no cache holds are blocks' work.
 enum { kTile128 = 0, kTile128x64, kTile64, kTile128x256, kTile256x192, kTile192x256, kTile256, kTileStreamK };
 struct TileCost { int bm, bn, share; float stage[3], end, cut; };
 static const TileCost kTileCosts[] = {{128, 128, 1, {0.482f}, 3.24f, 1.46f}, {128, 64, 2, {0.36f, 0.568f}, 2.02f, 0.929f}, {64, 64, 3, {0.256f, 0.382f, 0.614f}, 0.81f, 0.428f},
                                       {128, 256, 1, {0.785f}, 6.77f, 2.27f}, {256, 192, 1, {1.21f}, 7.82f, 0.293f},        {192, 256, 1, {1.16f}, 7.58f, 0.472f},
                                       {256, 256, 1, {1.33f}, 10.1f, 0.493f}};
-constexpr float kPersistEnd = 8.f, kLaunchUs = 2.43f, kCutUs = 4.04f, kPartUsPerMB = 0.555f, kMostPartMB = 80.f, kShareUs = 20.9f;
+constexpr float kPersistEnd = 8.f, kLaunchUs = 2.43f, kCutUs = 4.04f, kPartUsPerMB = 0.555f, kMostPartMB = 80.f, kShareUs = 20.9f, kPersistShareUs = 25.f;
 
 // Stream-K over 256 x 256 tiles, where its last round is exactly half full and so each of that round's tiles the work of two CUs, a half of
-// K each: no CU is left idle, for an exchange of the halves (us, stream-K, the best whole tiles when both were blocks of a tile each: 4096 x 10240 x 2560 200,
-// 212; 16384 x 1536 x 8960 374, 419; 1200 x 32768 x 2048 168, 174; so 186, 386, 152).  Shares that begin anywhere in K lose more in the L2s, where blocks no longer read
+// K each: no CU is left idle, for an exchange of the halves (us, stream-K, the best whole tiles, all as blocks of a tile each: 4096 x 10240 x 2560
+// 200, 212; 16384 x 1536 x 8960 374, 419; 1200 x 32768 x 2048 168, 174).  Shares that begin anywhere in K lose more in the L2s, where blocks no longer read
 // the same columns together, than they win in idle CUs: of 168 such products with 40 stages and more the median took 1.14 times the best
 // whole tiles' time (7770 x 2560 x 10240 476 us for 369, 7443 x 2560 x 2560 133 for 104), three less than 0.96 of it (14476 x 1536 x 8960
-// 344 for 388).  0: does not pay or does not apply.
+// 344 for 388).  On one block per CU a shared tile costs what a block's does, a whole one less, and the exchange is the dearer for it
+// (2827 x 24480 x 2048 263, whole 246; 884 x 40776 x 2048 158, 146; 1341 x 16320 x 3584 151, on 192 x 256 tiles 138; but 16384 x 1536 x 4096 169, 178).
+// 0: does not pay or does not apply.
 static float streamk_us(const LinearArgs &a) {
   const int tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256);
   StreamKPlan plan;
   if (!has_huge_tiles(a) || tiles % kNumCU != kNumCU / 2 || a.K / 64 % 2 || !streamk_applies(a, 64, &plan)) return 0.f;
-  const float tile = kPersistEnd + kTileCosts[kTile256].stage[0] * ((float)a.K / 64), shared = tile * ((float)tiles / kNumCU) + kShareUs;
-  return shared < tile * ((tiles + kNumCU - 1) / kNumCU) ? kLaunchUs + shared : 0.f;
+  const bool persist = persists(a);
+  const float multiply = kTileCosts[kTile256].stage[0] * ((float)a.K / 64), end = kTileCosts[kTile256].end;
+  const float shared = (end + multiply) * ((float)tiles / kNumCU) + (persist ? kPersistShareUs : kShareUs);
+  return shared < ((persist ? kPersistEnd : end) + multiply) * ((tiles + kNumCU - 1) / kNumCU) ? kLaunchUs + shared : 0.f;
 }
 // With K stages of 32 (K no multiple of 64) whole 256 x 256 tiles are all there is beside it, and any shares pay where the CU time saved
 // exceeds the exchange of two or three to a tile; a K tile of 32 takes some 1 us with all CUs busy (us, stream-K, whole tiles: 16384 x

@@ -133,6 +133,27 @@ def test_what_the_rule_picks(R, m, k, n, tile, cut):
     assert np.all(np.abs(got - full) <= 2.0 ** -8 * np.abs(full) + 2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)
 
 
+@pytest.mark.parametrize("tile", ["256x256k64", "streamk64"])
+def test_operands_that_no_cache_holds(R, monkeypatch, tile):
+    """290 MB of operands: 256 x 256 tiles of a block each, and their shares; ragged rows, columns and number of stages."""
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", tile)
+    m, k, n, few = 16200, 8256, 1400, 300
+    g = np.random.Generator(np.random.PCG64(m + k))
+    x, w, b, r = rand(g, (few, k), "bf16"), rand(g, (n, k), "bf16", k ** -0.5), rand(g, (n,), "bf16"), rand(g, (few, n), "bf16")
+    want = x @ w.T   # in f32: both sides' sums are within the spread of the exact ones
+    tol = 2 * (k + 20) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T + 1)
+    again = lambda a: np.tile(a, (m // few, 1))  # noqa: E731
+    xd, wd = up(again(x), "bf16"), up(w, "bf16")
+    got = down(R.linear(xd, wd))
+    assert np.all(np.abs(got[:few] - want) <= 2.0 ** -8 * np.abs(want) + tol)
+    z = want + b
+    full = z / (1 + np.exp(-z)) + r   # silu's slope stays below 1.1, its own error below 2^-18 of it
+    fused = down(R.linear(xd, wd, up(b, "bf16"), "silu", up(again(r), "bf16")))
+    assert np.all(np.abs(fused[:few] - full) <= 2.0 ** -8 * np.abs(full) + 2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)
+    # every row block, against the first (a shared tile's sums are grouped in another way: 2 tol, one rounding)
+    assert np.all(np.abs(got - again(got[:few])) <= 2.0 ** -7 * np.abs(again(want)) + 2 * again(tol))
+
+
 def test_plan_is_what_runs(R, monkeypatch):
     """A product whose sums differ by tile and parts: the rule's name and parts, forced, give the bits of the call that is not."""
     m, k, n = 409, 5760, 8416

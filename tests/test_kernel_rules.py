@@ -93,13 +93,16 @@ int main() {
   a.K = 4064; printf("%d ", persists(a));
   a.K = 4096; a.lda = 1 << 22; printf("%d ", persists(a));
   a.lda = 4096; a.ld1 = 1ll << 28; printf("%d ", persists(a));
-  puts("");
+  printf("%d %d %d\\n", persists(product(16384, 16384, 4096)), persists(product(16385, 16384, 4096)), persists(product(1 << 20, 1 << 20, 65536)));
 }""")
-    assert lines == ["1 0 0 0 "]
+    assert lines == ["1 0 0 0 1 0 0"]
 
 
 @pytest.mark.parametrize("m,n,k,want", [
     # K an odd number of 32s: 256 x 256 tiles are a block's each and cost as much
-    (4397, 19664, 288, "192x256"), (14470, 5768, 224, "192x256"), (16384, 8960, 1504, "256x256k64")])
+    (4397, 19664, 288, "192x256"), (14470, 5768, 224, "192x256"), (16384, 8960, 1504, "256x256k64"),
+    # a half-full last round: shares, whole 256 x 256 tiles, others
+    (16384, 1536, 8960, "streamk64"), (4096, 6144, 4096, "streamk64"), (2827, 24480, 2048, "256x256k64"), (16384, 17920, 1536, "256x256k64"),
+    (1341, 16320, 3584, "192x256"), (5900, 3936, 3840, "192x256")])
 def test_tile_of_a_product(tmp_path, m, n, k, want):
     assert run(tmp_path, RULES + f'int main() {{ puts(tile({m}, {n}, {k})); }}') == [want]
