@@ -79,7 +79,6 @@ __device__ __forceinline__ void gemm_tile_epilogue(const LinearArgs &a, f32x16 (
       if (lane >= RP * CG || m >= a.M || n >= a.N) continue;
       const f32x4 v0 = *reinterpret_cast<const f32x4 *>(stage + row * EP + cg * 8);
       const f32x4 v1 = *reinterpret_cast<const f32x4 *>(stage + row * EP + cg * 8 + 4);
-      float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
       if (partial) {
         float *p = partial + ((int64_t)split * a.M + m) * a.N + n;
         if (a.N % 4 == 0) {
@@ -88,11 +87,11 @@ __device__ __forceinline__ void gemm_tile_epilogue(const LinearArgs &a, f32x16 (
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e)
-            if (n + e < a.N) p[e] = v[e];
+            if (n + e < a.N) p[e] = e < 4 ? v0[e & 3] : v1[e & 3];
         }
         continue;
       }
-      store_row8(a, v, bv, m, n, whole, vec_out);
+      store_row8(a, v0, v1, bv, m, n, whole, vec_out);
     }
   }
 }

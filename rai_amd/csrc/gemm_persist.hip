@@ -222,8 +222,7 @@ __device__ __forceinline__ void write_rows(const LinearArgs &a, Acc acc, float *
       const int r = p * 8 + (lane >> 3), m = m0 + q * 16 + r;
       const f32x4 v0 = *reinterpret_cast<const f32x4 *>(staging + r * kWN + ((((lane & 7) * 2) ^ r) << 2));
       const f32x4 v1 = *reinterpret_cast<const f32x4 *>(staging + r * kWN + ((((lane & 7) * 2 + 1) ^ r) << 2));
-      float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-      if (m < a.M && n < a.N) store_row8(a, v, bv, m, n, whole, vec_out);
+      if (m < a.M && n < a.N) store_row8(a, v0, v1, bv, m, n, whole, vec_out);
     }
   }
 }
