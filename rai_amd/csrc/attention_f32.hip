@@ -621,9 +621,12 @@ static bool takes(const AttnArgs &a) {
   return al(a.q, a.qs) && al(a.k, a.ks) && al(a.v, a.vs) && (uintptr_t)a.out % 16 == 0 && a.out_row_stride % 4 == 0 && (a.S + 31) / 32 <= 65535 && a.B <= 65535;
 }
 
-// A block per query row (attention.hip) is done sooner where there are few rows.  Up to 80 features a tile here is some 2 us, a row's
-// block as fast only on few keys: measured (us; block per row, here) 32 heads x 32 x 64 5.6, 5.6; 16 x 40 x 64 5.7, 5.8; 8 x 64 x 80 6.7,
-// 6.3; 8 x 100 x 80 9.0, 6.7; 32 x 16 x 80 on 100 keys 8.4, 6.7, on 400 30.3, 13.1; 16 on 40 keys for 8 x 16 heads of 64 9.1, 6.2.
+// A block per query row (attention.hip) is done sooner where there are few rows.  Up to 80 features it is up to 512 rows, as long as an XCD's L2
+// holds all keys and values, and up to 1024 rows on few keys: measured (us; block per row, here) 16 rows x 80 on 256 keys 7.4, 8.0, on 2000
+// 31.5, 38.8; 8 heads x 64 x 80 on 700 (3.6 MB) 15.4, 17.5, on 1000 (5.1 MB) 23.8, 21.9; 32 x 16 x 80 on 160 7.2, 8.5, on 256 10.7, 8.6; 32 x 33 x 64
+// on 64 5.9, 5.7, on 256 10.9, 7.7.  But its sums over the keys are longer chains: off by 1.88e-7 where the tiles are by 1.59e-7 (8 x 64 x 64 on 700),
+// 2.06e-7 and 1.64e-7 (8 x 64 x 80 on 700), 2.84e-7 and 1.91e-7 (16 x 80 on 2000).  So it has only what is short, fewer than 64 keys, where it
+// is ahead by a sixth (32 x 18 x 64 on 50 5.3, 5.9).
 //   Beyond, a tile is a chain of up to 8 us (256), which takes enough rows or keys to be worth it: 8 x 64 on 300 x 128 20.0, 29.3, 32 x 64 on
 // 300 38.1, 29.6; 32 x 64 on 300 x 256 66, 86, 2 x 8 x 512 x 256 174, 129.  The sums of a score are then longer chains than a row's
 // lanes make of them, and less exact than those until there are a few hundred keys (1.17e-7 and 1.11e-7 at 100 x 128, 1.67e-7 and
