@@ -29,14 +29,15 @@ __device__ __forceinline__ float af_gate(float z) { return 1.0f / (1.0f + expf(-
 // units in brackets): 16 x 12 x 1024 x 128 on 2 key heads 993 (3900), 2 x 8 x 512 x 256 130 (178).  Off by 1.28e-7 (1.36e-7),
 // 1.43e-7 (1.47e-7).  Two stages also with two waves at 128 features: 16 heads x 1024 112 -> 109.5.
 template <int D> struct F32Attn {
-  static constexpr int CPR = D / 4, DT = (D + 31) / 32, TILE = 32 * D, LOADS = D / 8;   // 1 KB pieces of a tile
-  static __device__ __forceinline__ int swizzle(int row) { return D == 80 ? (row >> 2) & 3 : D == 32 ? (row >> 1) & 7 : row & 15; }
+  static_assert(D >= 128 && D % 64 == 0, "whole 32-feature tiles, a row of K over all banks, as many pieces for every wave");
+  static constexpr int CPR = D / 4, DT = D / 32, TILE = 32 * D, LOADS = D / 8;   // 1 KB pieces of a tile
+  static __device__ __forceinline__ int swizzle(int row) { return row & 15; }
 };
 
 template <int D, int KSP, bool DB>
 __global__ void __launch_bounds__(256, 1) k_flash_prefill_f32(AttnArgs a) {
   typedef F32Attn<D> F;
-  constexpr int NG = 4 / KSP, KC = D / 8, CG = D <= 128 ? 2 : 4, DT = F::DT, STAGE = KSP * 2 * F::TILE, LW = (F::LOADS + 3) / 4;
+  constexpr int NG = 4 / KSP, KC = D / 8, CG = D <= 128 ? 2 : 4, DT = F::DT, STAGE = KSP * 2 * F::TILE, LW = F::LOADS / 4;
   extern __shared__ __attribute__((aligned(16))) float af_lds[];
   typedef __attribute__((address_space(3))) void *lds_ptr;
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kh = wave % KSP;
@@ -75,7 +76,7 @@ __global__ void __launch_bounds__(256, 1) k_flash_prefill_f32(AttnArgs a) {
     v_off[j] = (uint32_t)(row * (int)a.vs[2] + 4 * c);
   }
   // where this lane's chunks of a row of K lie: the swizzle stays within PAT chunks, what is beyond goes into the instruction
-  constexpr int PAT = D == 80 ? 4 : D == 32 ? 8 : 16;
+  constexpr int PAT = 16;
   int k_lane[PAT / 2];
 #pragma unroll
   for (int c = 0; c < PAT / 2; ++c) k_lane[c] = r * D + 4 * ((2 * c + h) ^ F::swizzle(r));
@@ -87,11 +88,10 @@ __global__ void __launch_bounds__(256, 1) k_flash_prefill_f32(AttnArgs a) {
       const float *kp = Kg + (int64_t)kt * a.ks[2], *vp = Vg + (int64_t)kt * a.vs[2];
       float *kd = af_lds + stage * STAGE + i * 2 * F::TILE, *vd = kd + F::TILE;
 #pragma unroll
-      for (int j = 0; j < LW; ++j)
-        if (F::LOADS % 4 == 0 || wave + 4 * j < F::LOADS) {
-          __builtin_amdgcn_global_load_lds((const void *)(kp + k_off[j]), (lds_ptr)(kd + (wave + 4 * j) * 256), 16, 0, 0);
-          __builtin_amdgcn_global_load_lds((const void *)(vp + v_off[j]), (lds_ptr)(vd + (wave + 4 * j) * 256), 16, 0, 0);
-        }
+      for (int j = 0; j < LW; ++j) {
+        __builtin_amdgcn_global_load_lds((const void *)(kp + k_off[j]), (lds_ptr)(kd + (wave + 4 * j) * 256), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void *)(vp + v_off[j]), (lds_ptr)(vd + (wave + 4 * j) * 256), 16, 0, 0);
+      }
     }
   };
   auto landed = [&]() {   // every wave's loads, for every wave
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(256, 1) k_flash_prefill_f32(AttnArgs a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) sg[i][e] = 0.f;
 #pragma unroll
-      for (int c = c0; c < KC && c < c0 + CG; ++c) {
+      for (int c = c0; c < c0 + CG; ++c) {
         const af_f32x4 kf = *reinterpret_cast<const af_f32x4 *>(Kt + k_lane[c % (PAT / 2)] + 4 * (2 * c & ~(PAT - 1)));
 #pragma unroll
         for (int j = 0; j < 4; ++j) sg[j & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j], qf[c][j], sg[j & 1], 0, 0, 0);
@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(256, 1) k_flash_prefill_f32(AttnArgs a) {
     // ---- O^T <- alpha O^T + V^T P^T, the products of sixteen keys in a chain
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
-      const float *vp = Vt + 4 * h * D + (D % 32 && t == DT - 1 ? min(32 * t + r, D - 1) : 32 * t + r);
+      const float *vp = Vt + 4 * h * D + 32 * t + r;
       float v[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) v[e] = vp[(8 * (e >> 2) + (e & 3)) * D];
@@ -232,11 +232,10 @@ __global__ void __launch_bounds__(256, 1) k_flash_prefill_f32(AttnArgs a) {
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
 #pragma unroll
-          for (int e = 0; e < 16; ++e)
-            if (32 * t + 8 * (e >> 2) < D) {
-              const float x = vp[32 * t + 8 * (e >> 2) + (e & 3)];
-              o[t][e] = fabsf(x) < INFINITY ? o[t][e] : fmaf(p, x, o[t][e]);
-            }
+          for (int e = 0; e < 16; ++e) {
+            const float x = vp[32 * t + 8 * (e >> 2) + (e & 3)];
+            o[t][e] = fabsf(x) < INFINITY ? o[t][e] : fmaf(p, x, o[t][e]);
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -294,7 +293,6 @@ __global__ void __launch_bounds__(256, 1) k_flash_prefill_f32(AttnArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; e += 4) {
       const int d = 32 * t + 2 * e + 4 * h;   // 8 (e / 4)
-      if (d >= D) continue;
       af_f32x4 w = {o[t][e] * inv, o[t][e + 1] * inv, o[t][e + 2] * inv, o[t][e + 3] * inv};
       if (gp) {
 #pragma unroll
@@ -319,6 +317,7 @@ __global__ void __launch_bounds__(256, 1) k_flash_prefill_f32(AttnArgs a) {
 // and each block reads its own keys from L2 (79 MB at 32 x 333, some 7 us of it).
 template <int D> struct F32Attn16 {
   static constexpr int CPR = D / 4, TILE = 32 * D, LOADS = D / 8, KC = D / 16;   // 1 KB pieces of a tile; 16-feature blocks
+  static __device__ __forceinline__ int kswizzle(int row) { return D == 80 ? (row >> 2) & 3 : D == 32 ? (row >> 1) & 7 : row & 15; }
   static __device__ __forceinline__ int vswizzle(int row) { return D == 80 ? 0 : D == 32 ? (row >> 1 & 1) << 2 : (row & 3) << 2; }   // of 16-byte chunks
 };
 __device__ __forceinline__ float af_quarter_fold_max(float v) {   // over the four lanes of a query
@@ -358,7 +357,7 @@ __global__ void __launch_bounds__(256, 2) k_flash_prefill_f32_q16(AttnArgs a) {
 #pragma unroll
   for (int j = 0; j < F::LOADS; ++j) {
     const int i = j * 64 + lane, row = i / F::CPR, c = i % F::CPR;
-    k_off[j] = (uint32_t)(row * (int)a.ks[2] + 4 * (c ^ F32Attn<D>::swizzle(row)));
+    k_off[j] = (uint32_t)(row * (int)a.ks[2] + 4 * (c ^ F::kswizzle(row)));
     v_off[j] = (uint32_t)(row * (int)a.vs[2] + 4 * (c ^ F::vswizzle(row)));
   }
   // a tile past the end of the keys starts early: what lies before its own first key is masked
@@ -400,7 +399,7 @@ __global__ void __launch_bounds__(256, 2) k_flash_prefill_f32_q16(AttnArgs a) {
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         const int row = 16 * hh + arow;
-        kf[hh] = *reinterpret_cast<const af_f32x4 *>(Kt + row * D + 4 * ((4 * c + g) ^ F32Attn<D>::swizzle(row)));
+        kf[hh] = *reinterpret_cast<const af_f32x4 *>(Kt + row * D + 4 * ((4 * c + g) ^ F::kswizzle(row)));
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)

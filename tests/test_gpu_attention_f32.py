@@ -1,4 +1,4 @@
-"""f32 prefill attention on the matrix instructions: query groups of 32, key tiles of 32; by the size of the call (small ones
+"""f32 prefill attention on the matrix instructions: query groups of 16 (up to 80 features) or 32, key tiles of 32; by the size of the call (small ones
 stay with the kernel that takes a row to a block), and every head size with one, two and four waves to a group forced."""
 import numpy as np
 import pytest
@@ -48,7 +48,7 @@ def test_against_64_bits(R, b, hq, hkv, s, t, d, causal):
     assert np.all(np.abs(got - want) <= tol)
 
 
-# Head sizes with the waves to a group they come with (two stages of tiles up to 128 features with one wave, one otherwise).
+# Head sizes with the waves to a group they come with.
 FORMS = [(d, waves) for d in (32, 64, 80, 128, 192, 256) for waves in (1, 2, 4) if waves < 4 or d <= 128]
 
 
@@ -84,7 +84,7 @@ def test_infinite_values_reach_only_queries_that_see_them(R, s, t, n, d=64):
     q, k, v = rand(g, (1, n, s, d), "f32"), rand(g, (1, n, t, d), "f32"), rand(g, (1, n, t, d), "f32")
     clean, tol = reference(q, k, v, d ** -0.5, 1)
     at = t - s // 2
-    v[0, 0, at, 5], v[0, 0, t - 1, 7], v[0, 1, at, d - 1] = np.inf, np.nan, -np.inf   # d - 1: the last feature, which 80's third tile repeats
+    v[0, 0, at, 5], v[0, 0, t - 1, 7], v[0, 1, at, d - 1] = np.inf, np.nan, -np.inf   # d - 1: the last feature
     got = down(R.attention(up(q, "f32"), up(k, "f32"), up(v, "f32"), d ** -0.5, 1, 1)).astype(np.float64)
     want = clean.copy()
     first = at - (t - s)   # the query at the key's own position
