@@ -82,3 +82,37 @@ def test_same_bits_whatever_way_the_rows_leave(R):
     full = down(R.linear(xd, up(w, "bf16")))
     for n in (575, 572, 568, 544):   # 16-byte pieces from the third on, whole 64-byte ones at the last
         np.testing.assert_array_equal(down(R.linear(xd, up(w[:n], "bf16"))), full[:, :n])
+
+
+# Stream-K: tiles that two and three blocks share (156 tiles), that two share besides a whole round (324), shares before whole tiles (720).
+# What the outputs need besides the sums is asked for once these are in.
+SHARED = [(3000, 2560, 3104), (4400, 320, 4608), (5000, 256, 9008)]
+
+
+@pytest.mark.parametrize("m,k,n", SHARED)
+def test_outputs_of_shared_tiles(R, monkeypatch, m, k, n):
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", "streamk64")
+    test_outputs(R, m, k, n)
+
+
+@pytest.mark.parametrize("m,k,n", SHARED)
+def test_gated_outputs_of_shared_tiles(R, monkeypatch, m, k, n):
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", "streamk64")
+    test_gated(R, m, k, n)
+
+
+@pytest.mark.parametrize("m,k,n", SHARED)
+def test_two_outputs_of_shared_tiles_and_the_same_bits_again(R, monkeypatch, m, k, n):
+    monkeypatch.setenv("RAI_HIP_GEMM_TILE", "streamk64")
+    x, w, b, r, want, tol = case(m, k, n)
+    xd, wd, bd, rd = up(x, "bf16"), up(w, "bf16"), up(b, "bf16"), up(r, "bf16")
+    n1, z = 1344, want + b
+    split = lambda: [down(o) for o in R.linear_packed(xd, wd, bias=bd, act="silu", act_from=n1, n1=n1)]  # noqa: E731
+    o1, o2 = split()
+    near(o1, z[:, :n1], tol[:, :n1])
+    near(o2, silu(z[:, n1:]), (2 * tol + 2.0 ** -18 * np.abs(z) + 2.0 ** -20)[:, n1:])
+    added = down(R.linear(xd, wd, residual=rd))
+    for _ in range(2):
+        again = split()
+        assert np.array_equal(again[0], o1) and np.array_equal(again[1], o2)
+        assert np.array_equal(down(R.linear(xd, wd, residual=rd)), added)
