@@ -622,84 +622,7 @@ __global__ void __launch_bounds__(512) k_gemm_bf16_mfma_dma_streamk(LinearArgs a
     __syncthreads();   // the previous segment's epilogue staging is done with the LDS
     if constexpr (NS == 2) dma_tile_mainloop_k64<BM, BN, WGN>(a, lds, m0, n0, kt0 * BK, kt1 - kt0, wave, lane, acc);
     else dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, kt0 * BK, kt1 - kt0, wave, lane, acc);
-    if (kt1 - kt0 != KT) {
-      // a share of the tile: which slot is ours, and how many there are
-      const int first = sk_block_of(sk, tile * KT), last = sk_block_of(sk, tile * KT + KT - 1);
-      const int parts = last - first + 1, slot = p - first;
-      // Slot layout [wave][accumulator register][lane]: one store or load instruction covers 256 consecutive bytes.
-      // The shares cross XCDs, whose L2s are not coherent with each other: they are written and read with
-      // device-scope accesses (write-through stores, loads that miss L2) instead of a release / acquire fence pair
-      // -- the fences write back and invalidate a whole L2 each and, issued by every block of an XCD at about the
-      // same time, queue up behind one another (measured: +130 us per launch).
-      float *tile_ws = sk.ws + (int64_t)tile * sk.max_parts * (BM * BN) + wave * (MT * NT * 16 * 64) + lane;
-      // Two counters per tile: `arrived` hands out tickets when a share has been computed, `stored` counts the
-      // shares that have reached memory.  The block with the last ticket keeps its share in registers and sums; the
-      // others store theirs.  Its wait is for blocks that already hold a ticket, i.e. are running and have nothing
-      // left to do but their stores, and it is bounded all the same.
-      int *arrived = sk.counters + 2 * tile, *stored = arrived + 1;
-      if (tid == 0) s_ticket = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      if (s_ticket != parts - 1) {
-        float *mine = tile_ws + (int64_t)slot * (BM * BN);
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-              __hip_atomic_store(mine + ((i * NT + j) * 16 + r) * 64, acc[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's share has left for memory
-        __syncthreads();
-        if (tid == 0 && tile != sk.drop_tile) __hip_atomic_fetch_add(stored, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        continue;
-      }
-      if (tid == 0) {
-        bool complete = false;
-        for (int spin = 0; spin < sk.spin_limit && !complete; ++spin) {
-          complete = __hip_atomic_load(stored, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
-          if (!complete) __builtin_amdgcn_s_sleep(2);
-        }
-        if (complete) {
-          __hip_atomic_store(arrived, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(stored, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-          // A share is missing.  Nothing is summed and nothing written for this tile, the counters stay as they are
-          // (a late block may still count itself in; the host zeroes them all before the next launch), and the
-          // host learns of it at its next synchronisation.
-          __hip_atomic_store(sk.fault, (int)RAI_FAULT_STREAMK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-          s_ticket = -1;
-        }
-      }
-      __syncthreads();
-      if (s_ticket < 0) continue;
-      // the other slots are complete.  Sum in slot order, our registers standing in for our slot, so the result does
-      // not depend on who came last.
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          f32x16 sum = acc[i][j];
-          for (int s = 0; s < parts; ++s) {
-            if (s == slot) {
-              if (s > 0) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sum[r] += acc[i][j][r];
-              }
-              continue;
-            }
-            const float *src = tile_ws + (int64_t)s * (BM * BN) + ((i * NT + j) * 16) * 64;
-            f32x16 v;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) v[r] = __hip_atomic_load(src + r * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (s == 0) sum = v;
-            else {
-#pragma unroll
-              for (int r = 0; r < 16; ++r) sum[r] += v[r];
-            }
-          }
-          acc[i][j] = sum;
-        }
-    }
+    if (kt1 - kt0 != KT && !sum_shares(sk, acc, &s_ticket, tile, KT, p, wave, lane)) continue;
     gemm_tile_epilogue<BM, BN, LDS_BYTES, WGN>(a, acc, lds, m0, n0, wave, lane, 0, nullptr);
   }
 }

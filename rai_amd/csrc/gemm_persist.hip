@@ -227,88 +227,6 @@ __device__ __forceinline__ void write_rows(const LinearArgs &a, Acc acc, float *
   }
 }
 
-// A tile that two or three blocks share (see StreamKArgs).  Slot layout [wave][accumulator register][lane]: one store or
-// load instruction covers 256 consecutive bytes.  The shares cross XCDs, whose L2s are not coherent with each other: they
-// are written and read with device-scope accesses (write-through stores, loads that miss L2) instead of a release /
-// acquire fence pair, which would write back and invalidate a whole L2 each and, issued by every block of an XCD at about
-// the same time, queue up behind one another (measured: +130 us per launch).
-// Two counters per tile: `arrived` hands out tickets when a share has been computed, `stored` counts the shares that have
-// reached memory.  The block with the last ticket keeps its share in registers and sums, in slot order, so that the result
-// does not depend on who was last; the others store theirs.  Its wait is for blocks that already hold a ticket, i.e. are
-// running and have nothing left to do but their stores, and it is bounded all the same.  True: this block writes the tile.
-__device__ __forceinline__ bool sum_shares(const StreamKArgs &sk, Acc acc, int *ticket, int tile, int stages, int p, int wave) {
-  const int lane = lane_again();
-  const int first = sk_block_of(sk, tile * stages), last = sk_block_of(sk, tile * stages + stages - 1);
-  const int parts = last - first + 1, slot = p - first;
-  float *tile_ws = sk.ws + (int64_t)tile * sk.max_parts * (kTileDim * kTileDim) + wave * (kMT * kNT * 4 * 64) + lane;
-  int *arrived = sk.counters + 2 * tile, *stored = arrived + 1;
-  __syncthreads();   // the staging area, which holds the ticket, is free
-  if (threadIdx.x == 0) *ticket = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __syncthreads();
-  if (*ticket != parts - 1) {
-    float *mine = tile_ws + (int64_t)slot * (kTileDim * kTileDim);
-#pragma unroll
-    for (int i = 0; i < kMT; ++i)
-#pragma unroll
-      for (int j = 0; j < kNT; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          __hip_atomic_store(mine + ((i * kNT + j) * 4 + r) * 64, acc[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's share has left for memory
-    __syncthreads();
-    if (threadIdx.x == 0 && tile != sk.drop_tile) __hip_atomic_fetch_add(stored, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return false;
-  }
-  __syncthreads();   // every wave has read the ticket
-  if (threadIdx.x == 0) {
-    bool complete = false;
-    for (int spin = 0; spin < sk.spin_limit && !complete; ++spin) {
-      complete = __hip_atomic_load(stored, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
-      if (!complete) __builtin_amdgcn_s_sleep(2);
-    }
-    if (complete) {
-      __hip_atomic_store(arrived, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(stored, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-      // A share is missing.  Nothing is summed and nothing written for this tile, the counters stay as they are (a late
-      // block may still count itself in; the host zeroes them all before the next launch), and the host learns of it at
-      // its next synchronisation.
-      __hip_atomic_store(sk.fault, (int)RAI_FAULT_STREAMK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    *ticket = complete;
-  }
-  __syncthreads();
-  const bool complete = *ticket != 0;
-  __syncthreads();   // before the staging area is written
-  if (!complete) return false;
-#pragma unroll
-  for (int i = 0; i < kMT; ++i)
-#pragma unroll
-    for (int j = 0; j < kNT; ++j) {
-      f32x4 sum = acc[i][j];
-      for (int s = 0; s < parts; ++s) {
-        if (s == slot) {
-          if (s > 0) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sum[r] += acc[i][j][r];
-          }
-          continue;
-        }
-        const float *src = tile_ws + (int64_t)s * (kTileDim * kTileDim) + ((i * kNT + j) * 4) * 64;
-        f32x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = __hip_atomic_load(src + r * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (s == 0) sum = v;
-        else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) sum[r] += v[r];
-        }
-      }
-      acc[i][j] = sum;
-    }
-  return true;
-}
-
 // Tile rows lie in LDS as in dma_tile_mainloop_k64 (gemm_mfma.hip): 128 bytes, 16-byte chunk c of row r at c ^ ((r >> 1) & 7).
 // SHARED: some tiles are shared out.
 template <int OUT, bool SHARED> __global__ void __launch_bounds__(kThreads) k_gemm_bf16_mfma_persist(LinearArgs a, StreamKArgs sk) {
@@ -463,7 +381,7 @@ template <int OUT, bool SHARED> __global__ void __launch_bounds__(kThreads) k_ge
     char *mine = reinterpret_cast<char *>(staging + wave * kStagingFloats);
     bool write = true;
     if (SHARED && seg.n != stages) {
-      write = sum_shares(sk, acc, reinterpret_cast<int *>(staging), seg.tile, stages, p, wave);
+      write = sum_shares(sk, acc, reinterpret_cast<int *>(staging), seg.tile, stages, p, wave, lane_again());
       if (write && OUT != kRows) {
         ask_for(a, mine, m0, n0);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
