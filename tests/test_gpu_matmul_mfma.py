@@ -65,7 +65,8 @@ def test_large_tiles(R, dt, b_t):
 @pytest.mark.parametrize("batch,m,n", [(3, 70, 61), (130, 255, 241)])
 @pytest.mark.parametrize("k", [4, 9, 32, 40, 41, 63, 64, 65, 80, 95, 96, 97, 128, 129, 160, 161, 193])
 def test_every_length_of_k_that_changes_the_form(R, dt, a_t, b_t, batch, m, n, k):
-    """K up to each size of a single stage and one beyond, in 64 x 64 and in 128 x 128 tiles; what lies around the operands is NaN."""
+    """K up to each size of a single stage (64, 96 and 128 of 16 bits, 32, 48 and 64 of f32) and beyond, in two stages; a few tiles and
+    three thousand; what lies around the operands is NaN."""
     g = np.random.Generator(np.random.PCG64(k))
     a, b = rand(g, (3, m, k), dt), rand(g, (3, k, n), dt)
     pad = lambda x: np.pad(x, ((0, 0), (1, 1), (3, 3)), constant_values=np.nan)  # noqa: E731
