@@ -287,6 +287,12 @@ __device__ __forceinline__ bool sum_shares(const StreamKArgs &sk, V (&acc)[MT][N
 // written (gemm_persist.hip); sk: which of them are shared out by K tile (sk_tiles == 0: none).
 // It addresses the rows of a tile by 32-bit offsets: of bytes in the operands, 256 rows, and of elements in the outputs, 16 rows.
 inline bool gemm_persist_serves(const LinearArgs &a) { return a.lda < (1 << 22) && a.ldw < (1 << 22) && a.ld1 < (1 << 28) && a.ld2 < (1 << 28); }
+// What its fast way out needs of the product as a whole (a wave has 64 columns of a tile).
+constexpr int kPersistColumns = 64;
+inline bool gemm_persist_plain(const LinearArgs &a) {
+  return rows_store_16(a) && !a.f32_out && !a.bias2 && !(a.residual && (a.bias || a.act >= 0)) && ((uintptr_t)a.bias & 3) == 0 &&
+         (a.n_split == a.N || a.n_split % kPersistColumns == 0) && a.act_from % kPersistColumns == 0 && (!a.glu || (a.N % 16 == 0 && a.act != kActClampedGlu));
+}
 int launch_gemm_bf16_persist(hipStream_t st, const LinearArgs &a, const StreamKArgs &sk);
 
 }  // namespace rai

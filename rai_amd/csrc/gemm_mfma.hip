@@ -996,11 +996,16 @@ template <int NS> static int launch_streamk_blocks(hipStream_t st, const LinearA
 // Whether the 256 x 256 tiles of stages of 64 are those of one block per CU (gemm_persist.hip); otherwise a block has one tile, or stream-K's
 // shares.  Those ask for a stage as soon as the one before the last is let go, all waves at once, and that is worth more where the operands
 // outgrow the memory-side cache of 256 MB and come from HBM again and again.  Measured (us, blocks / one per CU): stream-K 16384 x 1536 x 8960
-// (321 MB) 372, 382, 8032 x 8984 x 8832 (300 MB) 1033, 1065; whole 4318 x 16496 x 10432 (434 MB) 1279, 1324, 3784 x 15064 x 7680 (290 MB) 751, 773,
-// 4426 x 6392 x 12544 (271 MB) 608, 620.  From 200 MB on either may be ahead (8803 x 5064 x 7744, 215 MB, 560, 543; 16384 x 1536 x 6144, 220 MB, by
+// (321 MB) 378, 386, 8032 x 8984 x 8832 (300 MB) 1019, 1051; whole 4318 x 16496 x 10432 (434 MB) 1269, 1277, 3784 x 15064 x 7680 (290 MB) 745, 760,
+// 4426 x 6392 x 12544 (271 MB) 601, 611.  From 200 MB on either may be ahead (8803 x 5064 x 7744, 215 MB, 560, 543; 16384 x 1536 x 6144, 220 MB, by
 // stream-K 260, 267), below one per CU is (4096 x 4096 x 12288 312, 289; 8192 x 7168 x 4096 397, 370).
+//   With a residual one per CU has no such loss: a block's epilogue waits for its rows, there they are on their way (the same products 390,
+// 386; 1066, 1074; 1325, 1313; 780, 771; 625, 620).  Behind other work 16384 x 1536 x 8960 is further ahead: four layers of width 1536, 16 x 1024
+// tokens, 6680 us with blocks, 6575 with one per CU.
 constexpr int64_t kPersistBytes = 256 << 20;
-static bool persists(const LinearArgs &a) { return a.K % 64 == 0 && gemm_persist_serves(a) && ((int64_t)a.M + a.N) * a.K * 2 <= kPersistBytes; }
+static bool persists(const LinearArgs &a) {
+  return a.K % 64 == 0 && gemm_persist_serves(a) && (((int64_t)a.M + a.N) * a.K * 2 <= kPersistBytes || (a.residual && gemm_persist_plain(a)));
+}
 
 static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan, int bk) {
   int dev = 0;

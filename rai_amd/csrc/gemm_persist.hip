@@ -19,7 +19,7 @@ namespace rai {
 namespace {
 
 constexpr int kTileDim = 256, kStageK = 64, kWaves = 8, kThreads = 64 * kWaves;
-constexpr int kWM = 128, kWN = 64, kMT = kWM / 16, kNT = kWN / 16;   // a wave's part of the tile, waves 2 x 4, in 16 x 16 pieces
+constexpr int kWM = 128, kWN = kPersistColumns, kMT = kWM / 16, kNT = kWN / 16;   // a wave's part of the tile, waves 2 x 4, in 16 x 16 pieces
 constexpr int kLoads = kTileDim / (8 * kWaves);                     // per wave, stage and operand: 8 rows of 128 bytes each
 constexpr int kStageElems = 2 * kTileDim * kStageK;
 constexpr int kStagingFloats = 16 * kWN;                            // a wave's 16 rows of outputs
@@ -59,12 +59,8 @@ struct Walk {
 // put into the wave's own LDS eight bytes at a time and leave it as 16 bytes of a row.
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 
-// What the fast form needs of the product as a whole; the rest of it goes row by row through store_row8.
+// The fast forms, where gemm_persist_plain() holds; the rest goes row by row through store_row8.
 enum { kRows, kPlain, kPlainResidual };
-__host__ __device__ __forceinline__ bool plain_outputs(const LinearArgs &a) {
-  return rows_store_16(a) && !a.f32_out && !a.bias2 && !(a.residual && (a.bias || a.act >= 0)) && ((uintptr_t)a.bias & 3) == 0 && (a.n_split == a.N || a.n_split % kWN == 0) &&
-         a.act_from % kWN == 0 && (!a.glu || (a.N % 16 == 0 && a.act != kActClampedGlu));
-}
 
 // The wave's 64 biases, or the first 32 rows of its residual, go to its staging area a stage before the outputs are written:
 // ahead of the loads of the next tile, behind which they would wait.
@@ -420,7 +416,7 @@ int launch_gemm_bf16_persist(hipStream_t st, const LinearArgs &a, const StreamKA
   RAI_REQUIRE(dev >= 0 && dev < 64, RAI_ERR_BAD_ARG, "device %d out of range", dev);
   const int tiles = ((a.M + kTileDim - 1) / kTileDim) * ((a.N + kTileDim - 1) / kTileDim);
   const int grid = sk.sk_tiles || tiles >= kNumCU ? kNumCU : (tiles + kXcds - 1) / kXcds * kXcds;
-  const int out = plain_outputs(a) ? a.residual ? kPlainResidual : kPlain : kRows;
+  const int out = gemm_persist_plain(a) ? a.residual ? kPlainResidual : kPlain : kRows;
   if (sk.sk_tiles)
     return out == kPlain ? launch_persist<kPlain, true>(st, a, sk, dev, grid) : out == kRows ? launch_persist<kRows, true>(st, a, sk, dev, grid)
                                                                                              : launch_persist<kPlainResidual, true>(st, a, sk, dev, grid);

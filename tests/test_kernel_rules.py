@@ -93,9 +93,13 @@ int main() {
   a.K = 4064; printf("%d ", persists(a));
   a.K = 4096; a.lda = 1 << 22; printf("%d ", persists(a));
   a.lda = 4096; a.ld1 = 1ll << 28; printf("%d ", persists(a));
-  printf("%d %d %d\\n", persists(product(16384, 16384, 4096)), persists(product(16385, 16384, 4096)), persists(product(1 << 20, 1 << 20, 65536)));
+  printf("%d %d %d ", persists(product(16384, 16384, 4096)), persists(product(16385, 16384, 4096)), persists(product(1 << 20, 1 << 20, 65536)));
+  LinearArgs r = product(16385, 16384, 4096);   // a residual that is asked for ahead, whatever the operands' size
+  r.residual = (void *)64; r.ldr = 16384; printf("%d ", persists(r));
+  r.bias = (void *)64; printf("%d ", persists(r));
+  r.bias = nullptr; r.ldr = 16383; printf("%d\\n", persists(r));
 }""")
-    assert lines == ["1 0 0 0 1 0 0"]
+    assert lines == ["1 0 0 0 1 0 0 1 0 0"]
 
 
 @pytest.mark.parametrize("m,n,k,want", [
