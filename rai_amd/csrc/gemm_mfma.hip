@@ -1002,9 +1002,16 @@ template <int NS> static int launch_streamk_blocks(hipStream_t st, const LinearA
 //   With a residual one per CU has no such loss: a block's epilogue waits for its rows, there they are on their way (the same products 390,
 // 386; 1066, 1074; 1325, 1313; 780, 771; 625, 620).  Behind other work 16384 x 1536 x 8960 is further ahead: four layers of width 1536, 16 x 1024
 // tokens, 6680 us with blocks, 6575 with one per CU.
-constexpr int64_t kPersistBytes = 256 << 20;
-static bool persists(const LinearArgs &a) {
-  return a.K % 64 == 0 && gemm_persist_serves(a) && (((int64_t)a.M + a.N) * a.K * 2 <= kPersistBytes || (a.residual && gemm_persist_plain(a)));
+//   With stream-K's shares, which begin at different columns of K and so share less in the L2s, the line lies earlier, unless two whole rounds
+// follow (us, blocks / one per CU): 1.5 rounds, 16384 x 1536 x 4608 (165 MB) 199, 200, x 5632 (202 MB) 235, 242, x 6144 258,
+// 267, x 7168 304, 312, 8192 x 3072 x 8192 (185 MB) 320, 305, x 9216 (208 MB) 358, 366, x 10240 401, 418, 4096 x 6144 x 8192 (168 MB) 320, 304,
+// x 10240 393, 393, x 12288 (252 MB) 471, 478; 2.5 rounds, 4096 x 10240 x 7168 (206 MB) 462, 463, x 8192 (235 MB) 526, 518.  With new_gelu x 1536 x 5632 249,
+// 250, 8192 x 3072 x 9216 374, 378, x 10240 417, 426.
+constexpr int64_t kPersistBytes = 256 << 20, kPersistShareBytes = 192 << 20;
+static bool persists(const LinearArgs &a, bool shares = false) {
+  const bool few = ((a.M + 255) / 256) * ((a.N + 255) / 256) < 2 * kNumCU;   // (shares and less than two whole rounds)
+  return a.K % 64 == 0 && gemm_persist_serves(a) &&
+         (((int64_t)a.M + a.N) * a.K * 2 <= (shares && few ? kPersistShareBytes : kPersistBytes) || (a.residual && gemm_persist_plain(a)));
 }
 
 static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan, int bk) {
@@ -1023,7 +1030,7 @@ static int launch_streamk(hipStream_t st, const LinearArgs &a, StreamKPlan plan,
     if (sscanf(t, "%d,%d", &lim, &tile) == 2 && lim > 0) { plan.k.spin_limit = lim; plan.k.drop_tile = tile; }
   }
   if (bk == 32) return launch_streamk_blocks<4>(st, a, plan.k, dev);
-  return persists(a) ? launch_gemm_bf16_persist(st, a, plan.k) : launch_streamk_blocks<2>(st, a, plan.k, dev);
+  return persists(a, true) ? launch_gemm_bf16_persist(st, a, plan.k) : launch_streamk_blocks<2>(st, a, plan.k, dev);
 }
 
 // ---- small M (9..64 rows): weight streaming through 16x16x32 MFMA -----------------------
@@ -1614,7 +1621,7 @@ static bool has_huge_tiles(const LinearArgs &a) { return 32 * (((a.M + 255) / 25
 // leaves a last round nearly empty: 1200 x 16384 x 2048 108 to 97 us, 3000 x 4096 x 4096 105 to 88, 777 x 22528 x 2048 114 to 91.
 // Whole 256 x 256 tiles on one block per CU that keeps its pipeline full from tile to tile (gemm_persist.hip; persists()) cost kPersistEnd
 // besides (over 320 products with 100 such tiles and more what is picked takes 0.4 % more than the best in the mean, 1.2 % by the
-// figure of a block per tile).  K of an odd number of 32s, K parts and operands that no cache holds are blocks' work.
+// figure of a block per tile).  K of an odd number of 32s, K parts and, without a residual, operands that no cache holds are blocks' work.
 enum { kTile128 = 0, kTile128x64, kTile64, kTile128x256, kTile256x192, kTile192x256, kTile256, kTileStreamK };
 struct TileCost { int bm, bn, share; float stage[3], end, cut; };
 static const TileCost kTileCosts[] = {{128, 128, 1, {0.482f}, 3.24f, 1.46f}, {128, 64, 2, {0.36f, 0.568f}, 2.02f, 0.929f}, {64, 64, 3, {0.256f, 0.382f, 0.614f}, 0.81f, 0.428f},
@@ -1636,7 +1643,7 @@ static float streamk_us(const LinearArgs &a) {
   if (!has_huge_tiles(a) || tiles % kNumCU != kNumCU / 2 || a.K / 64 % 2 || !streamk_applies(a, 64, &plan)) return 0.f;
   const bool persist = persists(a);
   const float multiply = kTileCosts[kTile256].stage[0] * ((float)a.K / 64), end = kTileCosts[kTile256].end;
-  const float shared = (end + multiply) * ((float)tiles / kNumCU) + (persist ? kPersistShareUs : kShareUs);
+  const float shared = (end + multiply) * ((float)tiles / kNumCU) + (persists(a, true) ? kPersistShareUs : kShareUs);
   return shared < ((persist ? kPersistEnd : end) + multiply) * ((tiles + kNumCU - 1) / kNumCU) ? kLaunchUs + shared : 0.f;
 }
 // With K stages of 32 (K no multiple of 64) whole 256 x 256 tiles are all there is beside it, and any shares pay where the CU time saved

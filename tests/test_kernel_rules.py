@@ -102,11 +102,25 @@ int main() {
     assert lines == ["1 0 0 0 1 0 0 1 0 0"]
 
 
+def test_which_shares_go_from_tile_to_tile(tmp_path):
+    """From 192 MB of operands on shares that fewer than two whole rounds follow are blocks' again, unless a residual is asked for ahead."""
+    lines = run(tmp_path, RULES + """
+static int shares(LinearArgs a) { return 10 * persists(a) + persists(a, true); }
+int main() {
+  printf("%02d %02d %02d %02d ", shares(product(16384, 1536, 4608)), shares(product(16384, 1536, 5632)), shares(product(16384, 1536, 7168)), shares(product(16384, 1536, 8960)));
+  printf("%02d %02d %02d ", shares(product(8192, 3072, 8192)), shares(product(8192, 3072, 10240)), shares(product(4096, 10240, 8192)));
+  LinearArgs r = product(16384, 1536, 6144);
+  r.residual = (void *)64; r.ldr = 1536; printf("%02d ", shares(r));
+  r.K = 8960; printf("%02d\\n", shares(r));
+}""")
+    assert lines == ["11 10 10 00 11 10 11 11 11"]
+
+
 @pytest.mark.parametrize("m,n,k,want", [
     # K an odd number of 32s: 256 x 256 tiles are a block's each and cost as much
     (4397, 19664, 288, "192x256"), (14470, 5768, 224, "192x256"), (16384, 8960, 1504, "256x256k64"),
     # a half-full last round: shares, whole 256 x 256 tiles, others
-    (16384, 1536, 8960, "streamk64"), (4096, 6144, 4096, "streamk64"), (2827, 24480, 2048, "256x256k64"), (16384, 17920, 1536, "256x256k64"),
+    (16384, 1536, 8960, "streamk64"), (16384, 1536, 6144, "streamk64"), (4096, 6144, 4096, "streamk64"), (2827, 24480, 2048, "256x256k64"), (16384, 17920, 1536, "256x256k64"),
     (1341, 16320, 3584, "192x256"), (5900, 3936, 3840, "192x256")])
 def test_tile_of_a_product(tmp_path, m, n, k, want):
     assert run(tmp_path, RULES + f'int main() {{ puts(tile({m}, {n}, {k})); }}') == [want]
