@@ -366,8 +366,9 @@ __device__ __forceinline__ void dma_tile_mainloop(const LinearArgs &a, uint16_t 
 //     rows span the 64 banks) land on 16 different 16-byte slots.  (Swizzling by r & 7 left rows r and r + 8 on the
 //     same banks: SQ_LDS_BANK_CONFLICT at 23 % of the kernel's cycles.)
 //   - fragment sets alternate F0 / F1 over the four K steps of a stage; the reads run one set ahead of the multiplies.
-//   - `half`: stage 0 begins 32 before the operands' rows do, and reads zeros there (K of an odd number of 32s).  The first stage and
-//     not the last: it is asked for outside the loop, which then is the same.
+//   - `half`: stage 0 begins 32 before the operands' rows do, and reads zeros there (K of an odd number of 32s: ODD, kernels of their own).
+//     The first stage and not the last: it is asked for outside the loop, which need not know.  (With both ways to ask in one kernel the loop
+//     of 128 x 256 tiles came out in another order: 1024 x 8192 x 8192 131.6 us, so 130.0; the other tiles' times are the same.)
 static __device__ uint4 g_k_zeros[1];   // (sixteen bytes that nobody writes)
 template <int BM, int BN, int WGN, int WGM = 2, int NS = 2>
 __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint16_t *lds, int m0, int n0, int k_begin, int KT,
@@ -510,7 +511,7 @@ __device__ __forceinline__ void dma_tile_mainloop_k64(const LinearArgs &a, uint1
   __syncthreads();
 }
 
-template <int BM, int BN, int NS, int SH, int WGN = 2, int WGM = 2>
+template <int BM, int BN, int NS, int SH, int WGN, int WGM, bool ODD>
 __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArgs a, int longer, int k_per_split, float *partial) {
   // block = 2 x WGN waves.  WGN = 4 (eight waves, wave tile (BM/2) x (BN/4)) keeps two waves on every SIMD: one
   // multiplies while the other sits in its wait for the next tile, and twice as many waves issue loads.
@@ -532,13 +533,13 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArg
     k_span += split < longer ? 64 : 0;
   }
   // (stages of 64: K in whole stages, of which the first may begin 32 before it)
-  const int early = SH == 0 ? a.K & 32 : 0;
+  constexpr int early = SH == 0 && ODD ? 32 : 0;
   const int k_end = k_begin + k_span < a.K + early ? k_begin + k_span : a.K + early;
   const int KT = (k_end - k_begin) / BK;
 
   f32x16 acc[BM / (32 * WGM)][BN / (32 * WGN)];
   if constexpr (SH == 0) {   // stages of 64 (the launcher sends splits of whole stages here)
-    dma_tile_mainloop_k64<BM, BN, WGN, WGM, NS>(a, lds, m0, n0, k_begin - early, KT / 2, wave, lane, acc, early && split == 0);
+    dma_tile_mainloop_k64<BM, BN, WGN, WGM, NS>(a, lds, m0, n0, k_begin - early, KT / 2, wave, lane, acc, ODD && split == 0);
   } else {
     static_assert(WGM == 2, "the K-32 loop is written for two waves along M");
     dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, k_begin, KT, wave, lane, acc);
@@ -853,12 +854,12 @@ template <int BM, int BN, int BK, int SH = 0> static int launch_cfg(hipStream_t 
   return RAI_OK;
 }
 
-template <int BM, int BN, int NS, int SH, int WGN = 2, int WGM = 2>
-static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
+template <int BM, int BN, int NS, int SH, int WGN, int WGM, bool ODD>
+static int launch_cfg_dma_k(hipStream_t st, const LinearArgs &a, int splits) {
   constexpr size_t lds = dma_lds_bytes<BM, BN, NS, WGN, WGM, SH>();
   static bool attr_set = false;
   if (lds > 64 * 1024 && !attr_set) {
-    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_gemm_bf16_mfma_dma<BM, BN, NS, SH, WGN, WGM>,
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_gemm_bf16_mfma_dma<BM, BN, NS, SH, WGN, WGM, ODD>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_set = true;
   }
@@ -866,7 +867,7 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
   const int grid_x = ((tiles + kXcds - 1) / kXcds) * kXcds;
   const int stages = (a.K + 32) / 64;
   int k_per_split = SH == 0 ? stages * 64 : a.K, longer = 0;
-  const int most = stages - (a.K % 64 != 0);   // the part whose first stage begins before the rows has a second one
+  const int most = stages - ODD;   // the part whose first stage begins before the rows has a second one
   if (SH == 0 && splits > most) splits = most;
   if (splits > 1) {
     if constexpr (SH == 0) {   // stages of 64, dealt out evenly
@@ -879,11 +880,17 @@ static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
     }
   }
   float *partial = splits > 1 ? (float *)a.splitk_ws : nullptr;
-  hipLaunchKernelGGL((k_gemm_bf16_mfma_dma<BM, BN, NS, SH, WGN, WGM>), dim3(grid_x, splits), dim3(64 * WGM * WGN), lds, st, a,
+  hipLaunchKernelGGL((k_gemm_bf16_mfma_dma<BM, BN, NS, SH, WGN, WGM, ODD>), dim3(grid_x, splits), dim3(64 * WGM * WGN), lds, st, a,
                      longer, k_per_split, partial);
   RAI_TRY(launch_check("gemm_bf16_mfma_dma"));
   if (splits > 1) RAI_TRY(launch_splitk_epilogue(st, a, splits, (const float *)partial));
   return RAI_OK;
+}
+template <int BM, int BN, int NS, int SH, int WGN = 2, int WGM = 2> static int launch_cfg_dma(hipStream_t st, const LinearArgs &a, int splits) {
+  if constexpr (SH == 0) {
+    if (a.K % 64) return launch_cfg_dma_k<BM, BN, NS, SH, WGN, WGM, true>(st, a, splits);
+  }
+  return launch_cfg_dma_k<BM, BN, NS, SH, WGN, WGM, false>(st, a, splits);
 }
 
 // Arrival counters of the stream-K kernel, one per shared tile; every launch leaves them at zero.
