@@ -532,14 +532,15 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_bf16_mfma_dma(LinearArg
     k_begin += (split < longer ? split : longer) * 64;
     k_span += split < longer ? 64 : 0;
   }
-  // (stages of 64: K in whole stages, of which the first may begin 32 before it)
-  constexpr int early = SH == 0 && ODD ? 32 : 0;
+  // (stages of 64: K in whole stages, of which the first may begin 32 before it; ODD: 32, but with the constant small products take 0.1 to
+  // 0.2 us more, 500 x 1000 x 992 8.6, 8.9)
+  const int early = SH == 0 && ODD ? a.K & 32 : 0;
   const int k_end = k_begin + k_span < a.K + early ? k_begin + k_span : a.K + early;
   const int KT = (k_end - k_begin) / BK;
 
   f32x16 acc[BM / (32 * WGM)][BN / (32 * WGN)];
   if constexpr (SH == 0) {   // stages of 64 (the launcher sends splits of whole stages here)
-    dma_tile_mainloop_k64<BM, BN, WGN, WGM, NS>(a, lds, m0, n0, k_begin - early, KT / 2, wave, lane, acc, ODD && split == 0);
+    dma_tile_mainloop_k64<BM, BN, WGN, WGM, NS>(a, lds, m0, n0, k_begin - early, KT / 2, wave, lane, acc, early && split == 0);
   } else {
     static_assert(WGM == 2, "the K-32 loop is written for two waves along M");
     dma_tile_mainloop<BM, BN, NS, SH, WGN>(a, lds, m0, n0, k_begin, KT, wave, lane, acc);
