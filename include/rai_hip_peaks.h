@@ -32,7 +32,7 @@ typedef enum rai_hip_peak_kind {
 int rai_hip_measure_peak(int dev, int32_t kind, int64_t bytes, int32_t launches, double *seconds_per_launch,
                          double *work_per_launch);
 
-/* The tile that a bf16 Linear of m > 64 rows, n columns and k % 64 == 0 takes on `dev` with `scratch_bytes` of scratch lent to it, under
+/* The tile that a bf16 Linear of m > 64 rows, n columns and k % 64 == 0, without a residual, takes on `dev` with `scratch_bytes` of scratch lent to it, under
  * the name that RAI_HIP_GEMM_TILE has for it, and the parts that K is cut into.  rai_hip_linear lends 32 m n bytes, at
  * most 256 MiB.  Launches nothing. */
 int rai_hip_linear_plan(int dev, int32_t m, int32_t k, int32_t n, size_t scratch_bytes, char *tile, size_t tile_len,
