@@ -1,6 +1,8 @@
 // What the bf16 tile kernels (gemm_mfma.hip, gemm_persist.hip) share: tile order, activations of bf16 outputs, the
 // shares of stream-K.
 #pragma once
+#include <type_traits>
+
 #include "gemm.h"
 
 namespace rai {
@@ -63,6 +65,24 @@ __device__ __forceinline__ void act_n(int act, float (&x)[N], int n, int from) {
 #undef RAI_ACT_CASE
 }
 __device__ __forceinline__ void act8(int act, float (&x)[8], int n, int from) { act_n<8>(act, x, n, from); }
+// The same by the library's functions.
+template <int N>
+__device__ __forceinline__ void act_exact(int act, float (&x)[N], int n, int from) {
+#define RAI_ACT_CASE(K)                            \
+  case K:                                          \
+    _Pragma("unroll") for (int e = 0; e < N; ++e)  \
+      if (n + e >= from) x[e] = act_eval(K, x[e]); \
+    break;
+  switch (act) {
+    RAI_ACT_CASE(RAI_UN_GELU)
+    RAI_ACT_CASE(RAI_UN_NEW_GELU)
+    RAI_ACT_CASE(RAI_UN_SILU)
+    RAI_ACT_CASE(RAI_UN_RELU)
+    RAI_ACT_CASE(RAI_UN_TANH)
+    default: break;
+  }
+#undef RAI_ACT_CASE
+}
 __device__ __forceinline__ void unpack8(const u32x4 &p, float (&f)[8]) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) f[e] = bf16_bits_to_f32((uint16_t)(p[e >> 1] >> (16 * (e & 1))));
@@ -182,6 +202,23 @@ __device__ __forceinline__ void store_row8(const LinearArgs &a, const f32x4 v0, 
   }
 }
 
+// 16 bytes to or from memory past the (per-XCD, mutually incoherent) L2s: for data that another block of the same
+// launch reads or wrote (p is 16-byte aligned)
+__device__ __forceinline__ void store_f32x4_device(float *p, f32x4 v) {
+  unsigned long long *q = reinterpret_cast<unsigned long long *>(p);
+  __hip_atomic_store(q, (unsigned long long)__float_as_uint(v.x) | ((unsigned long long)__float_as_uint(v.y) << 32), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, (unsigned long long)__float_as_uint(v.z) | ((unsigned long long)__float_as_uint(v.w) << 32), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f32x4 load_f32x4_device(const float *p) {
+  const unsigned long long *q = reinterpret_cast<const unsigned long long *>(p);
+  const unsigned long long lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return f32x4{__uint_as_float((uint32_t)lo), __uint_as_float((uint32_t)(lo >> 32)), __uint_as_float((uint32_t)hi),
+               __uint_as_float((uint32_t)(hi >> 32))};
+}
+
 struct StreamKArgs {
   int sk_tiles;   // tiles 0 .. sk_tiles-1 are shared out by K tile; the rest run whole
   int q, rem;     // units per block: blocks 0 .. rem-1 take q + 1, the others q
@@ -294,5 +331,12 @@ inline bool gemm_persist_plain(const LinearArgs &a) {
          (a.n_split == a.N || a.n_split % kPersistColumns == 0) && a.act_from % kPersistColumns == 0 && (!a.glu || (a.N % 16 == 0 && a.act != kActClampedGlu));
 }
 int launch_gemm_bf16_persist(hipStream_t st, const LinearArgs &a, const StreamKArgs &sk);
+
+// The arrival counters of a device's K splits, zero between launches (null: device unknown).
+constexpr int kSplitTickets = 16384;
+int *splitk_tickets(const LinearArgs &a);
+// The streaming form for 9 to 32 rows on fragments (gemm_stream.hip).
+bool linear_stream_serves(const LinearArgs &a);
+int launch_linear_bf16_stream(hipStream_t st, const LinearArgs &a);
 
 }  // namespace rai

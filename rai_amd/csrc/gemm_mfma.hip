@@ -975,11 +975,15 @@ static int *streamk_counters_of(int dev) {
 // Tickets of the small-M streaming Linear's K split, one per group of weight tiles; zero between launches (the block
 // that takes a group's last ticket puts it back).  Launches that overlap on one GPU would share them: the library
 // runs a device's work on one stream.
-constexpr int kSplitTickets = 16384;
 static __device__ int g_splitk_tickets[kSplitTickets];
 static int *splitk_tickets_of(int dev) {
   static int *tickets[64];
   return device_ints_of(dev, tickets, HIP_SYMBOL(g_splitk_tickets));
+}
+
+int *splitk_tickets(const LinearArgs &a) {
+  int dev = -1;
+  return linear_device(a, &dev) == RAI_OK ? splitk_tickets_of(dev) : nullptr;
 }
 
 int streamk_counters_reset(int dev, hipStream_t st) {
@@ -1222,23 +1226,6 @@ int launch_linear_fragment_layout(hipStream_t st, const void *W, int64_t ldw, in
   hipLaunchKernelGGL(k_linear_fragment_layout, dim3((unsigned)(blocks < 65535 ? blocks : 65535)), dim3(256), 0, st,
                      (bf16x8 *)Wfrag, (const uint16_t *)W, ldw, N, K / 32, total);
   return launch_check("linear_fragment_layout");
-}
-
-// 16 bytes to or from memory past the (per-XCD, mutually incoherent) L2s: for data that another block of the same
-// launch reads or wrote (p is 16-byte aligned)
-__device__ __forceinline__ void store_f32x4_device(float *p, f32x4 v) {
-  unsigned long long *q = reinterpret_cast<unsigned long long *>(p);
-  __hip_atomic_store(q, (unsigned long long)__float_as_uint(v.x) | ((unsigned long long)__float_as_uint(v.y) << 32), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(q + 1, (unsigned long long)__float_as_uint(v.z) | ((unsigned long long)__float_as_uint(v.w) << 32), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ f32x4 load_f32x4_device(const float *p) {
-  const unsigned long long *q = reinterpret_cast<const unsigned long long *>(p);
-  const unsigned long long lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const unsigned long long hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return f32x4{__uint_as_float((uint32_t)lo), __uint_as_float((uint32_t)(lo >> 32)), __uint_as_float((uint32_t)hi),
-               __uint_as_float((uint32_t)(hi >> 32))};
 }
 
 // F32O: the f32 output of LinearArgs::f32_out (fragment-order weights only; a branch in the bf16 form costs it 1 %)
@@ -1563,10 +1550,7 @@ static int launch_mfma_stream_cfg(hipStream_t st, const LinearArgs &a, int split
   // launch) when the tickets reach and the partial rows are 16-byte aligned; RAI_HIP_NO_FUSED_SPLITK=1 keeps the
   // separate summing pass (the tests compare the two: same bits).
   int *tickets = nullptr;
-  if (splits > 1 && groups <= kSplitTickets && a.N % 4 == 0 && ((uintptr_t)partial & 15) == 0 && !getenv("RAI_HIP_NO_FUSED_SPLITK")) {
-    int dev = -1;
-    if (linear_device(a, &dev) == RAI_OK) tickets = splitk_tickets_of(dev);
-  }
+  if (splits > 1 && groups <= kSplitTickets && a.N % 4 == 0 && ((uintptr_t)partial & 15) == 0 && !getenv("RAI_HIP_NO_FUSED_SPLITK")) tickets = splitk_tickets(a);
   hipLaunchKernelGGL((k_linear_bf16_mfma_stream<MT, KS, G, FRAG, F32O>), dim3(blocks_x, splits), dim3(512), lds, st, a, tiles,
                      partial, tickets);
   RAI_TRY(launch_check("linear_bf16_mfma_stream"));
@@ -1839,6 +1823,7 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
       !no_skinny && !no_stream && (wide || deep))
     return launch_tile_k64(st, a, tile_plan_k64(a));
   if (a.M <= 64 && !no_skinny && !no_stream && (!a.f32_out || a.Wfrag)) {
+    if (linear_stream_serves(a)) return launch_linear_bf16_stream(st, a);
     int splits = 1;
     if (a.M <= 16 && mfma_stream_fits<1, 8>(a, &splits)) return launch_mfma_stream<1, 8>(st, a, splits);
     if (a.M > 16 && a.M <= 32 && mfma_stream_fits<2, 8>(a, &splits)) return launch_mfma_stream<2, 8>(st, a, splits);
