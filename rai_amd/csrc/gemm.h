@@ -125,6 +125,11 @@ int launch_gemv_group(hipStream_t st, GemvGroupArgs g);
 // where M x N alone leaves CUs idle, of `room` bytes at most; with less it cuts K less.
 int launch_linear_f32(hipStream_t st, const LinearArgs &a);
 size_t linear_f32_workspace_bytes(const LinearArgs &a, size_t room);
+// The streaming form for 2 to 32 rows (gemm_stream.hip), what it takes and where it is the fastest, and the scratch with which it also takes a K that it has to cut (0: none).
+bool linear_stream_serves(const LinearArgs &a);
+bool linear_stream_pays(const LinearArgs &a);
+size_t linear_stream_workspace_bytes(const LinearArgs &a);
+int launch_linear_bf16_stream(hipStream_t st, const LinearArgs &a);
 bool linear_mfma_fuses_norm(int M, int K, int ln_kind);
 
 // out[z] = A[z] B[z] (rai_hip_matmul), out contiguous.

@@ -738,6 +738,7 @@ int launch_linear_dual_row(hipStream_t st, int dev, const void *x1, int K1, cons
 }
 
 int launch_linear_bf16(hipStream_t st, const LinearArgs &a) {
+  if (linear_stream_serves(a) && linear_stream_pays(a)) return launch_linear_bf16_stream(st, a);
   if (a.M <= 8 && a.ln_kind < 0 && !a.K2) {
     RAI_TRY(check_linear_args(a, 2));
     if (a.glu) RAI_REQUIRE(a.N % 2 == 0 && !a.residual && a.n_split == a.N && a.act >= 0, RAI_ERR_BAD_ARG, "linear: bad gated-MLP arguments");
@@ -812,7 +813,8 @@ template <typename T> static void launch_transpose_2d(hipStream_t st, T *dst, co
 // all with what there is.  The caller keeps `hold` until the product's last kernel is enqueued.
 static void splitk_workspace(int dev, int dtype, LinearArgs *la, WorkspaceHold *hold) {
   const size_t cap = (size_t)256 << 20;
-  size_t want = dtype == RAI_F32 ? linear_f32_workspace_bytes(*la, cap) : (size_t)8 * la->M * la->N * sizeof(float);
+  size_t want = dtype == RAI_F32 ? linear_f32_workspace_bytes(*la, cap) : la->M > 8 ? (size_t)8 * la->M * la->N * sizeof(float) : 0;
+  if (dtype == RAI_BF16) want = std::max(want, linear_stream_workspace_bytes(*la));
   if (want > cap) want = cap;
   if (want) la->splitk_ws_bytes = workspace_if_room(dev, want, &la->splitk_ws, hold);
 }
@@ -883,7 +885,7 @@ int rai_hip_matmul(int dev, const rai_hip_tensor *a, const rai_hip_tensor *b, co
       la.n_split = (int)N;
       if (a->dtype == RAI_BF16 && la.M > 8 && la.K % 32 != 0) goto generic;
       WorkspaceHold hold;
-      if (a->dtype == RAI_F32 || la.M > 8) splitk_workspace(dev, a->dtype, &la, &hold);
+      splitk_workspace(dev, a->dtype, &la, &hold);
       return a->dtype == RAI_BF16 ? launch_linear_bf16(st, la) : launch_linear_f32(st, la);
     }
   }
@@ -998,7 +1000,7 @@ int rai_hip_linear(int dev, const rai_hip_tensor *x, const rai_hip_tensor *w, co
   if (x->dtype == RAI_BF16 && la.M > 8)
     RAI_REQUIRE(K % 32 == 0, RAI_ERR_UNSUPPORTED, "linear: bf16 with M > 8 needs K %% 32 == 0 (K=%lld)", (long long)K);
   WorkspaceHold hold;
-  if (x->dtype == RAI_F32 || la.M > 8) splitk_workspace(dev, x->dtype, &la, &hold);
+  splitk_workspace(dev, x->dtype, &la, &hold);
   return x->dtype == RAI_BF16 ? launch_linear_bf16(st, la) : launch_linear_f32(st, la);
 }
 

@@ -335,8 +335,5 @@ int launch_gemm_bf16_persist(hipStream_t st, const LinearArgs &a, const StreamKA
 // The arrival counters of a device's K splits, zero between launches (null: device unknown).
 constexpr int kSplitTickets = 16384;
 int *splitk_tickets(const LinearArgs &a);
-// The streaming form for 9 to 32 rows on fragments (gemm_stream.hip).
-bool linear_stream_serves(const LinearArgs &a);
-int launch_linear_bf16_stream(hipStream_t st, const LinearArgs &a);
 
 }  // namespace rai

@@ -1823,7 +1823,6 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
       !no_skinny && !no_stream && (wide || deep))
     return launch_tile_k64(st, a, tile_plan_k64(a));
   if (a.M <= 64 && !no_skinny && !no_stream && (!a.f32_out || a.Wfrag)) {
-    if (linear_stream_serves(a)) return launch_linear_bf16_stream(st, a);
     int splits = 1;
     if (a.M <= 16 && mfma_stream_fits<1, 8>(a, &splits)) return launch_mfma_stream<1, 8>(st, a, splits);
     if (a.M > 16 && a.M <= 32 && mfma_stream_fits<2, 8>(a, &splits)) return launch_mfma_stream<2, 8>(st, a, splits);

@@ -1,4 +1,4 @@
-// bf16 Linears of 9 to 32 rows (a batched decode step) on weights in fragment order, by v_mfma_f32_16x16x32_bf16.
+// bf16 Linears of 2 to 32 rows (a batched decode step) by v_mfma_f32_16x16x32_bf16, on weights in fragment order or in rows as they lie.
 #include "gemm_device.h"
 
 namespace rai {
@@ -7,8 +7,8 @@ typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 
 constexpr int kPastL2 = 17;   // cache policy bits sc0 and sc1: past the (per-XCD, mutually incoherent) L2s
 
-// A block's eight waves take the K steps of 32 in turn (step 8 i + wave, i = 0 .. KS - 1) with the activations of theirs in registers for the
-// whole launch; it walks over groups of G tiles of 16 weight rows, RT tiles on their way, and the eight partial sums of an output meet in LDS.
+// A block's eight waves take the K steps of 32 in turn (step 8 i + wave, i = 0 .. KS - 1; of rows as they lie, pairs of steps: whole lines) with the
+// activations of theirs in registers for the whole launch; it walks over groups of G tiles of 16 weight rows, RT tiles on their way, and the eight partial sums of an output meet in LDS.
 // K in parts (SPLIT): part s of n takes the eights of steps s, s + n, ...; a block has one group then, its tiles a grid apart, and two
 // blocks share a CU.
 // Bound by the stream of W behind a start (launch, activations, norm) and an end (the sums' way through LDS, with parts through memory) of some
@@ -20,8 +20,11 @@ constexpr int kPastL2 = 17;   // cache policy bits sc0 and sc1: past the (per-XC
 // 1536 x 8960 in five parts 14.1, 10.2; 2048 x 1536 normed 9.1, 6.2.
 // How the blocks' reads lie to each other counts as much: 2048 x 16384 took 21.4 with four neighbouring tiles to a block (each 512 KB), 17.2
 // with two, 16.3 with four a grid apart, but 32768 x 2048 (tiles of 64 KB) 24.8 with two neighbours, 26.5 with two a grid apart, 29 with four neighbours; eights
-// of steps of all tiles side by side 27.1.  A wave's steps in one piece instead of in turn: no difference.
-template <int MT, int KS, int G, bool NORM, bool GLU, bool SPLIT, bool F32O>
+// of steps of all tiles side by side 27.1.  A wave's steps in one piece instead of in turn: no difference.  Rows as they lie take some 13 %
+// more than fragments (four rows x 32768 x 2048 normed and gated 22.6, 26).
+// Registers: 128 at two blocks to a CU hold the activations, a tile and the sums of four, if nothing else is live then: uniform addresses, a load
+// behind the multiply whose operand it replaces, first sums on a zero that takes none (with spills 2048 x 16384 took 20.2 us).
+template <int MT, int KS, int G, bool FRAG, bool NORM, bool GLU, bool SPLIT, bool F32O>
 __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(LinearArgs a, int tiles, float *partial, int *tickets) {
   constexpr int NW = 8, RT = G < 2 || SPLIT ? 1 : 2, PCH = 4 * G + 1, ITEMS = MT * G * 64;
   static_assert(ITEMS <= 512 && !(F32O && (NORM || GLU)) && !(SPLIT && (NORM || GLU)), "a thread finishes one piece of a group");
@@ -32,15 +35,24 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lq = lane >> 4;
   const int parts = SPLIT ? gridDim.y : 1, part = SPLIT ? blockIdx.y : 0, ksteps = a.K / 32;
-  auto step_at = [&](int ks) { return (ks * parts + part) * NW + wave; };
-  const int last_step = step_at(KS - 1) < ksteps ? step_at(KS - 1) : 0;   // the others are within K
-  const bool beyond = step_at(KS - 1) >= ksteps;
+  constexpr int RUN = FRAG ? 1 : 2;   // neighbouring steps to a wave; all but the last run are within K
+  static_assert(KS % RUN == 0, "whole runs");
+  auto place = [&](int ks) { return ((ks / RUN * parts + part) * NW + wave) * RUN + ks % RUN; };
+  auto beyond = [&](int ks) { return ks >= KS - RUN && place(ks) >= ksteps; };
+  auto step_at = [&](int ks) { return beyond(ks) ? 0 : place(ks); };
 
   bf16x8 xf[MT][KS], wv[KS], w[RT][KS];
   const uint32_t lane_at = lane * 16;
-  auto load = [&](bf16x8 &dst, int tile, int ks) __attribute__((always_inline)) {   // one instruction reads 1 KB of consecutive memory
-    const char *p = (const char *)a.Wfrag + ((int64_t)(tile < tiles ? tile : tiles - 1) * ksteps + (ks < KS - 1 ? step_at(ks) : last_step)) * 1024;
-    dst = __builtin_nontemporal_load(reinterpret_cast<const bf16x8 *>(p + lane_at));
+  auto load = [&](bf16x8 &dst, int tile, int ks) __attribute__((always_inline)) {
+    tile = tile < tiles ? tile : tiles - 1;
+    if constexpr (FRAG) {   // one instruction reads 1 KB of consecutive memory
+      const char *p = (const char *)a.Wfrag + ((int64_t)tile * ksteps + step_at(ks)) * 1024;
+      dst = __builtin_nontemporal_load(reinterpret_cast<const bf16x8 *>(p + lane_at));
+    } else {                // 64 bytes of sixteen rows, the second half of their lines with the next step: through the caches
+      const char *p = (const char *)a.W + ((int64_t)tile * 16 * a.ldw + step_at(ks) * 32) * 2;
+      const int rows = a.N - tile * 16;   // (addresses as a uniform part and 32 bits of a lane's own: no registers for pairs)
+      dst = *reinterpret_cast<const bf16x8 *>(p + (uint32_t)((lrow < rows ? lrow : rows - 1) * (int)a.ldw + lq * 8) * 2u);
+    }
   };
   const int stride = gridDim.x * G;
   auto tile_at = [&](int g0, int pos) { return SPLIT ? g0 + pos * (int)gridDim.x : pos < G ? g0 + pos : g0 + stride + pos - G; };
@@ -49,13 +61,13 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int m = mt * 16 + lrow;
-    const uint16_t *row = (const uint16_t *)a.A + (int64_t)(m < a.M ? m : a.M - 1) * a.lda + lq * 8;
+    const uint32_t row = (uint32_t)((m < a.M ? m : a.M - 1) * (int)a.lda + lq * 8) * 2u;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) xf[mt][ks] = *reinterpret_cast<const bf16x8 *>(row + (ks < KS - 1 ? step_at(ks) : last_step) * 32);
+    for (int ks = 0; ks < KS; ++ks) xf[mt][ks] = *reinterpret_cast<const bf16x8 *>((const char *)a.A + step_at(ks) * 64 + row);
   }
   if constexpr (NORM) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) wv[ks] = *reinterpret_cast<const bf16x8 *>((const uint16_t *)a.ln_w + (ks < KS - 1 ? step_at(ks) : last_step) * 32 + lq * 8);
+    for (int ks = 0; ks < KS; ++ks) wv[ks] = *reinterpret_cast<const bf16x8 *>((const char *)a.ln_w + step_at(ks) * 64 + lq * 16u);
   }
 #pragma unroll
   for (int pos = 0; pos < RT; ++pos)
@@ -63,13 +75,17 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
     for (int ks = 0; ks < KS; ++ks) load(w[pos][ks], tile_at(g0, pos), ks);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-    if (beyond) xf[mt][KS - 1] = bf16x8{};
+  for (int ks = KS - RUN; ks < KS; ++ks)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      if (beyond(ks)) xf[mt][ks] = bf16x8{};
   if constexpr (NORM) {
     // RMSNorm of the rows (ln_kind 1: x * w / rms, 2: x * (1 + w) / rms).  The fragments take the weight, in f32 and rounded once; the factor
     // 1 / rms is the finished sums', so that no wave waits for another's squares before it multiplies.  Every block norms all rows, so vector
     // instructions count: the squares are the diagonal of X X^T (lane (row, quarter) holds row 4 quarter + r of column `row`).
-    if (beyond) wv[KS - 1] = bf16x8{};   // an infinite weight would make the zeros NaN
+#pragma unroll
+    for (int ks = KS - RUN; ks < KS; ++ks)
+      if (beyond(ks)) wv[ks] = bf16x8{};   // an infinite weight would make the zeros NaN
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       f32x4 xx = {0.f, 0.f, 0.f, 0.f};
@@ -91,8 +107,7 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
     }
   }
   // what a thread finishes: four columns of row m, at column n of a group (ITEMS <= 512)
-  const int item = tid < ITEMS ? tid : 0, m = item / (G * 4), c = item % (G * 4);
-  const bool mine = tid < ITEMS && m < a.M;
+  const int lds_item = tid < ITEMS ? tid : 0;
   float scale = 1.f;
   // columns n .. n + 3 (N is a multiple of 4) and what is added to them
   auto word = [&](const void *p, int64_t at) { return *reinterpret_cast<const u32x2 *>(p ? (const char *)p + at * 2 : (const char *)a.A); };
@@ -102,7 +117,7 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
     if constexpr (F32O) return *reinterpret_cast<const f32x4 *>(a.residual ? (const float *)a.residual + at : (const float *)a.A);
     else return word(a.residual, at);
   };
-  auto finish = [&](int n, f32x4 s, const u32x2 &bv, const u32x2 &bv2, const Residual &rv) __attribute__((always_inline)) {
+  auto finish = [&](int m, int n, f32x4 s, const u32x2 &bv, const u32x2 &bv2, const Residual &rv) __attribute__((always_inline)) {
     float x[4] = {s.x, s.y, s.z, s.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] += (a.bias ? value(bv, e) : 0.f) + (a.bias2 ? value(bv2, e) : 0.f);
@@ -138,14 +153,17 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
   auto group = [&](auto last, const int g0, const bool first) __attribute__((always_inline)) {
     constexpr bool LAST = decltype(last)::value;   // nothing follows: no more loads
     f32x4 acc[G][MT];
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[j][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int n = (tile_at(g0, c >> 2) * 4 + (c & 3)) * 4, n_in = n < a.N ? n : 0, m_in = m < a.M ? m : 0;
+    int item, m, c, n, n_in, m_in;
+    auto whose = [&](int t) {
+      item = t; m = t / (G * 4); c = t % (G * 4);
+      n = (tile_at(g0, c >> 2) * 4 + (c & 3)) * 4;
+      n_in = n < a.N ? n : 0;
+      m_in = m < a.M ? m : 0;
+    };
     u32x2 bv, bv2;
     Residual rv;
     if constexpr (!SPLIT) {   // on their way while the weights are
+      whose(lds_item);
       bv = word(a.bias, n_in);
       bv2 = word(a.bias2, n_in);
       if (!GLU) rv = residual((int64_t)m_in * a.ldr + n_in);
@@ -156,10 +174,16 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j % RT][ks], xf[mt][ks], acc[j][mt], 0, 0, 0);
+        for (int mt = 0; mt < MT; ++mt) acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j % RT][ks], xf[mt][ks], ks ? acc[j][mt] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
         if (!LAST || j + RT < G) load(w[j % RT][ks], tile_at(g0, j + RT), ks);   // (left alone, it would sink to just before its use)
         __builtin_amdgcn_sched_barrier(0);
       }
+    if constexpr (SPLIT) {   // (not before: every register is taken)
+      int t = lds_item;
+      asm volatile("" : "+v"(t));
+      whose(t);
+    }
     // Parked as [row m][G tiles x 4 column quads], a pitch of an odd number of 16-byte chunks: the 16 lanes of a quad, a row each, hit
     // distinct banks; a thread then owns four consecutive columns of one row.
     if (!first) __syncthreads();   // the previous group's sums have been read
@@ -180,9 +204,9 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
       }
       s4 *= scale;
     }
-    const bool on = mine && n < a.N;
+    const bool on = tid < ITEMS && m < a.M && n < a.N;
     if constexpr (!SPLIT) {
-      if (on) finish(n, s4, bv, bv2, rv);
+      if (on) finish(m, n, s4, bv, bv2, rv);
     } else {
       // A block counts itself in once its partial sums have reached memory (past the L2s), and the block that counts last, whichever it is,
       // adds all of them in the order of the parts and finishes.  Nobody waits.
@@ -210,7 +234,7 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
         for (int i = 0; i < 8; ++i)
           if (sp + i < parts) s4 += t[i];
       }
-      finish(n, s4, bv, bv2, rv);
+      finish(m, n, s4, bv, bv2, rv);
     }
   };
   if constexpr (SPLIT) {
@@ -222,37 +246,38 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
   }
 }
 
-template <int MT, int KS, int G, bool NORM, bool GLU, bool SPLIT, bool F32O>
+template <int MT, int KS, int G, bool FRAG, bool NORM, bool GLU, bool SPLIT, bool F32O>
 static int launch_stream(hipStream_t st, const LinearArgs &a, int parts, int *tickets) {
   const int tiles = (a.N + 15) / 16, groups = (tiles + G - 1) / G;
   const size_t lds = (size_t)8 * MT * 16 * ((4 * G + 1) * sizeof(f32x4) + sizeof(float));
   static bool attr_set = false;
   if (lds > 64 * 1024 && !attr_set) {
-    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_linear_bf16_stream<MT, KS, G, NORM, GLU, SPLIT, F32O>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_linear_bf16_stream<MT, KS, G, FRAG, NORM, GLU, SPLIT, F32O>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_set = true;
   }
-  hipLaunchKernelGGL((k_linear_bf16_stream<MT, KS, G, NORM, GLU, SPLIT, F32O>), dim3(SPLIT || groups < kNumCU ? groups : kNumCU, parts), dim3(512), lds, st, a,
+  hipLaunchKernelGGL((k_linear_bf16_stream<MT, KS, G, FRAG, NORM, GLU, SPLIT, F32O>), dim3(SPLIT || groups < kNumCU ? groups : kNumCU, parts), dim3(512), lds, st, a,
                      tiles, (float *)a.splitk_ws, tickets);
   return launch_check("linear_bf16_stream");
 }
-template <int MT, int KS, bool F32O> static int launch_stream_form(hipStream_t st, const LinearArgs &a, int parts, int *tickets) {
+template <int MT, int KS, bool FRAG, bool F32O> static int launch_stream_form(hipStream_t st, const LinearArgs &a, int parts, int *tickets) {
   const int tiles = (a.N + 15) / 16;
   if constexpr (KS >= 6 && KS <= 8) {
     if (parts > 1) {   // one group to a block: as few tiles as two blocks to a CU allow
-      if (tiles * parts <= kNumCU) return launch_stream<MT, KS, 1, false, false, true, F32O>(st, a, parts, tickets);
-      if (tiles * parts <= 2 * kNumCU) return launch_stream<MT, KS, 2, false, false, true, F32O>(st, a, parts, tickets);
-      return launch_stream<MT, KS, 4, false, false, true, F32O>(st, a, parts, tickets);
+      if (tiles * parts <= kNumCU) return launch_stream<MT, KS, 1, FRAG, false, false, true, F32O>(st, a, parts, tickets);
+      if (tiles * parts <= 2 * kNumCU) return launch_stream<MT, KS, 2, FRAG, false, false, true, F32O>(st, a, parts, tickets);
+      return launch_stream<MT, KS, 4, FRAG, false, false, true, F32O>(st, a, parts, tickets);
     }
   }
   auto with = [&](auto g) -> int {
     constexpr int G = decltype(g)::value;
     if constexpr (!F32O) {
       if constexpr (KS <= 8) {
-        if (a.ln_kind > 0) return a.glu ? launch_stream<MT, KS, G, true, true, false, false>(st, a, 1, nullptr) : launch_stream<MT, KS, G, true, false, false, false>(st, a, 1, nullptr);
+        if (a.ln_kind > 0)
+          return a.glu ? launch_stream<MT, KS, G, FRAG, true, true, false, false>(st, a, 1, nullptr) : launch_stream<MT, KS, G, FRAG, true, false, false, false>(st, a, 1, nullptr);
       }
-      if (a.glu) return launch_stream<MT, KS, G, false, true, false, false>(st, a, 1, nullptr);
+      if (a.glu) return launch_stream<MT, KS, G, FRAG, false, true, false, false>(st, a, 1, nullptr);
     }
-    return launch_stream<MT, KS, G, false, false, false, F32O>(st, a, 1, nullptr);
+    return launch_stream<MT, KS, G, FRAG, false, false, false, F32O>(st, a, 1, nullptr);
   };
   return tiles <= kNumCU ? with(std::integral_constant<int, 1>{}) : with(std::integral_constant<int, 2>{});
 }
@@ -265,13 +290,35 @@ static size_t stream_parts_bytes(const LinearArgs &a) { return (size_t)stream_pa
 bool linear_stream_serves(const LinearArgs &a) {
   const int parts = stream_parts(a), piece = a.f32_out ? 16 : 8;
   auto whole = [](const void *p, int n) { return ((uintptr_t)p & (n - 1)) == 0; };
-  if (!a.Wfrag || a.M <= 8 || a.M > 32 || a.K % 32 || a.K <= 24 * 32 || a.N % 4 || a.n_split % 4 || a.ln_kind == 0) return false;
+  if (a.M < 2 || a.M > 32 || a.K % 32 || a.K <= 24 * 32 || a.N % 4 || a.n_split % 4 || a.ln_kind == 0 || a.K2 || a.force_splits > 0) return false;
   if ((a.ln_kind > 0 || a.glu) && (parts > 1 || a.f32_out)) return false;
+  if (!a.Wfrag && (a.ldw % 8 || a.ldw >= 1 << 26 || !whole(a.W, 16))) return false;
+  if (a.lda % 8 || a.lda >= 1 << 25 || !whole(a.A, 16) || (a.ln_kind > 0 && !whole(a.ln_w, 16))) return false;
   if (a.glu ? a.ld1 % 2 || !whole(a.out1, 4) : a.ld1 % 4 || !whole(a.out1, piece)) return false;
   if (a.n_split != a.N && (a.ld2 % 4 || !whole(a.out2, 8))) return false;
   if (!whole(a.bias, 8) || !whole(a.bias2, 8) || (a.residual && (a.ldr % 4 || !whole(a.residual, piece)))) return false;
   return parts == 1 || (a.splitk_ws && whole(a.splitk_ws, 16) && stream_parts_bytes(a) <= a.splitk_ws_bytes && stream_parts_bytes(a) < (1u << 31) &&
                         (a.N + 15) / 16 <= kSplitTickets);
+}
+// Where it is the fastest form.  On fragments and with a fused norm it always is (the latter, of rows as they lie, against k_linear_bf16_skinny, us: 2 rows x
+// 2560 x 2048 9.0, 7.3, x 32768 gated 41, 26.5; 8 rows 21.9, 7.8 and 60, 27).  Else, on rows as they lie, weights from HBM and, in brackets, from the caches
+// where the two disagree: two to four rows are k_linear_bf16_rows's (4 x 8960 x 1536 8.3, 10.1; 4 x 4096 x 4096 9.5, 9.6), which at five to eight
+// loses but for small matrices (8 x 2560 x 2048 7.9, 5.6; 8 x 16384 x 2048 21.0, 14.7; 8 x 1536 x 8960 12.2, 9.6; 8 x 512 x 1536 4.4, 4.5; 8 x
+// 1024 x 4096 6.4, 6.7); 9 to 32 rows, against tiles and the kernel in gemm_mfma.hip: 16 x 2048 x 2048 7.1, 5.9; 16 x 4096 x 1024 7.0, 4.2; 32 x 8960 x
+// 1536 14.6, 11.6; 24 x 2048 x 16384 22.7, 17.6; 24 x 16384 x 2048 19.0, 15.9 (12.5, 14.1); tiles keep wide matrices of ten steps a wave (24 x 10240 x
+// 2560 19.5, 17.3 (12.9, 15.2)) and, beyond 16 rows, large ones in parts (32 x 8192 x 8192 36.4, 38.0 (25.7, 28.5)).
+bool linear_stream_pays(const LinearArgs &a) {
+  const char *off = getenv("RAI_HIP_NO_MFMA_STREAM"), *off2 = getenv("RAI_HIP_NO_MFMA_SKINNY");   // read per call: tests force the other kernels
+  if (off || off2) return false;
+  if (a.Wfrag || a.ln_kind > 0) return true;
+  const int64_t size = (int64_t)a.N * a.K;
+  const bool parts = stream_parts(a) > 1;
+  if (a.M <= 4) return false;
+  if (a.M <= 8) return size >= (parts ? 8 << 20 : 3 << 19);
+  return !(a.M > 16 && parts && size >= 48 << 20) && !(!parts && a.K > 2048 && a.N >= 9000);
+}
+size_t linear_stream_workspace_bytes(const LinearArgs &a) {
+  return a.M > 4 && a.M <= 32 && a.K % 32 == 0 && stream_parts(a) > 1 && linear_stream_pays(a) ? stream_parts_bytes(a) : 0;
 }
 int launch_linear_bf16_stream(hipStream_t st, const LinearArgs &a) {
   const int parts = stream_parts(a), ks = (a.K / 32 + 8 * parts - 1) / (8 * parts);
@@ -283,14 +330,19 @@ int launch_linear_bf16_stream(hipStream_t st, const LinearArgs &a) {
   auto steps = [&](auto mt, auto f32o) -> int {
     constexpr int MT = decltype(mt)::value;
     constexpr bool F = decltype(f32o)::value;
+    if (!a.Wfrag) {   // rows as they lie: pairs of steps
+      if (ks > 8) return launch_stream_form<MT, 10, false, F>(st, a, parts, tickets);
+      if (ks > 6) return launch_stream_form<MT, 8, false, F>(st, a, parts, tickets);
+      return ks > 4 ? launch_stream_form<MT, 6, false, F>(st, a, parts, tickets) : launch_stream_form<MT, 4, false, F>(st, a, parts, tickets);
+    }
     switch (ks) {
-      case 10: return launch_stream_form<MT, 10, F>(st, a, parts, tickets);
-      case 9: return launch_stream_form<MT, 9, F>(st, a, parts, tickets);
-      case 8: return launch_stream_form<MT, 8, F>(st, a, parts, tickets);
-      case 7: return launch_stream_form<MT, 7, F>(st, a, parts, tickets);
-      case 6: return launch_stream_form<MT, 6, F>(st, a, parts, tickets);
-      case 5: return launch_stream_form<MT, 5, F>(st, a, parts, tickets);
-      default: return launch_stream_form<MT, 4, F>(st, a, parts, tickets);
+      case 10: return launch_stream_form<MT, 10, true, F>(st, a, parts, tickets);
+      case 9: return launch_stream_form<MT, 9, true, F>(st, a, parts, tickets);
+      case 8: return launch_stream_form<MT, 8, true, F>(st, a, parts, tickets);
+      case 7: return launch_stream_form<MT, 7, true, F>(st, a, parts, tickets);
+      case 6: return launch_stream_form<MT, 6, true, F>(st, a, parts, tickets);
+      case 5: return launch_stream_form<MT, 5, true, F>(st, a, parts, tickets);
+      default: return launch_stream_form<MT, 4, true, F>(st, a, parts, tickets);
     }
   };
   auto rows = [&](auto mt) -> int { return a.f32_out ? steps(mt, std::integral_constant<bool, true>{}) : steps(mt, std::integral_constant<bool, false>{}); };
