@@ -9,8 +9,8 @@
 // holding positions l * 8 + 512 u.  k_latent_in's blocks (a CU each) prepare that vector once for their eight waves while the
 // first weights fly, k_latent_mid's waves each by themselves.
 // Bound by the weights' stream behind a start of some 3 us (launch, activations, norm).  Width 2048, us, with a block of four waves that
-// each formed the norm and waited for the weights first (loads under masks are waited for where the mask ends) / so: 6464 rows
-// 9.9, 8.0; 16384 gated 15.1, 13.2; 22848 18.2, 17.2; a head of 32768 24.0, 22.7; [o | down] of 2048 x 10240 11.1, 9.9.
+// each formed the norm and waited for the weights first (loads under masks are waited for where the mask ends), 6464 rows 9.9; 16384 gated
+// 15.1; a head of 32768 24.0; [o | down] of 2048 x 10240 11.1; now 7.2, 13.1 (beside the delta step), 21.6, 8.7.
 #include <cstdlib>
 
 #include "latent_device.h"
@@ -325,9 +325,8 @@ template <int Q, bool EX> static int launch_latent_down_q(hipStream_t st, const 
 }
 template <bool EX> static int launch_latent_down_e(hipStream_t st, const LatentDownArgs &a, int chunks, size_t lds) {
   if (chunks <= 8) return launch_latent_down_q<8, EX>(st, a, lds);
-  if (chunks <= 16) return launch_latent_down_q<16, EX>(st, a, lds);
-  if (!EX && chunks <= 20) return launch_latent_down_q<20, false>(st, a, lds);   // (24, and 20 with the table, spill)
-  return launch_latent_down_q<16, EX>(st, a, lds);
+  // (chunks on their way at 2048 x 10240, us: 20 9.9, 16 10.6, 12 9.5, 10 8.8, 7 8.8, 5 8.7, 4 8.8)
+  return launch_latent_down_q<EX ? 16 : 5, EX>(st, a, lds);
 }
 int launch_latent_down(hipStream_t st, const LatentDownArgs &a) {
   const int chunks = (a.K0 + 511) / 512 + a.top * ((a.K1 + 511) / 512);

@@ -67,7 +67,10 @@ __device__ __forceinline__ void stream_rows(RowSet<KC, 2> &rs, const ld_u32x4 (&
 
 // Block `block` of `blocks` (eight waves each) of a LatentInArgs' launch, meant to have a CU to itself.  The block forms the
 // normalised vectors once, eight elements a thread, and its waves take them from LDS (2 K elements per product); a wave owns every
-// (8 blocks)-th pair of rows and keeps two pairs on their way, the first two from the block's first instructions on.
+// (8 blocks)-th pair of rows, neighbouring blocks neighbouring pairs, and keeps one pair on its way, from the block's first instructions on,
+// a row of the next asked for as soon as one of this is multiplied.  More on their way are slower: with two pairs, and neighbouring pairs to the waves of a
+// block, width 2048, us, before / so: 6464 rows 8.3, 7.2; 16384 gated beside the delta step 14.7, 13.1; 24576, most of them gated, 18.5, 17.1; a
+// head of 32768 22.7, 21.6; 2048 rows on f32 sums 5.5, 5.1.
 constexpr int kRowWaves = 8, kRowThreads = 64 * kRowWaves, kRowGroups = 16;
 inline size_t latent_in_lds(const LatentInArgs &a) { return ((size_t)a.K * ((a.N1 > 0) + (a.N2 > 0)) * 2 + 15) / 16 * 16 + (kRowWaves * (1 + kRowGroups)) * sizeof(float); }
 // Whether the wave at pair `at` takes the second product's vector, which lies K elements behind the first one's if both are there.  A
@@ -76,7 +79,7 @@ __host__ __device__ __forceinline__ bool latent_in_second(const LatentInArgs &a,
 template <int KC> __device__ __forceinline__ void latent_in_block(const LatentInArgs &a, int block, int blocks, char *lds) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int pairs1 = (a.N1 + 1) / 2, pairs = pairs1 + (a.N2 + 1) / 2, stride = blocks * kRowWaves;
-  int at = block * kRowWaves + wave;
+  int at = wave * blocks + block;
   uint16_t *xs1 = reinterpret_cast<uint16_t *>(lds), *xs2 = xs1 + (a.N1 > 0 ? a.K : 0);
   float *part = reinterpret_cast<float *>(lds + ((size_t)a.K * ((a.N1 > 0) + (a.N2 > 0)) * 2 + 15) / 16 * 16), *gpart = part + kRowWaves;
   // the small, L2-resident vectors first (loads return in order), then the first weights
@@ -95,14 +98,17 @@ template <int KC> __device__ __forceinline__ void latent_in_block(const LatentIn
     w1 = *reinterpret_cast<const ld_u32x4 *>((const uint16_t *)(a.N1 ? a.n1 : a.n2) + from);
     w2 = *reinterpret_cast<const ld_u32x4 *>((const uint16_t *)(a.N2 ? a.n2 : a.n1) + from);
   }
-  RowSet<KC, 2> rs[2];
+  RowSet<KC, 2> rs;
   // (behind the last pair: one line of the weights, again and again, so that the loads on their way can be counted)
-  auto request = [&](RowSet<KC, 2> &r, int pair) {
+  auto request = [&](int pair, int r) __attribute__((always_inline)) {
     const bool some = pair < pairs, second = some ? pair >= pairs1 : a.N1 == 0;
-    r.load((const uint16_t *)(second ? a.W2 : a.W1), a.ldw, !some ? 0 : 2 * (second ? pair - pairs1 : pair), !some ? 0 : (second ? a.N2 : a.N1) - 1, some ? a.K : 0, lane);
+    const int n = !some ? 0 : 2 * (second ? pair - pairs1 : pair) + r, last = !some ? 0 : (second ? a.N2 : a.N1) - 1, K = some ? a.K : 0;
+    const uint16_t *p = (const uint16_t *)(second ? a.W2 : a.W1) + (int64_t)(n < last ? n : last) * a.ldw;
+#pragma unroll
+    for (int u = 0; u < KC; ++u) rs.w[r][u] = __builtin_nontemporal_load(reinterpret_cast<const ld_u32x4 *>(p + (lane * 8 + u * 512 < K ? lane * 8 + u * 512 : 0)));
   };
-  request(rs[0], at);
-  request(rs[1], at + stride);
+  request(at, 0);
+  request(at, 1);
   float x[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = a.src_f32 ? (e < 4 ? x0[e & 3] : x1[e & 3]) : e & 1 ? hi_f32(raw[e >> 1]) : lo_f32(raw[e >> 1]);
@@ -166,15 +172,19 @@ template <int KC> __device__ __forceinline__ void latent_in_block(const LatentIn
   };
   bool second = latent_in_second(a, at);
   take(second);
-  auto finish = [&](RowSet<KC, 2> &r) {
+  auto finish = [&]() {
     if (!second && latent_in_second(a, at)) take(second = true);
     float v0 = 0.f, v1 = 0.f;
 #pragma unroll
-    for (int u = 0; u < KC; ++u) {
-      v0 = ld_dot8(r.piece(0, u, a.K, lane), xv[u], v0);
-      v1 = ld_dot8(r.piece(1, u, a.K, lane), xv[u], v1);
-    }
-    request(r, at + 2 * stride);
+    for (int u = 0; u < KC; ++u) v0 = ld_dot8(rs.piece(0, u, a.K, lane), xv[u], v0);
+    __builtin_amdgcn_sched_barrier(0);
+    request(at + stride, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < KC; ++u) v1 = ld_dot8(rs.piece(1, u, a.K, lane), xv[u], v1);
+    __builtin_amdgcn_sched_barrier(0);
+    request(at + stride, 1);
+    __builtin_amdgcn_sched_barrier(0);
     v0 = wave_sum(v0);
     v1 = wave_sum(v1);
     if (lane != 0) return;
@@ -193,13 +203,7 @@ template <int KC> __device__ __forceinline__ void latent_in_block(const LatentIn
       if (n + 1 < N) o[1] = v1;
     }
   };
-  while (at < pairs) {
-    finish(rs[0]);
-    at += stride;
-    if (at >= pairs) break;
-    finish(rs[1]);
-    at += stride;
-  }
+  for (; at < pairs; at += stride) finish();
 }
 
 }  // namespace rai
