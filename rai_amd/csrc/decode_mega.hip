@@ -986,9 +986,9 @@ __global__ void __launch_bounds__(kMegaThreads) k_phi2_decode_step(MegaArgs a) {
 
 // ---- the head behind the step -------------------------------------------------------------------------------------
 // logits = LayerNorm(x) . W^T + bias for one row, and the greedy choice on them, in one launch of one block per CU.
-// Every block normalises x once (as the step kernel does at the start of a layer), streams its share of the rows of W
-// through the same register ring (seven stream waves as there: with all eight streaming the launch took 48 us
-// instead of 43; the first sixteen tiles are requested before x is even read),
+// Every block normalises x once (as the step kernel does at the start of a layer).  Its eight waves stream pairs of rows of W, neighbouring blocks
+// neighbouring pairs, one pair on its way and replaced row by row: ten loads a wave, where the step kernel's ring of sixteen took longer
+// (32768 x 2560, 168 MB: 33.6 us, so 31.4; a kernel that only reads as much takes some 27).  A wave
 // rounds its logits to bf16, stores them and keeps the best of them: the first maximum, NaNs passed over, except
 // that a NaN in row 0 takes the choice (what a scan from element 0 that replaces on a strict comparison gives).  The
 // blocks' bests travel as 8-byte (value, row) words written past the L2; a block counts itself in when its word has
@@ -1011,7 +1011,6 @@ __global__ void __launch_bounds__(kMegaThreads) k_phi2_head_choice(HeadArgs a) {
   constexpr int H = KTA * 512;
   uint16_t *xr = reinterpret_cast<uint16_t *>(hd_smem);   // x as it is
   uint16_t *xn = xr + H;                                   // LayerNorm(x), bf16
-  float *part = reinterpret_cast<float *>(xn + H);         // [rows][kMegaWaves]
   __shared__ float s_v[kMegaWaves];
   __shared__ uint32_t s_i[kMegaWaves];
   __shared__ int s_ticket;
@@ -1019,38 +1018,37 @@ __global__ void __launch_bounds__(kMegaThreads) k_phi2_head_choice(HeadArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wg = blockIdx.x, G = gridDim.x;
-  const int r0 = (int)((int64_t)a.V * wg / G), r1 = (int)((int64_t)a.V * (wg + 1) / G);
-  const int nrows = r1 - r0;
-
-  const bool streams = wave < kMegaStream;
-  const int tt = nrows * KTA;
-  const int t0 = streams ? tt * wave / kMegaStream : 0, t1 = streams ? tt * (wave + 1) / kMegaStream : 0;
-  MgSplit sp;
-  sp.Wa0 = a.W; sp.Wb0 = a.W; sp.wa_stride = 0; sp.wb_stride = 0; sp.L = 1; sp.H = H; sp.KB = H; sp.KTA = KTA; sp.KTBC = 1;
-  sp.cnt0 = t1 - t0; sp.cnt1 = 0; sp.cnt2 = 0;
-  sp.kc0 = t0 % KTA; sp.kc1 = 0; sp.kc2 = 0;
-  sp.off0 = (int64_t)(r0 + t0 / KTA) * H; sp.off1 = 0; sp.off2 = 0;
-  sp.nx0 = 0; sp.nx1 = 0; sp.nx2 = 0;
-  MgCursor cur;
-  cur.layer = 0; cur.seg = 0; cur.kc = 0; cur.KT = 1; cur.left = 0; cur.jump = 0; cur.step = 0;
-  cur.ptr = a.W;
-  const bool streams_any = sp.cnt0 > 0;
-  if (streams_any) mg_seg_enter(cur, sp, 0, 0);
-  const MgPhase ph = mg_phase(t0, t1, 0, 0, KTA);
-  mg_u32x4 ring[kMegaRing];
+  // a wave's rows: every (8 G)-th pair, the pair under way and, row by row behind its multiplies, the next (behind the last: a row again)
+  const int pairs = (a.V + 1) / 2, stride = G * kMegaWaves;
+  int at = wave * G + wg;
+  mg_u32x4 w[2][KTA];
+  uint16_t braw[2];
+  auto request = [&](int pair, int r) __attribute__((always_inline)) {
+    const int n = pair < pairs ? 2 * pair + r : 0, row = n < a.V ? n : a.V - 1;
+    braw[r] = a.bias ? a.bias[row] : a.x[0];
+    const uint16_t *p = a.W + (int64_t)row * H;
 #pragma unroll
-  for (int p = 0; p < kMegaRing; ++p) ring[p] = streams_any ? mg_next_load(cur, sp, lane) : MG_ZERO4;
+    for (int u = 0; u < KTA; ++u) w[r][u] = mg_ldw(p + u * 512 + lane * 8);
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
-  // x into LDS, the partial sums to zero (a wave leaves one per row it touches)
-  for (int i = tid; i < H / 2; i += kMegaThreads) reinterpret_cast<uint32_t *>(xr)[i] = reinterpret_cast<const uint32_t *>(a.x)[i];
-  for (int e = tid; e < nrows * kMegaWaves; e += kMegaThreads) part[e] = 0.f;
+  // x, the first rows of weights behind it (loads return in order), x into LDS
+  uint32_t x0[(H / 2 + kMegaThreads - 1) / kMegaThreads];
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(x0) / 4); ++i) x0[i] = reinterpret_cast<const uint32_t *>(a.x)[tid + i * kMegaThreads < H / 2 ? tid + i * kMegaThreads : 0];
+  const int nf = (wave < KTA ? wave : 0) * 512 + lane * 8;
+  const mg_u32x4 lw = *reinterpret_cast<const mg_u32x4 *>(a.ln_w + nf), lb = *reinterpret_cast<const mg_u32x4 *>(a.ln_b + nf);
+  __builtin_amdgcn_sched_barrier(0);
+  request(at, 0);
+  request(at, 1);
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(x0) / 4); ++i)
+    if (tid + i * kMegaThreads < H / 2) reinterpret_cast<uint32_t *>(xr)[tid + i * kMegaThreads] = x0[i];
   wg_sync();
   if (wave < KTA) {   // wave u normalises features [512 u, 512 u + 512); every one of them computes the statistics
     mg_u32x4 xv[KTA];
 #pragma unroll
     for (int u = 0; u < KTA; ++u) xv[u] = *reinterpret_cast<const mg_u32x4 *>(xr + u * 512 + lane * 8);
-    const mg_u32x4 lw = *reinterpret_cast<const mg_u32x4 *>(a.ln_w + wave * 512 + lane * 8);
-    const mg_u32x4 lb = *reinterpret_cast<const mg_u32x4 *>(a.ln_b + wave * 512 + lane * 8);
     const uint32_t ones = 0x3f803f80u;
     float s1 = 0.f, s2 = 0.f;
     mg_u32x4 mine = MG_ZERO4;
@@ -1085,27 +1083,31 @@ __global__ void __launch_bounds__(kMegaThreads) k_phi2_head_choice(HeadArgs a) {
   }
   wg_sync();
 
-  bool staged = false;
-  (void)mg_run_phase(ring, cur, sp, ph, KTA, xn, part, part, nullptr, lane, wave, nullptr, staged);
-  wg_sync();
-
-  // this block's logits and the best of them
+  mg_u32x4 xv[KTA];
+#pragma unroll
+  for (int u = 0; u < KTA; ++u) xv[u] = *reinterpret_cast<const mg_u32x4 *>(xn + u * 512 + lane * 8);
+  // the logits of this wave's rows and the best of them (the same in every lane)
   float bv = -INFINITY;
   uint32_t bi = 0xffffffffu;
-  for (int e = tid; e < nrows; e += kMegaThreads) {
-    float sacc = 0.f;
+  for (; at < pairs; at += stride) {
 #pragma unroll
-    for (int w = 0; w < kMegaStream; ++w) sacc += part[e * kMegaWaves + w];
-    if (a.bias) sacc += bf16_bits_to_f32(a.bias[r0 + e]);
-    const uint16_t vb = f32_to_bf16_bits(sacc);
-    a.logits[r0 + e] = vb;
-    const float r = bf16_bits_to_f32(vb);
-    const uint32_t n = (uint32_t)(r0 + e);
-    if (r != r) {
-      if (n == 0u) { bv = r; bi = 0u; }
-    } else if (head_replaces(r, n, bv, bi)) {
-      bv = r;
-      bi = n;
+    for (int r = 0; r < 2; ++r) {
+      float acc = 0.f;
+#pragma unroll
+      for (int u = 0; u < KTA; ++u) acc = mg_dot8(w[r][u], xv[u], acc);
+      const float b = a.bias ? bf16_bits_to_f32(braw[r]) : 0.f;
+      asm volatile("" : "+v"(acc));   // (the products stay ahead of the loads that take their operands' place)
+      __builtin_amdgcn_sched_barrier(0);
+      request(at + stride, r);
+      const uint32_t n = 2u * at + r;
+      if (n >= (uint32_t)a.V) break;
+      const uint16_t vb = f32_to_bf16_bits(mg_wave_sum(acc) + b);
+      if (lane == 0) a.logits[n] = vb;
+      const float v = bf16_bits_to_f32(vb);
+      if (v != v ? n == 0u : head_replaces(v, n, bv, bi)) {
+        bv = v;
+        bi = n;
+      }
     }
   }
 #pragma unroll
@@ -1166,8 +1168,7 @@ __global__ void __launch_bounds__(kMegaThreads) k_phi2_head_choice(HeadArgs a) {
 }
 
 static size_t head_lds_bytes(const HeadArgs &a, int num_cu) {
-  const int rows = (a.V + num_cu - 1) / num_cu + 1;
-  return (size_t)a.H * 4 + (size_t)rows * kMegaWaves * sizeof(float);
+  return (size_t)a.H * 4;
 }
 
 bool head_choice_eligible(const HeadArgs &a, int num_cu) {
