@@ -95,7 +95,10 @@ __global__ void __launch_bounds__(256) k_reduce_thread(ReduceSpace s, T *out, co
 
 // ---------------------------------------------------------------- softmax
 // Row-major rows of length n with unit stride.  Each thread keeps up to
-// ITEMS*V values in registers, so the row is read exactly once.
+// ITEMS*V values in registers, so the row is read exactly once.  All of its loads go out before the
+// first is used, and the two reductions take a barrier each; bound by HBM for many rows, by the trip to memory and the barriers for few.
+// Measured by elements (us, before both; three passes over the row where n > 2048): bf16 7798 x 1367 19.3 -> 16.0, f32 8192 x 2047 35.8 -> 26.2 (5.1
+// TB/s), 3000 x 3381 31.2 -> 15.5 (5.2 TB/s), bf16 26.6 -> 13.2, 1 x 3381 8.6 -> 3.9.
 template <typename T, int V> struct alignas(sizeof(T) * V) RowPack { T v[V]; };
 
 __device__ __forceinline__ float block_reduce_max(float v, float *sh) {
@@ -121,26 +124,33 @@ __device__ __forceinline__ float block_reduce_sum(float v, float *sh) {
 
 template <typename T, int V, int ITEMS, bool LOG>
 __global__ void __launch_bounds__(256) k_softmax_row(T *out, const T *in, int64_t rows, int64_t n, int64_t in_row_stride) {
-  __shared__ float sh[4];
+  __shared__ float sh[2][4];   // a reduction each: what it holds is read before the other's barrier, so one barrier does for each
   const int64_t packs = n / V;
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
     const T *x = in + row * in_row_stride;
     T *y = out + row * n;
+    RowPack<T, V> pk[ITEMS];   // all of the row asked for before any of it is used
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+      const int64_t p = threadIdx.x + (int64_t)it * 256;
+      if (p < packs) pk[it] = *reinterpret_cast<const RowPack<T, V> *>(x + p * V);
+    }
     float vals[ITEMS][V];
     float m = -INFINITY;
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
-      int64_t p = threadIdx.x + (int64_t)it * 256;
-      if (p < packs) {
-        RowPack<T, V> pk = *reinterpret_cast<const RowPack<T, V> *>(x + p * V);
+      if (threadIdx.x + (int64_t)it * 256 < packs) {
 #pragma unroll
         for (int j = 0; j < V; ++j) {
-          vals[it][j] = (float)Scalar<T>::load(&pk.v[j]);
+          vals[it][j] = (float)Scalar<T>::load(&pk[it].v[j]);
           m = fmaxf(m, vals[it][j]);
         }
       }
     }
-    m = block_reduce_max(m, sh);
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(sh[0][0], sh[0][1]), fmaxf(sh[0][2], sh[0][3]));
     float sum = 0.f;
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
@@ -155,7 +165,10 @@ __global__ void __launch_bounds__(256) k_softmax_row(T *out, const T *in, int64_
         }
       }
     }
-    sum = block_reduce_sum(sum, sh);
+    sum = wave_sum(sum);
+    if ((threadIdx.x & 63) == 0) sh[1][threadIdx.x >> 6] = sum;
+    __syncthreads();
+    sum = ((sh[1][0] + sh[1][1]) + sh[1][2]) + sh[1][3];
     const float inv = 1.0f / sum, lse = logf(sum);
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
@@ -544,10 +557,13 @@ template <bool LOG> static int softmax_impl(int dev, const rai_hip_tensor *in, i
     if (packs <= 256) SM_LAUNCH(T, V, 1);                   \
     else if (packs <= 512) SM_LAUNCH(T, V, 2);              \
     else if (packs <= 1024) SM_LAUNCH(T, V, 4);             \
-    else SM_LAUNCH(T, V, 8);                                \
+    else if (packs <= 2048) SM_LAUNCH(T, V, 8);             \
+    else SM_LAUNCH(T, 1, 16);                               \
   } while (0)
-      // rows of up to 512 packs (4096 bf16 / 2048 f32 elements), several of them: one wave per row
-      if (aligned && packs <= 512 && rows >= 4) {
+      // Rows of up to 512 packs (4096 bf16 / 2048 f32 elements) or, where they are not whole 16-byte pieces, 512 elements, several of them: one wave
+      // per row.  Measured by elements (us, block, wave): bf16 8192 x 300 9.6, 5.4, 8192 x 511 10.6, 6.0, f32 8192 x 130 8.3, 4.0,
+      // 8192 x 511 11.3, 7.3; 500 rows and fewer alike, within the launch.
+      if (packs <= 512 && rows >= 4) {
         const int64_t wblocks = (rows + 3) / 4;
         const int wgrid = (int)(wblocks < kNumCU * 32 ? wblocks : kNumCU * 32);
 #define SMW_LAUNCH(T, V, ITEMS)                                                                                 \
@@ -560,14 +576,14 @@ template <bool LOG> static int softmax_impl(int dev, const rai_hip_tensor *in, i
     else if (packs <= 256) SMW_LAUNCH(T, V, 4);     \
     else SMW_LAUNCH(T, V, 8);                       \
   } while (0)
-        if (in->dtype == RAI_F32) SMW_BY_ITEMS(float, 4);
-        else if (in->dtype == RAI_BF16) SMW_BY_ITEMS(bf16_raw, 8);
-        else SMW_BY_ITEMS(f16_raw, 8);
+        if (in->dtype == RAI_F32) { if (aligned) SMW_BY_ITEMS(float, 4); else SMW_BY_ITEMS(float, 1); }
+        else if (in->dtype == RAI_BF16) { if (aligned) SMW_BY_ITEMS(bf16_raw, 8); else SMW_BY_ITEMS(bf16_raw, 1); }
+        else { if (aligned) SMW_BY_ITEMS(f16_raw, 8); else SMW_BY_ITEMS(f16_raw, 1); }
 #undef SMW_BY_ITEMS
 #undef SMW_LAUNCH
         return launch_check("softmax_wave");
       }
-      if (packs <= 2048) {
+      if (packs <= (aligned ? 2048 : 4096)) {   // (an unaligned row: as many elements as a block holds)
         if (in->dtype == RAI_F32) { if (aligned) SM_BY_ITEMS(float, 4); else SM_BY_ITEMS(float, 1); }
         else if (in->dtype == RAI_BF16) { if (aligned) SM_BY_ITEMS(bf16_raw, 8); else SM_BY_ITEMS(bf16_raw, 1); }
         else { if (aligned) SM_BY_ITEMS(f16_raw, 8); else SM_BY_ITEMS(f16_raw, 1); }
