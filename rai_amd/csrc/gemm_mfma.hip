@@ -629,8 +629,65 @@ __global__ void __launch_bounds__(512) k_gemm_bf16_mfma_dma_streamk(LinearArgs a
   }
 }
 
-// Sums the per-split partial products and applies the Linear epilogue.
+// Sums the per-split partial products and applies the Linear epilogue: four columns of a row to a thread, P of its parts asked for at a time
+// and added in their order.  Bound by the partial sums' way through the caches.  Measured
+// against an element at a time, the whole product (us): 333 x 8960 x 1536 of five parts 26.5 -> 24.4, 131 x 8512 x 5936 38.6 -> 36.4, 70 x 3072 x 1000
+// 10.1 -> 9.2, 800 x 16384 x 2048 71.4 -> 68.9.
+typedef __attribute__((ext_vector_type(2))) uint32_t sum_u32x2;
+template <int P>
 __global__ void __launch_bounds__(256) k_splitk_epilogue(LinearArgs a, int splits, const float *partial) {
+  const uint32_t total = (uint32_t)a.M * (uint32_t)a.N, row_quads = (uint32_t)a.N / 4, q = blockIdx.x * 256 + threadIdx.x;   // (fewer than 2^32 floats)
+  if (q >= total / 4) return;
+  const int m = (int)(q / row_quads), n = (int)(q % row_quads) * 4;
+  const uint16_t *bias = (const uint16_t *)a.bias, *bias2 = (const uint16_t *)a.bias2, *res = (const uint16_t *)a.residual;
+  sum_u32x2 b1 = {0u, 0u}, b2 = {0u, 0u}, rb = {0u, 0u};   // zero bits where there is none: +0.0
+  f32x4 rf = {0.f, 0.f, 0.f, 0.f};
+  if (bias) b1 = *reinterpret_cast<const sum_u32x2 *>(bias + n);
+  if (bias2) b2 = *reinterpret_cast<const sum_u32x2 *>(bias2 + n);
+  if (a.residual && a.f32_out) rf = *reinterpret_cast<const f32x4 *>((const float *)a.residual + (int64_t)m * a.ldr + n);
+  else if (a.residual) rb = *reinterpret_cast<const sum_u32x2 *>(res + (int64_t)m * a.ldr + n);
+  float x[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < splits; s0 += P) {
+    f32x4 p[P];
+#pragma unroll
+    for (int u = 0; u < P; ++u) p[u] = *reinterpret_cast<const f32x4 *>(partial + (size_t)min(s0 + u, splits - 1) * total + 4 * (size_t)q);
+#pragma unroll
+    for (int u = 0; u < P; ++u)
+      if (s0 + u < splits) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] += p[u][e];
+      }
+  }
+  auto half = [](sum_u32x2 v, int e) { return bf16_bits_to_f32((uint16_t)(v[e >> 1] >> (e & 1) * 16)); };
+  if (a.glu) {   // two (gate, up) pairs
+    uint32_t o = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) o |= (uint32_t)f32_to_bf16_bits(glu_bf16(a, x[e] + half(b1, e), x[e + 1] + half(b1, e + 1))) << 8 * e;
+    *reinterpret_cast<uint32_t *>((uint16_t *)a.out1 + (int64_t)m * a.ld1 + (n >> 1)) = o;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] += half(b1, e) + half(b2, e);
+  if (a.act >= 0) act_exact<4>(a.act, x, n, a.act_from);
+  if (a.f32_out) {
+    f32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = fmaf(a.out_scale, x[e], rf[e]);
+    *reinterpret_cast<f32x4 *>((float *)a.out1 + (int64_t)m * a.ld1 + n) = o;
+    return;
+  }
+  if (res) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] += half(rb, e);
+  }
+  const sum_u32x2 o = {(uint32_t)f32_to_bf16_bits(x[0]) | (uint32_t)f32_to_bf16_bits(x[1]) << 16,
+                   (uint32_t)f32_to_bf16_bits(x[2]) | (uint32_t)f32_to_bf16_bits(x[3]) << 16};
+  uint16_t *dst = n < a.n_split ? (uint16_t *)a.out1 + (int64_t)m * a.ld1 + n : (uint16_t *)a.out2 + (int64_t)m * a.ld2 + (n - a.n_split);
+  *reinterpret_cast<sum_u32x2 *>(dst) = o;
+}
+
+// The same an element at a time: where a piece below would be cut or off its boundary.
+__global__ void __launch_bounds__(256) k_splitk_epilogue_any(LinearArgs a, int splits, const float *partial) {
   const int64_t total = (int64_t)a.M * a.N;
   const uint16_t *bias = (const uint16_t *)a.bias;
   const uint16_t *bias2 = (const uint16_t *)a.bias2;
@@ -814,6 +871,27 @@ static bool post_norm_fits(const LinearArgs &a) {
          (!a.residual || (a.ldr % 8 == 0 && al16(a.residual))) && (!a.post_ln_w || al16(a.post_ln_w)) &&
          (!a.post_ln_b || al16(a.post_ln_b)) && a.splitk_ws && ((uintptr_t)a.splitk_ws & 15) == 0;
 }
+// Whether whole pieces of four columns lie on their boundaries in the partial sums and everything they meet.
+static bool quads_fit(const LinearArgs &a, const float *partial) {
+  auto al = [](const void *p, int64_t ld, unsigned bytes, unsigned size) { return ((uintptr_t)p & (bytes - 1)) == 0 && ld * size % bytes == 0; };
+  if (a.N % 4 || (int64_t)a.M * a.N >= (int64_t)1 << 32 || ((uintptr_t)partial & 15) || !al(a.bias, 0, 8, 2) || !al(a.bias2, 0, 8, 2)) return false;
+  if (a.glu) return al(a.out1, a.ld1, 4, 2);
+  if (a.f32_out) return al(a.out1, a.ld1, 16, 4) && al(a.residual, a.residual ? a.ldr : 0, 16, 4);
+  return al(a.out1, a.ld1, 8, 2) && al(a.residual, a.residual ? a.ldr : 0, 8, 2) && (a.n_split >= a.N || (a.n_split % 4 == 0 && al(a.out2, a.ld2, 8, 2)));
+}
+static int launch_sum_of_parts(hipStream_t st, const LinearArgs &a, int splits, const float *partial) {
+  const int64_t total = (int64_t)a.M * a.N;
+  if (quads_fit(a, partial)) {
+    const dim3 grid((unsigned)((total / 4 + 255) / 256)), block(256);
+    if (splits == 2) hipLaunchKernelGGL(k_splitk_epilogue<2>, grid, block, 0, st, a, splits, partial);
+    else if (splits == 3) hipLaunchKernelGGL(k_splitk_epilogue<3>, grid, block, 0, st, a, splits, partial);
+    else hipLaunchKernelGGL(k_splitk_epilogue<4>, grid, block, 0, st, a, splits, partial);
+    return launch_check("splitk_epilogue");
+  }
+  const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
+  hipLaunchKernelGGL(k_splitk_epilogue_any, dim3(blocks), dim3(256), 0, st, a, splits, partial);
+  return launch_check("splitk_epilogue");
+}
 // Sums the partial products of a tile GEMM that split K (and normalises the rows when asked to and possible).
 static int launch_splitk_epilogue(hipStream_t st, const LinearArgs &a, int splits, const float *partial) {
   if (post_norm_fits(a)) {
@@ -824,10 +902,7 @@ static int launch_splitk_epilogue(hipStream_t st, const LinearArgs &a, int split
     else hipLaunchKernelGGL(k_splitk_epilogue_ln<8>, grid, block, 0, st, a, splits, partial);
     return launch_check("splitk_epilogue_ln");
   }
-  const int64_t total = (int64_t)a.M * a.N;
-  const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
-  hipLaunchKernelGGL(k_splitk_epilogue, dim3(blocks), dim3(256), 0, st, a, splits, partial);
-  return launch_check("splitk_epilogue");
+  return launch_sum_of_parts(st, a, splits, partial);
 }
 
 template <int BM, int BN, int BK, int SH = 0> static int launch_cfg(hipStream_t st, const LinearArgs &a, int splits) {
@@ -1185,10 +1260,7 @@ template <int MT> static int launch_mfma_skinny(hipStream_t st, const LinearArgs
                      partial);
   RAI_TRY(launch_check("linear_bf16_mfma_skinny"));
   if (splits > 1) {
-    const int64_t total = (int64_t)a.M * a.N;
-    const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
-    hipLaunchKernelGGL(k_splitk_epilogue, dim3(blocks), dim3(256), 0, st, a, splits, (const float *)partial);
-    RAI_TRY(launch_check("splitk_epilogue"));
+    RAI_TRY(launch_sum_of_parts(st, a, splits, partial));
   }
   return RAI_OK;
 }
@@ -1555,10 +1627,7 @@ static int launch_mfma_stream_cfg(hipStream_t st, const LinearArgs &a, int split
                      partial, tickets);
   RAI_TRY(launch_check("linear_bf16_mfma_stream"));
   if (splits > 1 && !tickets) {
-    const int64_t total = (int64_t)a.M * a.N;
-    const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
-    hipLaunchKernelGGL(k_splitk_epilogue, dim3(blocks), dim3(256), 0, st, a, splits, (const float *)partial);
-    RAI_TRY(launch_check("splitk_epilogue"));
+    RAI_TRY(launch_sum_of_parts(st, a, splits, partial));
   }
   return RAI_OK;
 }
