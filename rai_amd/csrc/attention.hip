@@ -613,12 +613,12 @@ size_t attention_decode_counter_bytes(int B, int Hq) { return sizeof(int) * (siz
 // heads of one KV head over at most CH (64 or 128) consecutive keys:
 //   - every K and V load of the block is issued before anything is computed.  K goes
 //     straight from global memory into MFMA A fragments (lane l: key l%16 of a 16-key
-//     tile, features 32*step + 8*(l/16) ..), two tiles per wave; V goes through LDS;
+//     tile, features 32*step + 8*(l/16) ..), one or two tiles per wave; V goes through LDS;
 //   - scores^T[key, head] = K . Q^T per tile; accumulator register r of lane l is key
 //     4*(l/16)+r, head l%16.  The rotated queries are the B fragments, held in registers;
 //   - per-head max / exp / sum over the block's keys (one wave per head), exp values
 //     rounded to bf16 for the second product (the reference rounds P to V's dtype);
-//   - O[head, feature] = P . V: wave w owns features [w*D/4, (w+1)*D/4), P fragments are
+//   - O[head, feature] = P . V: wave w of NW owns features [w*D/NW, (w+1)*D/NW), P fragments are
 //     16-byte LDS reads, V fragments are gathered from LDS two bytes at a time (the
 //     transposition costs LDS reads, of which there are few: the kernel is bound by
 //     the K/V stream);
@@ -627,14 +627,15 @@ typedef __attribute__((ext_vector_type(8))) __bf16 ad_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float ad_f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t ad_u32x4;
 
-template <int D, int CH>
-__global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeArgs a) {
+template <int D, int CH, int NT>
+__global__ void __launch_bounds__(NT) k_attn_decode_mfma(AttnDecodeArgs a) {
   typedef bf16_raw T;
-  constexpr int KS = D / 32, KT = (CH + 63) / 64;  // 16-key tiles per wave (CH = 96: the last tile of waves 2, 3 is empty)
+  constexpr int NW = NT / 64;
+  constexpr int KS = D / 32, KT = (CH / 16 + NW - 1) / NW;  // 16-key tiles per wave (the last may be empty)
   constexpr int VP = D + 8, PP = CH + 8;           // LDS pitches (bf16 elements)
   constexpr int CPR = D / 8;                        // 16-byte chunks per K/V row
-  constexpr int VL = CH * CPR / kDecodeThreads;     // V chunks per thread
-  constexpr int DT = D / 64;                        // 16-feature tiles per wave in P.V
+  constexpr int VL = CH * CPR / NT;                  // V chunks per thread
+  constexpr int DT = D / 16 / NW;                    // 16-feature tiles per wave in P.V
   extern __shared__ __attribute__((aligned(16))) float smem[];
   uint16_t *Vs = reinterpret_cast<uint16_t *>(smem);          // [CH][VP]; the first 16 rows hold Q until the scores are done
   const int R = a.Hq / a.Hkv;
@@ -656,8 +657,8 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
   const T *vrow = (a.k_new ? (const T *)a.v_new + (int64_t)b * a.v_row_stride : qrow + QD + KD) + hk * D;
   // ---- asked for before the position is here, every load whole: feature tid of the new token's key and value, the query rows
   // (eight features per item; `by8`: a rotary half is whole items)
-  static_assert(D <= kDecodeThreads, "a thread per feature");
-  constexpr int QI = (16 * CPR + kDecodeThreads - 1) / kDecodeThreads;
+  static_assert(D <= NT && CH * CPR % NT == 0 && D % (16 * NW) == 0, "a thread per feature, whole rounds of V, whole tiles of features");
+  constexpr int QI = (16 * CPR + NT - 1) / NT;
   const bool by8 = a.rot % 16 == 0;
   const int rot8 = by8 ? a.rot : 0, half = rot8 >> 1, kd = tid < D ? tid : D - 1;
   RopeRaw<T> kx;
@@ -666,7 +667,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
   ad_u32x4 qx[QI], qo[QI], qc[QI][2], qn[QI][2];
 #pragma unroll
   for (int i = 0; i < QI; ++i) {
-    const int item = tid + i * kDecodeThreads, r = item / CPR, d = (item - r * CPR) * 8;
+    const int item = tid + i * NT, r = item / CPR, d = (item - r * CPR) * 8;
     const T *row = qrow + (hq0 + min(r, R - 1)) * D;
     qx[i] = *reinterpret_cast<const ad_u32x4 *>(row + d);
     qo[i] = *reinterpret_cast<const ad_u32x4 *>(row + (d < half ? d + half : d < rot8 ? d - half : d));
@@ -690,7 +691,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
   // ---- the tables (eight values are 16 or 32 bytes), then all K and V loads of the block (past the end: the last key once more)
 #pragma unroll
   for (int i = 0; i < QI; ++i) {
-    const int item = tid + i * kDecodeThreads, d = item % CPR * 8, size = a.tab_f32 ? 4 : 2;
+    const int item = tid + i * NT, d = item % CPR * 8, size = a.tab_f32 ? 4 : 2;
     const int64_t at = ((int64_t)pos * rot8 + (d < rot8 ? d : 0)) * size;
     const char *c = by8 && rot8 ? (const char *)a.cos_t + at : (const char *)qrow, *sn = by8 && rot8 ? (const char *)a.sin_t + at : (const char *)qrow;
     const int second = a.tab_f32 && by8 && rot8 ? 16 : 0;
@@ -706,18 +707,18 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
   for (int i = 0; i < KT; ++i)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
-      kreg[i][ks] = *reinterpret_cast<const ad_bf16x8 *>(Kc + (int64_t)min(t0 + (wave + 4 * i) * 16 + lrow, last) * D + ks * 32 + lq * 8);
+      kreg[i][ks] = *reinterpret_cast<const ad_bf16x8 *>(Kc + (int64_t)min(t0 + (wave + NW * i) * 16 + lrow, last) * D + ks * 32 + lq * 8);
   ad_u32x4 vreg[VL];
 #pragma unroll
   for (int j = 0; j < VL; ++j) {
-    const int c = tid + j * kDecodeThreads, r = c / CPR, c8 = c - r * CPR;
+    const int c = tid + j * NT, r = c / CPR, c8 = c - r * CPR;
     vreg[j] = *reinterpret_cast<const ad_u32x4 *>(Vc + (int64_t)min(t0 + r, last) * D + c8 * 8);
   }
   // ---- rotated queries (rows >= R are zero)
   if (by8) {
 #pragma unroll
     for (int i = 0; i < QI; ++i) {
-      const int item = tid + i * kDecodeThreads, r = item / CPR, d = (item - r * CPR) * 8;
+      const int item = tid + i * NT, r = item / CPR, d = (item - r * CPR) * 8;
       if (item >= 16 * CPR) continue;
       ad_u32x4 out = r < R ? qx[i] : ad_u32x4{0u, 0u, 0u, 0u};
       if (r < R && d < a.rot && a.tab_f32) {   // f32 tables: products and sum in f32, one rounding
@@ -753,13 +754,13 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
       *reinterpret_cast<ad_u32x4 *>(Vs + r * VP + d) = out;
     }
   } else {
-    for (int e = tid; e < 16 * D; e += kDecodeThreads) {
+    for (int e = tid; e < 16 * D; e += NT) {
       const int r = e / D, d = e - r * D;
       const float q = r < R ? rope_feature<T>(qrow + (hq0 + r) * D, d, a.rot, cos_t, sin_t, pos, a.tab_f32) : 0.f;
       Vs[r * VP + d] = f32_to_bf16_bits(q);
     }
   }
-  for (int e = tid; e < 16 * PP; e += kDecodeThreads) ps[e] = 0;
+  for (int e = tid; e < 16 * PP; e += NT) ps[e] = 0;
   if (has_new && tid < D) {
     const uint16_t kr = f32_to_bf16_bits(rope_finish(kx, kd, a.rot, a.tab_f32));
     knew[tid] = kr;
@@ -776,7 +777,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
     for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const ad_bf16x8 *>(Vs + lrow * VP + ks * 32 + lq * 8);
 #pragma unroll
     for (int i = 0; i < KT; ++i) {
-      const int tile = wave + 4 * i;
+      const int tile = wave + NW * i;
       if (tile * 16 >= CH) continue;
       if (has_new && new_row == tile * 16 + lrow) {   // the lanes that hold the new token's key row
 #pragma unroll
@@ -798,12 +799,12 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
   // ---- V into LDS (the new token's row from the activations), softmax statistics
 #pragma unroll
   for (int j = 0; j < VL; ++j) {
-    const int c = tid + j * kDecodeThreads, r = c / CPR, c8 = c - r * CPR;
+    const int c = tid + j * NT, r = c / CPR, c8 = c - r * CPR;
     ad_u32x4 v = t0 + r < t1c ? vreg[j] : ad_u32x4{0u, 0u, 0u, 0u};
     if (has_new && r == new_row) v = *reinterpret_cast<const ad_u32x4 *>(vnew + c8 * 8);
     *reinterpret_cast<ad_u32x4 *>(Vs + r * VP + c8 * 8) = v;
   }
-  for (int r = wave; r < R; r += 4) {
+  for (int r = wave; r < R; r += NW) {
     float m = -INFINITY;
     for (int t = lane; t < n; t += 64) m = fmaxf(m, scores[r * CH + t]);
     m = wave_max(m);
@@ -825,7 +826,7 @@ __global__ void __launch_bounds__(kDecodeThreads) k_attn_decode_mfma(AttnDecodeA
     ad_f32x4 o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) o[dt] = ad_f32x4{0.f, 0.f, 0.f, 0.f};
-    const int d0 = wave * (D / 4);
+    const int d0 = wave * (D / NW);
     for (int k0 = 0; k0 < n; k0 += 32) {
       const ad_bf16x8 pf = *reinterpret_cast<const ad_bf16x8 *>(ps + lrow * PP + k0 + lq * 8);
 #pragma unroll
@@ -901,7 +902,7 @@ __global__ void __launch_bounds__(256) k_attn_decode_merge_bf16(AttnDecodeArgs a
 
 // Splits of the context over blocks of `ch` keys.  A block that holds the longest context the cache has room for (the context itself is the
 // device's to know) writes the result itself, without the launch that merges: 24 sequences on 51 to 83 keys (8 heads of 256 on one) 10.4 us
-// for 7.2 + 4.7 in two blocks a sequence.  One to 32 sequences of 52 to 122 keys decoded so, against two blocks each: 128 features 0.2 to
+// for 7.2 + 4.7 in two blocks a sequence (four waves each).  One to 32 sequences of 52 to 122 keys decoded so, against two blocks each: 128 features 0.2 to
 // 3 % sooner, 256 features 0.3 to 2 % up to 96 keys and within 1 % either way beyond.
 static int mfma_decode_splits(const AttnDecodeArgs &a, int ch) {
   if (a.Tmax <= ch && !getenv("RAI_HIP_ATTN_SPLITS")) return 1;
@@ -909,23 +910,34 @@ static int mfma_decode_splits(const AttnDecodeArgs &a, int ch) {
   return ns < need ? need : ns;
 }
 
-template <int D, int CH> static int launch_decode_mfma_cfg(hipStream_t st, AttnDecodeArgs a) {
+template <int D, int CH, int NT> static int launch_decode_mfma_cfg(hipStream_t st, AttnDecodeArgs a) {
   const int R = a.Hq / a.Hkv;
-  a.ns = mfma_decode_splits(a, CH);
   a.chunk_cap = CH;
   const size_t lds = (size_t)CH * (D + 8) * 2 + (size_t)R * CH * 4 + 16 * (CH + 8) * 2 + 2 * D * 2;
   static bool attr_set = false;
   if (lds > 64 * 1024 && !attr_set) {
-    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_attn_decode_mfma<D, CH>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_attn_decode_mfma<D, CH, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)((size_t)CH * (D + 8) * 2 + 16 * CH * 4 + 16 * (CH + 8) * 2 + 2 * D * 2)));
     attr_set = true;
   }
   RAI_REQUIRE(a.Hkv <= 65535 && a.B <= 65535, RAI_ERR_UNSUPPORTED, "attention decode: grid too large");
-  hipLaunchKernelGGL((k_attn_decode_mfma<D, CH>), dim3(a.ns, a.Hkv, a.B), dim3(kDecodeThreads), lds, st, a);
+  hipLaunchKernelGGL((k_attn_decode_mfma<D, CH, NT>), dim3(a.ns, a.Hkv, a.B), dim3(NT), lds, st, a);
   RAI_TRY(launch_check("attention_decode_mfma"));
   if (a.ns == 1) return RAI_OK;
   hipLaunchKernelGGL(k_attn_decode_merge_bf16, dim3(a.Hq, a.B), dim3(D), 0, st, a);
   return launch_check("attention_decode_merge");
+}
+
+// Eight waves to a block where all blocks are on the chip with them, four beyond, where more blocks share a CU and its registers.  A block is a chain
+// of a few trips to memory and of its own steps, which eight waves halve.  Measured (us, four waves, eight): 256 features, 24 blocks
+// of 96 keys 10.3, 7.7, 16 of 64 7.1, 6.1, 240 8.4, 7.6, 512 12.0, 10.9; 128 features, 32 blocks 5.6, 5.1, 256 6.3, 5.6, 320 7.2, 7.1, 1024
+// 11.9, 13.5.  (128 keys of 256 features take more registers than two blocks of eight waves have.)
+template <int D, int CH> static int launch_decode_mfma_waves(hipStream_t st, AttnDecodeArgs a) {
+  a.ns = mfma_decode_splits(a, CH);
+  if constexpr (D >= 128) {
+    if ((int64_t)a.ns * a.Hkv * a.B <= (D == 256 && CH < 128 ? 2 : 1) * kNumCU) return launch_decode_mfma_cfg<D, CH, 512>(st, a);
+  }
+  return launch_decode_mfma_cfg<D, CH, 256>(st, a);
 }
 
 // Keys per block: 64, 96 or 128.  Every block issues all its loads up front and a CU holds as many blocks as their LDS
@@ -952,9 +964,9 @@ template <int D> static int launch_decode_mfma(hipStream_t st, const AttnDecodeA
     if (!best || rounds < best_rounds) { best = ch; best_rounds = rounds; }
     if (ns == 1 && !forced) { best = ch; break; }   // the smallest block that holds every key
   }
-  if (best == 64) return launch_decode_mfma_cfg<D, 64>(st, a);
-  if (best == 96) return launch_decode_mfma_cfg<D, 96>(st, a);
-  return launch_decode_mfma_cfg<D, 128>(st, a);
+  if (best == 64) return launch_decode_mfma_waves<D, 64>(st, a);
+  if (best == 96) return launch_decode_mfma_waves<D, 96>(st, a);
+  return launch_decode_mfma_waves<D, 128>(st, a);
 }
 
 // The MFMA kernel serves bf16 grouped-query shapes whose longest context fits
