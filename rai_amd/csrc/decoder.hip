@@ -1351,6 +1351,10 @@ int decoder_alloc_common(rai_hip_decoder *d) {
   // the stream-K form of the tile kernel (prefill products of 136 tiles and more) parks partial tiles here
   if (cfg->dtype == RAI_BF16 && d->max_rows >= 256 && d->splitk_ws_bytes < ((size_t)192 << 20))
     d->splitk_ws_bytes = (size_t)192 << 20;
+  // f32 tiles of a short prompt's wide products leave the last round of blocks half empty without a few parts of K (128 x 2560 x 17920: 147 us,
+  // in three parts 113 and the sum)
+  if (cfg->dtype == RAI_F32)
+    d->splitk_ws_bytes = std::max(d->splitk_ws_bytes, std::min((size_t)64 << 20, (size_t)4 * d->max_rows * (d->QD + 2 * d->KD + 2 * d->I) * sizeof(float)));
   RAI_TRY(dalloc(d, d->splitk_ws_bytes, &d->splitk_ws));
   RAI_TRY(dalloc(d, (size_t)cfg->max_batch * kChoiceMaxSplits * sizeof(float), &tmp));
   d->choice_val = (float *)tmp;
