@@ -34,8 +34,8 @@ template <> __device__ __forceinline__ mm_f32x16 mm_mfma<f16_raw>(mm_chunk a, mm
 // as it lies, BK rows of ROWS elements + 16 bytes, and the fragments are put together on the way out: 16-bit elements
 // with the transposing LDS read (lane i of 16 receives element i % 4 of the 8 bytes that lanes 4j + i / 4, j = 0..3, point
 // at: with lane a pointing at row a / 4, columns 4 (a % 4), it receives column i of four rows), f32 one by one.
-// Memory is read in pieces of 16 bytes whatever their alignment; where K ends inside one (KC), the last 16 bytes of the row are
-// read and moved down, or a K of less than a piece by pairs (element by element, 16-bit operands with K of 9 to 15 took up to
+// Memory is read in pieces of 16 bytes whatever their alignment; where K ends inside one (KC), or the outputs do (otherwise), the last 16 bytes of
+// the row are read and moved down when they go to LDS, or a K of less than a piece by pairs (element by element, 16-bit operands with K of 9 to 15 took up to
 // 1.1 us more than multiply-adds on the vector units: 11 x 1 x 11 x 93 in bf16 4.2 us there, 5.3, now 4.5).
 template <typename T, int ROWS, bool KC, int KB>
 struct MmOperand {
@@ -45,15 +45,42 @@ struct MmOperand {
   const T *base;      // the tile's first output row (column), k = 0
   int64_t stride;     // KC: between outputs; otherwise: between consecutive k
   int valid, K;       // outputs that exist from the tile's first on; the length of K
+  int before;         // outputs before the tile's first
   mm_chunk reg[P];
 
   // place of this thread's piece p: KC: (output, chunk of K); otherwise (k, chunk of outputs)
   static __device__ __forceinline__ int row(int p) { return (threadIdx.x + 256 * p) / CPR; }
   static __device__ __forceinline__ int col(int p) { return ((threadIdx.x + 256 * p) % CPR) * V; }
 
+  // Every row has a piece, so that one can be read for every place.
+  __device__ __forceinline__ bool pieces() const { return KC ? K >= V : before + valid >= V; }
   // The whole tile lies inside the operand (outputs past the end aside, which are read from the last one).
   __device__ __forceinline__ bool whole(int k0) const { return k0 + BK <= K && (KC || valid >= ROWS); }
-  __device__ __forceinline__ void fetch(int k0) {
+  // How a tile's step is fetched and put into LDS: all of it inside the operand; whole steps of a tile whose outputs may end inside (whose rows
+  // have a piece); any.  The first two have no branch, so that they stay between the products of the step before.
+  enum { kInside, kOutputsEnd, kAny };
+  template <int MODE> __device__ __forceinline__ void fetch(int k0) {
+    if constexpr (MODE != kAny) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const T *at = KC ? base + (int64_t)min(row(p), valid - 1) * stride + k0 + col(p)
+                         : base + (int64_t)(k0 + row(p)) * stride + (MODE == kInside ? col(p) : min(col(p), valid - V));
+        __builtin_memcpy(&reg[p], at, 16);
+      }
+    } else {
+      fetch_any(k0);
+    }
+  }
+  template <int MODE> __device__ __forceinline__ void park(char *st, int k0) const {
+    if constexpr (MODE == kAny) {
+      park_any(st, k0);
+    } else {
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+        *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = KC || MODE == kInside ? reg[p] : end_of_row(reg[p], col(p) + V - valid);
+    }
+  }
+  __device__ __forceinline__ void fetch_any(int k0) {
     if (whole(k0)) {
 #pragma unroll
       for (int p = 0; p < P; ++p) {
@@ -62,17 +89,20 @@ struct MmOperand {
       }
       return;
     }
+    if (pieces()) {   // at the ends: the last 16 bytes of the row, or the last row, again
 #pragma unroll
-    for (int p = 0; p < P; ++p) {   // at the ends: zeros past K, the last output repeated
+      for (int p = 0; p < P; ++p) {
+        const T *at = KC ? base + (int64_t)min(row(p), valid - 1) * stride + min(k0 + col(p), K - V)
+                         : base + (int64_t)min(k0 + row(p), K - 1) * stride + min(col(p), valid - V);
+        __builtin_memcpy(&reg[p], at, 16);
+      }
+      return;
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {   // rows of less than a piece: zeros past K, the last output repeated
       const int k = KC ? k0 + col(p) : k0 + row(p), o = KC ? min(row(p), valid - 1) : col(p);
-      const T *at = KC ? base + (int64_t)o * stride + k : base + (int64_t)k * stride + o;
       if (k >= K) {
         reg[p] = mm_chunk{0u, 0u, 0u, 0u};
-      } else if (KC ? k + V <= K : o + V <= valid) {
-        __builtin_memcpy(&reg[p], at, 16);
-      } else if (KC && K >= V) {   // the piece that ends with K, moved down
-        __builtin_memcpy(&reg[p], base + (int64_t)o * stride + (K - V), 16);
-        reg[p] = end_of_k(reg[p], k + V - K);
       } else if (KC && sizeof(T) == 2 && K > 1) {   // a shorter K, by pairs
         const T *at_o = base + (int64_t)o * stride;
 #pragma unroll
@@ -94,8 +124,9 @@ struct MmOperand {
       }
     }
   }
-  // A piece that was read `past` elements (below V) ahead of its place: what lies past the end is zero.
-  static __device__ __forceinline__ mm_chunk end_of_k(mm_chunk v, int past) {
+  // A piece that was read `past` elements (none: past <= 0) ahead of its place: what lies past the end is zero.  (V and more: not zero, of no use.)
+  static __device__ __forceinline__ mm_chunk end_of_row(mm_chunk v, int past) {
+    past = max(past, 0);
     const int words = past * (int)sizeof(T) / 4;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -103,7 +134,17 @@ struct MmOperand {
     if (sizeof(T) == 2 && (past & 1)) v = mm_chunk{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
     return v;
   }
-  __device__ __forceinline__ void park(char *st) const {
+  // To LDS, what was fetched for k0; a piece that was read ahead of its place goes there now.
+  __device__ __forceinline__ void park_any(char *st, int k0) const {
+    if (!whole(k0) && pieces()) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int k = KC ? k0 + col(p) : k0 + row(p);
+        const mm_chunk v = end_of_row(reg[p], KC ? k + V - K : col(p) + V - valid);
+        *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = k < K ? v : mm_chunk{0u, 0u, 0u, 0u};
+      }
+      return;
+    }
 #pragma unroll
     for (int p = 0; p < P; ++p) *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = reg[p];
   }
@@ -151,6 +192,11 @@ template <typename T> __device__ __forceinline__ void mm_store(T *dst, const flo
 //   Measured (us; 64 x 64 tiles of multiply-adds on the vector units before): bf16 32 x 512 x 80 x 512 (scores) 11.2 (40.5),
 // 32 x 512 x 512 x 80 (values, [K, N]) 13.4 (94.8), 64 x 1024 x 1024 x 1024 200 to 316 (2900 to 3035), one row against 32 x
 // 777 x 128 10.4 (77.5), odd 18 x 410 x 141 x 349 10.8 (31.8); f32 32 x 512 x 80 x 512 24.4 (47.9).
+//   The steps of a long K are free of branches but for the last three (us, a fetch that asks each step and piece whether it ends inside,
+// and now): bf16 64 x 1024 x 1024 x 1024, [K, N] 299, 207, K-contiguous 304, 277, 64 x 1000 x 999 x 1001 454, 266 and 367, 333, 7 x 481 x
+// 944 x 246 27.9, 11.9, 18 x 169 x 639 x 234 19.2, 9.7, f16 5 x 9 x 723 x 56 14.6, 8.8; f32 3 x 15 x 737 x 625 24.0, 22.3, K-contiguous 6 x 14 x
+// 538 x 677 16.8, 14.9, whole tiles of [K, N] alike.  f32, whose products take longer, loads a step ahead from its first products on
+// (from the third: 64 x 128 x 512 x 128 17.1, 16.5).  Stages of 256 bytes: 0.95 to 1.33 of the time.
 template <typename T, bool AKC, bool BKC, int F, int KB, bool ONE>
 __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T *B, MatmulArgs g, int tiles_m, int tiles_n) {
   constexpr int BT = 64 * F;
@@ -177,11 +223,13 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
   a.base = A + aoff + (AKC ? (int64_t)m0 * g.a_rs : (int64_t)m0);
   a.valid = (int)min<int64_t>(BT, g.M - m0);
   a.K = (int)g.K;
+  a.before = m0;
   OpB b;
   b.stride = BKC ? g.b_cs : g.b_rs;
   b.base = B + boff + (BKC ? (int64_t)n0 * g.b_cs : (int64_t)n0);
   b.valid = (int)min<int64_t>(BT, g.N - n0);
   b.K = (int)g.K;
+  b.before = n0;
 
   const int wave = threadIdx.x >> 6, wm = (wave >> 1) * 32 * F, wn = (wave & 1) * 32 * F;
   mm_f32x16 acc[F][F];
@@ -192,13 +240,16 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   const int steps = ONE ? 1 : ((int)g.K + OpA::BK - 1) / OpA::BK;
-  a.fetch(0);
-  b.fetch(0);
-  a.park(lds);
-  b.park(lds + OpA::BYTES);
-  if (steps > 1) { a.fetch(OpA::BK); b.fetch(OpA::BK); }
+  constexpr int kInside = OpA::kInside, kOutputsEnd = OpA::kOutputsEnd, kAny = OpA::kAny;
+  a.template fetch<kAny>(0);
+  b.template fetch<kAny>(0);
+  a.template park<kAny>(lds, 0);
+  b.template park<kAny>(lds + OpA::BYTES, 0);
+  if (steps > 1) { a.template fetch<kAny>(OpA::BK); b.template fetch<kAny>(OpA::BK); }
   __syncthreads();
-  for (int s = 0; s < steps; ++s) {
+  int s = 0;
+  auto step = [&](auto how) __attribute__((always_inline)) {
+    constexpr int MODE = decltype(how)::value;
     const char *sa = lds + (s & 1) * STAGE, *sb = sa + OpA::BYTES;
     mm_chunk fa[2][F], fb[2][F];
     auto read = [&](int kk) {
@@ -212,11 +263,13 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
     for (int kk = 0; kk < PAIRS; ++kk) {
       if (ONE && kk * (32 / (int)sizeof(T)) >= (int)g.K) break;
       if (kk + 1 < PAIRS) read(kk + 1);
-      if (kk == 2 && s + 1 < steps) {   // to the stage that every wave left before the last barrier
+      if (kk == (sizeof(T) == 4 ? 0 : 2) && (MODE != kAny || s + 1 < steps)) {   // to the stage that every wave left before the last barrier
         char *next = lds + ((s + 1) & 1) * STAGE;
-        a.park(next);
-        b.park(next + OpA::BYTES);
-        if (s + 2 < steps) { a.fetch((s + 2) * OpA::BK); b.fetch((s + 2) * OpA::BK); }
+        if constexpr (F == 1) __builtin_amdgcn_sched_barrier(0);   // (what the compiler moves across costs short products 1 to 5 %)
+        a.template park<MODE>(next, (s + 1) * OpA::BK);
+        b.template park<MODE>(next + OpA::BYTES, (s + 1) * OpA::BK);
+        if (MODE != kAny || s + 2 < steps) { a.template fetch<MODE>((s + 2) * OpA::BK); b.template fetch<MODE>((s + 2) * OpA::BK); }
+        if constexpr (F == 1) __builtin_amdgcn_sched_barrier(0);   // (what the compiler moves across costs short products 1 to 5 %)
       }
 #pragma unroll
       for (int i = 0; i < F; ++i)
@@ -224,7 +277,18 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
         for (int j = 0; j < F; ++j) acc[i][j] = mm_mfma<T>(fa[kk & 1][i], fb[kk & 1][j], acc[i][j]);
     }
     __syncthreads();
+  };
+  // the steps that fetch one before the last, whole in K
+  if constexpr (!ONE) {
+    if (a.pieces() && b.pieces()) {
+      if ((AKC || a.valid >= BT) && (BKC || b.valid >= BT)) {
+        for (; s + 3 < steps; ++s) step(std::integral_constant<int, kInside>{});
+      } else {
+        for (; s + 3 < steps; ++s) step(std::integral_constant<int, kOutputsEnd>{});
+      }
+    }
   }
+  for (; s < steps; ++s) step(std::integral_constant<int, kAny>{});
   // accumulator register e of lane (r, h) is row 8 (e / 4) + 4 h + e % 4, column r
   float *f = reinterpret_cast<float *>(lds);
   const int r = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
