@@ -54,50 +54,38 @@ struct MmOperand {
 
   // Every row has a piece, so that one can be read for every place.
   __device__ __forceinline__ bool pieces() const { return KC ? K >= V : before + valid >= V; }
-  // The whole tile lies inside the operand (outputs past the end aside, which are read from the last one).
-  __device__ __forceinline__ bool whole(int k0) const { return k0 + BK <= K && (KC || valid >= ROWS); }
-  // How a tile's step is fetched and put into LDS: all of it inside the operand; whole steps of a tile whose outputs may end inside (whose rows
-  // have a piece); any.  The first two have no branch, so that they stay between the products of the step before.
-  enum { kInside, kOutputsEnd, kAny };
+  // How a step is fetched and put into LDS: all of it inside the operand; whole in K, where the outputs may end inside; any.  None of these has a
+  // branch, so that it stays between the products of the step before.  kShort: rows of this operand or the other have no piece.
+  enum { kInside, kOutputsEnd, kEnds, kShort };
   template <int MODE> __device__ __forceinline__ void fetch(int k0) {
-    if constexpr (MODE != kAny) {
+    if constexpr (MODE == kShort) {
+      if (pieces()) fetch<kEnds>(k0);
+      else fetch_short(k0);
+    } else {
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const T *at = KC ? base + (int64_t)min(row(p), valid - 1) * stride + k0 + col(p)
-                         : base + (int64_t)(k0 + row(p)) * stride + (MODE == kInside ? col(p) : min(col(p), valid - V));
+      for (int p = 0; p < P; ++p) {   // at an end: the last 16 bytes of the row, or the last row, again
+        const int k = KC ? k0 + col(p) : k0 + row(p), o = KC ? min(row(p), valid - 1) : col(p);
+        const T *at = KC ? base + (int64_t)o * stride + (MODE == kEnds ? min(k, K - V) : k)
+                         : base + (int64_t)(MODE == kEnds ? min(k, K - 1) : k) * stride + (MODE == kInside ? o : min(o, valid - V));
         __builtin_memcpy(&reg[p], at, 16);
       }
-    } else {
-      fetch_any(k0);
     }
   }
+  // To LDS, what was fetched for k0; a piece that was read ahead of its place goes there now.
   template <int MODE> __device__ __forceinline__ void park(char *st, int k0) const {
-    if constexpr (MODE == kAny) {
-      park_any(st, k0);
-    } else {
+    if constexpr (MODE == kShort) {
+      if (pieces()) return park<kEnds>(st, k0);
+    }
 #pragma unroll
-      for (int p = 0; p < P; ++p)
-        *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = KC || MODE == kInside ? reg[p] : end_of_row(reg[p], col(p) + V - valid);
+    for (int p = 0; p < P; ++p) {
+      const int k = KC ? k0 + col(p) : k0 + row(p);
+      mm_chunk v = reg[p];
+      if (MODE == kEnds || (MODE == kOutputsEnd && !KC)) v = end_of_row(v, KC ? k + V - K : col(p) + V - valid);
+      if (MODE == kEnds) v = k < K ? v : mm_chunk{0u, 0u, 0u, 0u};
+      *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = v;
     }
   }
-  __device__ __forceinline__ void fetch_any(int k0) {
-    if (whole(k0)) {
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const T *at = KC ? base + (int64_t)min(row(p), valid - 1) * stride + k0 + col(p) : base + (int64_t)(k0 + row(p)) * stride + col(p);
-        __builtin_memcpy(&reg[p], at, 16);
-      }
-      return;
-    }
-    if (pieces()) {   // at the ends: the last 16 bytes of the row, or the last row, again
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const T *at = KC ? base + (int64_t)min(row(p), valid - 1) * stride + min(k0 + col(p), K - V)
-                         : base + (int64_t)min(k0 + row(p), K - 1) * stride + min(col(p), valid - V);
-        __builtin_memcpy(&reg[p], at, 16);
-      }
-      return;
-    }
+  __device__ __forceinline__ void fetch_short(int k0) {
 #pragma unroll
     for (int p = 0; p < P; ++p) {   // rows of less than a piece: zeros past K, the last output repeated
       const int k = KC ? k0 + col(p) : k0 + row(p), o = KC ? min(row(p), valid - 1) : col(p);
@@ -133,20 +121,6 @@ struct MmOperand {
       if (words > i) v = mm_chunk{v[1], v[2], v[3], 0u};
     if (sizeof(T) == 2 && (past & 1)) v = mm_chunk{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
     return v;
-  }
-  // To LDS, what was fetched for k0; a piece that was read ahead of its place goes there now.
-  __device__ __forceinline__ void park_any(char *st, int k0) const {
-    if (!whole(k0) && pieces()) {
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const int k = KC ? k0 + col(p) : k0 + row(p);
-        const mm_chunk v = end_of_row(reg[p], KC ? k + V - K : col(p) + V - valid);
-        *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = k < K ? v : mm_chunk{0u, 0u, 0u, 0u};
-      }
-      return;
-    }
-#pragma unroll
-    for (int p = 0; p < P; ++p) *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = reg[p];
   }
   // Outputs first .. first + 31, chunk pair kk of K: lane (r, h) gets chunk 2 kk + h of output first + r.
   static __device__ __forceinline__ mm_chunk fragment(const char *st, int first, int kk) {
@@ -192,11 +166,11 @@ template <typename T> __device__ __forceinline__ void mm_store(T *dst, const flo
 //   Measured (us; 64 x 64 tiles of multiply-adds on the vector units before): bf16 32 x 512 x 80 x 512 (scores) 11.2 (40.5),
 // 32 x 512 x 512 x 80 (values, [K, N]) 13.4 (94.8), 64 x 1024 x 1024 x 1024 200 to 316 (2900 to 3035), one row against 32 x
 // 777 x 128 10.4 (77.5), odd 18 x 410 x 141 x 349 10.8 (31.8); f32 32 x 512 x 80 x 512 24.4 (47.9).
-//   The steps of a long K are free of branches but for the last three (us, a fetch that asks each step and piece whether it ends inside,
-// and now): bf16 64 x 1024 x 1024 x 1024, [K, N] 299, 207, K-contiguous 304, 277, 64 x 1000 x 999 x 1001 454, 266 and 367, 333, 7 x 481 x
-// 944 x 246 27.9, 11.9, 18 x 169 x 639 x 234 19.2, 9.7, f16 5 x 9 x 723 x 56 14.6, 8.8; f32 3 x 15 x 737 x 625 24.0, 22.3, K-contiguous 6 x 14 x
-// 538 x 677 16.8, 14.9, whole tiles of [K, N] alike.  f32, whose products take longer, loads a step ahead from its first products on
-// (from the third: 64 x 128 x 512 x 128 17.1, 16.5).  Stages of 256 bytes: 0.95 to 1.33 of the time.
+//   A step has no branch: the ends of rows are put right by moving what was read, not by asking where it lies (us, with branches, and now): bf16 64 x
+// 1024 x 1024 x 1024, [K, N] 300, 207 to 212, K-contiguous 305, 202, 64 x 1000 x 999 x 1001 454, 266 and 367, 263, 7 x 481 x 944 x 246 27.9, 11.2,
+// 18 x 169 x 639 x 234 19.3, 9.1, 19 x 30 x 192 x 34 6.3, 4.8, f16 5 x 9 x 723 x 56 14.6, 8.0; f32 3 x 15 x 737 x 625 24.1, 21.1, 64 x 128 x 512 x 128
+// 16.6, 15.8.  f32, whose products take longer, loads a step ahead from its first products on (from the third: 17.1).  Stages of
+// 256 bytes: 0.95 to 1.33 of the time.
 template <typename T, bool AKC, bool BKC, int F, int KB, bool ONE>
 __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T *B, MatmulArgs g, int tiles_m, int tiles_n) {
   constexpr int BT = 64 * F;
@@ -240,13 +214,17 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   const int steps = ONE ? 1 : ((int)g.K + OpA::BK - 1) / OpA::BK;
-  constexpr int kInside = OpA::kInside, kOutputsEnd = OpA::kOutputsEnd, kAny = OpA::kAny;
-  a.template fetch<kAny>(0);
-  b.template fetch<kAny>(0);
-  a.template park<kAny>(lds, 0);
-  b.template park<kAny>(lds + OpA::BYTES, 0);
-  if (steps > 1) { a.template fetch<kAny>(OpA::BK); b.template fetch<kAny>(OpA::BK); }
-  __syncthreads();
+  constexpr int kInside = OpA::kInside, kOutputsEnd = OpA::kOutputsEnd, kEnds = OpA::kEnds, kShort = OpA::kShort;
+  const bool pieces = a.pieces() && b.pieces();
+  auto begin = [&](auto how) __attribute__((always_inline)) {
+    constexpr int MODE = decltype(how)::value;
+    a.template fetch<MODE>(0);
+    b.template fetch<MODE>(0);
+    a.template park<MODE>(lds, 0);
+    b.template park<MODE>(lds + OpA::BYTES, 0);
+    if (steps > 1) { a.template fetch<MODE>(OpA::BK); b.template fetch<MODE>(OpA::BK); }
+    __syncthreads();
+  };
   int s = 0;
   auto step = [&](auto how) __attribute__((always_inline)) {
     constexpr int MODE = decltype(how)::value;
@@ -263,12 +241,12 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
     for (int kk = 0; kk < PAIRS; ++kk) {
       if (ONE && kk * (32 / (int)sizeof(T)) >= (int)g.K) break;
       if (kk + 1 < PAIRS) read(kk + 1);
-      if (kk == (sizeof(T) == 4 ? 0 : 2) && (MODE != kAny || s + 1 < steps)) {   // to the stage that every wave left before the last barrier
+      if (kk == (sizeof(T) == 4 ? 0 : 2) && (MODE < kEnds || s + 1 < steps)) {   // to the stage that every wave left before the last barrier
         char *next = lds + ((s + 1) & 1) * STAGE;
         if constexpr (F == 1) __builtin_amdgcn_sched_barrier(0);   // (what the compiler moves across costs short products 1 to 5 %)
         a.template park<MODE>(next, (s + 1) * OpA::BK);
         b.template park<MODE>(next + OpA::BYTES, (s + 1) * OpA::BK);
-        if (MODE != kAny || s + 2 < steps) { a.template fetch<MODE>((s + 2) * OpA::BK); b.template fetch<MODE>((s + 2) * OpA::BK); }
+        if (MODE < kEnds || s + 2 < steps) { a.template fetch<MODE>((s + 2) * OpA::BK); b.template fetch<MODE>((s + 2) * OpA::BK); }
         if constexpr (F == 1) __builtin_amdgcn_sched_barrier(0);   // (what the compiler moves across costs short products 1 to 5 %)
       }
 #pragma unroll
@@ -278,17 +256,20 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
     }
     __syncthreads();
   };
-  // the steps that fetch one before the last, whole in K
-  if constexpr (!ONE) {
-    if (a.pieces() && b.pieces()) {
+  if (!pieces) {
+    begin(std::integral_constant<int, kShort>{});
+    for (; s < steps; ++s) step(std::integral_constant<int, kShort>{});
+  } else {
+    begin(std::integral_constant<int, kEnds>{});
+    if constexpr (!ONE) {   // the steps that fetch one before the last, whole in K
       if ((AKC || a.valid >= BT) && (BKC || b.valid >= BT)) {
         for (; s + 3 < steps; ++s) step(std::integral_constant<int, kInside>{});
       } else {
         for (; s + 3 < steps; ++s) step(std::integral_constant<int, kOutputsEnd>{});
       }
     }
+    for (; s < steps; ++s) step(std::integral_constant<int, kEnds>{});
   }
-  for (; s < steps; ++s) step(std::integral_constant<int, kAny>{});
   // accumulator register e of lane (r, h) is row 8 (e / 4) + 4 h + e % 4, column r
   float *f = reinterpret_cast<float *>(lds);
   const int r = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
