@@ -709,6 +709,7 @@ static rai_hip_tensor desc1(void *p, int dtype, int64_t n) {
 int decoder_linear(rai_hip_decoder *d, hipStream_t st, const LinearArgs &a0) {
   LinearArgs a = a0;
   a.dev = d->dev;
+  a.fixed_sums = 1;
   return d->cfg.dtype == RAI_BF16 ? launch_linear_bf16(st, a) : launch_linear_f32(st, a);
 }
 
@@ -824,9 +825,7 @@ static int forward_phi2(rai_hip_decoder *d, int B, int S, bool advance_step, boo
   const int H = d->H, QD = d->QD, KD = d->KD, I = d->I;
   const int64_t M = (int64_t)B * S;
   const int ldq = QD + 2 * KD;
-  // One row's norm runs inside its Linear.  Several rows take it first: the Linears without are that much faster (two layers of Phi-2,
-  // 40 tokens and 16 more: 2 sequences 3514, 2527 us, 4 4163, 2909, 8 5103, 3222).
-  const bool fuse_ln = dt == RAI_BF16 && M == 1;
+  const bool fuse_ln = dt == RAI_BF16 && M <= 8;
   const int T_after = d->ctx_len + S;
   const bool frag = wants_fragments(d, M);
   if (frag) RAI_TRY(ensure_fragments(d, st));
@@ -932,7 +931,7 @@ static int forward_phi2(rai_hip_decoder *d, int B, int S, bool advance_step, boo
   // (phi2.rs:345-346: narrow(1, S-1, 1) before lm_head).
   LinearArgs h = linear_args_default();
   char *last_rows = x + (size_t)(S - 1) * H * d->es;  // row b*S + S-1, stride S*H
-  if (dt == RAI_BF16 && B == 1) {
+  if (dt == RAI_BF16 && B <= 8) {
     h.A = last_rows; h.lda = (int64_t)S * H;
     h.ln_kind = 0; h.ln_w = d->lnf_w; h.ln_b = d->lnf_b; h.ln_eps = (float)d->cfg.norm_eps;
   } else {

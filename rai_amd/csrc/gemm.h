@@ -55,6 +55,10 @@ struct LinearArgs {
   // 16 rows x 32 columns that one wave loads with one instruction are 1 KB of consecutive memory
   // ([N / 16 row tiles][K / 32 steps][64 lanes][8 elements], see linear_fragment_layout); null: read W itself.
   const void *Wfrag;
+  // != 0: the caller's results rest on the order in which the row kernels, tiles and k_linear_bf16_mfma_stream add (a decoder's: another order
+  // changes one output in some thousand by a unit of bf16, which all layers behind it carry on).  The streaming form is then left to weights in
+  // fragment order, where its sums are theirs.
+  int fixed_sums;
   // Optional LayerNorm of the finished output rows, written to post_ln_out ([M, N], dense) next to out1: the pass
   // that sums the split-K partial products has the whole row at hand, so the norm that consumes the output (the next
   // block's input LayerNorm) costs no launch of its own.  Only that pass offers it: ask linear_fuses_post_norm()
@@ -93,7 +97,7 @@ int launch_linear_fragment_layout(hipStream_t st, const void *W, int64_t ldw, in
 int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a);
 // bf16 weight-streaming kernels for M <= 8 with a fused norm or a second product (decode): HBM-bound.
 int launch_linear_bf16_skinny(hipStream_t st, const LinearArgs &a);
-// Up to eight rows without either: a kernel of their own (gemm.hip); otherwise one of the two above.
+// The streaming form (below) where it serves and pays; else up to eight rows without either: a kernel of their own (gemm.hip); otherwise one of the two above.
 int launch_linear_bf16(hipStream_t st, const LinearArgs &a);
 
 // Up to kGemvGroupMax bf16 Linears of one activation row (M == 1, K <= 4096, a multiple of 8) in one launch: member i
@@ -125,7 +129,8 @@ int launch_gemv_group(hipStream_t st, GemvGroupArgs g);
 // where M x N alone leaves CUs idle, of `room` bytes at most; with less it cuts K less.
 int launch_linear_f32(hipStream_t st, const LinearArgs &a);
 size_t linear_f32_workspace_bytes(const LinearArgs &a, size_t room);
-// The streaming form for 2 to 32 rows (gemm_stream.hip), what it takes and where it is the fastest, and the scratch with which it also takes a K that it has to cut (0: none).
+// The streaming form (gemm_stream.hip: 9 to 32 rows on fragments, 5 to 32 on rows as they lie), what it takes and where it is the fastest, and the scratch with which
+// it also takes a K that it has to cut (0: none).
 bool linear_stream_serves(const LinearArgs &a);
 bool linear_stream_pays(const LinearArgs &a);
 size_t linear_stream_workspace_bytes(const LinearArgs &a);

@@ -1,4 +1,4 @@
-// bf16 Linears of 2 to 32 rows (a batched decode step) by v_mfma_f32_16x16x32_bf16, on weights in fragment order or in rows as they lie.
+// bf16 Linears of 5 to 32 rows (a batched decode step; one of 9 and more for weights in fragment order) by v_mfma_f32_16x16x32_bf16, on weights in fragment order or in rows as they lie.
 #include "gemm_device.h"
 
 namespace rai {
@@ -21,7 +21,7 @@ constexpr int kPastL2 = 17;   // cache policy bits sc0 and sc1: past the (per-XC
 // How the blocks' reads lie to each other counts as much: 2048 x 16384 took 21.4 with four neighbouring tiles to a block (each 512 KB), 17.2
 // with two, 16.3 with four a grid apart, but 32768 x 2048 (tiles of 64 KB) 24.8 with two neighbours, 26.5 with two a grid apart, 29 with four neighbours; eights
 // of steps of all tiles side by side 27.1.  A wave's steps in one piece instead of in turn: no difference.  Rows as they lie take some 13 %
-// more than fragments (four rows x 32768 x 2048 normed and gated 22.6, 26).
+// more than fragments.
 // Registers: 128 at two blocks to a CU hold the activations, a tile and the sums of four, if nothing else is live then: uniform addresses, a load
 // behind the multiply whose operand it replaces, first sums on a zero that takes none (with spills 2048 x 16384 took 20.2 us).
 template <int MT, int KS, int G, bool FRAG, bool NORM, bool GLU, bool SPLIT, bool F32O>
@@ -271,7 +271,7 @@ template <int MT, int KS, bool FRAG, bool F32O> static int launch_stream_form(hi
   auto with = [&](auto g) -> int {
     constexpr int G = decltype(g)::value;
     if constexpr (!F32O) {
-      if constexpr (KS <= 8) {
+      if constexpr (FRAG && KS <= 8) {
         if (a.ln_kind > 0)
           return a.glu ? launch_stream<MT, KS, G, FRAG, true, true, false, false>(st, a, 1, nullptr) : launch_stream<MT, KS, G, FRAG, true, false, false, false>(st, a, 1, nullptr);
       }
@@ -286,11 +286,13 @@ template <int MT, int KS, bool FRAG, bool F32O> static int launch_stream_form(hi
 // gives and the steps dealt out evenly (K = 1536 in six, 8960 in five parts of seven).
 static int stream_parts(const LinearArgs &a) { return a.K <= (a.ln_kind > 0 ? 2048 : 2560) ? 1 : (a.K / 32 + 63) / 64; }
 static size_t stream_parts_bytes(const LinearArgs &a) { return (size_t)stream_parts(a) * ((a.N + 63) / 64 * 64) * ((a.M + 15) / 16 * 16) * sizeof(float); }
-// What it takes: whole pieces of four columns everywhere, K long enough for four steps a wave and, where K is cut, room for the parts.
+// What it takes: whole pieces of four columns everywhere, K long enough for four steps a wave and, where K is cut, room for the parts; weights in rows as they lie without
+// a norm or an f32 output, and not where the caller keeps to the other kernels' sums.
 bool linear_stream_serves(const LinearArgs &a) {
   const int parts = stream_parts(a), piece = a.f32_out ? 16 : 8;
   auto whole = [](const void *p, int n) { return ((uintptr_t)p & (n - 1)) == 0; };
   if (a.M < 2 || a.M > 32 || a.K % 32 || a.K <= 24 * 32 || a.N % 4 || a.n_split % 4 || a.ln_kind == 0 || a.K2 || a.force_splits > 0) return false;
+  if (a.Wfrag ? a.M <= 8 : a.fixed_sums || a.ln_kind > 0 || a.f32_out) return false;
   if ((a.ln_kind > 0 || a.glu) && (parts > 1 || a.f32_out)) return false;
   if (!a.Wfrag && (a.ldw % 8 || a.ldw >= 1 << 26 || !whole(a.W, 16))) return false;
   if (a.lda % 8 || a.lda >= 1 << 25 || !whole(a.A, 16) || (a.ln_kind > 0 && !whole(a.ln_w, 16))) return false;
@@ -300,8 +302,7 @@ bool linear_stream_serves(const LinearArgs &a) {
   return parts == 1 || (a.splitk_ws && whole(a.splitk_ws, 16) && stream_parts_bytes(a) <= a.splitk_ws_bytes && stream_parts_bytes(a) < (1u << 31) &&
                         (a.N + 15) / 16 <= kSplitTickets);
 }
-// Where it is the fastest form.  On fragments and with a fused norm it always is (the latter, of rows as they lie, against k_linear_bf16_skinny, us: 2 rows x
-// 2560 x 2048 9.0, 7.3, x 32768 gated 41, 26.5; 8 rows 21.9, 7.8 and 60, 27).  Else, on rows as they lie, weights from HBM and, in brackets, from the caches
+// Where it is the fastest form.  On fragments it always is.  On rows as they lie, weights from HBM and, in brackets, from the caches
 // where the two disagree: two to four rows are k_linear_bf16_rows's (4 x 8960 x 1536 8.3, 10.1; 4 x 4096 x 4096 9.5, 9.6), which at five to eight
 // loses but for small matrices (8 x 2560 x 2048 7.9, 5.6; 8 x 16384 x 2048 21.0, 14.7; 8 x 1536 x 8960 12.2, 9.6; 8 x 512 x 1536 4.4, 4.5; 8 x
 // 1024 x 4096 6.4, 6.7); 9 to 32 rows, against tiles and the kernel in gemm_mfma.hip: 16 x 2048 x 2048 7.1, 5.9; 16 x 4096 x 1024 7.0, 4.2; 32 x 8960 x
@@ -310,7 +311,7 @@ bool linear_stream_serves(const LinearArgs &a) {
 bool linear_stream_pays(const LinearArgs &a) {
   const char *off = getenv("RAI_HIP_NO_MFMA_STREAM"), *off2 = getenv("RAI_HIP_NO_MFMA_SKINNY");   // read per call: tests force the other kernels
   if (off || off2) return false;
-  if (a.Wfrag || a.ln_kind > 0) return true;
+  if (a.Wfrag) return true;
   const int64_t size = (int64_t)a.N * a.K;
   const bool parts = stream_parts(a) > 1;
   if (a.M <= 4) return false;
@@ -331,9 +332,9 @@ int launch_linear_bf16_stream(hipStream_t st, const LinearArgs &a) {
     constexpr int MT = decltype(mt)::value;
     constexpr bool F = decltype(f32o)::value;
     if (!a.Wfrag) {   // rows as they lie: pairs of steps
-      if (ks > 8) return launch_stream_form<MT, 10, false, F>(st, a, parts, tickets);
-      if (ks > 6) return launch_stream_form<MT, 8, false, F>(st, a, parts, tickets);
-      return ks > 4 ? launch_stream_form<MT, 6, false, F>(st, a, parts, tickets) : launch_stream_form<MT, 4, false, F>(st, a, parts, tickets);
+      if (ks > 8) return launch_stream_form<MT, 10, false, false>(st, a, parts, tickets);
+      if (ks > 6) return launch_stream_form<MT, 8, false, false>(st, a, parts, tickets);
+      return ks > 4 ? launch_stream_form<MT, 6, false, false>(st, a, parts, tickets) : launch_stream_form<MT, 4, false, false>(st, a, parts, tickets);
     }
     switch (ks) {
       case 10: return launch_stream_form<MT, 10, true, F>(st, a, parts, tickets);
