@@ -1,4 +1,4 @@
-// bf16 Linears of 5 to 32 rows (a batched decode step; one of 9 and more for weights in fragment order) by v_mfma_f32_16x16x32_bf16, on weights in fragment order or in rows as they lie.
+// bf16 Linears of a batched decode step by v_mfma_f32_16x16x32_bf16: 9 to 32 rows on weights in fragment order, 5 to 32 on rows as they lie.
 #include "gemm_device.h"
 
 namespace rai {
@@ -7,27 +7,29 @@ typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 
 constexpr int kPastL2 = 17;   // cache policy bits sc0 and sc1: past the (per-XCD, mutually incoherent) L2s
 
-// A block's eight waves take the K steps of 32 in turn (step 8 i + wave, i = 0 .. KS - 1; of rows as they lie, pairs of steps: whole lines) with the
-// activations of theirs in registers for the whole launch; it walks over groups of G tiles of 16 weight rows, RT tiles on their way, and the eight partial sums of an output meet in LDS.
-// K in parts (SPLIT): part s of n takes the eights of steps s, s + n, ...; a block has one group then, its tiles a grid apart, and two
-// blocks share a CU.
+// A wave takes eight K steps of 32 with their activations in registers for the whole launch: NW waves to a block, as many as K has eights.  The block walks over
+// groups of G tiles of 16 weight rows, RT tiles on their way, and the waves' partial sums of an output meet in LDS.  K beyond 2560 in parts of 64
+// steps (SPLIT): a block has one group of one part then, its tiles a grid apart, and two blocks share a CU.
+// On fragments a wave's steps are neighbours.  The order of every f32 sum and the one rounding of a normed activation are then those of
+// k_linear_bf16_mfma_stream (gemm_mfma.hip), bit for bit, which a decoder's results rest on (LinearArgs::fixed_sums): steps dealt out otherwise, and the norm's
+// factor on the finished sums, saved 0.3 to 1.5 us a launch and moved the logits of four layers of Gemma by 1 %, none of them nearer to the exact ones.
+// On rows as they lie the waves take pairs of steps (whole lines) in turn: 8 rows x 16384 x 2048 14.3 us, in pieces 17.6.
 // Bound by the stream of W behind a start (launch, activations, norm) and an end (the sums' way through LDS, with parts through memory) of some
 // 5 us together.  The compiler's wait for a load that may not have been made counts none that follow: a residual asked for under a condition
-// drained the ring at every group's start.  So nothing is loaded under a condition; rows beyond M and steps beyond K are those at the
-// end once more.  Measured on weights from HBM, 24 rows, in a graph, against the kernel in gemm_mfma.hip, which is also bigger by its outputs of any
-// alignment (us, it, this): 32768 x 2048 normed and gated 28.9, 24.8 (134 MB: 5.4 TB/s; a kernel that only reads them takes 21 to 23), plain 25.4,
-// 23.5; 2560 x 2048 normed 9.9, 7.9; 2048 x 2048 with residual 6.6, 6.3; 2048 x 16384 in eight parts 19.5, 16.3; 17920 x 1536 normed and gated 21.1, 13.6;
-// 1536 x 8960 in five parts 14.1, 10.2; 2048 x 1536 normed 9.1, 6.2.
+// drained the ring at every group's start.  So nothing is loaded under a condition; rows beyond M are the last once more, steps beyond K the first,
+// times zeros.  Measured on fragments from HBM, 24 rows, against the kernel in gemm_mfma.hip, which is also bigger by its outputs of any alignment (us, it, this):
+// 32768 x 2048 normed and gated 28.9, 26.1 (134 MB: 5.1 TB/s; a kernel that only reads them takes 21 to 23); 2560 x 2048 normed 9.9, 9.0; 2048 x 2048
+// with residual 6.6, 6.6; 2048 x 16384 in eight parts 19.5, 16.0; 17920 x 1536 normed and gated 21.1, 15.2; 1536 x 8960 in five parts 14.1, 10.4; 2048 x 1536
+// normed 9.1, 7.9; Phi-2's 12800 x 2560 and 2560 x 12800 29.7 in the mean, 20.7 and 21.0.
 // How the blocks' reads lie to each other counts as much: 2048 x 16384 took 21.4 with four neighbouring tiles to a block (each 512 KB), 17.2
-// with two, 16.3 with four a grid apart, but 32768 x 2048 (tiles of 64 KB) 24.8 with two neighbours, 26.5 with two a grid apart, 29 with four neighbours; eights
-// of steps of all tiles side by side 27.1.  A wave's steps in one piece instead of in turn: no difference.  Rows as they lie take some 13 %
-// more than fragments.
+// with two, 16.3 with four a grid apart, but 32768 x 2048 (tiles of 64 KB) 24.8 with two neighbours, 26.5 with two a grid apart, 29 with four neighbours.
 // Registers: 128 at two blocks to a CU hold the activations, a tile and the sums of four, if nothing else is live then: uniform addresses, a load
-// behind the multiply whose operand it replaces, first sums on a zero that takes none (with spills 2048 x 16384 took 20.2 us).
-template <int MT, int KS, int G, bool FRAG, bool NORM, bool GLU, bool SPLIT, bool F32O>
-__global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(LinearArgs a, int tiles, float *partial, int *tickets) {
-  constexpr int NW = 8, RT = G < 2 || SPLIT ? 1 : 2, PCH = 4 * G + 1, ITEMS = MT * G * 64;
-  static_assert(ITEMS <= 512 && !(F32O && (NORM || GLU)) && !(SPLIT && (NORM || GLU)), "a thread finishes one piece of a group");
+// behind the multiply whose operand it replaces, first sums on a zero that takes none (with spills 2048 x 16384 took 20.2 us).  Beyond eight waves and 16
+// rows one tile is on its way: of two, the second spills.
+template <int MT, int NW, int G, bool FRAG, bool NORM, bool GLU, bool SPLIT, bool F32O>
+__global__ void __launch_bounds__(64 * NW, SPLIT ? 4 : (NW + 3) / 4) k_linear_bf16_stream(LinearArgs a, int tiles, float *partial, int *tickets) {
+  constexpr int KS = 8, RT = G < 2 || SPLIT || (NW > 8 && MT > 1) ? 1 : 2, PCH = 4 * G + 1, ITEMS = MT * G * 64;
+  static_assert(ITEMS <= 64 * NW && !(F32O && (NORM || GLU)) && !(SPLIT && (NORM || GLU || NW != 8)), "a thread finishes one piece of a group");
   extern __shared__ __attribute__((aligned(16))) char stream_lds[];
   f32x4 *red = reinterpret_cast<f32x4 *>(stream_lds);                     // [NW][MT * 16 rows][PCH]
   float *squares = reinterpret_cast<float *>(red + NW * MT * 16 * PCH);   // [NW][MT * 16 rows]
@@ -35,12 +37,10 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, lq = lane >> 4;
   const int parts = SPLIT ? gridDim.y : 1, part = SPLIT ? blockIdx.y : 0, ksteps = a.K / 32;
-  constexpr int RUN = FRAG ? 1 : 2;   // neighbouring steps to a wave; all but the last run are within K
-  static_assert(KS % RUN == 0, "whole runs");
-  auto place = [&](int ks) { return ((ks / RUN * parts + part) * NW + wave) * RUN + ks % RUN; };
-  auto beyond = [&](int ks) { return ks >= KS - RUN && place(ks) >= ksteps; };
-  auto step_at = [&](int ks) { return beyond(ks) ? 0 : place(ks); };
-
+  auto place = [&](int ks) { return FRAG ? (part * NW + wave) * KS + ks : ((ks / 2 * parts + part) * NW + wave) * 2 + ks % 2; };
+  constexpr int SURE = FRAG ? 0 : SPLIT ? 4 : 6;   // as many are within K wherever it ends
+  auto within = [&](int ks) { return ks < SURE || place(ks) < ksteps; };
+  auto step_at = [&](int ks) { return within(ks) ? place(ks) : 0; };
   bf16x8 xf[MT][KS], wv[KS], w[RT][KS];
   const uint32_t lane_at = lane * 16;
   auto load = [&](bf16x8 &dst, int tile, int ks) __attribute__((always_inline)) {
@@ -75,40 +75,59 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
     for (int ks = 0; ks < KS; ++ks) load(w[pos][ks], tile_at(g0, pos), ks);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int ks = KS - RUN; ks < KS; ++ks)
+  for (int ks = SURE; ks < KS; ++ks) {   // (zeros beyond K, of the norm's weight too: an infinite one would make them NaN)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      if (beyond(ks)) xf[mt][ks] = bf16x8{};
+      if (!within(ks)) xf[mt][ks] = bf16x8{};
+    if constexpr (NORM)
+      if (!within(ks)) wv[ks] = bf16x8{};
+  }
   if constexpr (NORM) {
-    // RMSNorm of the rows (ln_kind 1: x * w / rms, 2: x * (1 + w) / rms).  The fragments take the weight, in f32 and rounded once; the factor
-    // 1 / rms is the finished sums', so that no wave waits for another's squares before it multiplies.  Every block norms all rows, so vector
-    // instructions count: the squares are the diagonal of X X^T (lane (row, quarter) holds row 4 quarter + r of column `row`).
+    // RMSNorm of the rows (ln_kind 1: x * w / rms, 2: x * (1 + w) / rms): the sum of squares of a row is gathered from the waves that hold its pieces,
+    // then every fragment is scaled and rounded once, as the stand-alone kernel does.  Every block norms all rows, so vector
+    // instructions count: the squares are the diagonal of X X^T (lane (row, quarter) holds row 4 quarter + r of column `row`), and the weight is widened
+    // ahead of the barrier that they wait for.
+    f32x4 xx[MT];
 #pragma unroll
-    for (int ks = KS - RUN; ks < KS; ++ks)
-      if (beyond(ks)) wv[ks] = bf16x8{};   // an infinite weight would make the zeros NaN
+    for (int mt = 0; mt < MT; ++mt) xx[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) xx[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[mt][ks], xf[mt][ks], xx[mt], 0, 0, 0);
+    float wf[KS][8];
+    const float one = a.ln_kind == 2 ? 1.f : 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        wf[ks][j] = (float)wv[ks][j] + one;
+        asm volatile("" : "+v"(wf[ks][j]));
+      }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      f32x4 xx = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) xx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[mt][ks], xf[mt][ks], xx, 0, 0, 0);
-      const float lo = lrow & 1 ? xx.y : xx.x, hi = lrow & 1 ? xx.w : xx.z;
+      const float lo = lrow & 1 ? xx[mt].y : xx[mt].x, hi = lrow & 1 ? xx[mt].w : xx[mt].z;
       if (lq == lrow >> 2) squares[wave * (MT * 16) + mt * 16 + lrow] = lrow & 2 ? hi : lo;
     }
-    const float one = a.ln_kind == 2 ? 1.f : 0.f;
+    __syncthreads();
+    float scale[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      float tot = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) tot += squares[w * (MT * 16) + mt * 16 + lrow];
+      scale[mt] = 1.0f / sqrtf(tot / (float)a.K + a.ln_eps);
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float wf = (float)wv[ks][j] + one;
+      for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) xf[mt][ks][j] = (__bf16)((float)xf[mt][ks][j] * wf);
-      }
+        for (int mt = 0; mt < MT; ++mt) xf[mt][ks][j] = (__bf16)((float)xf[mt][ks][j] * scale[mt] * wf[ks][j]);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
   // what a thread finishes: four columns of row m, at column n of a group (ITEMS <= 512)
   const int lds_item = tid < ITEMS ? tid : 0;
-  float scale = 1.f;
   // columns n .. n + 3 (N is a multiple of 4) and what is added to them
   auto word = [&](const void *p, int64_t at) { return *reinterpret_cast<const u32x2 *>(p ? (const char *)p + at * 2 : (const char *)a.A); };
   auto value = [&](const u32x2 &v, int e) { return bf16_bits_to_f32((uint16_t)((e < 2 ? v.x : v.y) >> (16 * (e & 1)))); };
@@ -194,15 +213,12 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
     __syncthreads();
     f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < NW; ++w) s4 += red[(w * MT * 16 + m) * PCH + c];
-    if constexpr (NORM) {
-      if (first) {
-        float tot = 0.f;
+    for (int w = 0; w < 8 && w < NW; ++w) s4 += red[(w * MT * 16 + m) * PCH + c];
+    if constexpr (NW > 8) {   // what a second part would hold
+      f32x4 second = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < NW; ++w) tot += squares[w * (MT * 16) + m];
-        scale = 1.0f / sqrtf(tot / (float)a.K + a.ln_eps);
-      }
-      s4 *= scale;
+      for (int w = 8; w < NW; ++w) second += red[(w * MT * 16 + m) * PCH + c];
+      s4 += second;
     }
     const bool on = tid < ITEMS && m < a.M && n < a.N;
     if constexpr (!SPLIT) {
@@ -246,54 +262,53 @@ __global__ void __launch_bounds__(512, SPLIT ? 4 : 2) k_linear_bf16_stream(Linea
   }
 }
 
-template <int MT, int KS, int G, bool FRAG, bool NORM, bool GLU, bool SPLIT, bool F32O>
+template <int MT, int NW, int G, bool FRAG, bool NORM, bool GLU, bool SPLIT, bool F32O>
 static int launch_stream(hipStream_t st, const LinearArgs &a, int parts, int *tickets) {
   const int tiles = (a.N + 15) / 16, groups = (tiles + G - 1) / G;
-  const size_t lds = (size_t)8 * MT * 16 * ((4 * G + 1) * sizeof(f32x4) + sizeof(float));
+  const size_t lds = (size_t)NW * MT * 16 * ((4 * G + 1) * sizeof(f32x4) + sizeof(float));
   static bool attr_set = false;
   if (lds > 64 * 1024 && !attr_set) {
-    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_linear_bf16_stream<MT, KS, G, FRAG, NORM, GLU, SPLIT, F32O>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    RAI_HIP_TRY(hipFuncSetAttribute((const void *)k_linear_bf16_stream<MT, NW, G, FRAG, NORM, GLU, SPLIT, F32O>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     attr_set = true;
   }
-  hipLaunchKernelGGL((k_linear_bf16_stream<MT, KS, G, FRAG, NORM, GLU, SPLIT, F32O>), dim3(SPLIT || groups < kNumCU ? groups : kNumCU, parts), dim3(512), lds, st, a,
+  hipLaunchKernelGGL((k_linear_bf16_stream<MT, NW, G, FRAG, NORM, GLU, SPLIT, F32O>), dim3(SPLIT || groups < kNumCU ? groups : kNumCU, parts), dim3(64 * NW), lds, st, a,
                      tiles, (float *)a.splitk_ws, tickets);
   return launch_check("linear_bf16_stream");
 }
-template <int MT, int KS, bool FRAG, bool F32O> static int launch_stream_form(hipStream_t st, const LinearArgs &a, int parts, int *tickets) {
-  const int tiles = (a.N + 15) / 16;
-  if constexpr (KS >= 6 && KS <= 8) {
-    if (parts > 1) {   // one group to a block: as few tiles as two blocks to a CU allow
-      if (tiles * parts <= kNumCU) return launch_stream<MT, KS, 1, FRAG, false, false, true, F32O>(st, a, parts, tickets);
-      if (tiles * parts <= 2 * kNumCU) return launch_stream<MT, KS, 2, FRAG, false, false, true, F32O>(st, a, parts, tickets);
-      return launch_stream<MT, KS, 4, FRAG, false, false, true, F32O>(st, a, parts, tickets);
-    }
-  }
+template <int MT, bool FRAG, bool F32O> static int launch_stream_parts(hipStream_t st, const LinearArgs &a, int parts, int *tickets) {
+  const int tiles = (a.N + 15) / 16;   // one group to a block: as few tiles as two blocks to a CU allow
+  if (tiles * parts <= kNumCU) return launch_stream<MT, 8, 1, FRAG, false, false, true, F32O>(st, a, parts, tickets);
+  if (tiles * parts <= 2 * kNumCU) return launch_stream<MT, 8, 2, FRAG, false, false, true, F32O>(st, a, parts, tickets);
+  return launch_stream<MT, 8, 4, FRAG, false, false, true, F32O>(st, a, parts, tickets);
+}
+template <int MT, int NW, bool FRAG, bool F32O> static int launch_stream_whole(hipStream_t st, const LinearArgs &a) {
   auto with = [&](auto g) -> int {
     constexpr int G = decltype(g)::value;
     if constexpr (!F32O) {
-      if constexpr (FRAG && KS <= 8) {
-        if (a.ln_kind > 0)
-          return a.glu ? launch_stream<MT, KS, G, FRAG, true, true, false, false>(st, a, 1, nullptr) : launch_stream<MT, KS, G, FRAG, true, false, false, false>(st, a, 1, nullptr);
+      if constexpr (FRAG && NW <= 8) {
+        if (a.ln_kind > 0) return a.glu ? launch_stream<MT, NW, G, true, true, true, false, false>(st, a, 1, nullptr) : launch_stream<MT, NW, G, true, true, false, false, false>(st, a, 1, nullptr);
       }
-      if (a.glu) return launch_stream<MT, KS, G, FRAG, false, true, false, false>(st, a, 1, nullptr);
+      if (a.glu) return launch_stream<MT, NW, G, FRAG, false, true, false, false>(st, a, 1, nullptr);
     }
-    return launch_stream<MT, KS, G, FRAG, false, false, false, F32O>(st, a, 1, nullptr);
+    return launch_stream<MT, NW, G, FRAG, false, false, false, F32O>(st, a, 1, nullptr);
   };
-  return tiles <= kNumCU ? with(std::integral_constant<int, 1>{}) : with(std::integral_constant<int, 2>{});
+  return (a.N + 15) / 16 <= kNumCU ? with(std::integral_constant<int, 1>{}) : with(std::integral_constant<int, 2>{});
 }
 
-// K steps to a wave: ten at most with K whole (eight with a norm, whose weight takes registers too), eight with K in parts, as few parts as that
-// gives and the steps dealt out evenly (K = 1536 in six, 8960 in five parts of seven).
-static int stream_parts(const LinearArgs &a) { return a.K <= (a.ln_kind > 0 ? 2048 : 2560) ? 1 : (a.K / 32 + 63) / 64; }
+// K whole up to ten eights of steps (eight with a norm, whose weight takes registers too), beyond that in parts of eight.
+static int stream_parts(const LinearArgs &a) { return a.K <= 2560 ? 1 : (a.K + 2047) / 2048; }
 static size_t stream_parts_bytes(const LinearArgs &a) { return (size_t)stream_parts(a) * ((a.N + 63) / 64 * 64) * ((a.M + 15) / 16 * 16) * sizeof(float); }
-// What it takes: whole pieces of four columns everywhere, K long enough for four steps a wave and, where K is cut, room for the parts; weights in rows as they lie without
+// What it takes: whole pieces of four columns everywhere, K of four eights of steps and more and, where K is cut, room for the parts; weights in rows as they lie without
 // a norm or an f32 output, and not where the caller keeps to the other kernels' sums.
 bool linear_stream_serves(const LinearArgs &a) {
   const int parts = stream_parts(a), piece = a.f32_out ? 16 : 8;
   auto whole = [](const void *p, int n) { return ((uintptr_t)p & (n - 1)) == 0; };
-  if (a.M < 2 || a.M > 32 || a.K % 32 || a.K <= 24 * 32 || a.N % 4 || a.n_split % 4 || a.ln_kind == 0 || a.K2 || a.force_splits > 0) return false;
+  if (a.M < 2 || a.M > 32 || a.K % 32 || a.K <= 3 * 256 || a.N % 4 || a.n_split % 4 || a.ln_kind == 0 || a.K2 || a.force_splits > 0) return false;
   if (a.Wfrag ? a.M <= 8 : a.fixed_sums || a.ln_kind > 0 || a.f32_out) return false;
-  if ((a.ln_kind > 0 || a.glu) && (parts > 1 || a.f32_out)) return false;
+  if (a.ln_kind > 0 && (a.K > 2048 || a.f32_out)) return false;
+  if (a.glu && (parts > 1 || a.f32_out)) return false;
+  // fragments and a K that k_linear_bf16_mfma_stream cuts: without the scratch that it takes, k_linear_bf16_mfma_skinny has been the one to serve it
+  if (a.Wfrag && a.K > 2048 && (!a.splitk_ws || (size_t)((a.K + 2047) / 2048) * a.M * a.N * sizeof(float) > a.splitk_ws_bytes)) return false;
   if (!a.Wfrag && (a.ldw % 8 || a.ldw >= 1 << 26 || !whole(a.W, 16))) return false;
   if (a.lda % 8 || a.lda >= 1 << 25 || !whole(a.A, 16) || (a.ln_kind > 0 && !whole(a.ln_w, 16))) return false;
   if (a.glu ? a.ld1 % 2 || !whole(a.out1, 4) : a.ld1 % 4 || !whole(a.out1, piece)) return false;
@@ -303,11 +318,11 @@ bool linear_stream_serves(const LinearArgs &a) {
                         (a.N + 15) / 16 <= kSplitTickets);
 }
 // Where it is the fastest form.  On fragments it always is.  On rows as they lie, weights from HBM and, in brackets, from the caches
-// where the two disagree: two to four rows are k_linear_bf16_rows's (4 x 8960 x 1536 8.3, 10.1; 4 x 4096 x 4096 9.5, 9.6), which at five to eight
-// loses but for small matrices (8 x 2560 x 2048 7.9, 5.6; 8 x 16384 x 2048 21.0, 14.7; 8 x 1536 x 8960 12.2, 9.6; 8 x 512 x 1536 4.4, 4.5; 8 x
-// 1024 x 4096 6.4, 6.7); 9 to 32 rows, against tiles and the kernel in gemm_mfma.hip: 16 x 2048 x 2048 7.1, 5.9; 16 x 4096 x 1024 7.0, 4.2; 32 x 8960 x
-// 1536 14.6, 11.6; 24 x 2048 x 16384 22.7, 17.6; 24 x 16384 x 2048 19.0, 15.9 (12.5, 14.1); tiles keep wide matrices of ten steps a wave (24 x 10240 x
-// 2560 19.5, 17.3 (12.9, 15.2)) and, beyond 16 rows, large ones in parts (32 x 8192 x 8192 36.4, 38.0 (25.7, 28.5)).
+// where the two disagree (us): two to four rows are k_linear_bf16_rows's (4 x 8960 x 1536 8.3, 10.1; 4 x 4096 x 4096 9.5, 9.6), which at five to eight
+// loses but for small matrices (8 x 2560 x 2048 8.1, 5.1; 8 x 16384 x 2048 21.1, 14.3; 8 x 1536 x 8960 12.2, 9.5; 8 x 512 x 1536 4.4, 4.5; 8 x
+// 1024 x 4096 6.3, 6.7); 9 to 32 rows, against tiles and the kernel in gemm_mfma.hip: 16 x 2048 x 2048 6.9, 5.5; 16 x 4096 x 1024 7.0, 3.6; 32 x 8960 x
+// 1536 14.2, 11.5; 24 x 2048 x 16384 22.7, 18.9; 24 x 16384 x 2048 18.1, 15.5 (12.4, 13.6); tiles keep wide matrices of more than eight waves (24 x 10240 x
+// 2560 19.5, 17.3 (12.9, 15.2)) and, beyond 16 rows, large ones in parts (32 x 8192 x 8192 36.1, 38.0 (25.4, 28.5)).
 bool linear_stream_pays(const LinearArgs &a) {
   const char *off = getenv("RAI_HIP_NO_MFMA_STREAM"), *off2 = getenv("RAI_HIP_NO_MFMA_SKINNY");   // read per call: tests force the other kernels
   if (off || off2) return false;
@@ -322,31 +337,29 @@ size_t linear_stream_workspace_bytes(const LinearArgs &a) {
   return a.M > 4 && a.M <= 32 && a.K % 32 == 0 && stream_parts(a) > 1 && linear_stream_pays(a) ? stream_parts_bytes(a) : 0;
 }
 int launch_linear_bf16_stream(hipStream_t st, const LinearArgs &a) {
-  const int parts = stream_parts(a), ks = (a.K / 32 + 8 * parts - 1) / (8 * parts);
+  const int parts = stream_parts(a), waves = (a.K + 255) / 256;
   int *tickets = nullptr;
   if (parts > 1) {
     tickets = splitk_tickets(a);
     RAI_REQUIRE(tickets, RAI_ERR_HIP, "linear: the device's split counters were not found");
   }
-  auto steps = [&](auto mt, auto f32o) -> int {
+  auto go = [&](auto mt, auto frag, auto f32o) -> int {
     constexpr int MT = decltype(mt)::value;
-    constexpr bool F = decltype(f32o)::value;
-    if (!a.Wfrag) {   // rows as they lie: pairs of steps
-      if (ks > 8) return launch_stream_form<MT, 10, false, false>(st, a, parts, tickets);
-      if (ks > 6) return launch_stream_form<MT, 8, false, false>(st, a, parts, tickets);
-      return ks > 4 ? launch_stream_form<MT, 6, false, false>(st, a, parts, tickets) : launch_stream_form<MT, 4, false, false>(st, a, parts, tickets);
-    }
-    switch (ks) {
-      case 10: return launch_stream_form<MT, 10, true, F>(st, a, parts, tickets);
-      case 9: return launch_stream_form<MT, 9, true, F>(st, a, parts, tickets);
-      case 8: return launch_stream_form<MT, 8, true, F>(st, a, parts, tickets);
-      case 7: return launch_stream_form<MT, 7, true, F>(st, a, parts, tickets);
-      case 6: return launch_stream_form<MT, 6, true, F>(st, a, parts, tickets);
-      case 5: return launch_stream_form<MT, 5, true, F>(st, a, parts, tickets);
-      default: return launch_stream_form<MT, 4, true, F>(st, a, parts, tickets);
+    constexpr bool FRAG = decltype(frag)::value, F = decltype(f32o)::value;
+    if (parts > 1) return launch_stream_parts<MT, FRAG, F>(st, a, parts, tickets);
+    switch (waves) {
+      case 10: return launch_stream_whole<MT, 10, FRAG, F>(st, a);
+      case 9: return launch_stream_whole<MT, 9, FRAG, F>(st, a);
+      case 8: return launch_stream_whole<MT, 8, FRAG, F>(st, a);
+      case 7: return launch_stream_whole<MT, 7, FRAG, F>(st, a);
+      case 6: return launch_stream_whole<MT, 6, FRAG, F>(st, a);
+      case 5: return launch_stream_whole<MT, 5, FRAG, F>(st, a);
+      default: return launch_stream_whole<MT, 4, FRAG, F>(st, a);
     }
   };
-  auto rows = [&](auto mt) -> int { return a.f32_out ? steps(mt, std::integral_constant<bool, true>{}) : steps(mt, std::integral_constant<bool, false>{}); };
+  const std::integral_constant<bool, true> yes;
+  const std::integral_constant<bool, false> no;
+  auto rows = [&](auto mt) -> int { return !a.Wfrag ? go(mt, no, no) : a.f32_out ? go(mt, yes, yes) : go(mt, yes, no); };
   return a.M <= 16 ? rows(std::integral_constant<int, 1>{}) : rows(std::integral_constant<int, 2>{});
 }
 

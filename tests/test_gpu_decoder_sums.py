@@ -36,7 +36,7 @@ def hybrid(width, ff):
 # K of four to ten runs of eight steps and of two and three parts, whole and with a last run or a last part that is not
 FAMILIES = {"gemma_2048": seq("gemma", 2048, 4096, 4, 1, 256), "qwen2_1536": seq("qwen2", 1536, 4480, 12, 2, 128), "qwen2_1568": seq("qwen2", 1568, 2592, 4, 2, 256),
             "phi2_2560": parallel(32, 2560), "phi2_960": parallel(12, 2176), "bezadra_1024": hybrid(1024, 1888)}
-BATCHES = [2, 5, 8]
+BATCHES = [2, 5, 8, 9, 16, 17, 32]
 
 
 def logits(family, batch):
@@ -55,7 +55,7 @@ def test_bits(hip, family, batch):
     assert got.shape == want.shape and np.array_equal(got, want), f"{(got != want).sum()} of {want.size} logits have other bits"
 
 
-@pytest.mark.parametrize("batch", [2, 8])
+@pytest.mark.parametrize("batch", [2, 8, 9, 16, 17, 32])
 @pytest.mark.parametrize("arch,width", [("qwen2", 1056), ("gemma", 1056), ("qwen2", 2048), ("gemma", 2048)])
 def test_norm_rounds_once(hip, arch, width, batch):
     """No layer adds anything and the head reads single features, so that a logit is a feature of the normed embedding: x * scale * w (Gemma: 1 + w), rounded once
