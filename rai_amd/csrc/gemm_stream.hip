@@ -16,8 +16,7 @@ constexpr int kPastL2 = 17;   // cache policy bits sc0 and sc1: past the (per-XC
 // On rows as they lie the waves take pairs of steps (whole lines) in turn: 8 rows x 16384 x 2048 14.3 us, in pieces 17.6.
 // Bound by the stream of W behind a start (launch, activations, norm) and an end (the sums' way through LDS, with parts through memory) of some
 // 5 us together.  The compiler's wait for a load that may not have been made counts none that follow: a residual asked for under a condition
-// drained the ring at every group's start.  So nothing is loaded under a condition; rows beyond M are the last once more, steps beyond K the first,
-// times zeros.  Measured on fragments from HBM, 24 rows, against the kernel in gemm_mfma.hip, which is also bigger by its outputs of any alignment (us, it, this):
+// drained the ring at every group's start.  So nothing is loaded under a condition; rows beyond M are the last once more, steps beyond K are zeros.  Measured on fragments from HBM, 24 rows, against the kernel in gemm_mfma.hip, which is also bigger by its outputs of any alignment (us, it, this):
 // 32768 x 2048 normed and gated 28.9, 26.1 (134 MB: 5.1 TB/s; a kernel that only reads them takes 21 to 23); 2560 x 2048 normed 9.9, 9.0; 2048 x 2048
 // with residual 6.6, 6.6; 2048 x 16384 in eight parts 19.5, 16.0; 17920 x 1536 normed and gated 21.1, 15.2; 1536 x 8960 in five parts 14.1, 10.4; 2048 x 1536
 // normed 9.1, 7.9; Phi-2's 12800 x 2560 and 2560 x 12800 29.7 in the mean, 20.7 and 21.0.
@@ -26,6 +25,8 @@ constexpr int kPastL2 = 17;   // cache policy bits sc0 and sc1: past the (per-XC
 // Registers: 128 at two blocks to a CU hold the activations, a tile and the sums of four, if nothing else is live then: uniform addresses, a load
 // behind the multiply whose operand it replaces, first sums on a zero that takes none (with spills 2048 x 16384 took 20.2 us).  Beyond eight waves and 16
 // rows one tile is on its way: of two, the second spills.
+static __device__ u32x4 g_stream_zeros[64];   // never written
+
 template <int MT, int NW, int G, bool FRAG, bool NORM, bool GLU, bool SPLIT, bool F32O>
 __global__ void __launch_bounds__(64 * NW, SPLIT ? 4 : (NW + 3) / 4) k_linear_bf16_stream(LinearArgs a, int tiles, float *partial, int *tickets) {
   constexpr int KS = 8, RT = G < 2 || SPLIT || (NW > 8 && MT > 1) ? 1 : 2, PCH = 4 * G + 1, ITEMS = MT * G * 64;
@@ -41,12 +42,18 @@ __global__ void __launch_bounds__(64 * NW, SPLIT ? 4 : (NW + 3) / 4) k_linear_bf
   constexpr int SURE = FRAG ? 0 : SPLIT ? 4 : 6;   // as many are within K wherever it ends
   auto within = [&](int ks) { return ks < SURE || place(ks) < ksteps; };
   auto step_at = [&](int ks) { return within(ks) ? place(ks) : 0; };
+  // Beyond K both operands are zeros, or an infinity in one would make the other's NaN: activations by a mask, fragments from a page of them (for
+  // nothing; a branch around the products cost 0.2 to 0.6 us a launch), rows as they lie, where only the last steps can be beyond, by a mask as well.
   bf16x8 xf[MT][KS], wv[KS], w[RT][KS];
+  uint32_t kept[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) kept[ks] = within(ks) ? ~0u : 0u;
+  auto keep = [&](bf16x8 v, int ks) { return ks < SURE ? v : __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v) & kept[ks]); };
   const uint32_t lane_at = lane * 16;
   auto load = [&](bf16x8 &dst, int tile, int ks) __attribute__((always_inline)) {
     tile = tile < tiles ? tile : tiles - 1;
     if constexpr (FRAG) {   // one instruction reads 1 KB of consecutive memory
-      const char *p = (const char *)a.Wfrag + ((int64_t)tile * ksteps + step_at(ks)) * 1024;
+      const char *p = within(ks) ? (const char *)a.Wfrag + ((int64_t)tile * ksteps + place(ks)) * 1024 : (const char *)g_stream_zeros;
       dst = __builtin_nontemporal_load(reinterpret_cast<const bf16x8 *>(p + lane_at));
     } else {                // 64 bytes of sixteen rows, the second half of their lines with the next step: through the caches
       const char *p = (const char *)a.W + ((int64_t)tile * 16 * a.ldw + step_at(ks) * 32) * 2;
@@ -75,12 +82,10 @@ __global__ void __launch_bounds__(64 * NW, SPLIT ? 4 : (NW + 3) / 4) k_linear_bf
     for (int ks = 0; ks < KS; ++ks) load(w[pos][ks], tile_at(g0, pos), ks);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int ks = SURE; ks < KS; ++ks) {   // (zeros beyond K, of the norm's weight too: an infinite one would make them NaN)
+  for (int ks = SURE; ks < KS; ++ks) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      if (!within(ks)) xf[mt][ks] = bf16x8{};
-    if constexpr (NORM)
-      if (!within(ks)) wv[ks] = bf16x8{};
+    for (int mt = 0; mt < MT; ++mt) xf[mt][ks] = keep(xf[mt][ks], ks);
+    if constexpr (NORM) wv[ks] = keep(wv[ks], ks);
   }
   if constexpr (NORM) {
     // RMSNorm of the rows (ln_kind 1: x * w / rms, 2: x * (1 + w) / rms): the sum of squares of a row is gathered from the waves that hold its pieces,
@@ -192,8 +197,9 @@ __global__ void __launch_bounds__(64 * NW, SPLIT ? 4 : (NW + 3) / 4) k_linear_bf
     for (int j = 0; j < G; ++j)
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8 wk = FRAG ? w[j % RT][ks] : keep(w[j % RT][ks], ks);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j % RT][ks], xf[mt][ks], ks ? acc[j][mt] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        for (int mt = 0; mt < MT; ++mt) acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wk, xf[mt][ks], ks ? acc[j][mt] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         if (!LAST || j + RT < G) load(w[j % RT][ks], tile_at(g0, j + RT), ks);   // (left alone, it would sink to just before its use)
         __builtin_amdgcn_sched_barrier(0);
