@@ -37,7 +37,12 @@ template <> __device__ __forceinline__ mm_f32x16 mm_mfma<f16_raw>(mm_chunk a, mm
 // Memory is read in pieces of 16 bytes whatever their alignment; where K ends inside one (KC), or the outputs do (otherwise), the last 16 bytes of
 // the row are read and moved down when they go to LDS, or a K of less than a piece by pairs (element by element, 16-bit operands with K of 9 to 15 took up to
 // 1.1 us more than multiply-adds on the vector units: 11 x 1 x 11 x 93 in bf16 4.2 us there, 5.3, now 4.5).
-template <typename T, int ROWS, bool KC, int KB>
+// A K of two stages and more, both operands contiguous along it, of 16 bits and off 16-byte boundaries (OFF): the fetch that asks where a tile ends.  A loop that
+// read them without a condition (products formed transposed, 128 x 128 tiles) once gave 130 x 255 x 129 x 241 wrong in one call of three, one piece of one
+// operand in one tile, and no cause was found in its source or its assembly: its loads write over their own addresses, but so do those of
+// forms that have never failed.  Its single stages did not fail, and none of the other layouts.  What it costs (us): 64 x 1000 x 999 x 1001
+// 263, 356; 130 x 255 x 129 x 241 16.4, 18.6; 7 x 481 x 943 x 246 9.1, 9.9.
+template <typename T, int ROWS, bool KC, int KB, bool OFF>
 struct MmOperand {
   static constexpr int V = 16 / sizeof(T), BK = KB / sizeof(T), CPR = KC ? KB / 16 : ROWS / V, P = ROWS * KB / 16 / 256;
   static constexpr int PITCH = (KC ? KB : ROWS * (int)sizeof(T)) + 16;
@@ -55,12 +60,12 @@ struct MmOperand {
   // Every row has a piece, so that one can be read for every place.
   __device__ __forceinline__ bool pieces() const { return KC ? K >= V : before + valid >= V; }
   // How a step is fetched and put into LDS: all of it inside the operand; whole in K, where the outputs may end inside; any.  None of these has a
-  // branch, so that it stays between the products of the step before.  kShort: rows of this operand or the other have no piece.
-  enum { kInside, kOutputsEnd, kEnds, kShort };
+  // branch, so that it stays between the products of the step before.  kGuarded: rows of this operand or the other have no piece, or OFF.
+  enum { kInside, kOutputsEnd, kEnds, kGuarded };
   template <int MODE> __device__ __forceinline__ void fetch(int k0) {
-    if constexpr (MODE == kShort) {
-      if (pieces()) fetch<kEnds>(k0);
-      else fetch_short(k0);
+    if constexpr (MODE == kGuarded) {
+      if (!OFF && pieces()) fetch<kEnds>(k0);
+      else fetch_guarded(k0);
     } else {
 #pragma unroll
       for (int p = 0; p < P; ++p) {   // at an end: the last 16 bytes of the row, or the last row, again
@@ -73,8 +78,8 @@ struct MmOperand {
   }
   // To LDS, what was fetched for k0; a piece that was read ahead of its place goes there now.
   template <int MODE> __device__ __forceinline__ void park(char *st, int k0) const {
-    if constexpr (MODE == kShort) {
-      if (pieces()) return park<kEnds>(st, k0);
+    if constexpr (MODE == kGuarded) {
+      if (!OFF && pieces()) return park<kEnds>(st, k0);
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
@@ -85,12 +90,22 @@ struct MmOperand {
       *reinterpret_cast<mm_chunk *>(st + row(p) * PITCH + col(p) * (int)sizeof(T)) = v;
     }
   }
-  __device__ __forceinline__ void fetch_short(int k0) {
+  __device__ __forceinline__ void fetch_guarded(int k0) {
+    if (KC && OFF && k0 + BK <= K) {
 #pragma unroll
-    for (int p = 0; p < P; ++p) {   // rows of less than a piece: zeros past K, the last output repeated
+      for (int p = 0; p < P; ++p) __builtin_memcpy(&reg[p], base + (int64_t)min(row(p), valid - 1) * stride + k0 + col(p), 16);
+      return;
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {   // at the ends, or rows of less than a piece: zeros past K, the last output repeated
       const int k = KC ? k0 + col(p) : k0 + row(p), o = KC ? min(row(p), valid - 1) : col(p);
       if (k >= K) {
         reg[p] = mm_chunk{0u, 0u, 0u, 0u};
+      } else if (KC && OFF && k + V <= K) {
+        __builtin_memcpy(&reg[p], base + (int64_t)o * stride + k, 16);
+      } else if (KC && OFF && K >= V) {   // the piece that ends with K, moved down
+        __builtin_memcpy(&reg[p], base + (int64_t)o * stride + (K - V), 16);
+        reg[p] = end_of_row(reg[p], k + V - K);
       } else if (KC && sizeof(T) == 2 && K > 1) {   // a shorter K, by pairs
         const T *at_o = base + (int64_t)o * stride;
 #pragma unroll
@@ -167,15 +182,15 @@ template <typename T> __device__ __forceinline__ void mm_store(T *dst, const flo
 // 32 x 512 x 512 x 80 (values, [K, N]) 13.4 (94.8), 64 x 1024 x 1024 x 1024 200 to 316 (2900 to 3035), one row against 32 x
 // 777 x 128 10.4 (77.5), odd 18 x 410 x 141 x 349 10.8 (31.8); f32 32 x 512 x 80 x 512 24.4 (47.9).
 //   A step has no branch: the ends of rows are put right by moving what was read, not by asking where it lies (us, with branches, and now): bf16 64 x
-// 1024 x 1024 x 1024, [K, N] 300, 207 to 212, K-contiguous 305, 202, 64 x 1000 x 999 x 1001 454, 266 and 367, 263, 7 x 481 x 944 x 246 27.9, 11.2,
+// 1024 x 1024 x 1024, [K, N] 300, 207 to 212, K-contiguous 305, 202, 64 x 1000 x 999 x 1001, [K, N] 454, 266, 7 x 481 x 944 x 246 27.9, 11.2,
 // 18 x 169 x 639 x 234 19.3, 9.1, 19 x 30 x 192 x 34 6.3, 4.8, f16 5 x 9 x 723 x 56 14.6, 8.0; f32 3 x 15 x 737 x 625 24.1, 21.1, 64 x 128 x 512 x 128
 // 16.6, 15.8.  f32, whose products take longer, loads a step ahead from its first products on (from the third: 17.1).  Stages of
 // 256 bytes: 0.95 to 1.33 of the time.
-template <typename T, bool AKC, bool BKC, int F, int KB, bool ONE>
+template <typename T, bool AKC, bool BKC, int F, int KB, bool ONE, bool OFF = false>
 __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T *B, MatmulArgs g, int tiles_m, int tiles_n) {
   constexpr int BT = 64 * F;
-  typedef MmOperand<T, BT, AKC, KB> OpA;
-  typedef MmOperand<T, BT, BKC, KB> OpB;
+  typedef MmOperand<T, BT, AKC, KB, OFF> OpA;
+  typedef MmOperand<T, BT, BKC, KB, OFF> OpB;
   constexpr int STAGE = OpA::BYTES + OpB::BYTES, OP = BT + 4, PAIRS = KB / 32;
   constexpr int LDS = (ONE ? 1 : 2) * STAGE > BT * OP * 4 ? (ONE ? 1 : 2) * STAGE : BT * OP * 4;
   __shared__ __attribute__((aligned(16))) char lds[LDS];
@@ -214,8 +229,8 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   const int steps = ONE ? 1 : ((int)g.K + OpA::BK - 1) / OpA::BK;
-  constexpr int kInside = OpA::kInside, kOutputsEnd = OpA::kOutputsEnd, kEnds = OpA::kEnds, kShort = OpA::kShort;
-  const bool pieces = a.pieces() && b.pieces();
+  constexpr int kInside = OpA::kInside, kOutputsEnd = OpA::kOutputsEnd, kEnds = OpA::kEnds, kGuarded = OpA::kGuarded;
+  const bool pieces = !OFF && a.pieces() && b.pieces();
   auto begin = [&](auto how) __attribute__((always_inline)) {
     constexpr int MODE = decltype(how)::value;
     a.template fetch<MODE>(0);
@@ -257,8 +272,8 @@ __global__ void __launch_bounds__(256) k_matmul_mfma(T *out, const T *A, const T
     __syncthreads();
   };
   if (!pieces) {
-    begin(std::integral_constant<int, kShort>{});
-    for (; s < steps; ++s) step(std::integral_constant<int, kShort>{});
+    begin(std::integral_constant<int, kGuarded>{});
+    for (; s < steps; ++s) step(std::integral_constant<int, kGuarded>{});
   } else {
     begin(std::integral_constant<int, kEnds>{});
     if constexpr (!ONE) {   // the steps that fetch one before the last, whole in K
@@ -404,17 +419,18 @@ static int launch_mm(hipStream_t st, void *out, const void *A, const void *B, co
   const int64_t t64 = batch * ((g.M + 63) / 64) * ((g.N + 63) / 64), tm128 = (g.M + 127) / 128, tn128 = (g.N + 127) / 128;
   const int kb = (int)(g.K * (int64_t)sizeof(T) < 512 ? g.K * sizeof(T) : 512);
   const int tm = (int)((g.M + 63) / 64), tn = (int)((g.N + 63) / 64);
+  auto wide = [&](const void *p, int64_t stride, const int64_t *bs) {
+    bool ok = (uintptr_t)p % 16 == 0 && stride % 8 == 0;
+    for (int d = 0; d < g.batch_rank; ++d) ok = ok && (bs[d] % 8 == 0 || g.batch_shape[d] == 1);
+    return ok;
+  };
+  const bool aligned = wide(A, g.a_rs, g.a_bs) && wide(B, g.b_cs, g.b_bs);
   auto go = [&](auto kernel, int64_t blocks, int tiles_m, int tiles_n) -> int {
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, (T *)out, (const T *)A, (const T *)B, g, tiles_m, tiles_n);
     return launch_check("matmul_mfma");
   };
   if constexpr (sizeof(T) == 2 && AKC && BKC) {
-    auto wide = [&](const void *p, int64_t stride, const int64_t *bs) {
-      bool ok = (uintptr_t)p % 16 == 0 && stride % 8 == 0;
-      for (int d = 0; d < g.batch_rank; ++d) ok = ok && (bs[d] % 8 == 0 || g.batch_shape[d] == 1);
-      return ok;
-    };
-    if (g.K <= 128 && g.K % 8 == 0 && wide(A, g.a_rs, g.a_bs) && wide(B, g.b_cs, g.b_bs)) {
+    if (g.K <= 128 && g.K % 8 == 0 && aligned) {
       // (tiles half of which lie past an end: 50 x 874 x 40 x 41 5.4 us in the form above, 6.3 by large ones)
       const int64_t t128 = batch * tm128 * tn128;
       const bool large = t128 >= kNumCU && 8 * t128 <= 3 * t64;
@@ -434,13 +450,20 @@ static int launch_mm(hipStream_t st, void *out, const void *A, const void *B, co
       }
     }
   }
-  if constexpr (sizeof(T) == 2) {
-    if (batch * tm128 * tn128 >= 2 * kNumCU && g.K >= 256) return go(k_matmul_mfma<T, AKC, BKC, 2, 128, false>, batch * tm128 * tn128, (int)tm128, (int)tn128);
-  }
   if (kb <= 128) return go(k_matmul_mfma<T, AKC, BKC, 1, 128, true>, t64, tm, tn);
   if (kb <= 192) return go(k_matmul_mfma<T, AKC, BKC, 1, 192, true>, t64, tm, tn);
   if (kb <= 256) return go(k_matmul_mfma<T, AKC, BKC, 1, 256, true>, t64, tm, tn);
-  return go(k_matmul_mfma<T, AKC, BKC, 1, 128, false>, t64, tm, tn);
+  auto stages = [&](auto off) -> int {   // two and more
+    constexpr bool OFF = decltype(off)::value;
+    if constexpr (sizeof(T) == 2) {
+      if (batch * tm128 * tn128 >= 2 * kNumCU && g.K >= 256) return go(k_matmul_mfma<T, AKC, BKC, 2, 128, false, OFF>, batch * tm128 * tn128, (int)tm128, (int)tn128);
+    }
+    return go(k_matmul_mfma<T, AKC, BKC, 1, 128, false, OFF>, t64, tm, tn);
+  };
+  if constexpr (sizeof(T) == 2 && AKC && BKC) {
+    if (!aligned) return stages(std::integral_constant<bool, true>{});
+  }
+  return stages(std::integral_constant<bool, false>{});
 }
 
 bool matmul_mfma_serves(int dtype, const MatmulArgs &g, int64_t batch) {

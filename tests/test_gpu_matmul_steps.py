@@ -48,3 +48,23 @@ def test_large_tiles(hip, dt, b_t):
     a, b = a.astype(np.float64), b.astype(np.float64)
     want = a @ b
     assert np.all(np.abs(got - want) <= 2 * (325 + 8) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + U[dt] * np.abs(want))
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("k,lie", [(257, 257), (264, 267), (129, 129), (104, 107)])
+def test_contiguous_along_k_off_boundaries(hip, dt, k, lie):
+    """Both operands contiguous along K in rows off 16-byte boundaries: 128 x 128 tiles from K = 256 on, 64 x 64 below; every call the same bits."""
+    from rai_amd import ops as R
+
+    g = np.random.Generator(np.random.PCG64(k))
+    some = np.arange(130) % 3
+    a, b = rand(g, (3, 255, lie), dt), rand(g, (3, 241, lie), dt)
+    a[..., k:], b[..., k:] = np.nan, np.nan
+    ad, bd = up(a[some], dt).narrow(2, 0, k), up(b[some], dt).narrow(2, 0, k).transpose(1, 2)
+    first = down(R.matmul(ad, bd))
+    a, b = a[..., :k].astype(np.float64), b[..., :k].astype(np.float64).swapaxes(1, 2)
+    want = a @ b
+    assert np.all(np.abs(first[:3] - want) <= 2 * (k + 8) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + U[dt] * np.abs(want))
+    assert np.array_equal(first, first[:3][some])
+    for _ in range(4):
+        assert np.array_equal(down(R.matmul(ad, bd)), first)
