@@ -310,6 +310,9 @@ bool linear_stream_serves(const LinearArgs &a) {
   const int parts = stream_parts(a), piece = a.f32_out ? 16 : 8;
   auto whole = [](const void *p, int n) { return ((uintptr_t)p & (n - 1)) == 0; };
   if (a.M < 2 || a.M > 32 || a.K % 32 || a.K <= 3 * 256 || a.N % 4 || a.n_split % 4 || a.ln_kind == 0 || a.K2 || a.force_splits > 0) return false;
+  // what the other kernels refuse is theirs to refuse
+  if (a.N <= 0 || !a.A || !a.W || !a.out1 || a.n_split < 0 || a.n_split > a.N || (a.n_split != a.N && (!a.out2 || a.f32_out))) return false;
+  if (a.glu && (a.act < 0 || a.residual || a.n_split != a.N || (a.M > 8 && a.N % 8))) return false;
   if (a.Wfrag ? a.M <= 8 : a.fixed_sums || a.ln_kind > 0 || a.f32_out) return false;
   if (a.ln_kind > 0 && (a.K > 2048 || a.f32_out)) return false;
   if (a.glu && (parts > 1 || a.f32_out)) return false;

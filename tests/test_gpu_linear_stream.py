@@ -100,3 +100,17 @@ def test_gated(R, m, k, n):
     want = gate / (1 + np.exp(-gate)) * upv
     got = down(R.linear_packed(up(x, "bf16"), up(w, "bf16"), act="silu", glu=True)).astype(np.float64)
     assert np.all(np.abs(got - want) <= 4 * 2.0 ** -8 * (np.abs(gate) + 1) * (np.abs(upv) + 1))
+
+
+@pytest.mark.parametrize("m,k,n,taken", [(8, 1024, 1028, True), (9, 1024, 1028, False), (32, 2048, 2052, False), (16, 1024, 1032, True), (16, 736, 1028, False)])
+def test_gated_columns_that_are_refused(R, m, k, n, taken):
+    """Beyond eight rows gated products come in whole eights of columns, whichever kernel would serve them."""
+    from rai_amd._lib import RaiHipError
+
+    g = np.random.Generator(np.random.PCG64(m))
+    x, w = up(rand(g, (m, k), "bf16"), "bf16"), up(rand(g, (n, k), "bf16"), "bf16")
+    if taken:
+        assert R.linear_packed(x, w, act="silu", glu=True).shape == (m, n // 2)
+    else:
+        with pytest.raises(RaiHipError, match="gated"):
+            R.linear_packed(x, w, act="silu", glu=True)
