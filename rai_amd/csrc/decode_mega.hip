@@ -994,7 +994,7 @@ __global__ void __launch_bounds__(kMegaThreads) k_phi2_decode_step(MegaArgs a) {
 // blocks' bests travel as 8-byte (value, row) words written past the L2; a block counts itself in when its word has
 // reached memory, and the block that counts last, whichever it is, picks among the words, writes the token, copies
 // its embedding row to the next step's input and advances the device-side counters.  Nobody waits for anybody.
-constexpr int kHeadRowsMax = 256;
+constexpr int kHeadRowsMax = 256;   // rows to a block: the vocabularies of more keep the Linear, the choice and their sums
 
 // whether candidate (v, i) replaces (bv, bi): a NaN value only ever comes with row 0 and is final; row 0xffffffff
 // means nothing seen yet
@@ -1167,13 +1167,13 @@ __global__ void __launch_bounds__(kMegaThreads) k_phi2_head_choice(HeadArgs a) {
   }
 }
 
-static size_t head_lds_bytes(const HeadArgs &a, int num_cu) {
+static size_t head_lds_bytes(const HeadArgs &a) {   // x as it is and normed
   return (size_t)a.H * 4;
 }
 
 bool head_choice_eligible(const HeadArgs &a, int num_cu) {
   if (!(a.H == 2560 || a.H == 2048) || num_cu < 1 || num_cu > 256) return false;
-  if (a.V < num_cu * 16 || (a.V + num_cu - 1) / num_cu + 1 > kHeadRowsMax) return false;   // at least a pass over the ring per wave
+  if (a.V < num_cu * 16 || (a.V + num_cu - 1) / num_cu + 1 > kHeadRowsMax) return false;   // at least a pair of rows to each of a block's eight waves
   auto al16 = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
   return a.W && a.x && a.ln_w && a.ln_b && a.logits && a.best && a.token && a.state && al16(a.W) && al16(a.x) && al16(a.ln_w) &&
          al16(a.ln_b) && (!a.x_next || a.embed);
@@ -1181,7 +1181,7 @@ bool head_choice_eligible(const HeadArgs &a, int num_cu) {
 
 int launch_phi2_head_choice(hipStream_t st, const HeadArgs &a, int num_cu) {
   RAI_REQUIRE(head_choice_eligible(a, num_cu), RAI_ERR_UNSUPPORTED, "head with choice: H=%d V=%d on %d CUs not served", a.H, a.V, num_cu);
-  const size_t lds = head_lds_bytes(a, num_cu);
+  const size_t lds = head_lds_bytes(a);
   if (a.H == 2560) hipLaunchKernelGGL((k_phi2_head_choice<5>), dim3(num_cu), dim3(kMegaThreads), lds, st, a);
   else hipLaunchKernelGGL((k_phi2_head_choice<4>), dim3(num_cu), dim3(kMegaThreads), lds, st, a);
   return launch_check("phi2_head_choice");

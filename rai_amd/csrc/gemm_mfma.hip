@@ -1878,7 +1878,8 @@ int launch_linear_bf16_mfma(hipStream_t st, const LinearArgs &a) {
               RAI_ERR_BAD_STRIDE, "linear mfma: operands must be 16-byte aligned with row strides multiple of 8");
   const bool no_skinny = getenv("RAI_HIP_NO_MFMA_SKINNY") != nullptr;
   const bool no_stream = getenv("RAI_HIP_NO_MFMA_STREAM") != nullptr;
-  // A row-major W and 9 to 64 rows: the streaming kernel reads 512-byte pieces of W's rows, at 2 to 3 TB/s; tiles with all of
+  // A row-major W and 9 to 64 rows (up to 32 those that the streaming form of gemm_stream.hip leaves: a decoder's head on chosen rows, short K,
+  // columns in no whole fours, and where it does not pay): the streaming kernel here reads 512-byte pieces of W's rows, at 2 to 3 TB/s; tiles with all of
   // their loads in flight do better once there are enough of them, and split K by themselves (us, stream, tiles, weights from
   // HBM: 16 x 512 x 8960 11.2, 6.2; 16 x 8192 x 8960 45, 35; 64 x 8192 x 8960 77, 40; 64 x 2048 x 2048 9.8, 9.2; 16 x 8192 x 2048 15.2,
   // 14.4; but 16 x 2048 x 2048 7.1, 8.0; 48 x 512 x 2048 4.8, 5.8; 16 x 8192 x 512 9.7, 13.4).  Where K needs no cut in the streaming
