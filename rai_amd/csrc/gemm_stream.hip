@@ -16,7 +16,8 @@ constexpr int kPastL2 = 17;   // cache policy bits sc0 and sc1: past the (per-XC
 // On rows as they lie the waves take pairs of steps (whole lines) in turn: 8 rows x 16384 x 2048 14.3 us, in pieces 17.6.
 // Bound by the stream of W behind a start (launch, activations, norm) and an end (the sums' way through LDS, with parts through memory) of some
 // 5 us together.  The compiler's wait for a load that may not have been made counts none that follow: a residual asked for under a condition
-// drained the ring at every group's start.  So nothing is loaded under a condition; rows beyond M are the last once more, steps beyond K are zeros.  Measured on fragments from HBM, 24 rows, against the kernel in gemm_mfma.hip, which is also bigger by its outputs of any alignment (us, it, this):
+// drained the ring at every group's start.  So nothing is loaded under a condition; rows beyond M are the last once more, steps beyond K are zeros.
+// Measured on fragments from HBM, 24 rows, against the kernel in gemm_mfma.hip, which is also bigger by its outputs of any alignment (us, it, this):
 // 32768 x 2048 normed and gated 28.9, 26.1 (134 MB: 5.1 TB/s; a kernel that only reads them takes 21 to 23); 2560 x 2048 normed 9.9, 9.0; 2048 x 2048
 // with residual 6.6, 6.6; 2048 x 16384 in eight parts 19.5, 16.0; 17920 x 1536 normed and gated 21.1, 15.2; 1536 x 8960 in five parts 14.1, 10.4; 2048 x 1536
 // normed 9.1, 7.9; Phi-2's 12800 x 2560 and 2560 x 12800 29.7 in the mean, 20.7 and 21.0.
@@ -329,8 +330,8 @@ bool linear_stream_serves(const LinearArgs &a) {
 // Where it is the fastest form.  On fragments it always is.  On rows as they lie, weights from HBM and, in brackets, from the caches
 // where the two disagree (us): two to four rows are k_linear_bf16_rows's (4 x 8960 x 1536 8.3, 10.1; 4 x 4096 x 4096 9.5, 9.6), which at five to eight
 // loses but for small matrices (8 x 2560 x 2048 8.1, 5.1; 8 x 16384 x 2048 21.1, 14.3; 8 x 1536 x 8960 12.2, 9.5; 8 x 512 x 1536 4.4, 4.5; 8 x
-// 1024 x 4096 6.3, 6.7); 9 to 32 rows, against tiles and the kernel in gemm_mfma.hip: 16 x 2048 x 2048 6.9, 5.5; 16 x 4096 x 1024 7.0, 3.6; 32 x 8960 x
-// 1536 14.2, 11.5; 24 x 2048 x 16384 22.7, 18.9; 24 x 16384 x 2048 18.1, 15.5 (12.4, 13.6); tiles keep wide matrices of more than eight waves (24 x 10240 x
+// 1024 x 4096 6.3, 6.7); 9 to 32 rows, against tiles and the kernel in gemm_mfma.hip: 16 x 2048 x 2048 6.9, 5.5; 16 x 4096 x 1024 7.0, 3.7; 32 x 8960 x
+// 1536 14.2, 11.5; 24 x 2048 x 16384 22.7, 16.7; 24 x 16384 x 2048 18.1, 15.5 (12.4, 13.4); tiles keep wide matrices of more than eight waves (24 x 10240 x
 // 2560 19.5, 17.3 (12.9, 15.2)) and, beyond 16 rows, large ones in parts (32 x 8192 x 8192 36.1, 38.0 (25.4, 28.5)).
 bool linear_stream_pays(const LinearArgs &a) {
   const char *off = getenv("RAI_HIP_NO_MFMA_STREAM"), *off2 = getenv("RAI_HIP_NO_MFMA_SKINNY");   // read per call: tests force the other kernels
